@@ -28,6 +28,8 @@ SIGNATURES = {
     "dpep_layout": (_I, (_P, _P, _I, _I, _I, _I, _I, _P, _P, _P, _P, _P, _P, _P)),
     "dpep_layout_static": (_I, (_P, _I, _I, _I, _I, _I, _P, _P, _P, _P, _P, _P, _P)),
     "dpep_layout_wait": (_I, (_P, _P, _I, ctypes.POINTER(ctypes.c_int32), ctypes.c_longlong)),
+    "dpep_layout_ready": (_I, (_P,)),
+    "dpep_dispatch_fresh": (_I, (_P, _P, _P)),
     "dpep_dispatch_store_policy": (_I, (_I,)),
     "dpep_dispatch_copy": (_I, (_P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P, _P, _P, _P)),
     "dpep_dispatch_quant_fp8": (_I, (_P, _P, _P, _P, _I, _I, _I, _I, _P, _P, _P, _P)),
@@ -71,6 +73,16 @@ def load():
                 fn.argtypes = list(argtypes)
             _lib = lib
     return _lib
+
+
+def host():
+    """The native host path (csrc/host.cpp), a CPython extension over this library.  Raises if it is not built."""
+    load()
+    try:
+        from . import _host
+    except ImportError as error:
+        raise ImportError(f"deepep_amd/_host.so cannot be loaded ({error}): build it with `python -m deepep_amd.build`") from error
+    return _host
 
 
 class NativeError(RuntimeError):

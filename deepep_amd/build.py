@@ -1,4 +1,5 @@
-"""Compile the HIP sources for gfx950 into deepep_amd/libdeepep_amd.so (in-tree).
+"""Compile the HIP sources for gfx950 into deepep_amd/libdeepep_amd.so, and the native host path over it into
+deepep_amd/_host.so (both in-tree).
 
 Usage: ``python -m deepep_amd.build``.  hipcc cross-compiles without a GPU.
 """
@@ -36,6 +37,27 @@ FLAGS = (
 FILE_FLAGS = {"megamoe.hip": ("-mllvm", "-greedy-reverse-local-assignment=1")}
 
 
+HOST_SOURCE = "host.cpp"
+HOST_OUT = os.path.join(HERE, "_host.so")
+
+
+def _build_host() -> None:
+    """The CPython extension: plain C++ against torch's headers; finds libdeepep_amd.so beside itself."""
+    import sysconfig
+
+    from torch.utils import cpp_extension
+
+    includes = [*cpp_extension.include_paths("cuda"), sysconfig.get_paths()["include"]]
+    libraries = cpp_extension.library_paths("cuda")
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM",
+           *(flag for path in includes for flag in ("-isystem", path)), os.path.join(CSRC, HOST_SOURCE), "-o", HOST_OUT,
+           "-L" + HERE, "-ldeepep_amd", *("-L" + path for path in libraries), "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_hip",
+           "-ltorch_python", "-lamdhip64", "-Wl,-rpath,$ORIGIN"]
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError(f"g++ failed for {HOST_SOURCE}:\n{proc.stdout}\n{proc.stderr}")
+
+
 def _hipcc():
     for candidate in (os.environ.get("HIPCC"), "/opt/rocm/bin/hipcc", "hipcc"):
         if candidate and (os.path.isabs(candidate) and os.path.exists(candidate) or not os.path.isabs(candidate)):
@@ -67,6 +89,7 @@ def build(verbose: bool = False) -> str:
     proc = subprocess.run(link, capture_output=True, text=True)
     if proc.returncode != 0:
         raise RuntimeError(f"link failed:\n{proc.stdout}\n{proc.stderr}")
+    _build_host()
     return OUT
 
 

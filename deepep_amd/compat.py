@@ -15,10 +15,12 @@ import functools
 def accept_aliases(**alias_to_public):
     """Decorator: ``alias=value`` is forwarded as ``public=value``; the signature is unchanged."""
 
+    pairs = tuple(alias_to_public.items())
+
     def wrap(function):
         @functools.wraps(function)
         def call(*args, **kwargs):
-            for alias, public in alias_to_public.items():
+            for alias, public in pairs:
                 if alias in kwargs:
                     value = kwargs.pop(alias)
                     if public in kwargs and kwargs[public] != value:

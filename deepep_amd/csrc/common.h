@@ -115,6 +115,20 @@ __device__ __forceinline__ int local_expert(long long e, int route, int end, int
     return valid ? static_cast<int>(local) : -1;
 }
 
+// Rows of experts 0..e on this rank for EVERY expert e of the job (a low-latency handle's send_counts): zero in front of the
+// local experts, their inclusive prefix, the total behind them.  counts == nullptr: not wanted.
+struct SendCounts {
+    int* counts;
+    int expert_begin, num_experts;
+};
+// The entries of experts that are not local, by `threads` threads that know the total.
+__device__ __forceinline__ void send_counts_of_others(const SendCounts& send, int num_local, int total, int tid, int threads)
+{
+    if (send.counts == nullptr) return;
+    for (int e = tid; e < send.num_experts; e += threads)
+        if (e < send.expert_begin || e >= send.expert_begin + num_local) send.counts[e] = e < send.expert_begin ? 0 : total;
+}
+
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 

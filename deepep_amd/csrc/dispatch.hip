@@ -53,7 +53,7 @@ template <int kPolicy>
 __global__ __launch_bounds__(kMaxThreads) void dispatch_copy_token_kernel(
     const u32x4* __restrict__ x, const float* __restrict__ scales, const float* __restrict__ weights,
     const int* __restrict__ route_to_row, int num_topk, int vec_per_row, int vec_per_part, int parts, int scale_cols,
-    u32x4* __restrict__ out, float* __restrict__ out_scales, float* __restrict__ out_weights)
+    int capacity, u32x4* __restrict__ out, float* __restrict__ out_scales, float* __restrict__ out_weights)
 {
     __shared__ int rows[DPEP_MAX_TOPK];
     __shared__ int any_valid;
@@ -68,7 +68,8 @@ __global__ __launch_bounds__(kMaxThreads) void dispatch_copy_token_kernel(
     if (threadIdx.x == 0) any_valid = 0;
     __syncthreads();
     if (threadIdx.x < num_topk) {
-        const int row = route_to_row[static_cast<size_t>(token) * num_topk + threadIdx.x];
+        int row = route_to_row[static_cast<size_t>(token) * num_topk + threadIdx.x];
+        if (row >= capacity) row = -1;  // outputs allocated before R was known: rows beyond them are dropped
         rows[threadIdx.x] = row;
         if (row >= 0) any_valid = 1;
     }
@@ -96,27 +97,43 @@ __global__ __launch_bounds__(kMaxThreads) void dispatch_copy_token_kernel(
     }
 }
 
-// ---- row-major copy: one workgroup per (output row, column part); for sparse receive shares -------
+// ---- row-major: one workgroup per (output row, column part); for sparse receive shares -------------
+// Rows [0, rows): `rows` from the host, or, rows_on_device, the smaller of that bound and the count the layout left on the
+// device (a payload queued before the host knows R).  Such a launch has workgroups for about the expected number of rows;
+// they walk on by the grid's rows until the real count is reached, and the first row's route is asked for together with
+// the count (row_to_route has an entry for every row of the grid, so the load is in bounds whatever the count says).
+struct RowRange {
+    int rows;
+    const int* rows_on_device;
+    __device__ __forceinline__ int count() const { return rows_on_device != nullptr ? min(*rows_on_device, rows) : rows; }
+};
+
 template <int kPolicy>
 __global__ __launch_bounds__(kMaxThreads) void dispatch_copy_row_kernel(
     const u32x4* __restrict__ x, const float* __restrict__ scales, const float* __restrict__ weights,
-    const int* __restrict__ row_to_route, int num_tokens, int num_topk, int vec_per_row, int vec_per_part, int parts,
-    int scale_cols, u32x4* __restrict__ out, float* __restrict__ out_scales, float* __restrict__ out_weights)
+    const int* __restrict__ row_to_route, RowRange range, int num_tokens, int num_topk, int vec_per_row, int vec_per_part,
+    int parts, int scale_cols, u32x4* __restrict__ out, float* __restrict__ out_scales, float* __restrict__ out_weights)
 {
-    const int row = blockIdx.x / parts, part = blockIdx.x % parts;
-    // (clamped: a map left incomplete by a layout launch that reported a time-out must not become a wild address)
-    const int route = min(max(row_to_route[row], 0), num_tokens * num_topk - 1);
-    const int token = route / num_topk;
+    const int part = blockIdx.x % parts, stride = gridDim.x / parts;
     const int v_begin = part * vec_per_part;
     const int v_end = min(v_begin + vec_per_part, vec_per_row);
-    const u32x4* src = x + static_cast<size_t>(token) * vec_per_row;
-    u32x4* dst = out + static_cast<size_t>(row) * vec_per_row;
-    for (int v = v_begin + threadIdx.x; v < v_end; v += blockDim.x) store16_as<kPolicy>(dst + v, load16(src + v));
-    if (part == 0) {
-        if (scales != nullptr)
-            for (int c = threadIdx.x; c < scale_cols; c += blockDim.x)
-                out_scales[static_cast<size_t>(row) * scale_cols + c] = scales[static_cast<size_t>(token) * scale_cols + c];
-        if (weights != nullptr && threadIdx.x == 0) out_weights[row] = weights[route];
+    int row = blockIdx.x / parts;
+    int next_route = row_to_route[row];
+    const int rows = range.count();
+    for (; row < rows; row += stride) {
+        // (clamped: a map left incomplete by a layout launch that reported a time-out must not become a wild address)
+        const int route = min(max(next_route, 0), num_tokens * num_topk - 1);
+        if (row + stride < rows) next_route = row_to_route[row + stride];
+        const int token = route / num_topk;
+        const u32x4* src = x + static_cast<size_t>(token) * vec_per_row;
+        u32x4* dst = out + static_cast<size_t>(row) * vec_per_row;
+        for (int v = v_begin + threadIdx.x; v < v_end; v += blockDim.x) store16_as<kPolicy>(dst + v, load16(src + v));
+        if (part == 0) {
+            if (scales != nullptr)
+                for (int c = threadIdx.x; c < scale_cols; c += blockDim.x)
+                    out_scales[static_cast<size_t>(row) * scale_cols + c] = scales[static_cast<size_t>(token) * scale_cols + c];
+            if (weights != nullptr && threadIdx.x == 0) out_weights[row] = weights[route];
+        }
     }
 }
 
@@ -188,7 +205,7 @@ __device__ __forceinline__ Quant16 quantize16(u32x4 lo, u32x4 hi)
 template <int kPolicy>
 __global__ __launch_bounds__(kMaxThreads) void dispatch_quant_token_kernel(
     const u32x4* __restrict__ x, const float* __restrict__ weights, const int* __restrict__ route_to_row, int num_topk,
-    int units_per_row, int units_per_part, int parts, u32x4* __restrict__ out, float* __restrict__ out_scales,
+    int units_per_row, int units_per_part, int parts, int capacity, u32x4* __restrict__ out, float* __restrict__ out_scales,
     float* __restrict__ out_weights)
 {
     __shared__ int rows[DPEP_MAX_TOPK];
@@ -214,7 +231,8 @@ __global__ __launch_bounds__(kMaxThreads) void dispatch_quant_token_kernel(
     if (threadIdx.x == 0) any_valid = 0;
     __syncthreads();
     if (threadIdx.x < num_topk) {
-        const int row = route_to_row[static_cast<size_t>(token) * num_topk + threadIdx.x];
+        int row = route_to_row[static_cast<size_t>(token) * num_topk + threadIdx.x];
+        if (row >= capacity) row = -1;  // outputs allocated before R was known: rows beyond them are dropped
         rows[threadIdx.x] = row;
         if (row >= 0) any_valid = 1;
     }
@@ -263,27 +281,33 @@ __global__ __launch_bounds__(kMaxThreads) void dispatch_quant_token_kernel(
         out_weights[rows[threadIdx.x]] = weights[static_cast<size_t>(token) * num_topk + threadIdx.x];
 }
 
-// row-major: one workgroup per (output row, column part); row_to_route == nullptr means identity
+// row-major: one workgroup per (output row, column part), rows as above; row_to_route == nullptr means identity
 // (row == token), which is the stand-alone quantiser.
 template <int kPolicy>
 __global__ __launch_bounds__(kMaxThreads) void dispatch_quant_row_kernel(
-    const u32x4* __restrict__ x, const float* __restrict__ weights, const int* __restrict__ row_to_route, int num_tokens,
-    int num_topk, int units_per_row, int units_per_part, int parts, u32x4* __restrict__ out, float* __restrict__ out_scales,
-    float* __restrict__ out_weights)
+    const u32x4* __restrict__ x, const float* __restrict__ weights, const int* __restrict__ row_to_route, RowRange range,
+    int num_tokens, int num_topk, int units_per_row, int units_per_part, int parts, u32x4* __restrict__ out,
+    float* __restrict__ out_scales, float* __restrict__ out_weights)
 {
-    const int row = blockIdx.x / parts, part = blockIdx.x % parts;
-    const int route = row_to_route != nullptr ? min(max(row_to_route[row], 0), num_tokens * num_topk - 1) : row;
-    const int token = row_to_route != nullptr ? route / num_topk : row;
+    const int part = blockIdx.x % parts, stride = gridDim.x / parts;
     const int u_begin = part * units_per_part;
     const int u_end = min(u_begin + units_per_part, units_per_row);
     const int scale_cols = units_per_row / 8;
-    const u32x4* src = x + static_cast<size_t>(token) * units_per_row * 2;
-    for (int u = u_begin + threadIdx.x; u < u_end; u += blockDim.x) {
-        const Quant16 q = quantize16(load16(src + 2 * u), load16(src + 2 * u + 1));
-        store16_as<kPolicy>(out + static_cast<size_t>(row) * units_per_row + u, q.codes);
-        if ((u & 7) == 0) out_scales[static_cast<size_t>(row) * scale_cols + (u >> 3)] = q.scale;
+    int row = blockIdx.x / parts;
+    int next_route = row_to_route != nullptr ? row_to_route[row] : row;
+    const int rows = range.count();
+    for (; row < rows; row += stride) {
+        const int route = row_to_route != nullptr ? min(max(next_route, 0), num_tokens * num_topk - 1) : row;
+        if (row_to_route != nullptr && row + stride < rows) next_route = row_to_route[row + stride];
+        const int token = row_to_route != nullptr ? route / num_topk : row;
+        const u32x4* src = x + static_cast<size_t>(token) * units_per_row * 2;
+        for (int u = u_begin + threadIdx.x; u < u_end; u += blockDim.x) {
+            const Quant16 q = quantize16(load16(src + 2 * u), load16(src + 2 * u + 1));
+            store16_as<kPolicy>(out + static_cast<size_t>(row) * units_per_row + u, q.codes);
+            if ((u & 7) == 0) out_scales[static_cast<size_t>(row) * scale_cols + (u >> 3)] = q.scale;
+        }
+        if (part == 0 && weights != nullptr && threadIdx.x == 0) out_weights[row] = weights[route];
     }
-    if (part == 0 && weights != nullptr && threadIdx.x == 0) out_weights[row] = weights[route];
 }
 
 // Stand-alone quantiser for rows whose width is not a multiple of 128: the last block of a row is short and is
@@ -357,10 +381,10 @@ constexpr int kSmallRoutes = 2048;
 
 template <bool kQuant, int kSlots>  // kSlots: compile-time bound of top-k (8 or DPEP_MAX_TOPK)
 __global__ __launch_bounds__(kMaxThreads) void layout_dispatch_small_kernel(
-    const long long* __restrict__ idx, int n_routes, int num_experts, int expert_begin, int num_local, int num_topk,
-    const u32x4* __restrict__ x, const float* __restrict__ scales, const float* __restrict__ weights, int units_per_row,
-    int units_per_part, int parts, int scale_cols, int* __restrict__ counts, int* __restrict__ psum, int* __restrict__ offsets,
-    int* __restrict__ num_rows, int* __restrict__ route_to_row, int* __restrict__ row_to_route, u32x4* __restrict__ out,
+    const long long* __restrict__ idx, long long* __restrict__ idx_copy, int n_routes, int num_experts, int expert_begin,
+    int num_local, int num_topk, const u32x4* __restrict__ x, const float* __restrict__ scales, const float* __restrict__ weights, int units_per_row,
+    int units_per_part, int parts, int scale_cols, int capacity, SendCounts send, int* __restrict__ counts,
+    int* __restrict__ psum, int* __restrict__ offsets, int* __restrict__ num_rows, int* __restrict__ route_to_row, int* __restrict__ row_to_route, u32x4* __restrict__ out,
     float* __restrict__ out_scales, float* __restrict__ out_weights, uint32_t* __restrict__ mailbox, uint32_t sequence)
 {
     __shared__ short local_id[kSmallRoutes];
@@ -389,8 +413,11 @@ __global__ __launch_bounds__(kMaxThreads) void layout_dispatch_small_kernel(
     for (int e = tid; e < num_local; e += kMaxThreads) first_row[e] = 0;
     if (tid < DPEP_MAX_TOPK) before[tid] = 0;
     __syncthreads();
+    const bool reporter = blockIdx.x == 0;
     for (int j = tid; j < n_routes; j += kMaxThreads) {
-        const int e = local_expert(idx[j], j, n_routes, num_experts, expert_begin, num_local);
+        const long long id = idx[j];
+        if (reporter && idx_copy != nullptr) idx_copy[j] = id;
+        const int e = local_expert(id, j, n_routes, num_experts, expert_begin, num_local);
         local_id[j] = static_cast<short>(e);
         if (e >= 0) atomicAdd(&first_row[e], 1);
     }
@@ -413,7 +440,6 @@ __global__ __launch_bounds__(kMaxThreads) void layout_dispatch_small_kernel(
     __syncthreads();
     int offset = incl - sum;
     for (int w = 0; w < wave; ++w) offset += wave_sums[w];
-    const bool reporter = blockIdx.x == 0;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
         const int e = tid * 4 + j;
@@ -423,6 +449,7 @@ __global__ __launch_bounds__(kMaxThreads) void layout_dispatch_small_kernel(
                 counts[e] = mine[j];
                 psum[e] = offset + mine[j];
                 offsets[e + 1] = offset + mine[j];
+                if (send.counts != nullptr) send.counts[send.expert_begin + e] = offset + mine[j];
             }
         }
         offset += mine[j];
@@ -431,6 +458,7 @@ __global__ __launch_bounds__(kMaxThreads) void layout_dispatch_small_kernel(
         offsets[0] = 0;
         num_rows[0] = offset;  // the last thread's running offset is the total
     }
+    if (reporter) send_counts_of_others(send, num_local, wave_sums[0] + wave_sums[1] + wave_sums[2] + wave_sums[3], tid, kMaxThreads);
     if (reporter && mailbox != nullptr && tid * 4 < num_local) mailbox_store_counts(mailbox, tid * 4, mine);
     if (reporter && mailbox != nullptr) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this thread's counts have reached the host
     __syncthreads();
@@ -458,12 +486,12 @@ __global__ __launch_bounds__(kMaxThreads) void layout_dispatch_small_kernel(
     if (tid < num_topk) {
         const int e = local_id[my_first + tid];
         const int row = e >= 0 ? first_row[e] + before[tid] : -1;
-        rows[tid] = row;
+        rows[tid] = row < capacity ? row : -1;
         if (part == 0) {
             route_to_row[my_first + tid] = row;
             if (row >= 0) {
                 row_to_route[row] = my_first + tid;
-                if (weights != nullptr) out_weights[row] = weights[my_first + tid];
+                if (weights != nullptr && row < capacity) out_weights[row] = weights[my_first + tid];
             }
         }
     }
@@ -544,7 +572,131 @@ int check_common(const char* what, int num_tokens, int num_topk, int num_rows, c
     return DPEP_OK;
 }
 
+// One payload launch.  units per row: 16-byte vectors (copy), or 16-value groups (quantise).
+struct Payload {
+    const void* x;
+    const float* scales;
+    const float* weights;
+    int num_tokens, num_topk, units, scale_cols;
+    bool quantize;
+    void* out;
+    float* out_scales;
+    float* out_weights;
+};
+
+// token-major: the grid does not depend on R; rows at or beyond `capacity` are dropped.
+int launch_token_major(const Payload& p, const int32_t* route_to_row, int capacity, hipStream_t s)
+{
+    const Split sp = choose_split(p.num_tokens, p.units, p.quantize ? 8 : 1);
+    const dim3 grid(p.num_tokens * sp.parts), block(sp.threads);
+    with_store_policy([&](auto policy) {
+        constexpr int kPolicy = decltype(policy)::value;
+        if (p.quantize)
+            hipLaunchKernelGGL(dispatch_quant_token_kernel<kPolicy>, grid, block, 0, s, static_cast<const u32x4*>(p.x), p.weights,
+                               route_to_row, p.num_topk, p.units, sp.per_part, sp.parts, capacity, static_cast<u32x4*>(p.out),
+                               p.out_scales, p.out_weights);
+        else
+            hipLaunchKernelGGL(dispatch_copy_token_kernel<kPolicy>, grid, block, 0, s, static_cast<const u32x4*>(p.x), p.scales,
+                               p.weights, route_to_row, p.num_topk, p.units, sp.per_part, sp.parts, p.scale_cols, capacity,
+                               static_cast<u32x4*>(p.out), p.out_scales, p.out_weights);
+    });
+    return launch_status("dispatch_token");
+}
+
+// row-major: workgroups for `grid_rows` rows (row_to_route has at least as many entries), which walk on to the range's end.
+int launch_row_major(const Payload& p, const int32_t* row_to_route, const RowRange& range, int grid_rows, hipStream_t s)
+{
+    const Split sp = choose_split(grid_rows, p.units, p.quantize ? 8 : 1);
+    const dim3 grid(grid_rows * sp.parts), block(sp.threads);
+    with_store_policy([&](auto policy) {
+        constexpr int kPolicy = decltype(policy)::value;
+        if (p.quantize)
+            hipLaunchKernelGGL(dispatch_quant_row_kernel<kPolicy>, grid, block, 0, s, static_cast<const u32x4*>(p.x), p.weights,
+                               row_to_route, range, p.num_tokens, p.num_topk, p.units, sp.per_part, sp.parts,
+                               static_cast<u32x4*>(p.out), p.out_scales, p.out_weights);
+        else
+            hipLaunchKernelGGL(dispatch_copy_row_kernel<kPolicy>, grid, block, 0, s, static_cast<const u32x4*>(p.x), p.scales,
+                               p.weights, row_to_route, range, p.num_tokens, p.num_topk, p.units, sp.per_part, sp.parts,
+                               p.scale_cols, static_cast<u32x4*>(p.out), p.out_scales, p.out_weights);
+    });
+    return launch_status("dispatch_row");
+}
+
+// R known (num_rows >= 0), or not known and outputs of T*K rows (num_rows < 0: the token-major grid, which does not
+// depend on R).
+int launch_payload(const Payload& p, const int32_t* route_to_row, const int32_t* row_to_route, int num_rows, hipStream_t s)
+{
+    if (num_rows < 0 || static_cast<long long>(num_rows) > static_cast<long long>(kRowMajorRatio) * p.num_tokens)
+        return launch_token_major(p, route_to_row, 0x7fffffff, s);
+    return launch_row_major(p, row_to_route, RowRange{num_rows, nullptr}, num_rows, s);
+}
+
+int launch_small(Workspace* w, const dpep_fresh_dispatch& c, int units, hipStream_t s)
+{
+    if (c.report_to_host) {
+        w->sequence = w->sequence == 0xffffffffu ? 1u : w->sequence + 1u;  // never 0: that is "nothing launched"
+        w->mailbox_local = c.num_local;
+    }
+    const Split sp = choose_split(c.num_tokens, units, 8);
+    auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(c.num_tokens * sp.parts), dim3(kMaxThreads), 0, s,
+                           reinterpret_cast<const long long*>(c.topk_idx), reinterpret_cast<long long*>(c.topk_idx_copy),
+                           c.num_tokens * c.num_topk, c.num_experts, c.expert_begin, c.num_local, c.num_topk,
+                           static_cast<const u32x4*>(c.x), c.quantize ? nullptr : c.scales, c.topk_weights, units, sp.per_part,
+                           sp.parts, c.quantize ? 0 : c.scale_cols, c.capacity_rows,
+                           SendCounts{c.send_counts, c.expert_begin, c.num_experts}, c.counts, c.psum, c.offsets, c.num_rows,
+                           c.route_to_row, c.row_to_route, static_cast<u32x4*>(c.out), c.out_scales, c.out_weights,
+                           c.report_to_host ? w->mailbox_device : nullptr, w->sequence);
+    };
+    if (c.num_topk <= 8) {
+        if (c.quantize) launch(layout_dispatch_small_kernel<true, 8>);
+        else launch(layout_dispatch_small_kernel<false, 8>);
+    } else {
+        if (c.quantize) launch(layout_dispatch_small_kernel<true, DPEP_MAX_TOPK>);
+        else launch(layout_dispatch_small_kernel<false, DPEP_MAX_TOPK>);
+    }
+    return launch_status("layout_dispatch_small");
+}
+
+// What the payload side of a fresh dispatch requires; *units: 16-byte vectors or 16-value groups per row.
+int check_fresh_payload(const char* what, const dpep_fresh_dispatch& c, int* units)
+{
+    DPEP_REQUIRE(c.x && c.out && aligned16(c.x) && aligned16(c.out), "%s: x/out must be 16-byte aligned", what);
+    DPEP_REQUIRE((c.topk_weights == nullptr) == (c.out_weights == nullptr), "%s: weights and out_weights go together", what);
+    if (c.quantize) {
+        DPEP_REQUIRE(c.row_bytes > 0 && c.row_bytes % 256 == 0 && c.row_bytes / 256 <= kMaxScaleCols,
+                     "%s: a quantised row needs a BF16 width that is a multiple of 128 (row_bytes=%d)", what, c.row_bytes);
+        DPEP_REQUIRE(c.scales == nullptr && c.out_scales != nullptr, "%s: the fused quantiser takes no input scales and needs out_scales", what);
+        *units = c.row_bytes / 32;
+    } else {
+        DPEP_REQUIRE(c.row_bytes > 0 && c.row_bytes % 16 == 0, "%s: row_bytes=%d must be a positive multiple of 16", what, c.row_bytes);
+        DPEP_REQUIRE((c.scales == nullptr) == (c.out_scales == nullptr), "%s: scales and out_scales go together", what);
+        DPEP_REQUIRE(c.scales == nullptr || c.scale_cols > 0, "%s: scale_cols must be positive with scales", what);
+        *units = c.row_bytes / 16;
+    }
+    return DPEP_OK;
+}
+
+int fresh_in_one_launch(Workspace* w, const dpep_fresh_dispatch& c, hipStream_t stream)
+{
+    DPEP_REQUIRE(c.num_tokens >= 1 && c.num_topk >= 1 && c.num_topk <= DPEP_MAX_TOPK &&
+                     static_cast<long long>(c.num_tokens) * c.num_topk <= kSmallRoutes,
+                 "layout_dispatch_small: T=%d K=%d: needs 1 <= T*K <= %d routes (larger batches take dpep_layout and a "
+                 "dispatch call)", c.num_tokens, c.num_topk, kSmallRoutes);
+    DPEP_REQUIRE(c.num_experts >= 1 && c.expert_begin >= 0 && c.num_local >= 1 && c.num_local <= DPEP_MAX_LOCAL_EXPERTS &&
+                     c.expert_begin + c.num_local <= c.num_experts,
+                 "layout_dispatch_small: bad expert range E=%d begin=%d L=%d", c.num_experts, c.expert_begin, c.num_local);
+    DPEP_REQUIRE(c.topk_idx && c.counts && c.psum && c.offsets && c.route_to_row && c.row_to_route && c.num_rows,
+                 "layout_dispatch_small: NULL routing buffer");
+    int units = 0;
+    if (int rc = check_fresh_payload("layout_dispatch_small", c, &units)) return rc;
+    return launch_small(w, c, units, stream);
+}
+
 }  // namespace
+
+int layout_of_fresh(void* ws, const dpep_fresh_dispatch& c, hipStream_t stream);
+
 }  // namespace dpep
 
 extern "C" {
@@ -574,26 +726,8 @@ int dpep_dispatch_copy(const void* x, const float* scales, const float* topk_wei
     DPEP_REQUIRE(scales == nullptr || scale_cols > 0, "dispatch_copy: scale_cols must be positive with scales");
     DPEP_REQUIRE((topk_weights == nullptr) == (out_weights == nullptr), "dispatch_copy: weights and out_weights go together");
     DPEP_REQUIRE(x != nullptr && out != nullptr && aligned16(x) && aligned16(out), "dispatch_copy: x/out must be 16-byte aligned");
-    const int vec = row_bytes / 16;
-    hipStream_t s = static_cast<hipStream_t>(stream);
-    // the token-major grid does not depend on R, so a launch that does not know R yet takes it
-    if (num_rows < 0 || static_cast<long long>(num_rows) > static_cast<long long>(kRowMajorRatio) * num_tokens) {
-        const Split sp = choose_split(num_tokens, vec, 1);
-        with_store_policy([&](auto policy) {
-            hipLaunchKernelGGL(dispatch_copy_token_kernel<decltype(policy)::value>, dim3(num_tokens * sp.parts),
-                               dim3(sp.threads), 0, s, static_cast<const u32x4*>(x), scales, topk_weights, route_to_row,
-                               num_topk, vec, sp.per_part, sp.parts, scale_cols, static_cast<u32x4*>(out), out_scales,
-                               out_weights);
-        });
-        return launch_status("dispatch_copy_token");
-    }
-    const Split sp = choose_split(num_rows, vec, 1);
-    with_store_policy([&](auto policy) {
-        hipLaunchKernelGGL(dispatch_copy_row_kernel<decltype(policy)::value>, dim3(num_rows * sp.parts), dim3(sp.threads), 0,
-                           s, static_cast<const u32x4*>(x), scales, topk_weights, row_to_route, num_tokens, num_topk, vec,
-                           sp.per_part, sp.parts, scale_cols, static_cast<u32x4*>(out), out_scales, out_weights);
-    });
-    return launch_status("dispatch_copy_row");
+    const Payload p = {x, scales, topk_weights, num_tokens, num_topk, row_bytes / 16, scale_cols, false, out, out_scales, out_weights};
+    return launch_payload(p, route_to_row, row_to_route, num_rows, static_cast<hipStream_t>(stream));
 }
 
 int dpep_dispatch_quant_fp8(const void* x, const float* topk_weights, const int32_t* route_to_row,
@@ -607,25 +741,40 @@ int dpep_dispatch_quant_fp8(const void* x, const float* topk_weights, const int3
     if (num_rows == 0 || num_tokens == 0) return DPEP_OK;  // (empty outputs may be null pointers)
     DPEP_REQUIRE((topk_weights == nullptr) == (out_weights == nullptr), "dispatch_quant_fp8: weights and out_weights go together");
     DPEP_REQUIRE(x && out && out_scales && aligned16(x) && aligned16(out), "dispatch_quant_fp8: x/out must be 16-byte aligned");
-    const int units = hidden / 16;
+    const Payload p = {x, nullptr, topk_weights, num_tokens, num_topk, hidden / 16, 0, true, out, out_scales, out_weights};
+    return launch_payload(p, route_to_row, row_to_route, num_rows, static_cast<hipStream_t>(stream));
+}
+
+int dpep_dispatch_fresh(void* ws, const dpep_fresh_dispatch* call, void* stream)
+{
+    using namespace dpep;
+    Workspace* w = as_workspace(ws);
+    DPEP_REQUIRE(w != nullptr && call != nullptr, "dispatch_fresh: not a live workspace, or NULL call");
+    const dpep_fresh_dispatch& c = *call;
     hipStream_t s = static_cast<hipStream_t>(stream);
-    // the token-major grid does not depend on R, so a launch that does not know R yet takes it
-    if (num_rows < 0 || static_cast<long long>(num_rows) > static_cast<long long>(kRowMajorRatio) * num_tokens) {
-        const Split sp = choose_split(num_tokens, units, 8);
-        with_store_policy([&](auto policy) {
-            hipLaunchKernelGGL(dispatch_quant_token_kernel<decltype(policy)::value>, dim3(num_tokens * sp.parts),
-                               dim3(sp.threads), 0, s, static_cast<const u32x4*>(x), topk_weights, route_to_row, num_topk,
-                               units, sp.per_part, sp.parts, static_cast<u32x4*>(out), out_scales, out_weights);
-        });
-        return launch_status("dispatch_quant_token");
+    DPEP_REQUIRE(c.num_tokens >= 1 && c.num_topk >= 1 && c.num_topk <= DPEP_MAX_TOPK, "dispatch_fresh: bad T=%d K=%d", c.num_tokens,
+                 c.num_topk);
+    const long long n_routes = static_cast<long long>(c.num_tokens) * c.num_topk;
+    if (n_routes > kSmallRoutes) {
+        int units = 0;
+        if (int rc = check_fresh_payload("dispatch_fresh", c, &units)) return rc;
+        DPEP_REQUIRE(c.capacity_rows >= 0, "dispatch_fresh: capacity_rows=%d is negative", c.capacity_rows);
+        if (int rc = layout_of_fresh(ws, c, s)) return rc;  // (checks the routing arguments)
+        if (c.capacity_rows == 0) return DPEP_OK;
+        const Payload p = {c.x, c.scales, c.topk_weights, c.num_tokens, c.num_topk, units, c.quantize ? 0 : c.scale_cols,
+                           c.quantize != 0, c.out, c.out_scales, c.out_weights};
+        // Expected rows of this rank's share.  Many rows per token: token-major, which reads every token once.  Otherwise
+        // row-major over the rows that the layout finds: a token-major grid is mostly workgroups of tokens without a row
+        // (6144 tokens of which 560 own a row: 10.5 us).
+        const long long expected = n_routes * c.num_local / c.num_experts;
+        if (expected > static_cast<long long>(kRowMajorRatio) * c.num_tokens) return launch_token_major(p, c.route_to_row, c.capacity_rows, s);
+        long long grid_rows = expected + expected / 8 + 64;
+        if (grid_rows > c.capacity_rows) grid_rows = c.capacity_rows;
+        if (grid_rows > n_routes) grid_rows = n_routes;
+        const int bound = n_routes < c.capacity_rows ? static_cast<int>(n_routes) : c.capacity_rows;
+        return launch_row_major(p, c.row_to_route, RowRange{bound, c.num_rows}, static_cast<int>(grid_rows), s);
     }
-    const Split sp = choose_split(num_rows, units, 8);
-    with_store_policy([&](auto policy) {
-        hipLaunchKernelGGL(dispatch_quant_row_kernel<decltype(policy)::value>, dim3(num_rows * sp.parts), dim3(sp.threads),
-                           0, s, static_cast<const u32x4*>(x), topk_weights, row_to_route, num_tokens, num_topk, units,
-                           sp.per_part, sp.parts, static_cast<u32x4*>(out), out_scales, out_weights);
-    });
-    return launch_status("dispatch_quant_row");
+    return fresh_in_one_launch(w, c, s);
 }
 
 int dpep_layout_dispatch_small(void* ws, const int64_t* topk_idx, const void* x, const float* scales,
@@ -637,48 +786,11 @@ int dpep_layout_dispatch_small(void* ws, const int64_t* topk_idx, const void* x,
     using namespace dpep;
     Workspace* w = as_workspace(ws);
     DPEP_REQUIRE(w != nullptr, "layout_dispatch_small: not a live workspace");
-    DPEP_REQUIRE(num_tokens >= 1 && num_topk >= 1 && num_topk <= DPEP_MAX_TOPK &&
-                     static_cast<long long>(num_tokens) * num_topk <= kSmallRoutes,
-                 "layout_dispatch_small: T=%d K=%d: needs 1 <= T*K <= %d routes (larger batches take dpep_layout and a "
-                 "dispatch call)", num_tokens, num_topk, kSmallRoutes);
-    DPEP_REQUIRE(num_experts >= 1 && expert_begin >= 0 && num_local >= 1 && num_local <= DPEP_MAX_LOCAL_EXPERTS &&
-                     expert_begin + num_local <= num_experts,
-                 "layout_dispatch_small: bad expert range E=%d begin=%d L=%d", num_experts, expert_begin, num_local);
-    DPEP_REQUIRE(topk_idx && counts && psum && offsets && route_to_row && row_to_route && num_rows, "layout_dispatch_small: NULL routing buffer");
-    DPEP_REQUIRE(x && out && aligned16(x) && aligned16(out), "layout_dispatch_small: x/out must be 16-byte aligned");
-    DPEP_REQUIRE((topk_weights == nullptr) == (out_weights == nullptr), "layout_dispatch_small: weights and out_weights go together");
-    int units = 0;
-    if (quantize) {
-        DPEP_REQUIRE(row_bytes > 0 && row_bytes % 256 == 0 && row_bytes / 256 <= kMaxScaleCols,
-                     "layout_dispatch_small: a quantised row needs a BF16 width that is a multiple of 128 (row_bytes=%d)", row_bytes);
-        DPEP_REQUIRE(scales == nullptr && out_scales != nullptr, "layout_dispatch_small: the fused quantiser takes no input scales and needs out_scales");
-        units = row_bytes / 32;
-    } else {
-        DPEP_REQUIRE(row_bytes > 0 && row_bytes % 16 == 0, "layout_dispatch_small: row_bytes=%d must be a positive multiple of 16", row_bytes);
-        DPEP_REQUIRE((scales == nullptr) == (out_scales == nullptr), "layout_dispatch_small: scales and out_scales go together");
-        DPEP_REQUIRE(scales == nullptr || scale_cols > 0, "layout_dispatch_small: scale_cols must be positive with scales");
-        units = row_bytes / 16;
-    }
-    w->sequence = w->sequence == 0xffffffffu ? 1u : w->sequence + 1u;  // never 0: that is "nothing launched"
-    w->mailbox_local = num_local;
-    const Split sp = choose_split(num_tokens, units, 8);
-    const int n_routes = num_tokens * num_topk;
-    hipStream_t s = static_cast<hipStream_t>(stream);
-    auto launch = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, dim3(num_tokens * sp.parts), dim3(kMaxThreads), 0, s,
-                           reinterpret_cast<const long long*>(topk_idx), n_routes, num_experts, expert_begin, num_local, num_topk,
-                           static_cast<const u32x4*>(x), quantize ? nullptr : scales, topk_weights, units, sp.per_part, sp.parts,
-                           quantize ? 0 : scale_cols, counts, psum, offsets, num_rows, route_to_row, row_to_route,
-                           static_cast<u32x4*>(out), out_scales, out_weights, w->mailbox_device, w->sequence);
-    };
-    if (num_topk <= 8) {
-        if (quantize) launch(layout_dispatch_small_kernel<true, 8>);
-        else launch(layout_dispatch_small_kernel<false, 8>);
-    } else {
-        if (quantize) launch(layout_dispatch_small_kernel<true, DPEP_MAX_TOPK>);
-        else launch(layout_dispatch_small_kernel<false, DPEP_MAX_TOPK>);
-    }
-    return launch_status("layout_dispatch_small");
+    const dpep_fresh_dispatch c = {topk_idx, nullptr, x, scales, topk_weights, counts, psum, offsets, route_to_row, row_to_route,
+                                   num_rows, nullptr, out, out_scales, out_weights, num_tokens, num_topk, num_experts,
+                                   expert_begin, num_local, row_bytes, scale_cols, quantize, /*capacity_rows=*/0x7fffffff,
+                                   /*report_to_host=*/1};
+    return fresh_in_one_launch(w, c, static_cast<hipStream_t>(stream));
 }
 
 int dpep_cast_to_fp8(const void* x, int num_tokens, int hidden, void* out, float* out_scales, void* stream)
@@ -701,8 +813,8 @@ int dpep_cast_to_fp8(const void* x, int num_tokens, int hidden, void* out, float
     with_store_policy([&](auto policy) {
         hipLaunchKernelGGL(dispatch_quant_row_kernel<decltype(policy)::value>, dim3(num_tokens * sp.parts),
                            dim3(sp.threads), 0, static_cast<hipStream_t>(stream), static_cast<const u32x4*>(x), nullptr,
-                           nullptr, num_tokens, 1, units, sp.per_part, sp.parts, static_cast<u32x4*>(out), out_scales,
-                           nullptr);
+                           nullptr, RowRange{num_tokens, nullptr}, num_tokens, 1, units, sp.per_part, sp.parts,
+                           static_cast<u32x4*>(out), out_scales, nullptr);
     });
     return launch_status("cast_to_fp8");
 }

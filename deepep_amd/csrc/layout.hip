@@ -55,10 +55,12 @@ __device__ __forceinline__ void wave_sync()
 
 // Local experts of kSteps consecutive 64-route steps from `base` on.  All loads are issued before the first is
 // used (a route past the end reads the last id instead of branching around the load), so that the wave pays
-// one memory latency for the batch, not one per step.  Needs n_routes > 0.
+// one memory latency for the batch, not one per step.  Needs n_routes > 0.  idx_copy: where the ids are copied to
+// (a handle's own routing tensor; the copy rides on ids that are read anyway), or nullptr.
 template <int kSteps, typename IdxT>
 __device__ __forceinline__ void fetch_experts(int (&experts)[kSteps], const IdxT* __restrict__ idx, int base, int end,
-                                              int n_routes, int num_experts, int expert_begin, int num_local)
+                                              int n_routes, int num_experts, int expert_begin, int num_local,
+                                              IdxT* __restrict__ idx_copy = nullptr)
 {
     const int lane = threadIdx.x & 63;
     IdxT raw[kSteps];
@@ -68,6 +70,11 @@ __device__ __forceinline__ void fetch_experts(int (&experts)[kSteps], const IdxT
     for (int i = 0; i < kSteps; ++i)
         experts[i] = local_expert(static_cast<long long>(raw[i]), base + i * kWave + lane, end, num_experts, expert_begin,
                                   num_local);
+    if (idx_copy != nullptr) {
+#pragma unroll
+        for (int i = 0; i < kSteps; ++i)
+            if (base + i * kWave + lane < end) idx_copy[base + i * kWave + lane] = raw[i];
+    }
 }
 
 // LDS of one workgroup.  running[w][e]: wave w's histogram, later its next free row of expert e; match[w][e]: bit
@@ -147,7 +154,7 @@ template <typename IdxT>
 __global__ __launch_bounds__(kThreads) void layout_count_kernel(const IdxT* __restrict__ idx, int n_routes,
                                                                 int num_experts, int expert_begin, int num_local,
                                                                 int chunk, int num_chunks, int* __restrict__ wave_hist,
-                                                                int* __restrict__ block_hist)
+                                                                int* __restrict__ block_hist, IdxT* __restrict__ idx_copy)
 {
     __shared__ LayoutLds lds;
     const int wave = threadIdx.x >> 6;
@@ -157,7 +164,7 @@ __global__ __launch_bounds__(kThreads) void layout_count_kernel(const IdxT* __re
     clear_wave_lds(lds, num_local);
     for (int base = begin; base < end; base += kPrefetch * kWave) {
         int experts[kPrefetch];
-        fetch_experts(experts, idx, base, end, n_routes, num_experts, expert_begin, num_local);
+        fetch_experts(experts, idx, base, end, n_routes, num_experts, expert_begin, num_local, idx_copy);
 #pragma unroll
         for (int i = 0; i < kPrefetch; ++i) count_step(experts[i], lds.running[wave]);
     }
@@ -276,7 +283,7 @@ __device__ __forceinline__ bool expert_bases(LayoutLds& lds, const int* __restri
                                              const int* __restrict__ block_hist, int num_local, int padded_local,
                                              int num_chunks, int num_blocks, int* __restrict__ counts,
                                              int* __restrict__ psum, int* __restrict__ offsets, int* __restrict__ num_rows,
-                                             uint32_t* __restrict__ mailbox, uint32_t sequence,
+                                             const SendCounts& send, uint32_t* __restrict__ mailbox, uint32_t sequence,
                                              const TaggedSource* source = nullptr)
 {
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
@@ -377,6 +384,7 @@ __device__ __forceinline__ bool expert_bases(LayoutLds& lds, const int* __restri
                 counts[e] = mine[j];
                 psum[e] = offset + mine[j];
                 offsets[e + 1] = offset + mine[j];
+                if (send.counts != nullptr) send.counts[send.expert_begin + e] = offset + mine[j];
             }
         }
         offset += mine[j];
@@ -385,6 +393,7 @@ __device__ __forceinline__ bool expert_bases(LayoutLds& lds, const int* __restri
         offsets[0] = 0;
         num_rows[0] = offset;
     }
+    if (reporter) send_counts_of_others(send, num_local, lds.wave_sums[0] + lds.wave_sums[1] + lds.wave_sums[2] + lds.wave_sums[3], tid, kThreads);
     if (reporter && mailbox != nullptr && tid * 4 < num_local) mailbox_store_counts(mailbox, tid * 4, mine);
     // The host polls the mailbox's sequence word: publish it (with the row count, one 8-byte store) after
     // every per-expert count of this workgroup has reached host memory.  The counts went out as write-through
@@ -404,7 +413,8 @@ __global__ __launch_bounds__(kThreads) void layout_assign_kernel(
     const IdxT* __restrict__ idx, int n_routes, int num_experts, int expert_begin, int num_local, int padded_local,
     int chunk, int num_chunks, const int* __restrict__ wave_hist, const int* __restrict__ block_hist,
     int* __restrict__ counts, int* __restrict__ psum, int* __restrict__ offsets, int* __restrict__ num_rows,
-    int* __restrict__ route_to_row, int* __restrict__ row_to_route, uint32_t* __restrict__ mailbox, uint32_t sequence)
+    int* __restrict__ route_to_row, int* __restrict__ row_to_route, SendCounts send, uint32_t* __restrict__ mailbox,
+    uint32_t sequence)
 {
     __shared__ LayoutLds lds;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -416,7 +426,7 @@ __global__ __launch_bounds__(kThreads) void layout_assign_kernel(
     clear_wave_lds(lds, num_local);
     __syncthreads();  // expert_bases writes the rows of all waves
     expert_bases<false>(lds, wave_hist, block_hist, num_local, padded_local, num_chunks, gridDim.x - 1, counts, psum,
-                        offsets, num_rows, mailbox, sequence);
+                        offsets, num_rows, send, mailbox, sequence);
     for (int base = begin; base < end; base += kPrefetch * kWave) {
         if (base != begin) fetch_experts(experts, idx, base, end, n_routes, num_experts, expert_begin, num_local);
 #pragma unroll
@@ -444,8 +454,8 @@ template <typename IdxT>
 __global__ __launch_bounds__(kThreads) void layout_fused_kernel(
     const IdxT* __restrict__ idx, int n_routes, int num_experts, int expert_begin, int num_local, int padded_local,
     int chunk, int num_chunks, int* __restrict__ counts, int* __restrict__ psum, int* __restrict__ offsets,
-    int* __restrict__ num_rows, int* __restrict__ route_to_row, int* __restrict__ row_to_route,
-    uint32_t* __restrict__ mailbox, uint32_t sequence, unsigned long long* __restrict__ epoch,
+    int* __restrict__ num_rows, int* __restrict__ route_to_row, int* __restrict__ row_to_route, IdxT* __restrict__ idx_copy,
+    SendCounts send, uint32_t* __restrict__ mailbox, uint32_t sequence, unsigned long long* __restrict__ epoch,
     unsigned long long* __restrict__ tagged, int rows, long long limit_ticks, uint32_t* __restrict__ timeouts,
     uint32_t launch_id)
 {
@@ -464,7 +474,7 @@ __global__ __launch_bounds__(kThreads) void layout_fused_kernel(
         if (reporter) __hip_atomic_store(reporter_tag, lds.tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
     int experts[kKeep];
-    fetch_experts(experts, idx, begin, end, n_routes, num_experts, expert_begin, num_local);
+    fetch_experts(experts, idx, begin, end, n_routes, num_experts, expert_begin, num_local, idx_copy);
     clear_wave_lds(lds, num_local);
 #pragma unroll
     for (int i = 0; i < kKeep; ++i) count_step(experts[i], lds.running[wave]);
@@ -480,7 +490,7 @@ __global__ __launch_bounds__(kThreads) void layout_fused_kernel(
     // row_to_route clamp what they find there.
     const TaggedSource source = {tagged, tag, rows, reporter ? limit_ticks : 2 * limit_ticks, timeouts, launch_id};
     const bool in_time = expert_bases<true>(lds, nullptr, nullptr, num_local, padded_local, num_chunks, gridDim.x - 1, counts,
-                                            psum, offsets, num_rows, mailbox, sequence, &source);
+                                            psum, offsets, num_rows, send, mailbox, sequence, &source);
     // (asked for here, needed only at the very end: the load travels while the routes are assigned)
     unsigned long long reporter_seen = threadIdx.x == 0 && !reporter ? load_word(reporter_tag) : 0ull;
     if (in_time) {
@@ -553,27 +563,28 @@ int check_layout_arguments(const void* idx, int num_tokens, int num_topk, int nu
 template <typename IdxT>
 int enqueue_count_and_assign(const IdxT* idx, int n_routes, int num_experts, int expert_begin, int num_local, int padded, int chunk,
                              int num_chunks, int* wave_hist, int* block_hist, int32_t* counts, int32_t* psum, int32_t* offsets,
-                             int32_t* num_rows, int32_t* route_to_row, int32_t* row_to_route, uint32_t* mailbox, uint32_t sequence,
-                             hipStream_t stream)
+                             int32_t* num_rows, int32_t* route_to_row, int32_t* row_to_route, IdxT* idx_copy, const SendCounts& send,
+                             uint32_t* mailbox, uint32_t sequence, hipStream_t stream)
 {
     const int blocks = (num_chunks + kWaves - 1) / kWaves;
     if (blocks > 0) {
         hipLaunchKernelGGL(layout_count_kernel<IdxT>, dim3(blocks), dim3(kThreads), 0, stream, idx, n_routes, num_experts,
-                           expert_begin, num_local, chunk, num_chunks, wave_hist, block_hist);
+                           expert_begin, num_local, chunk, num_chunks, wave_hist, block_hist, idx_copy);
         if (int rc = launch_status("layout_count")) return rc;
     }
     // One workgroup more than there are chunks to assign: the reporter (with no routes, it alone publishes the
     // all-zero counts and prefix sums).
     hipLaunchKernelGGL(layout_assign_kernel<IdxT>, dim3(blocks + 1), dim3(kThreads), 0, stream, idx,
                        n_routes, num_experts, expert_begin, num_local, padded, chunk, num_chunks, wave_hist, block_hist, counts,
-                       psum, offsets, num_rows, route_to_row, row_to_route, mailbox, sequence);
+                       psum, offsets, num_rows, route_to_row, row_to_route, send, mailbox, sequence);
     return launch_status("layout_assign");
 }
 
 template <typename IdxT>
 int launch_layout(void* ws, const IdxT* idx, int num_tokens, int num_topk, int num_experts, int expert_begin,
                   int num_local, int32_t* counts, int32_t* psum, int32_t* offsets, int32_t* route_to_row,
-                  int32_t* row_to_route, int32_t* num_rows, bool report_to_host, hipStream_t stream)
+                  int32_t* row_to_route, int32_t* num_rows, IdxT* idx_copy, const SendCounts& send, bool report_to_host,
+                  hipStream_t stream)
 {
     Workspace* w = as_workspace(ws);
     DPEP_REQUIRE(w != nullptr, "layout: not a live workspace");
@@ -616,14 +627,14 @@ int launch_layout(void* ws, const IdxT* idx, int num_tokens, int num_topk, int n
         char* sync = static_cast<char*>(w->sync);
         hipLaunchKernelGGL(layout_fused_kernel<IdxT>, dim3(blocks + 1), dim3(kThreads), 0, stream, idx, n_routes, num_experts,
                            expert_begin, num_local, padded, chunk, num_chunks, counts, psum, offsets, num_rows, route_to_row,
-                           row_to_route, mailbox, w->sequence, reinterpret_cast<unsigned long long*>(sync),
+                           row_to_route, idx_copy, send, mailbox, w->sequence, reinterpret_cast<unsigned long long*>(sync),
                            reinterpret_cast<unsigned long long*>(sync + kSyncTagged), blocks + w->exchange_extra_rows,
                            w->exchange_ticks, w->mailbox_device + kMailboxTimeout, w->layout_launches);
         return launch_status("layout_fused");
     }
     return enqueue_count_and_assign<IdxT>(idx, n_routes, num_experts, expert_begin, num_local, padded, chunk, num_chunks, wave_hist,
-                                          block_hist, counts, psum, offsets, num_rows, route_to_row, row_to_route, mailbox,
-                                          w->sequence, stream);
+                                          block_hist, counts, psum, offsets, num_rows, route_to_row, row_to_route, idx_copy, send,
+                                          mailbox, w->sequence, stream);
 }
 
 }  // namespace
@@ -634,7 +645,15 @@ int layout_i32(void* ws, const int32_t* idx, int num_tokens, int num_topk, int n
                int32_t* row_to_route, int32_t* num_rows, hipStream_t stream)
 {
     return launch_layout<int32_t>(ws, idx, num_tokens, num_topk, num_experts, expert_begin, num_local, counts, psum,
-                                  offsets, route_to_row, row_to_route, num_rows, /*report_to_host=*/false, stream);
+                                  offsets, route_to_row, row_to_route, num_rows, nullptr, SendCounts{}, /*report_to_host=*/false, stream);
+}
+
+// The layout of a fresh dispatch (dpep_dispatch_fresh).
+int layout_of_fresh(void* ws, const dpep_fresh_dispatch& c, hipStream_t stream)
+{
+    return launch_layout<int64_t>(ws, c.topk_idx, c.num_tokens, c.num_topk, c.num_experts, c.expert_begin, c.num_local, c.counts,
+                                  c.psum, c.offsets, c.route_to_row, c.row_to_route, c.num_rows, c.topk_idx_copy,
+                                  SendCounts{c.send_counts, c.expert_begin, c.num_experts}, c.report_to_host != 0, stream);
 }
 
 }  // namespace dpep
@@ -690,7 +709,7 @@ int dpep_layout(void* ws, const int64_t* topk_idx, int num_tokens, int num_topk,
                 int32_t* row_to_route, int32_t* num_rows, void* stream)
 {
     return dpep::launch_layout<int64_t>(ws, topk_idx, num_tokens, num_topk, num_experts, expert_begin, num_local,
-                                        counts, psum, offsets, route_to_row, row_to_route, num_rows,
+                                        counts, psum, offsets, route_to_row, row_to_route, num_rows, nullptr, dpep::SendCounts{},
                                         /*report_to_host=*/true, static_cast<hipStream_t>(stream));
 }
 
@@ -716,7 +735,7 @@ int dpep_layout_static(const int64_t* topk_idx, int num_tokens, int num_topk, in
     if (int rc = scratch_of_current_device(&base)) return rc;
     return enqueue_count_and_assign<int64_t>(topk_idx, n_routes, num_experts, expert_begin, num_local, padded, chunk, num_chunks,
                                              base, base + kHistInts, counts, psum, offsets, num_rows, route_to_row, row_to_route,
-                                             /*mailbox=*/nullptr, 0u, static_cast<hipStream_t>(stream));
+                                             /*idx_copy=*/nullptr, SendCounts{}, /*mailbox=*/nullptr, 0u, static_cast<hipStream_t>(stream));
 }
 
 }  // extern "C"

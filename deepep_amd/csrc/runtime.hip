@@ -96,6 +96,12 @@ int dpep_workspace_destroy(void* ws)
     return DPEP_OK;
 }
 
+int dpep_layout_ready(void* ws)
+{
+    dpep::Workspace* w = dpep::as_workspace(ws);
+    return w != nullptr && w->sequence != 0 && static_cast<volatile uint32_t*>(w->mailbox_host)[1] == w->sequence;
+}
+
 int dpep_layout_wait(void* ws, int32_t* counts_host, int num_local, int32_t* num_rows_host, long long timeout_us)
 {
     dpep::Workspace* w = dpep::as_workspace(ws);

@@ -15,10 +15,15 @@ tuples and exception types.  What is different, deliberately:
     class also accepts);
   * a synchronous call (``async_with_compute_stream=False``) is queued on the caller's current stream; only
     asynchronous calls use the communication stream (see ``_Enqueue``).
+
+``dispatch`` and ``combine`` hand every call to the native host path first (csrc/host.cpp, ``_host.Exchange``), which takes all
+ordinary ones.  What follows in Python is for the calls it returns: invalid ones, whose faults are named here, and unusual
+ones (tensor subclasses, inference mode, handles whose attributes were replaced), which are carried out step by step.
 """
 
 from __future__ import annotations
 
+import functools
 import threading
 import warnings
 from typing import Optional, Tuple, Union
@@ -76,6 +81,17 @@ def _load_native():
 
     ops._lib.load()  # raises if libdeepep_amd.so is not built: there is no fallback path
     return ops
+
+
+@functools.lru_cache(maxsize=None)
+def _load_host():
+    """The native host path, told about the classes whose objects it makes."""
+    from . import _lib
+
+    host = _lib.host()
+    form = EPHandle(True, 0, 1, 0, 0, None, None, 0, [], None, None, None, None, None, None, None)
+    host.configure(EPHandle, vars(form), EventOverlap, EventHandle, _lib.NativeError)
+    return host
 
 
 class EPHandle:
@@ -136,6 +152,7 @@ class EPHandle:
         self.metadata_version = 7
         self._buffer_token = None
         self._routing_versions = {}
+        self._plan = None                 # the native host path's own record of the routing (_host.Plan)
 
     @property
     def num_sms(self):
@@ -197,7 +214,7 @@ class _Runtime:
     """Process-local owner of the HBM workspace and the communication stream (the single-GPU
     counterpart of deep_ep/_runtime.py:67-308 without SHMEM bootstrap)."""
 
-    def __init__(self, native, num_bytes, rank, world_size, combine_only):
+    def __init__(self, native, num_bytes, rank, world_size, combine_only, token, hidden, num_topk, bound, use_fp8_dispatch):
         self.native = native
         self.device = gpu_api().current_device()
         self.torch_device = torch.device("cuda", self.device)
@@ -205,14 +222,33 @@ class _Runtime:
         self.combine_only = combine_only
         self.capacity = num_bytes
         self.notify_lock = threading.RLock()
-        self.notify_failed = False
         self.notify_inflight = None
         # `capacity` is what the caller asked for (the low-latency path insists on exactly 8 GiB, as the reference
         # does); the HBM actually taken is bounded by what the single-GPU kernels use, the layout scratch.
         self.workspace = native.Workspace(min(num_bytes, WORKSPACE_ALLOCATION_CAP), self.torch_device)
         self.stream = gpu_api().Stream(device=self.torch_device)
-        self.last_stream = None  # the stream the buffer's most recent kernels were queued on
+        self.exchange = _load_host().Exchange(
+            self.workspace.handle.value, token, self.notify_lock, self.stream, self.device, rank, world_size, hidden, num_topk, bound,
+            use_fp8_dispatch, combine_only, num_bytes == LOW_LATENCY_WORKSPACE_BYTES)
         self.closed = False
+
+    @property
+    def notify_failed(self):
+        """A launch failed: the buffer takes no further calls."""
+        return self.exchange.failed
+
+    @notify_failed.setter
+    def notify_failed(self, value):
+        self.exchange.failed = value
+
+    @property
+    def last_stream(self):
+        """The stream the buffer's most recent kernels were queued on, or None."""
+        return self.exchange.last_stream
+
+    @last_stream.setter
+    def last_stream(self, stream):
+        self.exchange.last_stream = stream
 
     def ensure_alive(self):
         if self.closed:
@@ -220,6 +256,7 @@ class _Runtime:
 
     def close(self):
         if not self.closed:
+            self.exchange.close()
             self.stream.synchronize()
             if self.last_stream is not None:
                 self.last_stream.synchronize()
@@ -253,6 +290,8 @@ def _resolve_world(group, rank, world_size):
 
 class ElasticBuffer:
     """Dispatch / combine for one EP rank on one GPU; see the module docstring for the deviations."""
+
+    _exchange = None  # the native host path, set when the buffer owns a workspace
 
     @accept_aliases(num_device_timeout_secs="num_gpu_timeout_secs")
     def __init__(
@@ -314,7 +353,9 @@ class ElasticBuffer:
         self.use_fp8_dispatch = use_fp8_dispatch
         self.machine_type = "mi355x"
         self._handle_token = object()
-        self._runtime = _Runtime(native, num_bytes, resolved_rank, resolved_world, combine_only)
+        self._runtime = _Runtime(native, num_bytes, resolved_rank, resolved_world, combine_only, self._handle_token, hidden, num_topk,
+                                 num_max_tokens_per_rank, use_fp8_dispatch)
+        self._exchange = self._runtime.exchange
 
     def __del__(self):
         runtime = getattr(self, "_runtime", None)
@@ -427,7 +468,8 @@ class ElasticBuffer:
         )
 
     def _check_versions(self, handle):
-        for name, version in handle._routing_versions.items():
+        versions = handle._plan.versions() if handle._plan is not None else handle._routing_versions
+        for name, version in versions.items():
             tensor = getattr(handle, name)
             if torch.is_inference(tensor) or (tensor.data_ptr(), tensor._version) != version:
                 raise ValueError(f"Cached routing was modified: {name}")
@@ -462,6 +504,13 @@ class ElasticBuffer:
         A fresh call computes the layout and reads the per-expert counts back to the host (one
         synchronisation); ``handle=`` reuses a previous plan with a new payload.
         """
+        if self._exchange is not None:
+            done = self._exchange.dispatch(
+                x, topk_idx, topk_weights, cumulative_local_expert_recv_stats, num_experts, num_max_tokens_per_rank,
+                expert_alignment, num_sms, num_qps, previous_event, previous_event_before_epilogue, async_with_compute_stream,
+                allocate_on_comm_stream, handle, do_handle_copy, do_cpu_sync, do_expand, do_zero_padding, use_tma_aligned_col_major_sf)
+            if done is not None:
+                return done
         runtime = self._live_runtime()
         runtime.ensure_alive()
         native = runtime.native
@@ -866,6 +915,11 @@ class ElasticBuffer:
         ``[T,K]`` with 0 in slots without a row.  Low-latency style handles (``is_low_latency``):
         the saved ``handle.source_weights`` multiply each row before the sum.
         """
+        if self._exchange is not None:
+            done = self._exchange.combine(x, handle, topk_weights, bias, num_sms, num_qps, previous_event,
+                                          previous_event_before_epilogue, async_with_compute_stream, allocate_on_comm_stream)
+            if done is not None:
+                return done
         runtime = self._live_runtime()
         runtime.ensure_alive()
         native = runtime.native

@@ -4,7 +4,8 @@ protocol), over HIP events through ``torch.cuda``.
 
 How it is put together here: a ``_Marker`` is one recorded HIP event plus where it was recorded; a ``_Lease`` keeps
 objects alive and tells torch's caching allocator which streams use which tensors.  ``EventHandle`` is a marker with
-a public face, ``EventOverlap`` a marker, a lease and an optional hook.
+a public face, ``EventOverlap`` a marker, a lease and an optional hook.  The native host path makes markers and leases of
+its own (``_host.Marker``, ``_host.Lease``) with the same methods.
 """
 
 from __future__ import annotations
@@ -89,6 +90,13 @@ class EventOverlap:
     ``EventOverlap()`` with no event is valid and has nothing to wait for.  ``with overlap: ...`` waits when the block
     ends; ``with overlap(release_handle=True): ...`` also drops the event and the retained objects then.
     """
+
+    # (what an overlap without an event has; the native host path makes those without running __init__)
+    event: Optional[EventHandle] = None
+    extra_tensors: Optional[Tuple[torch.Tensor]] = None
+    hook_after_wait: Optional[Callable] = None
+    _lease: Optional[_Lease] = None
+    _release_on_exit = False
 
     def __init__(self, event: Optional[EventHandle] = None, extra_tensors: Optional[Tuple[torch.Tensor]] = None) -> None:
         self.event = event

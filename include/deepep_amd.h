@@ -95,6 +95,8 @@ int dpep_layout_static(const int64_t* topk_idx, int num_tokens, int num_topk, in
  *   timeout_us    DPEP_ERUNTIME if the kernel has not reported by then (a layout launch that failed never will)
  * One layout may be outstanding per workspace; the call does not wait for anything but the layout kernel. */
 int dpep_layout_wait(void* ws, int32_t* counts_host, int num_local, int32_t* num_rows_host, long long timeout_us);
+/* 1 if the most recent layout launched on ws has reported (dpep_layout_wait would not have to wait), else 0. */
+int dpep_layout_ready(void* ws);
 
 /* Expand-permute payload dispatch: out[row(t,s)] = x[t] for every route with a row.
  * Replaces dispatch() (csrc/ops/dispatch.cpp:82-211 -> dispatch_kernel, csrc/kernels/dispatch/dispatch.cpp:628)
@@ -150,6 +152,34 @@ int dpep_layout_dispatch_small(void* ws, const int64_t* topk_idx, const void* x,
                                int num_local, int row_bytes, int scale_cols, int quantize, int32_t* counts, int32_t* psum,
                                int32_t* offsets, int32_t* route_to_row, int32_t* row_to_route, int32_t* num_rows, void* out,
                                float* out_scales, float* out_weights, void* stream);
+
+/* One fresh dispatch as ElasticBuffer makes it (notify + dispatch, deep_ep/backends/mesh_clos/elastic.py:648-1008): the layout
+ * and, queued behind it before the host knows R, the payload; for a small batch both in one launch (see above).  The
+ * payload outputs hold capacity_rows rows, of which the first min(R, capacity_rows) are written: a caller that finds
+ * R > capacity_rows allocates R rows and calls dpep_dispatch_copy / dpep_dispatch_quant_fp8 with the same maps. */
+typedef struct dpep_fresh_dispatch {
+    const int64_t* topk_idx;    /* [T,K] */
+    int64_t* topk_idx_copy;     /* [T,K] receives a copy of topk_idx (the handle's own), or NULL */
+    const void* x;              /* [T] rows of row_bytes bytes */
+    const float* scales;        /* [T,scale_cols] 4-byte words moved with the rows, or NULL */
+    const float* topk_weights;  /* [T,K] or NULL */
+    int32_t* counts;            /* layout outputs as for dpep_layout */
+    int32_t* psum;
+    int32_t* offsets;
+    int32_t* route_to_row;
+    int32_t* row_to_route;
+    int32_t* num_rows;
+    int32_t* send_counts;       /* [E]: rows of experts 0..e that are local to this rank, or NULL */
+    void* out;                  /* payload outputs, capacity_rows rows each; out_scales and out_weights NULL where unused */
+    float* out_scales;
+    float* out_weights;
+    int32_t num_tokens, num_topk, num_experts, expert_begin, num_local;
+    int32_t row_bytes, scale_cols;
+    int32_t quantize;           /* != 0: x is BF16 and is quantised per 128 columns (scales NULL, out FP8, out_scales [.,H/128]) */
+    int32_t capacity_rows;
+    int32_t report_to_host;     /* != 0: counts and R also go to the host mailbox (dpep_layout_wait) */
+} dpep_fresh_dispatch;
+int dpep_dispatch_fresh(void* ws, const dpep_fresh_dispatch* call, void* stream);
 
 /* Stand-alone per-128 quantiser (deep_ep/utils/math.py:45-61): x bf16 [T,H] -> fp8 [T,H], fp32 [T,ceil(H/128)].
  * H % 16 == 0; a last block shorter than 128 is quantised as if padded with zeros (math.py:52-53). */

@@ -1,0 +1,204 @@
+"""The native host path of ElasticBuffer (csrc/host.cpp) where it can go wrong: outputs allocated before the row count is known
+and outgrown by it, row-major payloads that walk past their grid, the routing copy, ids per rank of the low-latency path,
+handles that leave the native path, and memory that is handed out again behind asynchronous calls."""
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import combine as ocombine
+from oracle import layout as olayout
+from oracle import quant as oquant
+from tests.gpu_util import bf16_bits, f32_bits, fp8_bits
+
+pytestmark = pytest.mark.gpu
+
+
+def _buffer(**options):
+    import deepep_amd
+
+    return deepep_amd.ElasticBuffer(None, explicitly_destroy=True, **options)
+
+
+def _batch(tokens, hidden, topk, seed):
+    gen = torch.Generator().manual_seed(seed)
+    return torch.randn(tokens, hidden, generator=gen).bfloat16(), torch.rand(tokens, topk, generator=gen)
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("world", [2, 4, 16])
+def test_rows_of_a_share_far_from_the_expected_number(world, fp8):
+    """One buffer, batches whose share of rows jumps: about the expected one, everything (outputs are outgrown, the payload is
+    dispatched again), nothing, one row, everything again (sized by the batch before), and a batch of the one-launch size."""
+    experts, topk, hidden = world * 4, 4, 256
+    rank = world - 1
+    local = range(rank * 4, rank * 4 + 4)
+    rng = np.random.default_rng(world)
+    buffer = _buffer(num_bytes=4 << 20, rank=rank, world_size=world, use_fp8_dispatch=fp8)
+    try:
+        for step, (tokens, kind) in enumerate([(1024, "usual"), (1024, "all"), (1024, "none"), (1024, "one"), (900, "all"), (1024, "usual"),
+                                               (64, "all"), (64, "usual")]):
+            ids = np.stack([rng.permutation(experts)[:topk] for _ in range(tokens)]).astype(np.int64)
+            if kind == "all":
+                ids = np.stack([rng.permutation(local)[:topk] for _ in range(tokens)]).astype(np.int64)
+            elif kind != "usual":
+                ids[np.isin(ids, local)] = -1
+                if kind == "one":
+                    ids[tokens - 1, topk - 1] = local[1]
+            x, w = _batch(tokens, hidden, topk, step)
+            idx = torch.from_numpy(ids).cuda()
+            weights = w.cuda() if world < 16 or fp8 else None  # (with weights, EP16 and BF16 this would be a low-latency call)
+            want = olayout.layout(ids, experts, rank * 4, 4)
+            recv, _, recv_w, handle, _ = buffer.dispatch(x.cuda(), topk_idx=idx, topk_weights=weights, num_experts=experts)
+            assert handle.num_expanded_tokens == want["num_rows"], (step, kind)
+            assert handle.num_recv_tokens_per_expert_list == want["counts"].tolist()
+            np.testing.assert_array_equal(handle.route_to_row.cpu().numpy(), want["route_to_row"])
+            np.testing.assert_array_equal(handle.weight_return_meta.cpu().numpy(), want["row_to_route"])
+            np.testing.assert_array_equal(handle.psum_num_recv_tokens_per_expert.cpu().numpy(), want["psum"])
+            np.testing.assert_array_equal(handle.expert_offsets.cpu().numpy(), want["offsets"])
+            assert torch.equal(handle.topk_idx, idx) and handle.topk_idx.data_ptr() != idx.data_ptr()
+            if fp8:
+                q, s = oquant.cast_to_fp8_torch(x)
+                np.testing.assert_array_equal(fp8_bits(recv[0]), olayout.expand_rows(fp8_bits(q), want["row_to_route"], topk))
+                np.testing.assert_array_equal(f32_bits(recv[1]), olayout.expand_rows(f32_bits(s), want["row_to_route"], topk))
+            else:
+                np.testing.assert_array_equal(bf16_bits(recv), olayout.expand_rows(bf16_bits(x), want["row_to_route"], topk))
+            if weights is not None:
+                np.testing.assert_array_equal(f32_bits(recv_w), olayout.expand_weights(w.numpy(), want["row_to_route"]).view(np.uint32))
+            y = torch.randn(want["num_rows"], hidden).bfloat16()
+            out, _, _ = buffer.combine(y.cuda(), handle)
+            np.testing.assert_array_equal(bf16_bits(out), ocombine.combine(bf16_bits(y), want["route_to_row"]))
+    finally:
+        buffer.destroy()
+
+
+@pytest.mark.parametrize("per_rank,skewed", [(3, False), (64, False), (64, True)])
+def test_low_latency_ids_and_send_counts(per_rank, skewed):
+    """Below and above the one-launch size, and with a share far above the expected one (row-major workgroups walk on)."""
+    world, rank, experts, topk, hidden = 16, 9, 64, 8, 512
+    rng = np.random.default_rng(per_rank)
+    tokens = world * per_rank
+    popularity = np.ones(experts)
+    if skewed:
+        popularity[rank * 4 : rank * 4 + 4] = 1000.0
+    ids = np.stack([rng.choice(experts, topk, replace=False, p=popularity / popularity.sum()) for _ in range(tokens)]).astype(np.int64)
+    x, w = _batch(tokens, hidden, topk, 5)
+    want = olayout.layout(ids, experts, rank * 4, 4)
+    buffer = _buffer(num_bytes=8 << 30, rank=rank, world_size=world)
+    try:
+        idx = torch.from_numpy(ids).cuda()
+        recv, _, _, handle, _ = buffer.dispatch(x.cuda(), topk_idx=idx, topk_weights=w.cuda(), num_experts=experts)
+        rows = want["num_rows"]
+        np.testing.assert_array_equal(bf16_bits(recv[:rows]), olayout.expand_rows(bf16_bits(x), want["row_to_route"], topk))
+        np.testing.assert_array_equal(f32_bits(handle.source_weights[:rows]), olayout.expand_weights(w.numpy(), want["row_to_route"]).view(np.uint32))
+        sent = np.zeros(experts, np.int32)
+        sent[rank * 4 : rank * 4 + 4] = want["psum"]
+        sent[rank * 4 + 4 :] = rows
+        np.testing.assert_array_equal(handle.send_counts.cpu().numpy(), sent)
+        np.testing.assert_array_equal(handle.route_to_row.cpu().numpy(), want["route_to_row"])
+        assert torch.equal(handle.topk_idx, idx)
+        y = torch.zeros_like(recv)
+        y[:rows] = recv[:rows]
+        out, _, _ = buffer.combine(y, handle)
+        np.testing.assert_array_equal(bf16_bits(out), ocombine.combine(bf16_bits(recv[:rows]), want["route_to_row"],
+                                                                       olayout.expand_weights(w.numpy(), want["row_to_route"])))
+    finally:
+        buffer.destroy()
+
+
+def test_changed_handles_and_unusual_tensors_take_the_slow_path():
+    x, w = _batch(40, 256, 2, 1)
+    idx = torch.stack([torch.randperm(8)[:2] for _ in range(40)]).cuda()
+    buffer = _buffer(num_bytes=4 << 20)
+    try:
+        recv, _, _, handle, _ = buffer.dispatch(x.cuda(), topk_idx=idx, topk_weights=w.cuda(), num_experts=8)
+        want, _, _ = buffer.combine(recv, handle)
+        # inference mode: carried out step by step, the same results
+        with torch.inference_mode():
+            again, _, _, other, _ = buffer.dispatch(x.cuda(), topk_idx=idx, topk_weights=w.cuda(), num_experts=8)
+            assert torch.equal(again, recv) and torch.equal(buffer.combine(again, handle)[0], want)
+        assert torch.equal(buffer.combine(recv, other)[0], want)
+        # a low-latency style handle: the saved weights multiply the rows
+        handle.is_low_latency, handle.source_weights = True, torch.full((handle.num_expanded_tokens,), 2.0, device="cuda")
+        assert torch.equal(buffer.combine(recv, handle)[0], (want.float() * 2).bfloat16())
+        handle.is_low_latency = False
+        with pytest.raises(ValueError, match="matching the handle"):
+            buffer.combine(recv[:-1], handle)
+        # an edit of the routing is found on the native path as well
+        handle.expert_totals.add_(0)
+        with pytest.raises(ValueError, match="Cached routing was modified: expert_totals"):
+            buffer.combine(recv, handle)
+        with pytest.raises(ValueError, match="Cached routing was modified"):
+            buffer.dispatch(x.cuda(), handle=handle)
+        other.route_to_row = other.route_to_row.clone()
+        with pytest.raises(ValueError, match="Cached routing was modified: route_to_row"):
+            buffer.combine(recv, other)
+    finally:
+        buffer.destroy()
+
+
+@pytest.mark.parametrize("wait", ["caller", "other", "never"])
+def test_memory_of_asynchronous_calls_is_not_handed_out_too_early(wait):
+    """Everything an asynchronous call used is dropped right after it, behind a kernel that keeps the communication stream
+    busy, and the allocator is asked for the same sizes at once: what the call wrote must still be right."""
+    tokens, hidden, topk, experts = 512, 1024, 4, 16
+    x, w = _batch(tokens, hidden, topk, 2)
+    ids = torch.stack([torch.randperm(experts)[:topk] for _ in range(tokens)])
+    want = olayout.layout(ids.numpy(), experts)
+    rows = olayout.expand_rows(bf16_bits(x), want["row_to_route"], topk)
+    buffer = _buffer(num_bytes=4 << 20)
+    side = torch.cuda.Stream()
+    try:
+        idx, xd = ids.cuda(), x.cuda()
+        _, _, _, handle, _ = buffer.dispatch(xd, topk_idx=idx, num_experts=experts)
+        for _ in range(8):
+            torch.cuda.synchronize()
+            with torch.cuda.stream(buffer.get_comm_stream()):
+                torch.cuda._sleep(2_000_000)
+            payload = xd.clone()
+            recv, _, _, _, event = buffer.dispatch(payload, handle=handle, async_with_compute_stream=True)
+            if wait == "never":
+                kept = recv  # waited for by hand below
+            elif wait == "caller":
+                event.current_stream_wait()
+                kept = recv.clone()
+                del recv
+            else:
+                with torch.cuda.stream(side):
+                    event.current_stream_wait()
+                    torch.cuda._sleep(1_000_000)
+                    kept = recv.clone()
+                del recv
+            del payload, event
+            noise = [torch.full((want["num_rows"], hidden), 7.0, dtype=torch.bfloat16, device="cuda") for _ in range(3)]
+            noise += [torch.full((tokens, hidden), 7.0, dtype=torch.bfloat16, device="cuda") for _ in range(3)]
+            buffer.get_comm_stream().synchronize()
+            torch.cuda.synchronize()
+            np.testing.assert_array_equal(bf16_bits(kept), rows)
+            del noise, kept
+            if wait == "never":
+                del recv
+    finally:
+        torch.cuda.synchronize()
+        buffer.destroy()
+
+
+def test_event_of_an_asynchronous_call_stands_in_for_torchs():
+    x, _ = _batch(64, 256, 2, 3)
+    idx = torch.stack([torch.randperm(8)[:2] for _ in range(64)]).cuda()
+    buffer = _buffer(num_bytes=4 << 20)
+    try:
+        recv, _, _, handle, overlap = buffer.dispatch(x.cuda(), topk_idx=idx, num_experts=8, async_with_compute_stream=True)
+        event = overlap.event.event
+        torch.cuda.Stream().wait_event(event)
+        event.wait()
+        event.synchronize()
+        assert event.query() and overlap.event._gpu_index == torch.cuda.current_device()
+        assert overlap.event._marker.stream == buffer.get_comm_stream()
+        out, _, second = buffer.combine(recv, handle, previous_event=overlap.event, async_with_compute_stream=True)
+        with second(release_handle=True):
+            pass
+        assert second.event is None and second._lease is None
+        assert torch.equal(out.float(), x.cuda().float() * 2)
+    finally:
+        buffer.destroy()
