@@ -6,6 +6,7 @@ There is no fallback: if the library is missing or a symbol is absent, loading r
 from __future__ import annotations
 
 import ctypes
+import functools
 import os
 import threading
 
@@ -50,6 +51,7 @@ SIGNATURES = {
                                       ctypes.POINTER(ctypes.c_int64), _P)),
     "dpep_megamoe_forward": (_I, (_P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I,
                                   _P, _P, _P)),
+    "dpep_megamoe_run": (_I, (_P, _P, _P)),
 }
 
 _lock = threading.Lock()
@@ -75,6 +77,7 @@ def load():
     return _lib
 
 
+@functools.lru_cache(maxsize=None)
 def host():
     """The native host path (csrc/host.cpp), a CPython extension over this library.  Raises if it is not built."""
     load()

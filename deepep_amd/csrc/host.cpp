@@ -71,7 +71,7 @@ inline PyObject* new_ref(PyObject* o)
     X(num_recv_tokens_per_expert_list) X(psum_num_recv_tokens_per_expert) X(num_unaligned_recv_tokens_per_expert)                \
     X(is_low_latency) X(route_to_row) X(weight_return_meta) X(expert_totals) X(expert_offsets) X(source_weights)                 \
     X(send_counts) X(rank) X(world_size) X(num_tokens) X(num_topk) X(hidden) X(metadata_only) X(metadata_version)                \
-    X(_buffer_token) X(_row_to_route_full) X(do_expand) X(expert_alignment)
+    X(_buffer_token) X(_row_to_route_full) X(do_expand) X(expert_alignment) X(gate_up) X(logical) X(_versions)
 struct Names {
 #define X(n) PyObject* n;
     DPEP_NAMES(X)
@@ -107,6 +107,7 @@ inline long long exact_int(PyObject* o, long long lower, long long upper, long l
 }
 inline bool is_bool(PyObject* o) { return o == Py_True || o == Py_False; }
 
+inline bool on_gpu(PyObject* o) { return THPVariable_CheckExact(o) && THPVariable_Unpack(o).is_cuda(); }
 // A plain device tensor: exactly torch.Tensor (or Parameter), strided, contiguous, on `device`, without grad.
 inline const at::Tensor* plain(PyObject* o, int device)
 {
@@ -1040,6 +1041,265 @@ PyGetSetDef exchange_getset[] = {{"failed", Exchange_get_failed, Exchange_set_fa
                                  {nullptr, nullptr, nullptr, nullptr, nullptr}};
 PyTypeObject ExchangeType = {PyVarObject_HEAD_INIT(nullptr, 0) "deepep_amd._host.Exchange", sizeof(Exchange)};
 
+// ---- the MegaMoE layer ------------------------------------------------------------------------------------------------------
+// One SymmBuffer's forward (deepep_amd.megamoe.api._run), and the FP8 casts.
+struct Mega {
+    PyObject_HEAD
+    std::shared_ptr<EventPool> pool;
+    PyObject* lock;      // the buffer's lock (a threading.Lock)
+    PyObject *logical1, *logical2, *shared1, *shared2;  // (experts, N, K) that l1 / l2 / shared l1 / shared l2 must have
+    void* workspace;     // of batches of `batch` rows; nullptr before the first
+    int batch;
+    int device, experts, first_expert, local, topk, hidden, inter, shared, capacity, padded;
+    Stream last;
+    bool has_last, closed;
+    hipEvent_t order;
+};
+extern PyTypeObject MegaType;
+PyTypeObject* g_pair_type;  // deepep_amd.megamoe.api._PreparedPair
+
+// The tensors of an unmodified prepared pair of the right kind and size.
+bool read_pair(PyObject* pair, bool gate_up, PyObject* logical, int device, const at::Tensor** w, const at::Tensor** s)
+{
+    if (Py_TYPE(pair) != g_pair_type || PyTuple_GET_SIZE(pair) != 2) return false;
+    *w = plain(PyTuple_GET_ITEM(pair, 0), device);
+    *s = plain(PyTuple_GET_ITEM(pair, 1), device);
+    if (*w == nullptr || *s == nullptr || (*w)->scalar_type() != at::kByte || (*s)->scalar_type() != at::kByte || !aligned16(**w) || !aligned16(**s) ||
+        (*w)->is_inference() || (*s)->is_inference())
+        return false;
+    Ref kind(PyObject_GetAttr(pair, N.gate_up)), sizes(PyObject_GetAttr(pair, N.logical)), versions(PyObject_GetAttr(pair, N._versions));
+    if (!kind || !sizes || !versions || PyObject_RichCompareBool(sizes.p, logical, Py_EQ) != 1 || !PyTuple_CheckExact(versions.p) ||
+        PyTuple_GET_SIZE(versions.p) != 2) {
+        PyErr_Clear();
+        return false;
+    }
+    return kind.p == (gate_up ? Py_True : Py_False) && exact_int(PyTuple_GET_ITEM(versions.p, 0), 0, 0xffffffffLL) == version_of(**w) &&
+           exact_int(PyTuple_GET_ITEM(versions.p, 1), 0, 0xffffffffLL) == version_of(**s);
+}
+
+inline bool overlap(const at::Tensor& a, const at::Tensor& b)
+{
+    const char *x = static_cast<const char*>(a.data_ptr()), *y = static_cast<const char*>(b.data_ptr());
+    return x < y + b.nbytes() && y < x + a.nbytes();
+}
+
+// forward(x, scales, topk_idx, topk_weights, l1, l2, shared_l1, shared_l2, out, staged) -> (y, counts), or None (see above).
+// scales None: x is BF16.  out None: allocated here.  staged: x / scales / topk_idx / topk_weights are the buffer's own input
+// tensors, of which the first rows (as many as out has) are meant.
+PyObject* Mega_forward(PyObject* self, PyObject* const* a, Py_ssize_t n)
+{
+    HANDLE_TH_ERRORS
+    Mega* m = reinterpret_cast<Mega*>(self);
+    if (n != 10) {
+        PyErr_SetString(PyExc_TypeError, "forward takes 10 arguments");
+        return nullptr;
+    }
+    const bool staged = a[9] == Py_True;
+    if (m->closed || m->workspace == nullptr || c10::hip::current_device() != m->device || c10::InferenceMode::is_enabled()) Py_RETURN_NONE;
+    const at::Tensor *x = plain(a[0], m->device), *scales = a[1] != Py_None ? plain(a[1], m->device) : nullptr, *idx = plain(a[2], m->device),
+                     *weights = plain(a[3], m->device), *out = a[8] != Py_None ? plain(a[8], m->device) : nullptr;
+    if (x == nullptr || idx == nullptr || weights == nullptr || (a[1] != Py_None && scales == nullptr) || (a[8] != Py_None && out == nullptr) ||
+        (staged && out == nullptr) || x->dim() != 2 || idx->dim() != 2 || weights->dim() != 2)
+        Py_RETURN_NONE;
+    const int64_t rows = staged ? out->dim() == 2 ? out->size(0) : 0 : x->size(0);
+    const bool bf16 = scales == nullptr;
+    auto fits = [&](const at::Tensor& t, int64_t columns) { return t.size(1) == columns && (staged ? t.size(0) >= rows : t.size(0) == rows); };
+    if (rows != m->batch || x->size(1) != m->hidden || !fits(*x, m->hidden) || !fits(*idx, m->topk) || !fits(*weights, m->topk) ||
+        idx->scalar_type() != at::kInt || weights->scalar_type() != at::kFloat || x->scalar_type() != (bf16 ? at::kBFloat16 : at::kFloat8_e4m3fn) ||
+        !aligned16(*x))
+        Py_RETURN_NONE;
+    if (!bf16 && (scales->dim() != 2 || !fits(*scales, m->hidden / 32) ||
+                  (scales->scalar_type() != at::kByte && scales->scalar_type() != at::kFloat8_e8m0fnu)))
+        Py_RETURN_NONE;
+    const at::Tensor *w1, *s1, *w2, *s2, *sw1 = nullptr, *ss1 = nullptr, *sw2 = nullptr, *ss2 = nullptr;
+    if (!read_pair(a[4], true, m->logical1, m->device, &w1, &s1) || !read_pair(a[5], false, m->logical2, m->device, &w2, &s2)) Py_RETURN_NONE;
+    if (m->shared > 0) {
+        if (!read_pair(a[6], true, m->shared1, m->device, &sw1, &ss1) || !read_pair(a[7], false, m->shared2, m->device, &sw2, &ss2)) Py_RETURN_NONE;
+    } else if (a[6] != Py_None || a[7] != Py_None) {
+        Py_RETURN_NONE;
+    }
+    if (out != nullptr) {
+        if (out->scalar_type() != at::kBFloat16 || !has_shape(*out, rows, m->hidden) || !aligned16(*out)) Py_RETURN_NONE;
+        for (const at::Tensor* t : {x, scales, idx, weights, w1, s1, w2, s2, sw1, ss1, sw2, ss2})
+            if (t != nullptr && overlap(*out, *t)) Py_RETURN_NONE;
+    }
+    Locked held(m->lock);
+    if (!held.held) return nullptr;
+    if (m->closed || m->workspace == nullptr || rows != m->batch) Py_RETURN_NONE;
+    const Stream stream = current_stream(m->device);
+    if (m->has_last && !(m->last == stream)) {
+        if (m->order == nullptr && (m->order = m->pool->take()) == nullptr) return raise_hip("hipEventCreate", hipErrorUnknown);
+        hipError_t err = hipEventRecord(m->order, m->last.raw);
+        if (err == hipSuccess) err = hipStreamWaitEvent(stream.raw, m->order, 0);
+        if (err != hipSuccess) return raise_hip("ordering two streams", err);
+    }
+    m->last = stream;
+    m->has_last = true;
+    at::Tensor y = out != nullptr ? *out : allocate({rows, m->hidden}, at::kBFloat16, m->device);
+    at::Tensor counts = allocate({m->local}, at::kInt, m->device), scratch;
+    dpep_megamoe_call c = {};
+    if (bf16) {
+        scratch = allocate({rows * m->padded + rows * (m->padded / 32)}, at::kByte, m->device);
+        c.x_bf16 = x->data_ptr();
+        c.x_codes_scratch = static_cast<uint8_t*>(scratch.data_ptr());
+        c.x_scales_scratch = c.x_codes_scratch + rows * m->padded;
+    } else {
+        c.x_codes = x->data_ptr();
+        c.x_scales = static_cast<const uint8_t*>(scales->data_ptr());
+    }
+    auto bytes = [](const at::Tensor* t) { return t != nullptr ? static_cast<const uint8_t*>(t->data_ptr()) : nullptr; };
+    c.topk_idx = static_cast<const int32_t*>(idx->data_ptr());
+    c.topk_weights = static_cast<const float*>(weights->data_ptr());
+    c.w1 = bytes(w1);
+    c.s1 = bytes(s1);
+    c.w2 = bytes(w2);
+    c.s2 = bytes(s2);
+    c.shared_w1 = bytes(sw1);
+    c.shared_s1 = bytes(ss1);
+    c.shared_w2 = bytes(sw2);
+    c.shared_s2 = bytes(ss2);
+    c.y = y.data_ptr();
+    c.expert_token_nums = static_cast<int32_t*>(counts.data_ptr());
+    c.num_shared = m->shared;
+    c.num_tokens = static_cast<int32_t>(rows);
+    c.hidden = m->hidden;
+    c.intermediate = m->inter;
+    c.num_topk = m->topk;
+    c.num_experts = m->experts;
+    c.expert_begin = m->first_expert;
+    c.num_local = m->local;
+    if (const int status = dpep_megamoe_run(m->workspace, &c, stream.raw)) return raise_native(status);
+    Ref first(out != nullptr ? new_ref(a[8]) : wrap(y)), second(wrap(counts));
+    return first && second ? PyTuple_Pack(2, first.p, second.p) : nullptr;
+    END_HANDLE_TH_ERRORS
+}
+PyObject* Mega_new(PyTypeObject* type, PyObject* args, PyObject*)
+{
+    PyObject* lock;
+    int device, experts, first, local, topk, hidden, inter, shared, capacity;
+    if (!PyArg_ParseTuple(args, "Oiiiiiiiii", &lock, &device, &experts, &first, &local, &topk, &hidden, &inter, &shared, &capacity)) return nullptr;
+    Mega* m = reinterpret_cast<Mega*>(type->tp_alloc(type, 0));
+    if (m == nullptr) return nullptr;
+    new (&m->pool) std::shared_ptr<EventPool>(std::make_shared<EventPool>());
+    m->lock = new_ref(lock);
+    m->device = device;
+    m->experts = experts;
+    m->first_expert = first;
+    m->local = local;
+    m->topk = topk;
+    m->hidden = hidden;
+    m->inter = inter;
+    m->shared = shared;
+    m->capacity = capacity;
+    m->padded = dpep_megamoe_padded_dim(hidden);
+    m->logical1 = Py_BuildValue("(iii)", local, 2 * inter, hidden);
+    m->logical2 = Py_BuildValue("(iii)", local, hidden, inter);
+    m->shared1 = Py_BuildValue("(iii)", shared, 2 * inter, hidden);
+    m->shared2 = Py_BuildValue("(iii)", shared, hidden, inter);
+    return reinterpret_cast<PyObject*>(m);
+}
+void Mega_dealloc(PyObject* o)
+{
+    Mega* m = reinterpret_cast<Mega*>(o);
+    if (m->order != nullptr) m->pool->give_back(m->order);
+    for (PyObject* p : {m->lock, m->logical1, m->logical2, m->shared1, m->shared2}) Py_XDECREF(p);
+    m->pool.~shared_ptr();
+    Py_TYPE(o)->tp_free(o);
+}
+// use(workspace handle, batch): the workspace of the batches to come; use(0, 0): none.
+PyObject* Mega_use(PyObject* o, PyObject* args)
+{
+    Mega* m = reinterpret_cast<Mega*>(o);
+    PyObject* workspace;
+    int batch;
+    if (!PyArg_ParseTuple(args, "Oi", &workspace, &batch)) return nullptr;
+    void* ws = PyLong_AsVoidPtr(workspace);
+    if (ws == nullptr && PyErr_Occurred()) return nullptr;
+    m->workspace = ws;
+    m->batch = batch;
+    Py_RETURN_NONE;
+}
+PyObject* Mega_close(PyObject* o, PyObject*)
+{
+    reinterpret_cast<Mega*>(o)->closed = true;
+    Py_RETURN_NONE;
+}
+PyObject* Mega_get_last(PyObject* o, void*)
+{
+    Mega* m = reinterpret_cast<Mega*>(o);
+    if (!m->has_last) Py_RETURN_NONE;
+    return stream_object(m->last, m->device);
+}
+int Mega_set_last(PyObject* o, PyObject* v, void*)
+{
+    Mega* m = reinterpret_cast<Mega*>(o);
+    m->has_last = v != nullptr && v != Py_None;
+    return !m->has_last || stream_from(v, &m->last) ? 0 : -1;
+}
+PyMethodDef mega_methods[] = {
+    {"forward", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(Mega_forward)), METH_FASTCALL, nullptr},
+    {"use", Mega_use, METH_VARARGS, nullptr},
+    {"close", Mega_close, METH_NOARGS, nullptr},
+    {nullptr, nullptr, 0, nullptr}};
+PyGetSetDef mega_getset[] = {{"last_stream", Mega_get_last, Mega_set_last, nullptr, nullptr}, {nullptr, nullptr, nullptr, nullptr, nullptr}};
+PyTypeObject MegaType = {PyVarObject_HEAD_INIT(nullptr, 0) "deepep_amd._host.Mega", sizeof(Mega)};
+
+// ---- FP8 casts -----------------------------------------------------------------------------------------------------------------
+// cast_to_fp8(x) -> (codes, scales): a plain BF16 [T,H] on the current GPU, H a positive multiple of 16; else None.
+PyObject* cast_to_fp8(PyObject*, PyObject* o)
+{
+    HANDLE_TH_ERRORS
+    if (!on_gpu(o)) Py_RETURN_NONE;
+    const int device = c10::hip::current_device();
+    const at::Tensor* x = plain(o, device);
+    if (x == nullptr || x->scalar_type() != at::kBFloat16 || x->dim() != 2 || x->size(1) == 0 || x->size(1) % 16 != 0 || x->size(0) > 0x7fffffff ||
+        x->size(1) > 0x7fffffff || !aligned16(*x) || c10::InferenceMode::is_enabled())
+        Py_RETURN_NONE;
+    const int64_t tokens = x->size(0), hidden = x->size(1);
+    at::Tensor codes = allocate({tokens, hidden}, at::kFloat8_e4m3fn, device), scales = allocate({tokens, (hidden + 127) / 128}, at::kFloat, device);
+    if (const int status = dpep_cast_to_fp8(x->data_ptr(), static_cast<int>(tokens), static_cast<int>(hidden), codes.data_ptr(),
+                                            static_cast<float*>(scales.data_ptr()), current_stream(device).raw))
+        return raise_native(status);
+    Ref first(wrap(codes)), second(wrap(scales));
+    return first && second ? PyTuple_Pack(2, first.p, second.p) : nullptr;
+    END_HANDLE_TH_ERRORS
+}
+// cast_back(codes, scales) -> BF16 [T,H]: plain e4m3fn codes and FP32 [T, ceil(H/128)] or packed int32 [T, ceil(H/128)/4] scales.
+PyObject* cast_back(PyObject*, PyObject* const* a, Py_ssize_t n)
+{
+    HANDLE_TH_ERRORS
+    if (n != 2) {
+        PyErr_SetString(PyExc_TypeError, "cast_back takes 2 arguments");
+        return nullptr;
+    }
+    if (!on_gpu(a[0])) Py_RETURN_NONE;
+    const int device = c10::hip::current_device();
+    const at::Tensor *codes = plain(a[0], device), *scales = plain(a[1], device);
+    if (codes == nullptr || scales == nullptr || codes->scalar_type() != at::kFloat8_e4m3fn || codes->dim() != 2 || codes->numel() == 0 ||
+        codes->size(1) % 16 != 0 || codes->size(0) > 0x7fffffff || codes->size(1) > 0x7fffffff || !aligned16(*codes) || c10::InferenceMode::is_enabled())
+        Py_RETURN_NONE;
+    const int64_t tokens = codes->size(0), hidden = codes->size(1), blocks = (hidden + 127) / 128;
+    const bool packed = scales->scalar_type() == at::kInt;
+    if (packed ? blocks % 4 != 0 || !has_shape(*scales, tokens, blocks / 4) : scales->scalar_type() != at::kFloat || !has_shape(*scales, tokens, blocks))
+        Py_RETURN_NONE;
+    at::Tensor out = allocate({tokens, hidden}, at::kBFloat16, device);
+    if (const int status = dpep_cast_back(codes->data_ptr(), scales->data_ptr(), packed, static_cast<int>(tokens), static_cast<int>(hidden),
+                                          out.data_ptr(), current_stream(device).raw))
+        return raise_native(status);
+    return wrap(out);
+    END_HANDLE_TH_ERRORS
+}
+
+// configure_mega(_PreparedPair, NativeError)
+PyObject* configure_mega(PyObject*, PyObject* args)
+{
+    PyObject *pair, *error;
+    if (!PyArg_ParseTuple(args, "O!O", &PyType_Type, &pair, &error)) return nullptr;
+    g_pair_type = reinterpret_cast<PyTypeObject*>(new_ref(pair));
+    g_native_error = new_ref(error);
+    Py_RETURN_NONE;
+}
+
 // configure(EPHandle, template dict, EventOverlap, EventHandle, NativeError): the Python classes whose objects are made here.
 PyObject* configure(PyObject*, PyObject* args)
 {
@@ -1055,7 +1315,11 @@ PyObject* configure(PyObject*, PyObject* args)
     Py_RETURN_NONE;
 }
 
-PyMethodDef module_methods[] = {{"configure", configure, METH_VARARGS, nullptr}, {nullptr, nullptr, 0, nullptr}};
+PyMethodDef module_methods[] = {{"configure", configure, METH_VARARGS, nullptr},
+                                {"configure_mega", configure_mega, METH_VARARGS, nullptr},
+                                {"cast_to_fp8", cast_to_fp8, METH_O, nullptr},
+                                {"cast_back", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(cast_back)), METH_FASTCALL, nullptr},
+                                {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "_host", "Native host path of deepep_amd (see csrc/host.cpp).", -1, module_methods};
 
 }  // namespace
@@ -1078,12 +1342,18 @@ PyMODINIT_FUNC PyInit__host()
     ExchangeType.tp_methods = exchange_methods;
     ExchangeType.tp_getset = exchange_getset;
     ExchangeType.tp_new = Exchange_new;
-    for (PyTypeObject* t : {&LeaseType, &MarkerType, &PlanType, &ExchangeType}) {
+    MegaType.tp_dealloc = Mega_dealloc;
+    MegaType.tp_methods = mega_methods;
+    MegaType.tp_getset = mega_getset;
+    MegaType.tp_new = Mega_new;
+    if ((g_native_error = new_ref(PyExc_RuntimeError)) == nullptr) return nullptr;  // (until the Python layer names its own)
+    for (PyTypeObject* t : {&LeaseType, &MarkerType, &PlanType, &ExchangeType, &MegaType}) {
         t->tp_flags = Py_TPFLAGS_DEFAULT;
         if (PyType_Ready(t) < 0) return nullptr;
     }
     PyObject* m = PyModule_Create(&module_def);
     if (m == nullptr) return nullptr;
     if (PyModule_AddObject(m, "Exchange", new_ref(reinterpret_cast<PyObject*>(&ExchangeType))) < 0) return nullptr;
+    if (PyModule_AddObject(m, "Mega", new_ref(reinterpret_cast<PyObject*>(&MegaType))) < 0) return nullptr;
     return m;
 }

@@ -24,6 +24,7 @@
 #include <mutex>
 
 #include "common.h"
+#include "mx.h"
 
 namespace dpep {
 namespace {
@@ -37,6 +38,7 @@ constexpr int kLargeBlockHistInts = kLargeHistInts / kWaves + DPEP_MAX_LOCAL_EXP
 constexpr int kMinChunk = 256;        // routes per wavefront, lower bound (multiple of 64)
 constexpr int kPrefetch = 8;          // 64-route steps whose ids are fetched at once
 constexpr int kKeep = 16;             // 64-route steps of a chunk that the one-launch kernel holds in registers
+constexpr int kMegaExperts = 128;     // local experts of a MegaMoE forward, at most
 constexpr int kColumnBatch = 16;      // histogram loads in flight per thread
 static_assert(kSyncTaggedWords >= static_cast<size_t>(kBlockHistInts), "the tagged histograms need a word per (workgroup, expert)");
 
@@ -80,17 +82,19 @@ __device__ __forceinline__ void fetch_experts(int (&experts)[kSteps], const IdxT
 // LDS of one workgroup.  running[w][e]: wave w's histogram, later its next free row of expert e; match[w][e]: bit
 // per lane of wave w whose route in the current step goes to expert e (all zero between steps); totals[e]: rows
 // of expert e.
+template <int kMaxLocal>
 struct LayoutLds {
-    int totals[DPEP_MAX_LOCAL_EXPERTS];
-    int running[kWaves][DPEP_MAX_LOCAL_EXPERTS];
-    unsigned long long match[kWaves][DPEP_MAX_LOCAL_EXPERTS];
+    int totals[kMaxLocal];
+    int running[kWaves][kMaxLocal];
+    unsigned long long match[kWaves][kMaxLocal];
     int partial[kThreads * 2];
     int wave_sums[kWaves];
     int timed_out;  // one-launch kernel: some thread's wait for another workgroup's histogram ran out
     unsigned long long tag;  // one-launch kernel: the tag of this launch, read once per workgroup
 };
 
-__device__ __forceinline__ void clear_wave_lds(LayoutLds& lds, int num_local)
+template <typename Lds>
+__device__ __forceinline__ void clear_wave_lds(Lds& lds, int num_local)
 {
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     for (int e = lane; e < num_local; e += kWave) {
@@ -106,7 +110,8 @@ __device__ __forceinline__ void count_step(int e, int* __restrict__ mine)
 }
 
 // The waves' histograms (lds.running) out to wave_hist, and their sum to block_hist.  Called by all threads.
-__device__ __forceinline__ void publish_histograms(LayoutLds& lds, int num_local, int num_chunks,
+template <typename Lds>
+__device__ __forceinline__ void publish_histograms(Lds& lds, int num_local, int num_chunks,
                                                    int* __restrict__ wave_hist, int* __restrict__ block_hist)
 {
     __syncthreads();
@@ -156,7 +161,7 @@ __global__ __launch_bounds__(kThreads) void layout_count_kernel(const IdxT* __re
                                                                 int chunk, int num_chunks, int* __restrict__ wave_hist,
                                                                 int* __restrict__ block_hist, IdxT* __restrict__ idx_copy)
 {
-    __shared__ LayoutLds lds;
+    __shared__ LayoutLds<DPEP_MAX_LOCAL_EXPERTS> lds;
     const int wave = threadIdx.x >> 6;
     const int g = blockIdx.x * kWaves + wave;
     const int begin = g < num_chunks ? g * chunk : 0;
@@ -209,7 +214,8 @@ __device__ __forceinline__ unsigned long long load_word(const unsigned long long
 
 // The workgroup's histogram (sum of its waves') out to its row of `tagged`.  Called by all threads, after a workgroup
 // barrier behind the counting.
-__device__ __forceinline__ void publish_tagged(LayoutLds& lds, int num_local, unsigned long long* __restrict__ tagged,
+template <typename Lds>
+__device__ __forceinline__ void publish_tagged(Lds& lds, int num_local, unsigned long long* __restrict__ tagged,
                                                unsigned long long tag)
 {
     for (int e = threadIdx.x; e < num_local; e += kThreads) {
@@ -278,8 +284,8 @@ struct TaggedSource {
 // num_blocks = workgroups that own chunks.  kTagged: the one-launch kernel (the workgroup's own wave histograms are
 // still in lds.running, the others' arrive as tagged words from `source`); else the count launch left everything in
 // wave_hist / block_hist.  Returns false if the wait for the tagged words ran out: every count is then reported as zero.
-template <bool kTagged>
-__device__ __forceinline__ bool expert_bases(LayoutLds& lds, const int* __restrict__ wave_hist,
+template <bool kTagged, typename Lds>
+__device__ __forceinline__ bool expert_bases(Lds& lds, const int* __restrict__ wave_hist,
                                              const int* __restrict__ block_hist, int num_local, int padded_local,
                                              int num_chunks, int num_blocks, int* __restrict__ counts,
                                              int* __restrict__ psum, int* __restrict__ offsets, int* __restrict__ num_rows,
@@ -287,7 +293,7 @@ __device__ __forceinline__ bool expert_bases(LayoutLds& lds, const int* __restri
                                              const TaggedSource* source = nullptr)
 {
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    const bool reporter = blockIdx.x == gridDim.x - 1;
+    const bool reporter = static_cast<int>(blockIdx.x) == num_blocks;
     // This workgroup's own rows are asked for before the column sums, so that all loads are in flight together.
     auto own_rows = [&](int e, int (&own)[kWaves]) {
 #pragma unroll
@@ -416,7 +422,7 @@ __global__ __launch_bounds__(kThreads) void layout_assign_kernel(
     int* __restrict__ route_to_row, int* __restrict__ row_to_route, SendCounts send, uint32_t* __restrict__ mailbox,
     uint32_t sequence)
 {
-    __shared__ LayoutLds lds;
+    __shared__ LayoutLds<DPEP_MAX_LOCAL_EXPERTS> lds;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int g = blockIdx.x * kWaves + wave;
     const int begin = g < num_chunks ? g * chunk : 0;
@@ -450,16 +456,25 @@ __global__ __launch_bounds__(kThreads) void layout_assign_kernel(
 // Count, exchange, assign in one launch; every wave keeps the ids of its chunk (at most kKeep steps) in registers.
 // `rows` = histogram rows to wait for (the workgroups that own chunks; one more in a test that wants the wait to run out),
 // `limit_ticks` the bound of that wait (100 MHz ticks).
-template <typename IdxT>
+// kMega: a MegaMoE forward's layout (at most 128 local experts).  Workgroups behind the reporter prepare the input rows
+// (quantise or pad them), which does not depend on the routing, and every workgroup of the layout writes a piece of the shared
+// experts' rows once it knows R: up to three launches fewer (777 tokens of 2880 BF16 columns with a shared expert: layout 8.3 +
+// quantise 4.1 + pad 3.3 + shared rows 1.9 us as launches of their own).
+template <typename IdxT, bool kMega>
 __global__ __launch_bounds__(kThreads) void layout_fused_kernel(
     const IdxT* __restrict__ idx, int n_routes, int num_experts, int expert_begin, int num_local, int padded_local,
     int chunk, int num_chunks, int* __restrict__ counts, int* __restrict__ psum, int* __restrict__ offsets,
     int* __restrict__ num_rows, int* __restrict__ route_to_row, int* __restrict__ row_to_route, IdxT* __restrict__ idx_copy,
     SendCounts send, uint32_t* __restrict__ mailbox, uint32_t sequence, unsigned long long* __restrict__ epoch,
-    unsigned long long* __restrict__ tagged, int rows, long long limit_ticks, uint32_t* __restrict__ timeouts,
-    uint32_t launch_id)
+    unsigned long long* __restrict__ tagged, int num_blocks, int rows, long long limit_ticks, uint32_t* __restrict__ timeouts,
+    uint32_t launch_id, MegaFront front)
 {
-    __shared__ LayoutLds lds;
+    __shared__ LayoutLds<kMega ? kMegaExperts : DPEP_MAX_LOCAL_EXPERTS> lds;
+    if (kMega && static_cast<int>(blockIdx.x) > num_blocks) {
+        __shared__ __attribute__((aligned(16))) uint8_t staged[kFrontThreads / 2];
+        prepare_rows(front, blockIdx.x - num_blocks - 1, staged);
+        return;
+    }
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int g = blockIdx.x * kWaves + wave;
     const int begin = g < num_chunks ? g * chunk : 0;
@@ -467,7 +482,7 @@ __global__ __launch_bounds__(kThreads) void layout_fused_kernel(
     // One thread reads the epoch for the whole workgroup (asked for together with the ids): every thread must use the
     // same tag, and the tag must be final before anything this workgroup publishes can be seen.
     unsigned long long* reporter_tag = epoch + kSyncReporterTag / sizeof(unsigned long long);
-    const bool reporter = blockIdx.x == gridDim.x - 1;
+    const bool reporter = static_cast<int>(blockIdx.x) == num_blocks;
     if (threadIdx.x == 0) {
         lds.tag = load_word(epoch) + 1ull;
         lds.timed_out = 0;
@@ -480,7 +495,7 @@ __global__ __launch_bounds__(kThreads) void layout_fused_kernel(
     for (int i = 0; i < kKeep; ++i) count_step(experts[i], lds.running[wave]);
     __syncthreads();
     const unsigned long long tag = lds.tag;
-    // (the reporter owns no chunk and publishes nothing: row gridDim.x - 1 is only ever waited for by a test that wants
+    // (the reporter owns no chunk and publishes nothing: row num_blocks is only ever waited for by a test that wants
     // the wait to run out)
     if (!reporter) publish_tagged(lds, num_local, tagged, tag);
     // The reporter gives up first (the others wait twice as long): a launch that the reporter passes as valid is then
@@ -489,8 +504,8 @@ __global__ __launch_bounds__(kThreads) void layout_fused_kernel(
     // on the consumers' side: such a workgroup marks its routes as having no row, and the kernels that read
     // row_to_route clamp what they find there.
     const TaggedSource source = {tagged, tag, rows, reporter ? limit_ticks : 2 * limit_ticks, timeouts, launch_id};
-    const bool in_time = expert_bases<true>(lds, nullptr, nullptr, num_local, padded_local, num_chunks, gridDim.x - 1, counts,
-                                            psum, offsets, num_rows, send, mailbox, sequence, &source);
+    const bool in_time = expert_bases<true>(lds, nullptr, nullptr, num_local, padded_local, num_chunks, num_blocks, counts, psum,
+                                            offsets, num_rows, send, mailbox, sequence, &source);
     // (asked for here, needed only at the very end: the load travels while the routes are assigned)
     unsigned long long reporter_seen = threadIdx.x == 0 && !reporter ? load_word(reporter_tag) : 0ull;
     if (in_time) {
@@ -504,6 +519,9 @@ __global__ __launch_bounds__(kThreads) void layout_fused_kernel(
         // (and the counts above are all zero).
         for (int route = begin + lane; route < end; route += kWave) route_to_row[route] = -1;
     }
+    if (kMega && front.num_shared > 0)  // (R = 0 where the exchange ran out of time)
+        shared_rows(front, lds.wave_sums[0] + lds.wave_sums[1] + lds.wave_sums[2] + lds.wave_sums[3], num_local, offsets, row_to_route,
+                    blockIdx.x * kThreads + threadIdx.x, (num_blocks + 1) * kThreads);
     if (threadIdx.x == 0) {
         // The epoch may only move once the reporter has read it (a reporter that read the raised epoch would wait for
         // words nobody publishes).  Tags only grow, so any value from this launch's tag on means that it has; the wait
@@ -522,6 +540,17 @@ __global__ __launch_bounds__(kThreads) void layout_fused_kernel(
         }
         __hip_atomic_fetch_max(epoch, tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
+}
+
+// The same preparation behind a layout that took two launches.
+__global__ __launch_bounds__(kFrontThreads) void mega_front_kernel(MegaFront front, const int* __restrict__ num_rows, int num_local,
+                                                                   int* __restrict__ offsets, int* __restrict__ row_to_route)
+{
+    __shared__ __attribute__((aligned(16))) uint8_t staged[kFrontThreads / 2];
+    const unsigned blocks = (front.units + kFrontThreads - 1) / kFrontThreads;
+    if (blockIdx.x < blocks) prepare_rows(front, blockIdx.x, staged);
+    else shared_rows(front, num_rows[0], num_local, offsets, row_to_route, (blockIdx.x - blocks) * kFrontThreads + threadIdx.x,
+                     (gridDim.x - blocks) * kFrontThreads);
 }
 
 int padded_experts(int num_local)
@@ -584,7 +613,7 @@ template <typename IdxT>
 int launch_layout(void* ws, const IdxT* idx, int num_tokens, int num_topk, int num_experts, int expert_begin,
                   int num_local, int32_t* counts, int32_t* psum, int32_t* offsets, int32_t* route_to_row,
                   int32_t* row_to_route, int32_t* num_rows, IdxT* idx_copy, const SendCounts& send, bool report_to_host,
-                  hipStream_t stream)
+                  const MegaFront* front, hipStream_t stream)
 {
     Workspace* w = as_workspace(ws);
     DPEP_REQUIRE(w != nullptr, "layout: not a live workspace");
@@ -625,27 +654,40 @@ int launch_layout(void* ws, const IdxT* idx, int num_tokens, int num_topk, int n
     uint32_t* mailbox = report_to_host ? w->mailbox_device : nullptr;
     if (one_launch) {
         char* sync = static_cast<char*>(w->sync);
-        hipLaunchKernelGGL(layout_fused_kernel<IdxT>, dim3(blocks + 1), dim3(kThreads), 0, stream, idx, n_routes, num_experts,
-                           expert_begin, num_local, padded, chunk, num_chunks, counts, psum, offsets, num_rows, route_to_row,
-                           row_to_route, idx_copy, send, mailbox, w->sequence, reinterpret_cast<unsigned long long*>(sync),
-                           reinterpret_cast<unsigned long long*>(sync + kSyncTagged), blocks + w->exchange_extra_rows,
-                           w->exchange_ticks, w->mailbox_device + kMailboxTimeout, w->layout_launches);
+        auto launch = [&](auto kernel, unsigned more, const MegaFront& f) {
+            hipLaunchKernelGGL(kernel, dim3(blocks + 1 + more), dim3(kThreads), 0, stream, idx, n_routes, num_experts, expert_begin,
+                               num_local, padded, chunk, num_chunks, counts, psum, offsets, num_rows, route_to_row, row_to_route,
+                               idx_copy, send, mailbox, w->sequence, reinterpret_cast<unsigned long long*>(sync),
+                               reinterpret_cast<unsigned long long*>(sync + kSyncTagged), blocks, blocks + w->exchange_extra_rows,
+                               w->exchange_ticks, w->mailbox_device + kMailboxTimeout, w->layout_launches, f);
+        };
+        if (front != nullptr) launch(layout_fused_kernel<IdxT, true>, front_blocks(*front), *front);
+        else launch(layout_fused_kernel<IdxT, false>, 0u, MegaFront{});
         return launch_status("layout_fused");
     }
-    return enqueue_count_and_assign<IdxT>(idx, n_routes, num_experts, expert_begin, num_local, padded, chunk, num_chunks, wave_hist,
-                                          block_hist, counts, psum, offsets, num_rows, route_to_row, row_to_route, idx_copy, send,
-                                          mailbox, w->sequence, stream);
+    if (int rc = enqueue_count_and_assign<IdxT>(idx, n_routes, num_experts, expert_begin, num_local, padded, chunk, num_chunks,
+                                                wave_hist, block_hist, counts, psum, offsets, num_rows, route_to_row, row_to_route,
+                                                idx_copy, send, mailbox, w->sequence, stream))
+        return rc;
+    if (front != nullptr && (front->units > 0 || front->num_shared > 0)) {
+        const unsigned rows_blocks = (static_cast<unsigned>(front->num_shared) * front->num_tokens + kFrontThreads - 1) / kFrontThreads;
+        hipLaunchKernelGGL(mega_front_kernel, dim3(front_blocks(*front) + rows_blocks), dim3(kFrontThreads), 0, stream, *front, num_rows,
+                           num_local, offsets, row_to_route);
+        return launch_status("mega_front");
+    }
+    return DPEP_OK;
 }
 
 }  // namespace
 
-// Shared with the MegaMoE forward, which routes on int32 ids.
+// Shared with the MegaMoE forward, which routes on int32 ids; front: what else is prepared in front of its GEMMs.
 int layout_i32(void* ws, const int32_t* idx, int num_tokens, int num_topk, int num_experts, int expert_begin,
                int num_local, int32_t* counts, int32_t* psum, int32_t* offsets, int32_t* route_to_row,
-               int32_t* row_to_route, int32_t* num_rows, hipStream_t stream)
+               int32_t* row_to_route, int32_t* num_rows, const MegaFront& front, hipStream_t stream)
 {
+    DPEP_REQUIRE(num_local <= kMegaExperts, "layout: %d local experts, at most %d", num_local, kMegaExperts);
     return launch_layout<int32_t>(ws, idx, num_tokens, num_topk, num_experts, expert_begin, num_local, counts, psum,
-                                  offsets, route_to_row, row_to_route, num_rows, nullptr, SendCounts{}, /*report_to_host=*/false, stream);
+                                  offsets, route_to_row, row_to_route, num_rows, nullptr, SendCounts{}, /*report_to_host=*/false, &front, stream);
 }
 
 // The layout of a fresh dispatch (dpep_dispatch_fresh).
@@ -653,7 +695,7 @@ int layout_of_fresh(void* ws, const dpep_fresh_dispatch& c, hipStream_t stream)
 {
     return launch_layout<int64_t>(ws, c.topk_idx, c.num_tokens, c.num_topk, c.num_experts, c.expert_begin, c.num_local, c.counts,
                                   c.psum, c.offsets, c.route_to_row, c.row_to_route, c.num_rows, c.topk_idx_copy,
-                                  SendCounts{c.send_counts, c.expert_begin, c.num_experts}, c.report_to_host != 0, stream);
+                                  SendCounts{c.send_counts, c.expert_begin, c.num_experts}, c.report_to_host != 0, nullptr, stream);
 }
 
 }  // namespace dpep
@@ -710,7 +752,7 @@ int dpep_layout(void* ws, const int64_t* topk_idx, int num_tokens, int num_topk,
 {
     return dpep::launch_layout<int64_t>(ws, topk_idx, num_tokens, num_topk, num_experts, expert_begin, num_local,
                                         counts, psum, offsets, route_to_row, row_to_route, num_rows, nullptr, dpep::SendCounts{},
-                                        /*report_to_host=*/true, static_cast<hipStream_t>(stream));
+                                        /*report_to_host=*/true, nullptr, static_cast<hipStream_t>(stream));
 }
 
 int dpep_layout_static(const int64_t* topk_idx, int num_tokens, int num_topk, int num_experts, int expert_begin,

@@ -17,6 +17,7 @@
 
 #include "common.h"
 #include "gemm_schedule.h"
+#include "mx.h"
 
 #pragma clang fp contract(off)
 
@@ -24,7 +25,7 @@ namespace dpep {
 
 int layout_i32(void* ws, const int32_t* idx, int num_tokens, int num_topk, int num_experts, int expert_begin,
                int num_local, int32_t* counts, int32_t* psum, int32_t* offsets, int32_t* route_to_row,
-               int32_t* row_to_route, int32_t* num_rows, hipStream_t stream);
+               int32_t* row_to_route, int32_t* num_rows, const MegaFront& front, hipStream_t stream);
 int combine_routes(const void* y, const float* route_weights, const int32_t* route_to_row, int num_tokens, int num_topk,
                    int num_rows_hint, int hidden, void* out, const int32_t* shared_first_row, int num_shared,
                    const int32_t* fill_state, int leave_unserved, hipStream_t stream);
@@ -50,27 +51,6 @@ __device__ __forceinline__ void static_for(F&& f)
 // =====================================================================================================
 // MXFP8 activation quantiser (block 32 along the row)
 // =====================================================================================================
-// e8m0 byte of a block with maximum magnitude amax: biased_exponent(max(amax, 2^-119)) - 8.
-__device__ __forceinline__ int mx_scale_byte(float amax)
-{
-    const float floored = fmaxf(amax, 0x1p-119f);
-    return static_cast<int>(__float_as_uint(floored) >> 23) - 8;
-}
-
-// v * 2^(127 - byte), magnitude clamped to 448, rounded to e4m3fn (nearest even).
-__device__ __forceinline__ float mx_scaled(float v, int byte)
-{
-    const float scaled = ldexpf(v, 127 - byte);
-    return fminf(fmaxf(scaled, -448.0f), 448.0f);
-}
-
-__device__ __forceinline__ uint32_t pack4_e4m3(float a, float b, float c, float d)
-{
-    int packed = __builtin_amdgcn_cvt_pk_fp8_f32(a, b, 0, false);
-    packed = __builtin_amdgcn_cvt_pk_fp8_f32(c, d, packed, true);
-    return static_cast<uint32_t>(packed);
-}
-
 // One lane owns 16 consecutive BF16 values (32 bytes in, one 16-byte vector of codes out, consecutive lanes writing
 // consecutive vectors); two adjacent lanes own one 32-element block.  The workgroup's 128 scale bytes are staged in LDS
 // and leave as eight 16-byte stores instead of one byte-wide store per block, which turned every scale row into
@@ -92,25 +72,9 @@ __global__ __launch_bounds__(kMxThreads) void mx_quant_kernel(const u32x4* __res
         raw[0] = load16_nt(x + 2 * u);
         raw[1] = load16_nt(x + 2 * u + 1);
     }
-    float v[16];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        v[2 * i] = bf16_to_f32(raw[i >> 2][i & 3] & 0xffffu);
-        v[2 * i + 1] = bf16_to_f32(raw[i >> 2][i & 3] >> 16);
-    }
-    float amax = 0.0f;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) amax = fmaxf(amax, fabsf(v[i]));
-    amax = fmaxf(amax, __shfl_xor(amax, 1));
-    const int byte = mx_scale_byte(amax);
-    if (live) {
-        u32x4 out;
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-            out[i] = pack4_e4m3(mx_scaled(v[4 * i], byte), mx_scaled(v[4 * i + 1], byte), mx_scaled(v[4 * i + 2], byte),
-                                mx_scaled(v[4 * i + 3], byte));
-        store16_nt(codes + u, out);
-    }
+    int byte;
+    const u32x4 out = mx_quantize16(raw[0], raw[1], byte);
+    if (live) store16_nt(codes + u, out);
     if ((threadIdx.x & 1) == 0) staged[threadIdx.x >> 1] = static_cast<uint8_t>(byte);
     __syncthreads();
     // blocks (= scale bytes) of this workgroup: [first, first + 128) clipped to the end
@@ -194,29 +158,6 @@ __global__ __launch_bounds__(256) void prepare_weights_kernel(const uint8_t* __r
         }
         s_out[id * 2] = lo;
         s_out[id * 2 + 1] = hi;
-    }
-}
-
-// Rows [T, h] of e4m3 codes with [T, h/32] scale bytes -> [T, hp] and [T, hp/32]: zero codes and the scale byte of
-// 1.0 behind column h.  One thread per 16 output bytes (codes), then per scale byte.
-__global__ __launch_bounds__(256) void pad_activations_kernel(const uint8_t* __restrict__ codes,
-                                                              const uint8_t* __restrict__ scales, int h, int hp,
-                                                              uint8_t* __restrict__ codes_out,
-                                                              uint8_t* __restrict__ scales_out, long long code_units,
-                                                              long long scale_bytes)
-{
-    const long long id = static_cast<long long>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (id < code_units) {
-        const long long row = id / (hp / 16);
-        const int unit = static_cast<int>(id % (hp / 16));
-        u32x4 v = {0u, 0u, 0u, 0u};
-        if (unit * 16 < h) v = *reinterpret_cast<const u32x4*>(codes + row * h + unit * 16);
-        reinterpret_cast<u32x4*>(codes_out)[id] = v;
-    }
-    if (id < scale_bytes) {
-        const long long row = id / (hp / 32);
-        const int block = static_cast<int>(id % (hp / 32));
-        scales_out[id] = block < h / 32 ? scales[row * (h / 32) + block] : static_cast<uint8_t>(127);
     }
 }
 
@@ -748,7 +689,7 @@ __global__ __launch_bounds__(kGemmThreads, 1) void grouped_gemm_kernel(GemmParam
                     u32x4 codes;
 #pragma unroll
                     for (int t = 0; t < 4; ++t)
-                        codes[t] = pack4_e4m3(mx_scaled(v[4 * t], byte), mx_scaled(v[4 * t + 1], byte),
+                        codes[t] = mx_pack4(mx_scaled(v[4 * t], byte), mx_scaled(v[4 * t + 1], byte),
                                               mx_scaled(v[4 * t + 2], byte), mx_scaled(v[4 * t + 3], byte));
                     if (r < tile_rows) {
                         *reinterpret_cast<u32x4*>(p.act_codes + (out_row0 + r) * act_width + act_col + half * 16) = codes;
@@ -1282,7 +1223,7 @@ __global__ __launch_bounds__(kGemmThreads, ColCfg<RT>::kWorkgroupsPerCu) void gr
                 uint32_t code[4];
 #pragma unroll
                 for (int q = 0; q < 4; ++q)
-                    code[q] = pack4_e4m3(mx_scaled(v[4 * q], byte), mx_scaled(v[4 * q + 1], byte), mx_scaled(v[4 * q + 2], byte),
+                    code[q] = mx_pack4(mx_scaled(v[4 * q], byte), mx_scaled(v[4 * q + 1], byte), mx_scaled(v[4 * q + 2], byte),
                                          mx_scaled(v[4 * q + 3], byte));
                 uint32_t first[2], second[2];
                 swap_halves(code[0], code[2], first);
@@ -1444,20 +1385,6 @@ __global__ __launch_bounds__(kGemmThreads, ColCfg<RT>::kWorkgroupsPerCu) void gr
     }
     // Nothing may still be in flight into this workgroup's LDS or registers when it retires.
     wait_copies_then_barrier<0>();
-}
-
-// Shared experts take every token: their rows follow the routed ones, expert-major, token order.
-// offsets[num_routed + 1 + s] = R + (s + 1) * B and row_to_route[R + s * B + t] = t * topk (so that the gather's
-// route / topk is t), with R read from the device.
-__global__ __launch_bounds__(256) void shared_rows_kernel(const int* __restrict__ num_rows, int num_tokens, int num_topk,
-                                                          int num_routed, int num_shared, int* __restrict__ offsets,
-                                                          int* __restrict__ row_to_route)
-{
-    const int first = num_rows[0];
-    const long long id = static_cast<long long>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (id < num_shared) offsets[num_routed + 1 + id] = first + static_cast<int>(id + 1) * num_tokens;
-    if (id < static_cast<long long>(num_shared) * num_tokens)
-        row_to_route[first + id] = static_cast<int>(id % num_tokens) * num_topk;
 }
 
 // What the GEMM works on for a logical dimension (hidden or intermediate): whole 256-column tiles and whole spans of
@@ -1933,9 +1860,26 @@ int dpep_megamoe_forward(void* ws, const void* x_codes, const uint8_t* x_scales,
                          int intermediate, int num_topk, int num_experts, int expert_begin, int num_local, void* y,
                          int32_t* expert_token_nums, void* stream)
 {
+    const dpep_megamoe_call call = {x_codes, x_scales, nullptr, nullptr, nullptr, topk_idx, topk_weights, w1, s1, w2, s2, shared_w1,
+                                    shared_s1, shared_w2, shared_s2, y, expert_token_nums, num_shared, num_tokens, hidden,
+                                    intermediate, num_topk, num_experts, expert_begin, num_local};
+    return dpep_megamoe_run(ws, &call, stream);
+}
+
+int dpep_megamoe_run(void* ws, const dpep_megamoe_call* call, void* stream)
+{
     using namespace dpep;
     Workspace* w = as_workspace(ws);
-    DPEP_REQUIRE(w != nullptr, "megamoe_forward: not a live workspace");
+    DPEP_REQUIRE(w != nullptr && call != nullptr, "megamoe_forward: not a live workspace, or NULL call");
+    const dpep_megamoe_call& c = *call;
+    const int num_shared = c.num_shared, num_tokens = c.num_tokens, hidden = c.hidden, intermediate = c.intermediate,
+              num_topk = c.num_topk, num_experts = c.num_experts, expert_begin = c.expert_begin, num_local = c.num_local;
+    const int32_t* topk_idx = c.topk_idx;
+    const float* topk_weights = c.topk_weights;
+    const uint8_t *w1 = c.w1, *s1 = c.s1, *w2 = c.w2, *s2 = c.s2;
+    const uint8_t *shared_w1 = c.shared_w1, *shared_s1 = c.shared_s1, *shared_w2 = c.shared_w2, *shared_s2 = c.shared_s2;
+    void* y = c.y;
+    int32_t* expert_token_nums = c.expert_token_nums;
     DPEP_REQUIRE(num_tokens >= 1 && num_topk >= 1 && num_topk <= DPEP_MAX_TOPK, "megamoe_forward: bad B=%d K=%d",
                  num_tokens, num_topk);
     DPEP_REQUIRE(hidden >= 64 && hidden % 64 == 0 && intermediate >= 128 && intermediate % 128 == 0,
@@ -1950,12 +1894,15 @@ int dpep_megamoe_forward(void* ws, const void* x_codes, const uint8_t* x_scales,
                      num_local + num_shared <= kMaxMoeExperts,
                  "megamoe_forward: %d shared experts with K=%d, L=%d (at most 8, K+S <= %d, L+S <= %d)", num_shared,
                  num_topk, num_local, DPEP_MAX_TOPK, kMaxMoeExperts);
-    DPEP_REQUIRE(x_codes && x_scales && topk_idx && topk_weights && w1 && s1 && w2 && s2 && y && expert_token_nums,
-                 "megamoe_forward: NULL buffer");
+    DPEP_REQUIRE(topk_idx && topk_weights && w1 && s1 && w2 && s2 && y && expert_token_nums, "megamoe_forward: NULL buffer");
+    DPEP_REQUIRE(c.x_bf16 == nullptr ? c.x_codes != nullptr && c.x_scales != nullptr && aligned16(c.x_codes)
+                                     : c.x_codes_scratch != nullptr && c.x_scales_scratch != nullptr && aligned16(c.x_bf16) &&
+                                           aligned16(c.x_codes_scratch) && aligned16(c.x_scales_scratch),
+                 "megamoe_forward: NULL or misaligned input rows");
     DPEP_REQUIRE(num_shared == 0 || (shared_w1 && shared_s1 && shared_w2 && shared_s2 && aligned16(shared_w1) &&
                                      aligned16(shared_w2) && aligned16(shared_s1) && aligned16(shared_s2)),
                  "megamoe_forward: shared experts need their four prepared weight buffers, 16-byte aligned");
-    DPEP_REQUIRE(aligned16(x_codes) && aligned16(w1) && aligned16(w2) && aligned16(s1) && aligned16(s2) && aligned16(y),
+    DPEP_REQUIRE(aligned16(w1) && aligned16(w2) && aligned16(s1) && aligned16(s2) && aligned16(y),
                  "megamoe_forward: misaligned buffer");
     // the GEMM's copies address activation rows with 32-bit byte offsets
     const long long max_rows = static_cast<long long>(num_tokens) * ((num_topk < num_local ? num_topk : num_local) + num_shared);
@@ -1971,27 +1918,33 @@ int dpep_megamoe_forward(void* ws, const void* x_codes, const uint8_t* x_scales,
     int32_t* num_rows = meta + 2 * num_local + num_shared + 1;    // rows of the routed experts
     int32_t* route_to_row = reinterpret_cast<int32_t*>(base + l.route_to_row);
     int32_t* row_to_route = reinterpret_cast<int32_t*>(base + l.row_to_route);
+    // Rows that are not what the GEMM works on (BF16, or sizes that are no whole tiles) are prepared by the layout's launch.
+    MegaFront front{};
+    front.num_shared = num_shared;
+    front.num_tokens = num_tokens;
+    front.num_topk = num_topk;
+    const bool from_bf16 = c.x_bf16 != nullptr;
+    const uint8_t* codes = static_cast<const uint8_t*>(c.x_codes);
+    const uint8_t* scales = c.x_scales;
+    if (from_bf16 || hp != hidden) {
+        front.bf16 = static_cast<const u32x4*>(c.x_bf16);
+        front.codes = codes;
+        front.scales = scales;
+        front.h = hidden;
+        front.hp = hp;
+        front.units = static_cast<unsigned>(static_cast<long long>(num_tokens) * (hp / 16));
+        uint8_t* const codes_out = from_bf16 ? c.x_codes_scratch : base + l.x_codes;
+        front.scales_out = from_bf16 ? c.x_scales_scratch : base + l.x_scales;
+        front.codes_out = reinterpret_cast<u32x4*>(codes_out);
+        codes = codes_out;
+        scales = front.scales_out;
+    }
     if (int rc = layout_i32(ws, topk_idx, num_tokens, num_topk, num_experts, expert_begin, num_local, expert_token_nums,
-                            psum, offsets, route_to_row, row_to_route, num_rows, s))
+                            psum, offsets, route_to_row, row_to_route, num_rows, front, s))
         return rc;
-    if (num_shared > 0) {
-        const long long shared_rows = static_cast<long long>(num_tokens) * num_shared;
-        hipLaunchKernelGGL(shared_rows_kernel, dim3(static_cast<unsigned>((shared_rows + 255) / 256)), dim3(256), 0, s,
-                           num_rows, num_tokens, num_topk, num_local, num_shared, offsets, row_to_route);
-        if (int rc = launch_status("shared_rows")) return rc;
-    }
     GemmParams g1{};
-    g1.a_codes = static_cast<const uint8_t*>(x_codes);
-    g1.a_scales = x_scales;
-    if (hp != hidden) {
-        const long long units = static_cast<long long>(num_tokens) * (hp / 16), bytes = static_cast<long long>(num_tokens) * (hp / 32);
-        hipLaunchKernelGGL(pad_activations_kernel, dim3(static_cast<unsigned>((units + 255) / 256)), dim3(256), 0, s,
-                           static_cast<const uint8_t*>(x_codes), x_scales, hidden, hp, base + l.x_codes, base + l.x_scales, units,
-                           bytes);
-        if (int rc = launch_status("pad_activations")) return rc;
-        g1.a_codes = base + l.x_codes;
-        g1.a_scales = base + l.x_scales;
-    }
+    g1.a_codes = codes;
+    g1.a_scales = scales;
     g1.row_to_route = row_to_route;
     g1.topk = num_topk;
     g1.a_rows = num_tokens;

@@ -16,12 +16,13 @@ transform_weights_for_mega_moe :311-379, mega_moe :382-413, fp8_fp4_mega_moe :52
 
 from __future__ import annotations
 
+import functools
 import threading
 import warnings
 
 import torch
 
-from .. import ops
+from .. import _lib, ops
 from .validation import check_routing
 
 SMALL_BATCH_MAX_TOKENS = 256
@@ -98,6 +99,14 @@ class _PreparedPair(tuple):
         return self[0], self[1]
 
 
+@functools.lru_cache(maxsize=None)
+def _load_host():
+    """The native host path (csrc/host.cpp), told about the prepared weights it is given."""
+    host = _lib.host()
+    host.configure_mega(_PreparedPair, _lib.NativeError)
+    return host
+
+
 class SymmBuffer:
     """Owner of the workspace and the input tensors of one rank.  One in-flight call per buffer."""
 
@@ -154,7 +163,9 @@ class SymmBuffer:
         self._workspace = None
         self._plan_bs = None
         self._closed = False
-        self._last_stream = None  # the stream the most recent call was queued on
+        self._native = _load_host().Mega(
+            self._lock, self._device.index, num_experts, group.rank() * self.num_local_experts, self.num_local_experts, num_topk, hidden,
+            intermediate_hidden, num_shared_experts, self.capacity_tokens)
         self.allocate_inputs()
 
     # -- lifetime ----------------------------------------------------------------------------------
@@ -180,12 +191,14 @@ class SymmBuffer:
             return
         # keep only the current BS's worst-case workspace
         if self._workspace is not None:
+            self._native.use(0, 0)
             self._workspace.destroy()
             self._workspace = None
         need = ops.megamoe_workspace_bytes(bs, self.num_topk, self.hidden, self.intermediate_hidden, self.num_local_experts,
                                            self.num_shared_experts)
         self._workspace = ops.Workspace(need, self._device)
         self._plan_bs = bs
+        self._native.use(self._workspace.handle.value, bs)
 
     def prepare(self, bs: int) -> "SymmBuffer":
         """Build or reuse the plan (workspace) of one batch size, outside the timed path."""
@@ -231,8 +244,10 @@ class SymmBuffer:
         with self._lock:
             if self._closed:
                 return
-            if self._last_stream is not None:
-                self._last_stream.synchronize()
+            self._native.close()
+            last_stream = self._native.last_stream
+            if last_stream is not None:
+                last_stream.synchronize()
             if self._workspace is not None:
                 self._workspace.destroy()
             self._workspace = self._plan_bs = None
@@ -304,6 +319,12 @@ def _run(x, topk_idx, topk_weights, l1_weights, l2_weights, sym_buffer, *, share
         raise RuntimeError("W4A8 timer requires DEEPEP_MEGAMOE_TIMER=ON (device timers are not built; use rocprofv3)")
     b = sym_buffer
     b._ensure_alive()
+    if cumulative_stats is None:
+        # Ordinary calls are made natively; what follows is for the ones that come back: faulty ones, whose faults are named
+        # here, the first of a batch size, and unusual tensors (see csrc/host.cpp).
+        done = b._native.forward(data, scales, topk_idx, topk_weights, l1_weights, l2_weights, shared_l1_weights, shared_l2_weights, out, False)
+        if done is not None:
+            return done
     if not isinstance(l1_weights, _PreparedPair) or not isinstance(l2_weights, _PreparedPair):
         raise ValueError(
             "MegaMoE requires prepared weights; call transform_weights_for_mega_moe on raw ND weights "
@@ -361,10 +382,10 @@ def _run(x, topk_idx, topk_weights, l1_weights, l2_weights, sym_buffer, *, share
         # The call is queued on the caller's current stream (every call is synchronous with it: the reference makes the
         # caller wait for its own stream before it returns).  Calls of one owner share its workspace, so a call that
         # arrives on another stream than the previous one waits for that stream first.
-        caller = torch.cuda.current_stream(b._device)
-        if b._last_stream is not None and b._last_stream != caller:
-            caller.wait_stream(b._last_stream)
-        b._last_stream = caller
+        caller, last_stream = torch.cuda.current_stream(b._device), b._native.last_stream
+        if last_stream is not None and last_stream != caller:
+            caller.wait_stream(last_stream)
+        b._native.last_stream = caller
         b._prepare(bs)
         if scales is None:
             data, scales = ops.mx_quant(data.contiguous())  # BF16 override: quantised here, not a BF16 GEMM
@@ -398,6 +419,12 @@ def fp8_fp4_mega_moe(y, l1_weights, l2_weights, sym_buffer, shared_l1_weights=No
     Inputs are the buffer's own x / x_sf / topk_idx / topk_weights (first y.shape[0] rows); ``x=`` is an
     optional BF16 [BS,H] override that is MX-quantised internally.  Route weights are applied after GMM2.
     """
+    if (x is None and timer is None and cumulative_local_expert_recv_stats is None and fast_math is True and recipe == (1, 1, 32)
+            and activation == "swiglu" and activation_clamp is None and isinstance(sym_buffer, SymmBuffer)):
+        b = sym_buffer
+        if b._native.forward(b.x, b.x_sf, b.topk_idx, b.topk_weights, l1_weights, l2_weights, shared_l1_weights, shared_l2_weights, y,
+                             True) is not None:
+            return
     fixed = {"recipe": (recipe, (1, 1, 32)), "activation": (activation, "swiglu"), "activation_clamp": (activation_clamp, None)}
     if fast_math is not True or any(given != only for given, only in fixed.values()):
         raise NotImplementedError("Supports recipe=(1,1,32), SwiGLU, no clamp, default math only")

@@ -6,7 +6,7 @@ from typing import Tuple
 
 import torch
 
-from . import ops
+from . import _lib, ops
 
 
 def per_token_cast_to_fp8(x: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]:
@@ -15,6 +15,9 @@ def per_token_cast_to_fp8(x: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]:
     Bit-identical to the reference's torch expression on CPU.  ``x`` is a BF16 [T, H] GPU tensor of any width: a last
     block shorter than 128 is quantised as if padded with zeros, as in the reference (the kernel takes widths that
     are multiples of 16; other widths are padded to the next one here and the codes cut back to H)."""
+    done = _lib.host().cast_to_fp8(x)  # the ordinary call, made natively
+    if done is not None:
+        return done
     if x.dim() != 2:
         raise AssertionError("x must be a 2D tensor")
     hidden = x.shape[1]
@@ -28,6 +31,9 @@ def per_token_cast_back(x_fp8: torch.Tensor, x_scales: torch.Tensor) -> torch.Te
     """bf16(fp32(q) * scale) per block of 128 columns (deep_ep/utils/math.py:64-79); an int32 scale holds the e8m0
     exponent bytes of four consecutive blocks.  Device tensors go through the HIP kernel (``dpep_cast_back``); host
     tensors are evaluated with torch, as the reference does on any device."""
+    done = _lib.host().cast_back(x_fp8, x_scales)  # the ordinary call, made natively
+    if done is not None:
+        return done
     if x_fp8.numel() == 0:
         return x_fp8.to(torch.bfloat16)
     if x_fp8.dim() != 2:
@@ -35,8 +41,6 @@ def per_token_cast_back(x_fp8: torch.Tensor, x_scales: torch.Tensor) -> torch.Te
     tokens, hidden = x_fp8.shape
     blocks = (hidden + 127) // 128
     if x_fp8.is_cuda and hidden % 16 == 0 and (x_scales.dtype != torch.int or blocks % 4 == 0):
-        from . import ops
-
         scales = x_scales.contiguous()
         scales = scales.view(tokens, -1) if scales.dtype == torch.int else scales.to(torch.float32).view(tokens, blocks)
         return ops.cast_back(x_fp8.contiguous(), scales)

@@ -293,6 +293,25 @@ int dpep_megamoe_forward(void* ws, const void* x_codes, const uint8_t* x_scales,
                          int intermediate, int num_topk, int num_experts, int expert_begin, int num_local, void* y,
                          int32_t* expert_token_nums, void* stream);
 
+/* The same forward with its arguments in a struct, and with the choice of BF16 input rows, which the forward then quantises
+ * itself (dpep_mx_quant's arithmetic, in the launch that also works out the layout): x_bf16 [B,H] instead of x_codes / x_scales,
+ * and scratch for the codes [B, dpep_megamoe_padded_dim(H)] and their scale bytes [B, dpep_megamoe_padded_dim(H) / 32]. */
+typedef struct dpep_megamoe_call {
+    const void* x_codes;
+    const uint8_t* x_scales;
+    const void* x_bf16;
+    uint8_t* x_codes_scratch;
+    uint8_t* x_scales_scratch;
+    const int32_t* topk_idx;
+    const float* topk_weights;
+    const uint8_t *w1, *s1, *w2, *s2;
+    const uint8_t *shared_w1, *shared_s1, *shared_w2, *shared_s2;
+    void* y;
+    int32_t* expert_token_nums;
+    int32_t num_shared, num_tokens, hidden, intermediate, num_topk, num_experts, expert_begin, num_local;
+} dpep_megamoe_call;
+int dpep_megamoe_run(void* ws, const dpep_megamoe_call* call, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

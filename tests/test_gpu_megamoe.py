@@ -746,3 +746,46 @@ def test_readme_example_runs_as_written(monkeypatch):
     want = mm.round_bf16(mm.local_reference(xq, idx, weights, mm.unpack_weight(*l1), mm.unpack_weight(*l2), 0,
                                             mm.unpack_weight(sp1, ss1), mm.unpack_weight(sp2, ss2)))
     assert mm.relative_frobenius(y.float().cpu().numpy(), want) <= 2e-2
+
+
+@pytest.mark.parametrize("tokens,hidden,inter,shared", [(1, 1024, 256, 0), (63, 1088, 384, 1), (130, 2880, 512, 2), (257, 1536, 256, 0)])
+def test_bf16_rows_quantised_by_the_layouts_launch(tokens, hidden, inter, shared):
+    """BF16 rows go through the workgroups behind the layout's (with the padding of sizes that are no whole tiles and the shared
+    experts' rows): the same bits as quantising them first, on the native host path, step by step in Python, and with a layout
+    that takes two launches."""
+    from deepep_amd import megamoe
+    from deepep_amd import ops as dops
+
+    experts, topk = 4, 2
+    gen = torch.Generator().manual_seed(tokens)
+    x = torch.randn(tokens, hidden, generator=gen).bfloat16().cuda()
+    x[0, :40] = 0
+    idx = torch.stack([torch.randperm(experts, generator=gen)[:topk] for _ in range(tokens)]).int().cuda()
+    w = torch.rand(tokens, topk, generator=gen).cuda()
+
+    def raw(e, n, k):
+        return (torch.randint(0, 256, (e, n, k // 2), dtype=torch.uint8, generator=gen).cuda(),
+                torch.randint(116, 121, (e, n, k // 64, 2), dtype=torch.uint8, generator=gen).cuda())
+
+    l1, l2 = megamoe.transform_weights_for_mega_moe(raw(experts, 2 * inter, hidden), raw(experts, hidden, inter))
+    kw = {}
+    if shared:
+        s1, s2 = megamoe.transform_weights_for_mega_moe(raw(shared, 2 * inter, hidden), raw(shared, hidden, inter), shared=True)
+        kw = dict(shared_l1_weights=s1, shared_l2_weights=s2)
+    buf = megamoe.SymmBuffer(None, experts, tokens, topk, hidden, inter, shared)
+    try:
+        slow, counts = megamoe.mega_moe(x, idx, w, l1, l2, buf, **kw)  # a batch size's first call: step by step
+        pair = dops.mx_quant(x)
+        outs = [megamoe.mega_moe(pair, idx, w, l1, l2, buf, **kw)[0], megamoe.mega_moe(x, idx, w, l1, l2, buf, **kw)[0]]
+        given = torch.full_like(slow, 3.0)
+        y, again = megamoe.mega_moe(x, idx, w, l1, l2, buf, out=given, **kw)
+        assert y is given and torch.equal(again, counts)
+        outs.append(given.clone())
+        buf._workspace.tune("layout_one_launch", 0)
+        outs.append(megamoe.mega_moe(x, idx, w, l1, l2, buf, **kw)[0])
+        for name, got in zip(("pair", "bf16", "out", "two launches"), outs):
+            assert torch.equal(got, slow), name
+        with pytest.raises(ValueError, match="alias"):
+            megamoe.mega_moe(x, idx, w, l1, l2, buf, out=x, **kw)
+    finally:
+        buf.destroy()
