@@ -202,3 +202,67 @@ def test_event_of_an_asynchronous_call_stands_in_for_torchs():
         assert torch.equal(out.float(), x.cuda().float() * 2)
     finally:
         buffer.destroy()
+
+
+def test_asynchronous_calls_from_changing_streams_keep_their_order():
+    """The caller's stream changes from call to call while the one before is still busy: every asynchronous call has to see
+    its own caller's input, whichever stream raised the buffer's counter last."""
+    tokens, hidden, topk, experts = 64, 256, 2, 8
+    idx = torch.stack([torch.randperm(experts)[:topk] for _ in range(tokens)]).cuda()
+    streams = [torch.cuda.Stream() for _ in range(3)]
+    buffer = _buffer(num_bytes=4 << 20)
+    try:
+        _, _, _, handle, _ = buffer.dispatch(torch.zeros(tokens, hidden, dtype=torch.bfloat16, device="cuda"), topk_idx=idx, num_experts=experts)
+        ones = torch.ones(tokens, hidden, dtype=torch.bfloat16, device="cuda")
+        torch.cuda.synchronize()
+        for order in ((0, 1, 2), (2, 1, 0), (0, 0, 1), (1, 2, 1)):
+            results = []
+            for at, which in enumerate(order):
+                with torch.cuda.stream(streams[which]):
+                    torch.cuda._sleep(3_000_000 if at == 0 else 1000)
+                    x = ones * (at + 1 + which)
+                    recv, _, _, _, event = buffer.dispatch(x, handle=handle, async_with_compute_stream=True)
+                    out, _, done = buffer.combine(recv, handle, previous_event=event.event, async_with_compute_stream=True)
+                    done.current_stream_wait()
+                    results.append((out * 1, 2.0 * (at + 1 + which)))
+            torch.cuda.synchronize()
+            for out, want in results:
+                assert torch.equal(out, torch.full_like(out, want)), order
+    finally:
+        torch.cuda.synchronize()
+        buffer.destroy()
+
+
+def test_asynchronous_cached_calls_in_a_hip_graph():
+    """Under capture streams are ordered by events: a cached dispatch and a combine on the communication stream, captured once
+    and replayed on new payloads, with the program's own work between the replays."""
+    tokens, hidden, topk, experts = 96, 512, 3, 8
+    gen = torch.Generator().manual_seed(4)
+    idx = torch.stack([torch.randperm(experts, generator=gen)[:topk] for _ in range(tokens)]).cuda()
+    x = torch.zeros(tokens, hidden, dtype=torch.bfloat16, device="cuda")
+    buffer = _buffer(num_bytes=4 << 20)
+    try:
+        _, _, _, handle, _ = buffer.dispatch(x, topk_idx=idx, num_experts=experts)
+        _, _, _, _, event = buffer.dispatch(x, handle=handle, async_with_compute_stream=True)
+        event.current_stream_wait()
+        torch.cuda.synchronize()
+        side = torch.cuda.Stream()
+        with torch.cuda.stream(side):
+            buffer.combine(torch.zeros(handle.num_expanded_tokens, hidden, dtype=torch.bfloat16, device="cuda"), handle)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=side):
+            recv, _, _, _, event = buffer.dispatch(x, handle=handle, async_with_compute_stream=True)
+            event.current_stream_wait()
+            out, _, event = buffer.combine(recv, handle, async_with_compute_stream=True)
+            event.current_stream_wait()
+        for _ in range(4):
+            x.copy_(torch.randn(tokens, hidden, generator=gen).bfloat16())
+            graph.replay()
+            torch.cuda.synchronize()
+            eager_rows, _, _, _, _ = buffer.dispatch(x, handle=handle)
+            assert torch.equal(recv, eager_rows)
+            assert torch.equal(out, buffer.combine(eager_rows, handle)[0])
+    finally:
+        torch.cuda.synchronize()
+        buffer.destroy()
