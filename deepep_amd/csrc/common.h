@@ -42,6 +42,7 @@ struct Workspace {
     uint32_t* mailbox_device;  // the same memory as the kernels address it
     uint32_t sequence;         // of the most recent layout launch
     int mailbox_local;         // its number of local experts
+    bool mailbox_narrow;       // and the form of its counts
     // One-launch layout: the memory its workgroups exchange histograms through, the bound of a workgroup's wait for the
     // others' histograms in 100 MHz ticks, and two switches for tests (take two launches instead; expect more
     // histogram rows than there are workgroups, so that the wait runs out).
@@ -70,10 +71,18 @@ constexpr size_t kSyncTaggedWords = 4096 + DPEP_MAX_LOCAL_EXPERTS;  // (workgrou
 constexpr size_t kSyncBytes = kSyncTagged + kSyncTaggedWords * 8;
 // The host mailbox (pinned memory, 32-bit words): word 0 = number of rows and word 1 = sequence number of the layout
 // that reported last (one 8-byte store); word kMailboxTimeout = launch number of a layout kernel whose wait for the
-// other workgroups' histograms ran out; from word kMailboxCounts on, 16-byte aligned, the per-expert counts.
+// other workgroups' histograms ran out; from word kMailboxCounts on the per-expert counts, 16 bytes for experts 4i .. 4i + 3:
+// (counts of two experts, sequence number, counts of the other two, sequence number) where every count fits 16 bits;
+// else (count, sequence number) of the first two there and of the other two in a second block of the same size.
+// Every 8 bytes say themselves which launch they belong to, so the device sends everything at once and the host waits
+// for what it reads (with one sequence number behind all counts the device had to wait for the counts' acknowledgement
+// first, a trip across PCIe and back).  Lanes write consecutive 16-byte pieces: the same words at a stride of 32 bytes
+// took 5 us longer for 256 experts.
 constexpr int kMailboxTimeout = 2;
 constexpr int kMailboxCounts = 4;
-constexpr int kMailboxWords = kMailboxCounts + (DPEP_MAX_LOCAL_EXPERTS + 3) / 4 * 4;
+constexpr int kMailboxBlock = DPEP_MAX_LOCAL_EXPERTS;  // words of one block of counts
+constexpr int kMailboxWords = kMailboxCounts + 2 * kMailboxBlock;
+inline __host__ __device__ bool mailbox_narrow(int n_routes) { return n_routes < 65536; }
 constexpr long long kLayoutExchangeTicks = 200000000;  // 2 s
 constexpr uint32_t kWorkspaceMagic = 0x44504550u;  // "DPEP"
 Workspace* as_workspace(void* ws);
@@ -144,15 +153,24 @@ __device__ __forceinline__ void store16_through(void* p, u32x4 v)
 }
 __device__ __forceinline__ u32x4 load16_nt(const void* p) { return __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p)); }
 
-// Counts of four consecutive local experts, first of them `first` (a multiple of 4), into the host mailbox as one
-// 16-byte store that goes through every cache (system scope).  One store per four experts instead of four: the
-// stores cross PCIe one by one, and a layout over 256 experts that sent a word at a time left the next launch
-// waiting behind them.  The caller waits with s_waitcnt vmcnt(0) before it publishes the sequence word.
-__device__ __forceinline__ void mailbox_store_counts(uint32_t* mailbox, int first, const int (&four)[4])
+// Counts of four consecutive local experts, first of them `first` (a multiple of 4), into the host mailbox as 16-byte
+// stores that go through every cache (system scope).
+__device__ __forceinline__ void mailbox_store_counts(uint32_t* mailbox, int first, const int (&four)[4], uint32_t sequence, bool narrow)
 {
-    const u32x4 v = {static_cast<uint32_t>(four[0]), static_cast<uint32_t>(four[1]), static_cast<uint32_t>(four[2]),
-                     static_cast<uint32_t>(four[3])};
-    asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1" ::"v"(mailbox + kMailboxCounts + first), "v"(v) : "memory");
+    const uint32_t c[4] = {static_cast<uint32_t>(four[0]), static_cast<uint32_t>(four[1]), static_cast<uint32_t>(four[2]), static_cast<uint32_t>(four[3])};
+    uint32_t* const to = mailbox + kMailboxCounts + first;
+    const u32x4 a = {narrow ? c[0] | (c[1] << 16) : c[0], sequence, narrow ? c[2] | (c[3] << 16) : c[1], sequence};
+    asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1" ::"v"(to), "v"(a) : "memory");
+    if (!narrow) {
+        const u32x4 b = {c[2], sequence, c[3], sequence};
+        asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1" ::"v"(to + kMailboxBlock), "v"(b) : "memory");
+    }
+}
+// The row count, with the sequence number the host polls for.
+__device__ __forceinline__ void mailbox_store_rows(uint32_t* mailbox, int rows, uint32_t sequence)
+{
+    const unsigned long long word = (static_cast<unsigned long long>(sequence) << 32) | static_cast<uint32_t>(rows);
+    __hip_atomic_store(reinterpret_cast<unsigned long long*>(mailbox), word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 }  // namespace dpep

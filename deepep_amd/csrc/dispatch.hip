@@ -399,7 +399,12 @@ __global__ __launch_bounds__(kMaxThreads) void layout_dispatch_small_kernel(
     const int u_begin = part * units_per_part, u_end = min(u_begin + units_per_part, units_per_row);
     constexpr int kIn = kQuant ? 2 : 1;
     const u32x4* src = x + static_cast<size_t>(token) * units_per_row * kIn;
-    // the payload is asked for first: it does not depend on the routing
+    // all ids at once (a route past the end reads the last id instead of branching around the load): one memory latency
+    constexpr int kIds = kSmallRoutes / kMaxThreads;
+    long long ids[kIds];
+#pragma unroll
+    for (int i = 0; i < kIds; ++i) ids[i] = idx[min(tid + i * kMaxThreads, n_routes - 1)];
+    // the payload is asked for right behind them: it does not depend on the routing
     constexpr int kEarly = 2;
     u32x4 early[kEarly][kIn];
 #pragma unroll
@@ -414,12 +419,15 @@ __global__ __launch_bounds__(kMaxThreads) void layout_dispatch_small_kernel(
     if (tid < DPEP_MAX_TOPK) before[tid] = 0;
     __syncthreads();
     const bool reporter = blockIdx.x == 0;
-    for (int j = tid; j < n_routes; j += kMaxThreads) {
-        const long long id = idx[j];
-        if (reporter && idx_copy != nullptr) idx_copy[j] = id;
-        const int e = local_expert(id, j, n_routes, num_experts, expert_begin, num_local);
-        local_id[j] = static_cast<short>(e);
-        if (e >= 0) atomicAdd(&first_row[e], 1);
+#pragma unroll
+    for (int i = 0; i < kIds; ++i) {
+        const int j = tid + i * kMaxThreads;
+        if (j < n_routes) {
+            if (reporter && idx_copy != nullptr) idx_copy[j] = ids[i];
+            const int e = local_expert(ids[i], j, n_routes, num_experts, expert_begin, num_local);
+            local_id[j] = static_cast<short>(e);
+            if (e >= 0) atomicAdd(&first_row[e], 1);
+        }
     }
     __syncthreads();
     // exclusive scan over the experts: four consecutive experts per thread, wave scan, then the waves' sums
@@ -459,13 +467,11 @@ __global__ __launch_bounds__(kMaxThreads) void layout_dispatch_small_kernel(
         num_rows[0] = offset;  // the last thread's running offset is the total
     }
     if (reporter) send_counts_of_others(send, num_local, wave_sums[0] + wave_sums[1] + wave_sums[2] + wave_sums[3], tid, kMaxThreads);
-    if (reporter && mailbox != nullptr && tid * 4 < num_local) mailbox_store_counts(mailbox, tid * 4, mine);
-    if (reporter && mailbox != nullptr) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this thread's counts have reached the host
-    __syncthreads();
-    if (reporter && mailbox != nullptr && tid == kMaxThreads - 1) {
-        const unsigned long long word = (static_cast<unsigned long long>(sequence) << 32) | static_cast<uint32_t>(offset);
-        __hip_atomic_store(reinterpret_cast<unsigned long long*>(mailbox), word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    if (reporter && mailbox != nullptr) {
+        if (tid * 4 < num_local) mailbox_store_counts(mailbox, tid * 4, mine, sequence, true);
+        if (tid == kMaxThreads - 1) mailbox_store_rows(mailbox, offset, sequence);
     }
+    __syncthreads();
     // earlier routes with the same expert, for each route of this token
     const int my_first = token * num_topk;
     int want[kSlots], seen[kSlots];
@@ -636,6 +642,7 @@ int launch_small(Workspace* w, const dpep_fresh_dispatch& c, int units, hipStrea
     if (c.report_to_host) {
         w->sequence = w->sequence == 0xffffffffu ? 1u : w->sequence + 1u;  // never 0: that is "nothing launched"
         w->mailbox_local = c.num_local;
+        w->mailbox_narrow = true;
     }
     const Split sp = choose_split(c.num_tokens, units, 8);
     auto launch = [&](auto kernel) {

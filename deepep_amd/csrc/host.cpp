@@ -704,14 +704,23 @@ PyObject* run_fresh(Exchange* e, const FreshCall& c, const Target& t, PyObject* 
     const bool small = routes <= 2048;
     const long long capacity = c.low_latency ? c.capacity_rows : capacity_for(e, routes, local, c.experts, small);
 
-    // One block for all of the routing: [ids 8 B][route_to_row][row_to_route][counts][psum][offsets][num_rows][send_counts].
+    // One block for all of the routing: [ids 8 B][route_to_row][row_to_route][counts][psum][offsets][num_rows][send_counts]
+    // [row weights], and one for the payload, which holds the scales too where both are small (an allocation takes 1 us).
     const int64_t at_forward = c.copy_idx ? routes * 8 : 0, at_rows = at_forward + routes * 4, at_counts = at_rows + routes * 4;
     const int64_t at_psum = at_counts + local * 4, at_offsets = at_psum + local * 4, at_num = at_offsets + (local + 1) * 4;
-    const int64_t at_send = at_num + 4, total = at_send + (c.low_latency ? c.experts * 4 : 0);
-    at::Tensor routing = allocate({total}, at::kByte, device);
-    at::Tensor out = allocate({capacity, width}, out_type, device), scales, weights;
-    if (scale_cols > 0) scales = allocate({capacity, scale_cols}, c.quantize ? at::kFloat : c.in.scales->scalar_type(), device);
-    if (c.weights != nullptr) weights = allocate({capacity}, at::kFloat, device);
+    const int64_t at_send = at_num + 4, at_weights = at_send + (c.low_latency ? c.experts * 4 : 0);
+    at::Tensor routing = allocate({at_weights + (c.weights != nullptr ? capacity * 4 : 0)}, at::kByte, device), out, scales, weights;
+    const at::ScalarType scale_type = c.quantize || c.in.scales == nullptr ? at::kFloat : c.in.scales->scalar_type();
+    const int64_t code_bytes = capacity * width, scale_bytes = capacity * scale_cols * 4;
+    if (scale_cols > 0 && code_bytes <= (1 << 20)) {  // (codes of one byte; width is a multiple of 16)
+        at::Tensor both = allocate({code_bytes + scale_bytes}, at::kByte, device);
+        out = over(both.storage(), 0, out_type, {capacity, width});
+        scales = over(both.storage(), code_bytes, scale_type, {capacity, scale_cols});
+    } else {
+        out = allocate({capacity, width}, out_type, device);
+        if (scale_cols > 0) scales = allocate({capacity, scale_cols}, scale_type, device);
+    }
+    if (c.weights != nullptr) weights = over(routing.storage(), at_weights, at::kFloat, {capacity});
     char* base = static_cast<char*>(routing.data_ptr());
 
     dpep_fresh_dispatch call = {};
@@ -811,7 +820,7 @@ PyObject* run_fresh(Exchange* e, const FreshCall& c, const Target& t, PyObject* 
         e->share = static_cast<double>(rows) / static_cast<double>(routes);
         if (rows > capacity) {  // more rows than the share suggested: once more, into outputs of the right size
             out = allocate({rows, width}, out_type, device);
-            if (scales.defined()) scales = allocate({rows, scale_cols}, scales.scalar_type(), device);
+            if (scales.defined()) scales = allocate({rows, scale_cols}, scale_type, device);
             if (weights.defined()) weights = allocate({rows}, at::kFloat, device);
             float* s_out = scales.defined() ? static_cast<float*>(scales.data_ptr()) : nullptr;
             float* w_out = weights.defined() ? static_cast<float*>(weights.data_ptr()) : nullptr;
@@ -822,8 +831,8 @@ PyObject* run_fresh(Exchange* e, const FreshCall& c, const Target& t, PyObject* 
             if (status) return raise_native(status);
         } else if (rows < capacity) {
             out = over(out.storage(), 0, out_type, {rows, width});
-            if (scales.defined()) scales = over(scales.storage(), 0, scales.scalar_type(), {rows, scale_cols});
-            if (weights.defined()) weights = over(weights.storage(), 0, at::kFloat, {rows});
+            if (scales.defined()) scales = over(scales.storage(), scales.storage_offset() * 4, scale_type, {rows, scale_cols});
+            if (weights.defined()) weights = over(storage, at_weights, at::kFloat, {rows});
         }
         Ref list(PyList_New(local));
         if (!list) return nullptr;

@@ -286,7 +286,7 @@ struct TaggedSource {
 // wave_hist / block_hist.  Returns false if the wait for the tagged words ran out: every count is then reported as zero.
 template <bool kTagged, typename Lds>
 __device__ __forceinline__ bool expert_bases(Lds& lds, const int* __restrict__ wave_hist,
-                                             const int* __restrict__ block_hist, int num_local, int padded_local,
+                                             const int* __restrict__ block_hist, int n_routes, int num_local, int padded_local,
                                              int num_chunks, int num_blocks, int* __restrict__ counts,
                                              int* __restrict__ psum, int* __restrict__ offsets, int* __restrict__ num_rows,
                                              const SendCounts& send, uint32_t* __restrict__ mailbox, uint32_t sequence,
@@ -350,10 +350,13 @@ __device__ __forceinline__ bool expert_bases(Lds& lds, const int* __restrict__ w
     const bool valid = !kTagged || lds.timed_out == 0;
     if (!valid) {
         // A histogram is missing: every count is reported as zero, and the host is told.  (The reporter's own store is
-        // acknowledged before it publishes the mailbox's sequence word below, so the host never sees a reporter's
+        // acknowledged before it reports to the mailbox below, so the host never sees a reporter's
         // time-out later than its report; another workgroup's time-out may reach the host after the report, and is
         // then found by the next call on the workspace.)
-        if (tid == 0) __hip_atomic_store(source->timeouts, source->launch_id, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        if (tid == 0) {
+            __hip_atomic_store(source->timeouts, source->launch_id, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        }
         for (int e = tid; e < num_local; e += kThreads) {
             lds.totals[e] = 0;
 #pragma unroll
@@ -400,17 +403,11 @@ __device__ __forceinline__ bool expert_bases(Lds& lds, const int* __restrict__ w
         num_rows[0] = offset;
     }
     if (reporter) send_counts_of_others(send, num_local, lds.wave_sums[0] + lds.wave_sums[1] + lds.wave_sums[2] + lds.wave_sums[3], tid, kThreads);
-    if (reporter && mailbox != nullptr && tid * 4 < num_local) mailbox_store_counts(mailbox, tid * 4, mine);
-    // The host polls the mailbox's sequence word: publish it (with the row count, one 8-byte store) after
-    // every per-expert count of this workgroup has reached host memory.  The counts went out as write-through
-    // stores, so each thread only has to wait until its own are acknowledged: no cache needs writing back, which
-    // is what a system-scope release fence would spend microseconds on after a kernel that left the L2 dirty.
-    if (reporter && mailbox != nullptr) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    if (reporter && mailbox != nullptr && tid == kThreads - 1) {
-        const unsigned long long word = (static_cast<unsigned long long>(sequence) << 32) | static_cast<uint32_t>(offset);
-        __hip_atomic_store(reinterpret_cast<unsigned long long*>(mailbox), word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    if (reporter && mailbox != nullptr) {
+        if (tid * 4 < num_local) mailbox_store_counts(mailbox, tid * 4, mine, sequence, mailbox_narrow(n_routes));
+        if (tid == kThreads - 1) mailbox_store_rows(mailbox, offset, sequence);
     }
+    __syncthreads();
     return valid;
 }
 
@@ -431,7 +428,7 @@ __global__ __launch_bounds__(kThreads) void layout_assign_kernel(
     if (begin < end) fetch_experts(experts, idx, begin, end, n_routes, num_experts, expert_begin, num_local);
     clear_wave_lds(lds, num_local);
     __syncthreads();  // expert_bases writes the rows of all waves
-    expert_bases<false>(lds, wave_hist, block_hist, num_local, padded_local, num_chunks, gridDim.x - 1, counts, psum,
+    expert_bases<false>(lds, wave_hist, block_hist, n_routes, num_local, padded_local, num_chunks, gridDim.x - 1, counts, psum,
                         offsets, num_rows, send, mailbox, sequence);
     for (int base = begin; base < end; base += kPrefetch * kWave) {
         if (base != begin) fetch_experts(experts, idx, base, end, n_routes, num_experts, expert_begin, num_local);
@@ -504,7 +501,7 @@ __global__ __launch_bounds__(kThreads) void layout_fused_kernel(
     // on the consumers' side: such a workgroup marks its routes as having no row, and the kernels that read
     // row_to_route clamp what they find there.
     const TaggedSource source = {tagged, tag, rows, reporter ? limit_ticks : 2 * limit_ticks, timeouts, launch_id};
-    const bool in_time = expert_bases<true>(lds, nullptr, nullptr, num_local, padded_local, num_chunks, num_blocks, counts, psum,
+    const bool in_time = expert_bases<true>(lds, nullptr, nullptr, n_routes, num_local, padded_local, num_chunks, num_blocks, counts, psum,
                                             offsets, num_rows, send, mailbox, sequence, &source);
     // (asked for here, needed only at the very end: the load travels while the routes are assigned)
     unsigned long long reporter_seen = threadIdx.x == 0 && !reporter ? load_word(reporter_tag) : 0ull;
@@ -650,6 +647,7 @@ int launch_layout(void* ws, const IdxT* idx, int num_tokens, int num_topk, int n
     if (report_to_host) {
         w->sequence = w->sequence == 0xffffffffu ? 1u : w->sequence + 1u;  // never 0: that is "nothing launched"
         w->mailbox_local = num_local;
+        w->mailbox_narrow = mailbox_narrow(n_routes);
     }
     uint32_t* mailbox = report_to_host ? w->mailbox_device : nullptr;
     if (one_launch) {

@@ -111,18 +111,22 @@ int dpep_layout_wait(void* ws, int32_t* counts_host, int num_local, int32_t* num
     DPEP_REQUIRE(counts_host == nullptr || num_local == w->mailbox_local,
                  "layout_wait: num_local=%d does not match the launched layout (%d)", num_local, w->mailbox_local);
     volatile uint32_t* box = w->mailbox_host;
-    timespec start;
-    clock_gettime(CLOCK_MONOTONIC, &start);
-    for (long long spins = 0; box[1] != w->sequence; ++spins) {
-        if ((spins & 1023) == 1023) {
-            timespec now;
-            clock_gettime(CLOCK_MONOTONIC, &now);
-            const long long waited = (now.tv_sec - start.tv_sec) * 1000000ll + (now.tv_nsec - start.tv_nsec) / 1000;
-            if (waited > timeout_us)
-                return dpep::fail(DPEP_ERUNTIME, "layout_wait: the layout kernel did not report within %lld us", timeout_us);
+    // Waits until the 8-byte word at `at` (value, sequence number) is this launch's; false after timeout_us.
+    timespec start = {0, 0};
+    auto arrived = [&](int at) {
+        for (long long spins = 0; box[at + 1] != w->sequence; ++spins) {
+            if ((spins & 1023) == 1023) {
+                timespec now;
+                clock_gettime(CLOCK_MONOTONIC, &now);
+                if (start.tv_sec == 0) start = now;
+                const long long waited = (now.tv_sec - start.tv_sec) * 1000000ll + (now.tv_nsec - start.tv_nsec) / 1000;
+                if (waited > timeout_us) return false;
+            }
+            __builtin_ia32_pause();
         }
-        __builtin_ia32_pause();
-    }
+        return true;
+    };
+    if (!arrived(0)) return dpep::fail(DPEP_ERUNTIME, "layout_wait: the layout kernel did not report within %lld us", timeout_us);
     __atomic_thread_fence(__ATOMIC_ACQUIRE);
     if (const uint32_t timed_out = box[dpep::kMailboxTimeout]; timed_out != w->timeout_seen) {
         w->timeout_seen = timed_out;
@@ -132,7 +136,16 @@ int dpep_layout_wait(void* ws, int32_t* counts_host, int num_local, int32_t* num
     }
     *num_rows_host = static_cast<int32_t>(box[0]);
     if (counts_host != nullptr)
-        for (int e = 0; e < num_local; ++e) counts_host[e] = static_cast<int32_t>(box[dpep::kMailboxCounts + e]);
+        for (int e = 0; e < num_local; ++e) {
+            // the word that holds expert e (see kMailboxCounts)
+            const bool narrow = w->mailbox_narrow;
+            const int block = !narrow && (e & 2) ? dpep::kMailboxBlock : 0;
+            const int at = dpep::kMailboxCounts + block + (e & ~3) + (narrow ? e & 2 : (e & 1) * 2);
+            if (!arrived(at))
+                return dpep::fail(DPEP_ERUNTIME, "layout_wait: the layout kernel did not report within %lld us", timeout_us);
+            const uint32_t word = box[at];
+            counts_host[e] = static_cast<int32_t>(narrow ? (word >> (16 * (e & 1))) & 0xffffu : word);
+        }
     return DPEP_OK;
 }
 
