@@ -7,6 +7,8 @@
 // tmp = float(y); tmp = tmp * w; acc = acc + tmp (separate multiply and add); final cast RNE.
 // Unweighted form: tests/elastic/test_combine.py:504-515; weighted form:
 // tests/elastic/test_ep_low_latency.py:449-463; weight-return channel: docs/elastic.md:71.
+#include <algorithm>
+
 #include "common.h"
 
 #pragma clang fp contract(off)
@@ -103,113 +105,32 @@ __global__ __launch_bounds__(kMaxThreads) void combine_kernel(
     }
 }
 
-// One wave reduces the 16-byte vectors [vec_begin, vec_end) of one token: lane s holds the row and weight of the
-// token's slot s (row < 0: no row), valid = the lanes that hold a row; rows are row_stride vectors apart.  Slots ascending, separate fp32 multiply and add, one
-// rounding to BF16.  kSparseBatch = 16-byte vectors per lane in flight per slot.
-template <int kWeights, bool kCached, int kSparseBatch>
-__device__ __forceinline__ void reduce_token_rows(const u32x4* __restrict__ y, int row, float weight, uint64_t valid,
-                                                  int row_stride, int vec_begin, int vec_end, u32x4* __restrict__ dst, int lane)
-{
-    for (int v0 = vec_begin; v0 < vec_end; v0 += 64 * kSparseBatch) {
-        float acc[kSparseBatch][8];
-#pragma unroll
-        for (int b = 0; b < kSparseBatch; ++b)
-#pragma unroll
-            for (int i = 0; i < 8; ++i) acc[b][i] = 0.0f;
-        for (uint64_t rest = valid; rest != 0ull; rest &= rest - 1ull) {
-            const int slot = __builtin_ctzll(rest);
-            const int r = __builtin_amdgcn_readlane(row, slot);
-            const float w = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, weight), slot));
-            const u32x4* src = y + static_cast<size_t>(r) * row_stride;
-            u32x4 val[kSparseBatch];
-#pragma unroll
-            for (int b = 0; b < kSparseBatch; ++b) {
-                const int v = v0 + b * 64 + lane;
-                if (v < vec_end) val[b] = kCached ? load16(src + v) : load16_nt(src + v);
-            }
-#pragma unroll
-            for (int b = 0; b < kSparseBatch; ++b) {
-                if (v0 + b * 64 + lane >= vec_end) continue;
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    float lo = bf16_to_f32(val[b][i] & 0xffffu);
-                    float hi = bf16_to_f32(val[b][i] >> 16);
-                    if (kWeights != 0) {
-                        lo = __fmul_rn(lo, w);
-                        hi = __fmul_rn(hi, w);
-                    }
-                    acc[b][2 * i] = __fadd_rn(acc[b][2 * i], lo);
-                    acc[b][2 * i + 1] = __fadd_rn(acc[b][2 * i + 1], hi);
-                }
-            }
-        }
-#pragma unroll
-        for (int b = 0; b < kSparseBatch; ++b) {
-            const int v = v0 + b * 64 + lane;
-            if (v >= vec_end) continue;
-            u32x4 packed;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) packed[i] = pack_bf16x2(acc[b][2 * i], acc[b][2 * i + 1]);
-            store16_nt(dst + v, packed);
-        }
-    }
-}
-
-// The reduce for sparse shares (most tokens own no row, none owns a shared expert's): one WAVE per token, so that a
-// token without rows costs one short-lived wave instead of a workgroup with a barrier, and four times as many tokens
-// are in flight per CU (the kernel above spends its time on the chain of dependent loads each of its workgroups
-// starts with).  Same arithmetic in the same order as combine_kernel: slots ascending, separate fp32 multiply and
-// add (no multiply at all without weights), one RNE rounding to BF16.  kWeights as above; kCached: the rows were
-// written by the kernel right before this one (the second GEMM) and are read through the caches.
-constexpr int kSparseWaves = 4;  // tokens (= waves) per workgroup
-template <int kWeights, bool kCached>
-__global__ __launch_bounds__(64 * kSparseWaves) void combine_sparse_kernel(
-    const u32x4* __restrict__ y, const float* __restrict__ weights, const int* __restrict__ route_to_row, int num_topk,
-    int vec_per_row, u32x4* __restrict__ out, int num_tokens, const int* __restrict__ fill_state,
-    const float* __restrict__ return_in, float* __restrict__ return_out, int num_rows)
-{
-    const int lane = threadIdx.x & 63;
-    const int token = blockIdx.x * kSparseWaves + (threadIdx.x >> 6);
-    if (token >= num_tokens) return;
-    int row = -1;
-    float weight = 0.0f;
-    if (lane < num_topk) {
-        const size_t route = static_cast<size_t>(token) * num_topk + lane;
-        row = route_to_row[route];
-        if (row >= num_rows) row = -1;  // a row the caller's y does not hold
-        if (kWeights == 1) weight = row >= 0 ? weights[row] : 0.0f;
-        if (kWeights == 2) weight = weights[route];
-        if (return_out != nullptr) return_out[route] = row >= 0 ? return_in[row] : 0.0f;
-    }
-    const uint64_t valid = __ballot(row >= 0);
-    u32x4* dst = out + static_cast<size_t>(token) * vec_per_row;
-    if (valid == 0ull) {
-        if (fill_state != nullptr) {  // rows that idle workgroups of the first GEMM have already zeroed
-            const int fillers = fill_state[0];
-            if (fillers > 0 && token / fillers < fill_state[1 + token % fillers]) return;
-        }
-        const u32x4 zero = {0u, 0u, 0u, 0u};
-        for (int v = lane; v < vec_per_row; v += 64) store16_nt(dst + v, zero);
-        return;
-    }
-    reduce_token_rows<kWeights, kCached, 8>(y, row, weight, valid, vec_per_row, 0, vec_per_row, dst, lane);
-}
-
-// Sparse shares whose unserved tokens are left alone (one rank's part of an EP job: the rows of tokens it does not
-// serve belong to other ranks).  A workgroup takes 64 / top-k consecutive tokens: every wave loads their (at most 64)
-// routes itself, one per lane, so that the tokens without a row (most of them) cost a lane of one load instead of a wave
-// each, and nothing goes through LDS or a barrier.  The four waves share every row, a quarter of its vectors each, and walk
-// the block's rows (set bits of the ballot, i.e. tokens ascending, slots ascending) with the loads of the next row in
-// flight while the current one is accumulated: a workgroup with several rows pays one memory round trip, not one per row.
-// Same arithmetic as combine_kernel: slots ascending, separate fp32 multiply and add, one rounding to BF16.
-constexpr int kServedWaves = 4;
-constexpr int kServedBatch = 4;  // 16-byte vectors per lane and row in flight
-template <int kWeights, bool kCached>
-__global__ __launch_bounds__(64 * kServedWaves) void combine_served_kernel(
+// Sparse shares: most tokens own no row (one rank's part of an EP job).  A workgroup takes a few consecutive tokens, at most
+// 64 / top-k: every wave loads their (at most 64) routes itself, one per lane, so that the tokens without a row (most of them)
+// cost a lane of one load instead of a wave each, and nothing goes through LDS or a barrier.  The four waves share every row,
+// a quarter of its vectors each, and walk the block's rows (set bits of the ballot, i.e. tokens ascending, slots ascending)
+// with the loads of the next row in flight while the current one is accumulated: a workgroup with several rows pays one
+// memory round trip, not one per row.  Tokens without a row are zeroed behind that (a wait for a load also waits for the
+// stores in front of it), or left alone: kLeave (the rows of tokens this rank does not serve belong to other ranks), or rows
+// that idle workgroups of the first GEMM have already zeroed (fill_state: filler f of n took tokens f, f + n, ... and got
+// through fill_state[1 + f] of them).
+// Same arithmetic as combine_kernel: slots ascending, separate fp32 multiply and add, one rounding.
+// stream_out: the output is larger than the memory-side cache should take (kStreamBytes); below that, write-through stores: 6144
+// tokens of 7168 columns of which 560 own a row 14.5 us against 22 with streaming ones, 2048 tokens 6.3 against 10.
+// kCached: the rows were written by the kernel right before this one (the second GEMM) and are read through the caches.
+constexpr int kShareWaves = 4;
+constexpr int kShareBatch = 4;  // 16-byte vectors per lane and row in flight
+constexpr int kShareBlocks = 1024;  // tokens are grouped while that leaves this many workgroups (four to a CU)
+template <int kWeights, bool kCached, bool kHalf>
+__global__ __launch_bounds__(64 * kShareWaves) void combine_share_kernel(
     const u32x4* __restrict__ y, const float* __restrict__ weights, const int* __restrict__ route_to_row, int num_topk,
     int tokens_per_block, int vec_per_row, u32x4* __restrict__ out, int num_tokens, const float* __restrict__ return_in,
-    float* __restrict__ return_out, int num_rows)
+    float* __restrict__ return_out, int num_rows, int leave_unserved, const int* __restrict__ fill_state, int stream_out)
 {
+    auto store = [&](u32x4* to, u32x4 v) {
+        if (stream_out) store16_nt(to, v);
+        else store16_through(to, v);
+    };
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int token0 = blockIdx.x * tokens_per_block;
@@ -225,37 +146,36 @@ __global__ __launch_bounds__(64 * kServedWaves) void combine_served_kernel(
         if (return_out != nullptr && wave == 0) return_out[route] = row >= 0 ? return_in[row] : 0.0f;
     }
     const uint64_t valid = __ballot(row >= 0);
-    if (valid == 0ull) return;
     const int token_of_lane = lane / num_topk;
-    const int quarter = (vec_per_row + kServedWaves - 1) / kServedWaves;
+    const int quarter = (vec_per_row + kShareWaves - 1) / kShareWaves;
     const int vec_begin = wave * quarter, vec_end = min(vec_begin + quarter, vec_per_row);
-    for (int v0 = vec_begin; v0 < vec_end; v0 += 64 * kServedBatch) {
-        u32x4 buffer[2][kServedBatch];
-        float acc[kServedBatch][8];
+    for (int v0 = valid != 0ull ? vec_begin : vec_end; v0 < vec_end; v0 += 64 * kShareBatch) {
+        u32x4 buffer[2][kShareBatch];
+        float acc[kShareBatch][8];
         auto clear = [&]() {
 #pragma unroll
-            for (int b = 0; b < kServedBatch; ++b)
+            for (int b = 0; b < kShareBatch; ++b)
 #pragma unroll
                 for (int i = 0; i < 8; ++i) acc[b][i] = 0.0f;
         };
-        auto issue = [&](u32x4 (&into)[kServedBatch], int at) {
+        auto issue = [&](u32x4 (&into)[kShareBatch], int at) {
             const u32x4* src = y + static_cast<size_t>(__builtin_amdgcn_readlane(row, at)) * vec_per_row;
 #pragma unroll
-            for (int b = 0; b < kServedBatch; ++b) {
+            for (int b = 0; b < kShareBatch; ++b) {
                 const int v = v0 + b * 64 + lane;
                 if (v < vec_end) into[b] = kCached ? load16(src + v) : load16_nt(src + v);
             }
         };
         // accumulates the row of lane `at`; stores the token when `next` (-1: none) belongs to another one
-        auto consume = [&](const u32x4 (&from)[kServedBatch], int at, int next) {
+        auto consume = [&](const u32x4 (&from)[kShareBatch], int at, int next) {
             const float w = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, weight), at));
 #pragma unroll
-            for (int b = 0; b < kServedBatch; ++b) {
+            for (int b = 0; b < kShareBatch; ++b) {
                 if (v0 + b * 64 + lane >= vec_end) continue;
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
-                    float lo = bf16_to_f32(from[b][i] & 0xffffu);
-                    float hi = bf16_to_f32(from[b][i] >> 16);
+                    float lo = kHalf ? f16_to_f32(from[b][i] & 0xffffu) : bf16_to_f32(from[b][i] & 0xffffu);
+                    float hi = kHalf ? f16_to_f32(from[b][i] >> 16) : bf16_to_f32(from[b][i] >> 16);
                     if (kWeights != 0) {
                         lo = __fmul_rn(lo, w);
                         hi = __fmul_rn(hi, w);
@@ -268,13 +188,14 @@ __global__ __launch_bounds__(64 * kServedWaves) void combine_served_kernel(
             if (next >= 0 && __builtin_amdgcn_readlane(token_of_lane, next) == token) return;
             u32x4* dst = out + static_cast<size_t>(token0 + token) * vec_per_row;
 #pragma unroll
-            for (int b = 0; b < kServedBatch; ++b) {
+            for (int b = 0; b < kShareBatch; ++b) {
                 const int v = v0 + b * 64 + lane;
                 if (v >= vec_end) continue;
                 u32x4 packed;
 #pragma unroll
-                for (int i = 0; i < 4; ++i) packed[i] = pack_bf16x2(acc[b][2 * i], acc[b][2 * i + 1]);
-                store16_nt(dst + v, packed);
+                for (int i = 0; i < 4; ++i)
+                    packed[i] = kHalf ? pack_f16x2(acc[b][2 * i], acc[b][2 * i + 1]) : pack_bf16x2(acc[b][2 * i], acc[b][2 * i + 1]);
+                store(dst + v, packed);
             }
             clear();
         };
@@ -298,16 +219,31 @@ __global__ __launch_bounds__(64 * kServedWaves) void combine_served_kernel(
             at = next;
         }
     }
+    if (leave_unserved) return;
+    const u32x4 zero = {0u, 0u, 0u, 0u};
+    const int fillers = fill_state != nullptr ? fill_state[0] : 0;
+    for (int t = 0; t < tokens; ++t) {
+        const uint64_t mine = num_topk < 64 ? ((1ull << num_topk) - 1ull) << (t * num_topk) : ~0ull;
+        if ((valid & mine) != 0ull) continue;
+        const int token = token0 + t;
+        if (fillers > 0 && token / fillers < fill_state[1 + token % fillers]) continue;
+        u32x4* dst = out + static_cast<size_t>(token) * vec_per_row;
+        for (int v = vec_begin + lane; v < vec_end; v += 64) store(dst + v, zero);
+    }
 }
 
-template <int kWeights, bool kCached>
-void launch_combine_served(hipStream_t stream, const void* y, const float* weights, const int32_t* route_to_row, int num_tokens,
-                           int num_topk, int vec, void* out, const float* return_in, float* return_out, int num_rows)
+template <int kWeights, bool kCached, bool kHalf = false>
+void launch_combine_share(hipStream_t stream, const void* y, const float* weights, const int32_t* route_to_row, int num_tokens,
+                          int num_topk, int vec, void* out, const float* return_in, float* return_out, int num_rows,
+                          int leave_unserved, const int32_t* fill_state = nullptr)
 {
-    const int tokens_per_block = 64 / num_topk;  // top-k is at most 32
-    hipLaunchKernelGGL((combine_served_kernel<kWeights, kCached>), dim3((num_tokens + tokens_per_block - 1) / tokens_per_block),
-                       dim3(64 * kServedWaves), 0, stream, static_cast<const u32x4*>(y), weights, route_to_row, num_topk,
-                       tokens_per_block, vec, static_cast<u32x4*>(out), num_tokens, return_in, return_out, num_rows);
+    // (tokens that are left alone cost nothing: as many to a workgroup as a wave has lanes for)
+    int tokens_per_block = 64 / num_topk;  // top-k is at most 32
+    if (!leave_unserved) tokens_per_block = std::max(1, std::min(tokens_per_block, num_tokens / kShareBlocks));
+    hipLaunchKernelGGL((combine_share_kernel<kWeights, kCached, kHalf>), dim3((num_tokens + tokens_per_block - 1) / tokens_per_block),
+                       dim3(64 * kShareWaves), 0, stream, static_cast<const u32x4*>(y), weights, route_to_row, num_topk,
+                       tokens_per_block, vec, static_cast<u32x4*>(out), num_tokens, return_in, return_out, num_rows, leave_unserved,
+                       fill_state, static_cast<size_t>(num_tokens) * vec * 16 > kStreamBytes);
 }
 
 struct CombineGrid {
@@ -354,16 +290,10 @@ int combine_routes(const void* y, const float* route_weights, const int32_t* rou
                    const int32_t* fill_state, int leave_unserved, hipStream_t stream)
 {
     const int vec = hidden / 8;
-    if (num_shared == 0 && leave_unserved && 2LL * num_rows_hint < num_tokens) {
-        launch_combine_served<2, true>(stream, y, route_weights, route_to_row, num_tokens, num_topk, vec, out, nullptr, nullptr,
-                                       0x7fffffff);
-        return launch_status("combine_routes_served");
-    }
     if (num_shared == 0 && 2LL * num_rows_hint < num_tokens) {  // a sparse share: most tokens own no row
-        hipLaunchKernelGGL((combine_sparse_kernel<2, true>), dim3((num_tokens + kSparseWaves - 1) / kSparseWaves),
-                           dim3(64 * kSparseWaves), 0, stream, static_cast<const u32x4*>(y), route_weights, route_to_row, num_topk,
-                           vec, static_cast<u32x4*>(out), num_tokens, fill_state, nullptr, nullptr, 0x7fffffff);
-        return launch_status("combine_routes_sparse");
+        launch_combine_share<2, true>(stream, y, route_weights, route_to_row, num_tokens, num_topk, vec, out, nullptr, nullptr,
+                                      0x7fffffff, leave_unserved, fill_state);
+        return launch_status("combine_routes_share");
     }
     const CombineGrid g = combine_grid(num_tokens, num_rows_hint, vec);
     launch_combine<2>(g, stream, y, route_weights, route_to_row, num_topk, vec, out, nullptr, nullptr, 0x7fffffff,
@@ -379,7 +309,7 @@ namespace {
 template <bool kHalf>
 int combine_entry(const char* what, const void* y, const float* row_weights, const int32_t* route_to_row, int num_tokens,
                   int num_topk, int num_rows, int hidden, void* out, const float* return_in, float* return_out, void* stream,
-                  int leave_unserved = 0)
+                  int leave_unserved = 0, int expected_rows = -1)
 {
     DPEP_REQUIRE(num_tokens >= 0 && num_topk >= 1 && num_topk <= DPEP_MAX_TOPK, "%s: bad T=%d K=%d", what, num_tokens,
                  num_topk);
@@ -395,18 +325,20 @@ int combine_entry(const char* what, const void* y, const float* row_weights, con
     DPEP_REQUIRE(num_rows == 0 || (y != nullptr && aligned16(y)), "%s: y must be 16-byte aligned", what);
     const int vec = hidden / 8;
     hipStream_t s = static_cast<hipStream_t>(stream);
-    if (!kHalf && leave_unserved && 2LL * num_rows < num_tokens) {
-        // a sparse share whose unserved tokens are skipped (with the zero rows to write as well, the workgroup-per-part
-        // kernel below measured faster than a wave per token: 53 against 56 us at 16384 tokens of which 2000 own rows)
+    // (of a capacity layout only the caller knows how many rows to expect)
+    const int hint = expected_rows >= 0 ? expected_rows : num_rows;
+    // (zero rows of more than kStreamBytes are written no faster by fewer, longer workgroups: 16384 tokens of 7168 columns of which
+    // 1900 own a row 57 us against 53 with a workgroup per token)
+    if (2LL * hint < num_tokens && (leave_unserved || static_cast<size_t>(num_tokens) * hidden * 2 <= kStreamBytes)) {
         if (row_weights != nullptr)
-            launch_combine_served<1, false>(s, y, row_weights, route_to_row, num_tokens, num_topk, vec, out, return_in, return_out,
-                                            num_rows);
+            launch_combine_share<1, false, kHalf>(s, y, row_weights, route_to_row, num_tokens, num_topk, vec, out, return_in, return_out,
+                                                  num_rows, leave_unserved);
         else
-            launch_combine_served<0, false>(s, y, nullptr, route_to_row, num_tokens, num_topk, vec, out, return_in, return_out,
-                                            num_rows);
+            launch_combine_share<0, false, kHalf>(s, y, nullptr, route_to_row, num_tokens, num_topk, vec, out, return_in, return_out,
+                                                  num_rows, leave_unserved);
         return launch_status(what);
     }
-    const CombineGrid g = combine_grid(num_tokens, num_rows, vec);
+    const CombineGrid g = combine_grid(num_tokens, hint, vec);
     if (row_weights != nullptr)
         launch_combine<1, kHalf>(g, s, y, row_weights, route_to_row, num_topk, vec, out, return_in, return_out, num_rows, nullptr, 0,
                                  0, nullptr, leave_unserved);
@@ -426,6 +358,15 @@ int dpep_combine(const void* y, const float* row_weights, const int32_t* route_t
 {
     return dpep::combine_entry<false>("combine", y, row_weights, route_to_row, num_tokens, num_topk, num_rows, hidden, out,
                                       return_in, return_out, stream);
+}
+
+int dpep_combine_expecting(const void* y, int half, const float* row_weights, const int32_t* route_to_row, int num_tokens, int num_topk,
+                           int num_rows, int expected_rows, int hidden, void* out, const float* return_in, float* return_out,
+                           void* stream)
+{
+    const auto entry = half ? dpep::combine_entry<true> : dpep::combine_entry<false>;
+    return entry("combine", y, row_weights, route_to_row, num_tokens, num_topk, num_rows, hidden, out, return_in, return_out, stream,
+                 /*leave_unserved=*/0, expected_rows < 0 ? 0 : expected_rows);
 }
 
 int dpep_combine_served(const void* y, const float* row_weights, const int32_t* route_to_row, int num_tokens, int num_topk,

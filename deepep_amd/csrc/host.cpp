@@ -1044,10 +1044,11 @@ PyObject* Exchange_combine(PyObject* self, PyObject* const* a, Py_ssize_t n)
         at::Tensor out = allocate({plan->tokens, plan->hidden}, type, e->device), returned;
         if (values != nullptr) returned = allocate({plan->tokens, plan->topk}, at::kFloat, e->device);
         const float* row_weights = plan->low_latency ? static_cast<const float*>(plan->weights->data_ptr()) : nullptr;
-        const auto entry = type == at::kHalf ? dpep_combine_fp16 : dpep_combine;
-        if (const int status = entry(rows->data_ptr(), row_weights, plan->route_to_row, plan->tokens, plan->topk, static_cast<int>(plan->rows),
-                                     plan->hidden, out.data_ptr(), values != nullptr ? static_cast<const float*>(values->data_ptr()) : nullptr,
-                                     returned.defined() ? static_cast<float*>(returned.data_ptr()) : nullptr, t.stream.raw))
+        const int expected = plan->low_latency ? static_cast<int>(static_cast<long long>(plan->tokens) * plan->topk / e->world) : static_cast<int>(plan->rows);
+        if (const int status = dpep_combine_expecting(rows->data_ptr(), type == at::kHalf, row_weights, plan->route_to_row, plan->tokens, plan->topk,
+                                                      static_cast<int>(plan->rows), expected, plan->hidden, out.data_ptr(),
+                                                      values != nullptr ? static_cast<const float*>(values->data_ptr()) : nullptr,
+                                                      returned.defined() ? static_cast<float*>(returned.data_ptr()) : nullptr, t.stream.raw))
             return raise_native(status);
         Ref event(event_of(e, t, {&out, &returned}, {rows, values, plan->routing, plan->weights}));
         Ref first(wrap(out)), second(returned.defined() ? wrap(returned) : new_ref(Py_None));

@@ -205,6 +205,12 @@ int dpep_combine(const void* y, const float* row_weights, const int32_t* route_t
                  int num_topk, int num_rows, int hidden, void* out, const float* return_in,
                  float* return_out, void* stream);
 
+/* dpep_combine (half != 0: dpep_combine_fp16) of a y that holds num_rows rows of which about expected_rows are in use, as
+ * in the low-latency path's capacity layout: the expectation decides how the work is split, never what is computed. */
+int dpep_combine_expecting(const void* y, int half, const float* row_weights, const int32_t* route_to_row, int num_tokens, int num_topk,
+                           int num_rows, int expected_rows, int hidden, void* out, const float* return_in, float* return_out,
+                           void* stream);
+
 /* dpep_combine that writes only the tokens that own at least one row and leaves the others' rows of `out` untouched.
  * For one rank's receive share of an EP job most candidate tokens own no row here, and in the reference nothing is
  * produced for them on this rank at all (a rank returns rows only for the routes it served,
