@@ -948,6 +948,265 @@ __device__ __forceinline__ int lane_now()
     return lane;
 }
 
+// ---- epilogue pieces: a 32-row tile straight from the accumulators -------------------------------------------------------
+// With the weights as the instruction's A operand a lane holds, for its row, columns q*8 + g*4 .. + 3 (q = 0..3) of a column
+// tile, its partner lane (l ^ 32) the four columns in between.  Two register swaps between the lane halves give the lower lane
+// columns 0..15 and the upper lane columns 16..31 of the row as consecutive bytes, which leave as 16-byte stores.
+__device__ __forceinline__ void swap_halves(uint32_t lower_q, uint32_t upper_q, uint32_t (&out)[2])
+{
+    // lanes 0..31 get (their own lower_q, the partner's lower_q), lanes 32..63 (the partner's upper_q, their own upper_q)
+    const auto swapped = __builtin_amdgcn_permlane32_swap(lower_q, upper_q, false, false);
+    out[0] = swapped[0];
+    out[1] = swapped[1];
+}
+// First GEMM: gate and up columns act_col .. act_col + 31 of one row -> SwiGLU -> one MXFP8 block.
+__device__ __forceinline__ void store_gate_up(const GemmParams& p, const v16f& gates, const v16f& ups, size_t row, bool row_exists, int act_col, int g)
+{
+    float v[16];
+    float amax = 0.0f;
+#pragma unroll
+    for (int j = 0; j < 16; j += 2) {
+        const uint32_t gate = pack_bf16x2(gates[j], gates[j + 1]), up = pack_bf16x2(ups[j], ups[j + 1]);
+        const uint32_t act = pack_bf16x2(silu_mul(__uint_as_float(gate << 16), __uint_as_float(up << 16)),
+                                         silu_mul(__uint_as_float(gate & 0xffff0000u), __uint_as_float(up & 0xffff0000u)));
+        v[j] = bf16_to_f32(act & 0xffffu);
+        v[j + 1] = bf16_to_f32(act >> 16);
+        amax = fmaxf(amax, fmaxf(fabsf(v[j]), fabsf(v[j + 1])));
+    }
+    amax = fmaxf(amax, __shfl_xor(amax, 32));  // the row's other sixteen columns
+    const int byte = mx_scale_byte(amax);
+    uint32_t code[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+        code[q] = mx_pack4(mx_scaled(v[4 * q], byte), mx_scaled(v[4 * q + 1], byte), mx_scaled(v[4 * q + 2], byte), mx_scaled(v[4 * q + 3], byte));
+    uint32_t first[2], second[2];
+    swap_halves(code[0], code[2], first);
+    swap_halves(code[1], code[3], second);
+    const u32x4 codes = {first[0], first[1], second[0], second[1]};
+    const int act_width = p.n / 2;
+    if (row_exists) {
+        *reinterpret_cast<u32x4*>(p.act_codes + row * act_width + act_col + g * 16) = codes;
+        if (g == 0) p.act_scales[row * (act_width / 32) + (act_col >> 5)] = static_cast<uint8_t>(byte);
+    }
+}
+// Second GEMM: columns col0 .. col0 + 31 of one row as BF16.
+__device__ __forceinline__ void store_output(const GemmParams& p, const v16f& acc, size_t row, bool row_exists, int col0, int g)
+{
+    uint32_t pairs[4][2];  // [q][columns +0,1 | +2,3]
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        pairs[q][0] = pack_bf16x2(acc[4 * q], acc[4 * q + 1]);
+        pairs[q][1] = pack_bf16x2(acc[4 * q + 2], acc[4 * q + 3]);
+    }
+    uint32_t s00[2], s01[2], s10[2], s11[2];
+    swap_halves(pairs[0][0], pairs[2][0], s00);
+    swap_halves(pairs[0][1], pairs[2][1], s01);
+    swap_halves(pairs[1][0], pairs[3][0], s10);
+    swap_halves(pairs[1][1], pairs[3][1], s11);
+    const u32x4 lower = {s00[0], s01[0], s00[1], s01[1]}, upper = {s10[0], s11[0], s10[1], s11[1]};
+    const int col = col0 + g * 16;
+    if (row_exists) {
+        // cached stores: the weighted reduce that follows reads these rows back at once
+        if (col < p.out_cols) *reinterpret_cast<u32x4*>(p.out + row * p.out_cols + col) = lower;
+        if (col + 8 < p.out_cols) *reinterpret_cast<u32x4*>(p.out + row * p.out_cols + col + 8) = upper;
+    }
+}
+
+// =====================================================================================================
+// Grouped GEMM for few rows per expert
+// =====================================================================================================
+// With fewer rows per expert than one row tile (a decode step, a small batch) the GEMM is the streaming of its weights: every
+// weight byte is read once and used for one 32-row MFMA tile, and what counts is how many requests are in flight and that
+// nothing else gets in their way.  A wave owns 64 columns (two column tiles; for the first GEMM a gate / up pair) and holds the
+// weight fragments of the next four k tiles in registers; the four waves of a workgroup share the activations, each fetching
+// one k tile of a span of four, through 32 KiB of LDS and one barrier per span (fetched by every wave for itself they cost as
+// many L1 requests as the weights: first GEMM below 82 us instead of 79).  Two workgroups fit on a CU, nothing is persistent
+// beyond the routing being worse than expected, and the hardware hands out the next workgroup when one ends.  The sums are
+// taken in the same order as in the other kernels, so the results are the same bits.
+// Measured on an MI355X, 32 of 256 experts of 7168 x 2048, 16 rows each: first GEMM 82 -> 79 us, second 53 -> 44 us; the bare
+// reads of the same bytes, by as many waves with as many requests in flight, take 78 and 43 us (6.4 and 5.8 TB/s, the launch
+// included).  Whole forward: 0.5 rows per expert 92 -> 62 us, 2: 134 -> 106, 8: 144 -> 130, 16: 153 -> 137.
+// (Tried and not kept: eight k tiles ahead at one workgroup per CU, 143 us; 64-row tiles, 154 us.)
+// kWaves = 1 spreads a column tile over four workgroups of one wave each, for launches that would leave CUs idle (below).
+typedef u32x4 u32x4_unaligned __attribute__((aligned(4)));
+template <int kWaves, bool kGateUp>
+__global__ __launch_bounds__(64 * kWaves, 2) void grouped_gemm_few_rows_kernel(GemmParams p)
+{
+    constexpr bool kGather = kGateUp;
+    constexpr int kRows = 32;
+    __shared__ __attribute__((aligned(16))) uint8_t lds[2][4][kRows * kBK];  // [span parity][k tile of the span][row][128 bytes]
+    const int lane = threadIdx.x & 63, g = lane >> 5, lr = lane & 31;
+    const int my_wave = kWaves == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    constexpr int kSplit = kGemmWaves / kWaves;  // workgroups per column tile
+    const int n_tiles = p.n / kBN, ktiles = p.k / kBK, spans = (ktiles + 3) / 4, scale_bytes = p.k / 32;
+    if (blockIdx.x == 0 && threadIdx.x == 0 && p.fill_state != nullptr) p.fill_state[0] = 0;
+
+    // Row tiles are numbered through the experts, so that the grid does not depend on how the routes fell; every wave works
+    // the numbering out for itself (a lane has experts lane and lane + 64).
+    static_assert(kMaxMoeExperts <= 128, "two experts per lane");
+    int tiles_through[2];
+    int total = 0;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        const int e = lane + 64 * h;
+        tiles_through[h] = 0;
+        if (64 * h >= p.num_local) continue;
+        int sum = e < p.num_local ? (p.offsets[e + 1] - p.offsets[e] + kRows - 1) / kRows : 0;
+#pragma unroll
+        for (int d = 1; d < 64; d *= 2) {
+            const int below = __shfl_up(sum, d);
+            if (lane >= d) sum += below;
+        }
+        tiles_through[h] = total + sum;
+        total = __builtin_amdgcn_readlane(tiles_through[h], 63);
+    }
+
+    for (int tile_id = blockIdx.x; tile_id < total * n_tiles * kSplit; tile_id += gridDim.x) {
+        const int unit = tile_id / (n_tiles * kSplit), piece = tile_id - unit * (n_tiles * kSplit);
+        const int nt = piece / kSplit, wave = kWaves == 1 ? piece % kSplit : my_wave;  // the column tile, the quarter of it
+        int expert = __popcll(__ballot(tiles_through[0] <= unit));  // experts that end at or before this row tile
+        int before = 0;
+        if (expert == 64) {
+            expert += __popcll(__ballot(tiles_through[1] <= unit));
+            before = expert == 64 ? __builtin_amdgcn_readlane(tiles_through[0], 63) : __builtin_amdgcn_readlane(tiles_through[1], expert - 65);
+        } else if (expert > 0) {
+            before = __builtin_amdgcn_readlane(tiles_through[0], expert - 1);
+        }
+        expert = min(expert, p.num_local - 1);
+        const int row0 = p.offsets[expert] + (unit - before) * kRows;
+        const int valid = min(kRows, p.offsets[expert + 1] - row0);
+        const bool shared = expert >= p.num_routed;
+        const size_t weight_index = shared ? expert - p.num_routed : expert;
+        const uint8_t* const w = (shared ? p.w_shared : p.w) + weight_index * p.n * (p.k / 2) + static_cast<size_t>(nt) * ktiles * 16384 +
+                                 wave * 4096 + lane * 16;
+        const uint8_t* const ws = (shared ? p.ws_shared : p.ws) + (weight_index * n_tiles + nt) * spans * 4096 + wave * 1024 + lane * 8;
+
+        u32x4 wreg[4][4];  // [k tile of the span][column tile * 2 + k step]
+        auto load_weights = [&](int slot, int kt) {
+            const uint8_t* at = w + static_cast<size_t>(min(kt, ktiles - 1)) * 16384;  // (past the end: the last k tile again, never used)
+#pragma unroll
+            for (int f = 0; f < 4; ++f) wreg[slot][f] = load16_nt(at + f * 1024);
+        };
+        // Activations: wave q fetches k tile q of a span for the whole workgroup.  Copy f: lane l asks for 16-byte chunk l % 8 of
+        // row 8 f + l / 8, so that eight lanes read a row's 128 bytes.  Rows past the end repeat the last one.
+        // (clamped: a map left incomplete by a layout launch that ran out of time must not become a wild address)
+        const uint8_t* const codes = kGather ? p.a_codes : p.a_codes + static_cast<size_t>(row0) * p.k;
+        const uint8_t* const row_scale_bytes = kGather ? p.a_scales : p.a_scales + static_cast<size_t>(row0) * scale_bytes;
+        auto source = [&](int r) {
+            r = min(r, valid - 1);
+            return static_cast<uint32_t>(kGather ? min(max(p.row_to_route[row0 + r] / p.topk, 0), p.a_rows - 1) : r);
+        };
+        uint32_t a_from[4];
+#pragma unroll
+        for (int f = 0; f < 4; ++f) a_from[f] = source(8 * f + (lane >> 3)) * static_cast<uint32_t>(p.k) + (lane & 7) * 16;
+        const uint32_t s_from = source(lr) * static_cast<uint32_t>(scale_bytes);
+        u32x4 areg[4 / kWaves][4];
+        auto load_activations = [&](int span) {
+#pragma unroll
+            for (int t = 0; t < 4 / kWaves; ++t) {
+                const uint8_t* at = codes + static_cast<size_t>(min(span * 4 + my_wave + t, ktiles - 1)) * kBK;
+#pragma unroll
+                for (int f = 0; f < 4; ++f) areg[t][f] = load16(at + a_from[f]);
+            }
+        };
+        const int put = (lane >> 3) * kBK + (((lane & 7) ^ (lane >> 3)) << 4);  // (row 8 f + i: + f * 1024, the same swizzle)
+        auto hand_over = [&](int parity) {
+#pragma unroll
+            for (int t = 0; t < 4 / kWaves; ++t)
+#pragma unroll
+                for (int f = 0; f < 4; ++f) *reinterpret_cast<u32x4*>(&lds[parity][my_wave + t][put + f * 1024]) = areg[t][f];
+            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        };
+        u32x4 row_scales[2];
+        u32x2 col_scales[2][2];  // [span parity][column tile]
+        auto load_scales = [&](int parity, int span) {
+            span = min(span, spans - 1);
+            row_scales[parity] = *reinterpret_cast<const u32x4_unaligned*>(row_scale_bytes + s_from + min(span * 16, scale_bytes - 16));
+#pragma unroll
+            for (int c = 0; c < 2; ++c)
+                col_scales[parity][c] = *reinterpret_cast<const u32x2*>(ws + static_cast<size_t>(span) * 4096 + c * 512);
+        };
+        v16f acc[2];
+#pragma unroll
+        for (int c = 0; c < 2; ++c)
+#pragma unroll
+            for (int j = 0; j < 16; ++j) acc[c][j] = 0.0f;
+        load_activations(0);
+        load_scales(0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) load_weights(q, q);
+        hand_over(0);
+        auto span_body = [&](auto parity_constant, auto more_constant, int span) {
+            constexpr int kParity = decltype(parity_constant)::value;
+            constexpr bool kMore = decltype(more_constant)::value;  // another span follows
+            if constexpr (kMore) {
+                load_activations(span + 1);
+                load_scales(kParity ^ 1, span + 1);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            const bool shifted_window = span * 16 > scale_bytes - 16;  // (k % 512 = 256: the last span's bytes sit two words up)
+            static_for<4>([&](auto q_constant) {
+                constexpr int q = decltype(q_constant)::value;
+                if (q < 2 || kMore || span * 4 + q < ktiles) {  // (k tiles come in twos)
+                    const uint32_t word = q < 2 && !kMore && shifted_window ? row_scales[kParity][q + 2] : row_scales[kParity][q];
+                    const int x_scale = static_cast<int>(word >> (8 * g));
+                    const uint8_t* const tile = &lds[kParity][q][lr * kBK];
+                    static_for<2>([&](auto step_constant) {
+                        constexpr int step = decltype(step_constant)::value;
+                        const u32x4 lo = *reinterpret_cast<const u32x4*>(tile + (((step * 4 + g) ^ (lr & 7)) << 4));
+                        const u32x4 hi = *reinterpret_cast<const u32x4*>(tile + (((step * 4 + 2 + g) ^ (lr & 7)) << 4));
+                        const v8i x = {(int)lo[0], (int)lo[1], (int)lo[2], (int)lo[3], (int)hi[0], (int)hi[1], (int)hi[2], (int)hi[3]};
+#pragma unroll
+                        for (int c = 0; c < 2; ++c) {
+                            const u32x4 f = wreg[q][2 * c + step];
+                            const v8i m = {(int)f[0], (int)f[1], (int)f[2], (int)f[3], 0, 0, 0, 0};
+                            acc[c] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(m, x, acc[c], 4, 0, 2 * (q & 1) + step,
+                                                                                     static_cast<int>(col_scales[kParity][c][q >> 1]), 2 * step, x_scale);
+                        }
+                    });
+                }
+                if constexpr (kMore) load_weights(q, (span + 1) * 4 + q);
+                __builtin_amdgcn_sched_barrier(0);
+            });
+            if constexpr (kMore) hand_over(kParity ^ 1);
+        };
+        constexpr std::integral_constant<int, 0> even{};
+        constexpr std::integral_constant<int, 1> odd{};
+        constexpr std::integral_constant<bool, true> more{};
+        constexpr std::integral_constant<bool, false> last{};
+        // (The first and the last spans stand outside the loop on purpose: the first one's operands were asked for in
+        // another order, and the compiler's counted waits have to suit every way into a body, so that a shared body waited
+        // for everything in flight; the last asks for nothing more.)
+        if (spans > 1) {
+            span_body(even, more, 0);
+            int span = 1;
+            for (; span + 2 < spans; span += 2) {
+                span_body(odd, more, span);
+                span_body(even, more, span + 1);
+            }
+            if (span + 1 < spans) {
+                span_body(odd, more, span);
+                span_body(even, last, span + 1);
+            } else {
+                span_body(odd, last, span);
+            }
+        } else {
+            span_body(even, last, 0);
+        }
+        // the next tile of this workgroup writes the LDS again
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        const bool row_exists = lr < valid;
+        const size_t row = static_cast<size_t>(row0) + lr;
+        if (kGateUp) {
+            store_gate_up(p, acc[0], acc[1], row, row_exists, (nt * (kBN / 64) + wave) * 32, g);
+        } else {
+#pragma unroll
+            for (int c = 0; c < 2; ++c) store_output(p, acc[c], row, row_exists, nt * kBN + (wave * 2 + c) * 32, g);
+        }
+    }
+}
+
 template <int RT, bool kGateUp>
 __global__ __launch_bounds__(kGemmThreads, ColCfg<RT>::kWorkgroupsPerCu) void grouped_gemm_colwave_kernel(GemmParams p)
 {
@@ -1183,16 +1442,7 @@ __global__ __launch_bounds__(kGemmThreads, ColCfg<RT>::kWorkgroupsPerCu) void gr
                 for (int j = 0; j < 16; ++j) acc[i][c][j] = 0.0f;
     };
 
-    // ---- epilogue of one tile: straight from the accumulators (see mfma_fp4_fp8_regs) ----------------------------------
-    // A lane holds, for its row, columns q*8 + g*4 .. + 3 (q = 0..3) of a column tile, its partner lane (l ^ 32) the four
-    // columns in between.  Two register swaps between the lane halves give the lower lane columns 0..15 and the upper lane
-    // columns 16..31 of the row as consecutive bytes, which leave as 16-byte stores.
-    auto swap_halves = [](uint32_t lower_q, uint32_t upper_q, uint32_t (&out)[2]) {
-        // lanes 0..31 get (their own lower_q, the partner's lower_q), lanes 32..63 (the partner's upper_q, their own upper_q)
-        const auto swapped = __builtin_amdgcn_permlane32_swap(lower_q, upper_q, false, false);
-        out[0] = swapped[0];
-        out[1] = swapped[1];
-    };
+    // ---- epilogue of one tile: straight from the accumulators (store_gate_up, store_output) ---------------------------------
     auto epilogue = [&](const TileInfo& info) {
         const int lane = lane_now(), g = lane >> 5, lr = lane & 31;  // (the epilogue's own copies: see lane_now)
 #pragma unroll
@@ -1206,57 +1456,10 @@ __global__ __launch_bounds__(kGemmThreads, ColCfg<RT>::kWorkgroupsPerCu) void gr
 #pragma unroll
             for (int c = 0; c < kCols; ++c) asm volatile("" : "+a"(acc[i][c]));
             if (kGateUp) {
-                // column tile 0 = gate, 1 = up of the same 32 activation columns
-                float v[16];
-                float amax = 0.0f;
-#pragma unroll
-                for (int j = 0; j < 16; j += 2) {
-                    const uint32_t gate = pack_bf16x2(acc[i][0][j], acc[i][0][j + 1]), up = pack_bf16x2(acc[i][1][j], acc[i][1][j + 1]);
-                    const uint32_t act = pack_bf16x2(silu_mul(__uint_as_float(gate << 16), __uint_as_float(up << 16)),
-                                                     silu_mul(__uint_as_float(gate & 0xffff0000u), __uint_as_float(up & 0xffff0000u)));
-                    v[j] = bf16_to_f32(act & 0xffffu);
-                    v[j + 1] = bf16_to_f32(act >> 16);
-                    amax = fmaxf(amax, fmaxf(fabsf(v[j]), fabsf(v[j + 1])));
-                }
-                amax = fmaxf(amax, __shfl_xor(amax, 32));  // the row's other sixteen columns
-                const int byte = mx_scale_byte(amax);
-                uint32_t code[4];
-#pragma unroll
-                for (int q = 0; q < 4; ++q)
-                    code[q] = mx_pack4(mx_scaled(v[4 * q], byte), mx_scaled(v[4 * q + 1], byte), mx_scaled(v[4 * q + 2], byte),
-                                         mx_scaled(v[4 * q + 3], byte));
-                uint32_t first[2], second[2];
-                swap_halves(code[0], code[2], first);
-                swap_halves(code[1], code[3], second);
-                const u32x4 codes = {first[0], first[1], second[0], second[1]};
-                const int act_width = p.n / 2;
-                const int act_col = (info.nt * (kBN / 64) + wave) * 32;
-                if (row_exists) {
-                    *reinterpret_cast<u32x4*>(p.act_codes + row * act_width + act_col + g * 16) = codes;
-                    if (g == 0) p.act_scales[row * (act_width / 32) + (act_col >> 5)] = static_cast<uint8_t>(byte);
-                }
+                store_gate_up(p, acc[i][0], acc[i][1], row, row_exists, (info.nt * (kBN / 64) + wave) * 32, g);
             } else {
 #pragma unroll
-                for (int c = 0; c < kCols; ++c) {
-                    uint32_t pairs[4][2];  // [q][columns +0,1 | +2,3]
-#pragma unroll
-                    for (int q = 0; q < 4; ++q) {
-                        pairs[q][0] = pack_bf16x2(acc[i][c][4 * q], acc[i][c][4 * q + 1]);
-                        pairs[q][1] = pack_bf16x2(acc[i][c][4 * q + 2], acc[i][c][4 * q + 3]);
-                    }
-                    uint32_t s00[2], s01[2], s10[2], s11[2];
-                    swap_halves(pairs[0][0], pairs[2][0], s00);
-                    swap_halves(pairs[0][1], pairs[2][1], s01);
-                    swap_halves(pairs[1][0], pairs[3][0], s10);
-                    swap_halves(pairs[1][1], pairs[3][1], s11);
-                    const u32x4 lower = {s00[0], s01[0], s00[1], s01[1]}, upper = {s10[0], s11[0], s10[1], s11[1]};
-                    const int col = info.nt * kBN + (wave * kCols + c) * 32 + g * 16;
-                    if (row_exists) {
-                        // cached stores: the weighted reduce that follows reads these rows back at once
-                        if (col < p.out_cols) *reinterpret_cast<u32x4*>(p.out + row * p.out_cols + col) = lower;
-                        if (col + 8 < p.out_cols) *reinterpret_cast<u32x4*>(p.out + row * p.out_cols + col + 8) = upper;
-                    }
-                }
+                for (int c = 0; c < kCols; ++c) store_output(p, acc[i][c], row, row_exists, info.nt * kBN + (wave * kCols + c) * 32, g);
             }
         }
     };
@@ -1461,6 +1664,22 @@ int launch_gemm(const GemmParams& p, int expected_rows_per_expert, hipStream_t s
 {
     const int cus = gemm_grid();
     const int n_tiles = p.n / kBN;
+    // Few rows: the counts scatter by about sqrt(mean), and every expert beyond 32 rows streams its weights once more, so the
+    // line lies where a tile of 32 still holds nearly all experts.  (7168 x 2048, 32 of 256 experts, whole forward, 64-row
+    // tiles -> few rows: mean 16: 153 -> 137 us, 20: 149 -> 138, 24: 148 -> 160, 32: 152 -> 208.)
+    // Source rows are addressed with 32 bits here.
+    if (expected_rows_per_expert <= 20 && p.column_waves && p.forced_rt == 0 &&
+        (!kGateUp || static_cast<long long>(p.a_rows) * p.k < (1LL << 32))) {
+        const int tiles = p.num_local * n_tiles;
+        // One workgroup per column tile fills half the CUs or fewer: a CU draws no more than about 50 GB/s from memory, so
+        // the columns are spread over four times as many (16 experts of 2048 x 768, 8 rows each: 96 + 128 tiles, 26.4 ->
+        // 24.7 us; at 7168 x 2048, 512 + 896 tiles, it costs 15 us: every wave then fetches the activations for itself).
+        if (tiles <= cus / 2)
+            hipLaunchKernelGGL((grouped_gemm_few_rows_kernel<1, kGateUp>), dim3(kGemmWaves * tiles), dim3(64), 0, stream, p);
+        else
+            hipLaunchKernelGGL((grouped_gemm_few_rows_kernel<kGemmWaves, kGateUp>), dim3(tiles), dim3(kGemmThreads), 0, stream, p);
+        return launch_status(what);
+    }
     const double mean = expected_rows_per_expert > 1 ? expected_rows_per_expert : 1;
     const double sigma = sqrt(mean);
     int best = 2;

@@ -208,6 +208,29 @@ def test_both_grouped_gemm_kernels_agree_bit_for_bit(ops, tokens, hidden, inter,
     np.testing.assert_array_equal(new.view(np.uint32), old.view(np.uint32))
 
 
+@pytest.mark.parametrize("hidden,inter,local,rows", [
+    (1024, 256, 3, [33, 1, 0]),              # a wave per workgroup; k = 1024 and 512
+    (1088, 384, 6, [0, 31, 32, 0, 64, 5]),   # k = 1280 ends in half a span of scales
+    (1088, 384, 40, [1, 0, 32, 33, 2] * 8),  # four waves per workgroup
+    (512, 640, 70, [0, 3, 7] + [0] * 60 + [1, 0, 97, 32, 2, 0, 4]),  # more experts than a wave has lanes, one far over the mean
+])
+def test_few_rows_per_expert(ops, hidden, inter, local, rows):
+    """Expected rows per expert below a row tile, actual ones from none to several tiles: against the oracle, and bit for bit
+    against the kernel with 64-row tiles."""
+    begin, experts, remote = 2, 16 * local, 40
+    tokens = sum(rows) + remote
+    x_codes, x_scales, l1, l2, idx, weights = _make_problem(tokens, hidden, inter, experts, begin, local, 1, seed=local)
+    routes = np.concatenate([np.repeat(np.arange(local) + begin, rows), np.full(remote, begin + local)]).astype(np.int32)
+    idx[:, 0] = np.random.default_rng(local).permutation(routes)
+    assert tokens // experts <= 20
+    y, counts = _run(ops, x_codes, x_scales, l1, l2, idx, weights, experts, begin, local)
+    np.testing.assert_array_equal(counts, rows)
+    ref = _oracle(x_codes, x_scales, l1, l2, idx, weights, begin)
+    assert np.linalg.norm(y - ref) <= 2e-2 * np.linalg.norm(ref)
+    tall, _ = _run(ops, x_codes, x_scales, l1, l2, idx, weights, experts, begin, local, tile_rows=64)
+    np.testing.assert_array_equal(y, tall)
+
+
 @pytest.mark.parametrize("tokens,hidden,inter,tile_rows", [
     (1000, 2304, 1280, 64),   # 320 + 288 tiles of 18 and 10 k tiles on 256 workgroups
     (1700, 1280, 768, 64),    # 10 and 6 k tiles: the shortest tile that still switches without letting the copies land
