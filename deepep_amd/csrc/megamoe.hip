@@ -364,6 +364,10 @@ __device__ __forceinline__ void mfma_fp8_fp4(v16f& acc, const v8i& a, const u32x
 }
 // 16-pass MFMA results may be read by other instruction types 19 wait states after issue at the earliest.
 __device__ __forceinline__ void settle_accumulators() { asm volatile("s_nop 15\n\ts_nop 7" ::: "memory"); }
+// The same behind builtin MFMAs, for accumulators that other code may read or move from here on.  The compiler inserts wait
+// states of its own, but counts an s_waitcnt as one of them, which it is not when nothing is left to wait for: a move of
+// an accumulator at the end of a branch, 18 states and an s_waitcnt behind the MFMA, read the last two registers stale.
+__device__ __forceinline__ void settle_accumulators(v16f (&acc)[2]) { asm volatile("s_nop 15\n\ts_nop 7" : "+v"(acc[0]), "+v"(acc[1])); }
 
 struct TileInfo {
     int expert, nt, row0, valid;  // row0 = first row of the tile in the expanded layout; valid rows <= kBM
@@ -1165,6 +1169,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void grouped_gemm_few_rows_kernel(G
                                                                                      static_cast<int>(col_scales[kParity][c][q >> 1]), 2 * step, x_scale);
                         }
                     });
+                    if constexpr (q > 0 && (q == 3 || !kMore)) settle_accumulators(acc);
                 }
                 if constexpr (kMore) load_weights(q, (span + 1) * 4 + q);
                 __builtin_amdgcn_sched_barrier(0);

@@ -211,6 +211,7 @@ def test_both_grouped_gemm_kernels_agree_bit_for_bit(ops, tokens, hidden, inter,
 @pytest.mark.parametrize("hidden,inter,local,rows", [
     (1024, 256, 3, [33, 1, 0]),              # a wave per workgroup; k = 1024 and 512
     (1088, 384, 6, [0, 31, 32, 0, 64, 5]),   # k = 1280 ends in half a span of scales
+    (1280, 1536, 6, [7, 40, 1, 0, 32, 2]),   # three whole spans
     (1088, 384, 40, [1, 0, 32, 33, 2] * 8),  # four waves per workgroup
     (512, 640, 70, [0, 3, 7] + [0] * 60 + [1, 0, 97, 32, 2, 0, 4]),  # more experts than a wave has lanes, one far over the mean
 ])
