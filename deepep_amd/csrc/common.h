@@ -92,6 +92,18 @@ constexpr int kWave = 64;
 // ---- device helpers -------------------------------------------------------------------------
 __device__ __forceinline__ float bf16_to_f32(uint32_t bits16) { return __uint_as_float(bits16 << 16); }
 
+// Inclusive sum over the wave's lanes, by row shifts and row broadcasts (an LDS permute per step costs 50 ns and more).
+__device__ __forceinline__ int wave_scan(int v)
+{
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);  // row_shr:1
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);  // row_shr:2
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);  // row_shr:4
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);  // row_shr:8
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // row_bcast:15 into rows 1 and 3
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // row_bcast:31 into rows 2 and 3
+    return v;
+}
+
 // Round-to-nearest-even fp32 -> bf16 bits, two at a time: lo in bits 0-15, hi in bits 16-31
 // (v_cvt_pk_bf16_f32; NaN stays a quiet NaN).
 typedef float dpep_f32x2 __attribute__((ext_vector_type(2)));

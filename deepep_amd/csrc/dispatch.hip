@@ -440,12 +440,7 @@ __global__ __launch_bounds__(kMaxThreads) void layout_dispatch_small_kernel(
         mine[j] = e < num_local ? first_row[e] : 0;
         sum += mine[j];
     }
-    int incl = sum;
-#pragma unroll
-    for (int d = 1; d < kWave; d <<= 1) {
-        const int up = __shfl_up(incl, d);
-        if (lane >= d) incl += up;
-    }
+    const int incl = wave_scan(sum);
     if (lane == kWave - 1) wave_sums[wave] = incl;
     __syncthreads();
     int offset = incl - sum;

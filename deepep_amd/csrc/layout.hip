@@ -14,6 +14,7 @@
 //            mask per expert in LDS (each lane ORs its bit in, then all read the mask back): a route's row is
 //            its expert's next free row plus the number of lower lanes in the mask.  The carry between steps
 //            lives in LDS.  There is no separate scan launch.
+// The smallest inputs take one workgroup, which holds everything (see "one workgroup" below).
 // Inputs whose chunks fit a wave's registers (at most kKeep steps of 64 routes) take ONE launch: the workgroups
 // (at most 65, far fewer than there are CUs, so all are resident together) count, publish their histograms as
 // self-validating words (count + the launch's tag in one 64-bit store), read each other's as soon as they appear, and
@@ -22,6 +23,7 @@
 // every route as having none, and leaves its number in the workspace's mailbox, where the host finds it; later layouts
 // on that workspace take two launches.  Larger inputs take two launches anyway.
 #include <mutex>
+#include <type_traits>
 
 #include "common.h"
 #include "mx.h"
@@ -82,11 +84,12 @@ __device__ __forceinline__ void fetch_experts(int (&experts)[kSteps], const IdxT
 // LDS of one workgroup.  running[w][e]: wave w's histogram, later its next free row of expert e; match[w][e]: bit
 // per lane of wave w whose route in the current step goes to expert e (all zero between steps); totals[e]: rows
 // of expert e.
-template <int kMaxLocal>
+template <int kMaxLocal, bool kOneLaunch>
 struct LayoutLds {
     int totals[kMaxLocal];
     int running[kWaves][kMaxLocal];
     unsigned long long match[kWaves][kMaxLocal];
+    int seen[kOneLaunch ? kWaves : 1][kOneLaunch ? kMaxLocal : 1];  // one-launch kernel: routes of expert e that wave w has ranked
     int partial[kThreads * 2];
     int wave_sums[kWaves];
     int timed_out;  // one-launch kernel: some thread's wait for another workgroup's histogram ran out
@@ -155,13 +158,35 @@ __device__ __forceinline__ void assign_step(int e, int route, int end, unsigned 
     }
 }
 
+// One 64-route step of the ranking: the number of routes of this wave, so far, with this lane's expert.
+__device__ __forceinline__ int rank_step(int e, unsigned long long* __restrict__ match, int* __restrict__ seen)
+{
+    if (e >= 0)
+        __hip_atomic_fetch_or(match + e, 1ull << (threadIdx.x & 63), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+    wave_sync();
+    int rank = 0, ahead = 0, group = 0;
+    if (e >= 0) {
+        const unsigned long long mask = match[e];
+        ahead = __popcll(mask & lanes_below());
+        group = __popcll(mask);
+        rank = seen[e] + ahead;
+    }
+    wave_sync();  // every lane has read its expert's mask and count before the first lane of the group moves them
+    if (e >= 0 && ahead == 0) {
+        seen[e] = rank + group;
+        match[e] = 0ull;
+    }
+    wave_sync();
+    return rank;
+}
+
 template <typename IdxT>
 __global__ __launch_bounds__(kThreads) void layout_count_kernel(const IdxT* __restrict__ idx, int n_routes,
                                                                 int num_experts, int expert_begin, int num_local,
                                                                 int chunk, int num_chunks, int* __restrict__ wave_hist,
                                                                 int* __restrict__ block_hist, IdxT* __restrict__ idx_copy)
 {
-    __shared__ LayoutLds<DPEP_MAX_LOCAL_EXPERTS> lds;
+    __shared__ LayoutLds<DPEP_MAX_LOCAL_EXPERTS, false> lds;
     const int wave = threadIdx.x >> 6;
     const int g = blockIdx.x * kWaves + wave;
     const int begin = g < num_chunks ? g * chunk : 0;
@@ -373,12 +398,7 @@ __device__ __forceinline__ bool expert_bases(Lds& lds, const int* __restrict__ w
         mine[j] = e < num_local ? lds.totals[e] : 0;
         local_sum += mine[j];
     }
-    int incl = local_sum;
-#pragma unroll
-    for (int d = 1; d < kWave; d <<= 1) {
-        const int up = __shfl_up(incl, d);
-        if (lane >= d) incl += up;
-    }
+    const int incl = wave_scan(local_sum);
     if (lane == kWave - 1) lds.wave_sums[wave] = incl;
     __syncthreads();
     int offset = incl - local_sum;
@@ -419,7 +439,7 @@ __global__ __launch_bounds__(kThreads) void layout_assign_kernel(
     int* __restrict__ route_to_row, int* __restrict__ row_to_route, SendCounts send, uint32_t* __restrict__ mailbox,
     uint32_t sequence)
 {
-    __shared__ LayoutLds<DPEP_MAX_LOCAL_EXPERTS> lds;
+    __shared__ LayoutLds<DPEP_MAX_LOCAL_EXPERTS, false> lds;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int g = blockIdx.x * kWaves + wave;
     const int begin = g < num_chunks ? g * chunk : 0;
@@ -450,14 +470,18 @@ __global__ __launch_bounds__(kThreads) void layout_assign_kernel(
 // thing they do, when it has long been there).  So all workgroups of a launch agree on the tag; a launch that ran
 // out of time may use two tags, and the atomic max still leaves the epoch above both.  Replays of a captured launch
 // therefore get fresh tags without any host involvement.  40 tag bits last 10^12 launches.
-// Count, exchange, assign in one launch; every wave keeps the ids of its chunk (at most kKeep steps) in registers.
+// Count, exchange, assign in one launch; every wave keeps the ids of its chunk (at most kSteps steps) in registers, and ranks
+// them within (wave, expert) while the words travel.  kSteps is the smallest of 4, 8 and kKeep that holds the chunk: the code is
+// straight-line, every launch finds the instruction caches cold, and steps that do nothing still had to be fetched (65 536
+// routes, 256 per wave, launches back to back: 6.8 us with sixteen steps that assigned behind the exchange, 6.3 with four
+// ranked ahead of it; with sixteen ranked ahead of it 7.7).
 // `rows` = histogram rows to wait for (the workgroups that own chunks; one more in a test that wants the wait to run out),
 // `limit_ticks` the bound of that wait (100 MHz ticks).
 // kMega: a MegaMoE forward's layout (at most 128 local experts).  Workgroups behind the reporter prepare the input rows
 // (quantise or pad them), which does not depend on the routing, and every workgroup of the layout writes a piece of the shared
 // experts' rows once it knows R: up to three launches fewer (777 tokens of 2880 BF16 columns with a shared expert: layout 8.3 +
 // quantise 4.1 + pad 3.3 + shared rows 1.9 us as launches of their own).
-template <typename IdxT, bool kMega>
+template <typename IdxT, bool kMega, int kSteps>
 __global__ __launch_bounds__(kThreads) void layout_fused_kernel(
     const IdxT* __restrict__ idx, int n_routes, int num_experts, int expert_begin, int num_local, int padded_local,
     int chunk, int num_chunks, int* __restrict__ counts, int* __restrict__ psum, int* __restrict__ offsets,
@@ -466,10 +490,10 @@ __global__ __launch_bounds__(kThreads) void layout_fused_kernel(
     unsigned long long* __restrict__ tagged, int num_blocks, int rows, long long limit_ticks, uint32_t* __restrict__ timeouts,
     uint32_t launch_id, MegaFront front)
 {
-    __shared__ LayoutLds<kMega ? kMegaExperts : DPEP_MAX_LOCAL_EXPERTS> lds;
+    __shared__ LayoutLds<kMega ? kMegaExperts : DPEP_MAX_LOCAL_EXPERTS, true> lds;
     if (kMega && static_cast<int>(blockIdx.x) > num_blocks) {
         __shared__ __attribute__((aligned(16))) uint8_t staged[kFrontThreads / 2];
-        prepare_rows(front, blockIdx.x - num_blocks - 1, staged);
+        prepare_rows<kFrontThreads>(front, blockIdx.x - num_blocks - 1, staged);
         return;
     }
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -485,16 +509,22 @@ __global__ __launch_bounds__(kThreads) void layout_fused_kernel(
         lds.timed_out = 0;
         if (reporter) __hip_atomic_store(reporter_tag, lds.tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-    int experts[kKeep];
+    int experts[kSteps];
     fetch_experts(experts, idx, begin, end, n_routes, num_experts, expert_begin, num_local, idx_copy);
     clear_wave_lds(lds, num_local);
+    for (int e = lane; e < num_local; e += kWave) lds.seen[wave][e] = 0;
 #pragma unroll
-    for (int i = 0; i < kKeep; ++i) count_step(experts[i], lds.running[wave]);
+    for (int i = 0; i < kSteps; ++i) count_step(experts[i], lds.running[wave]);
     __syncthreads();
     const unsigned long long tag = lds.tag;
     // (the reporter owns no chunk and publishes nothing: row num_blocks is only ever waited for by a test that wants
     // the wait to run out)
     if (!reporter) publish_tagged(lds, num_local, tagged, tag);
+    // Ranked while the words travel: behind the exchange a route's row is one LDS read away.
+    int rank[kSteps];
+#pragma unroll
+    for (int i = 0; i < kSteps; ++i)
+        if (begin + i * kWave < end) rank[i] = rank_step(experts[i], lds.match[wave], lds.seen[wave]);
     // The reporter gives up first (the others wait twice as long): a launch that the reporter passes as valid is then
     // one in which every histogram arrived within the reporter's bound, so another workgroup can only have run out of
     // time if its own wait began more than a whole bound before the reporter's.  What remains of that window is closed
@@ -507,10 +537,14 @@ __global__ __launch_bounds__(kThreads) void layout_fused_kernel(
     unsigned long long reporter_seen = threadIdx.x == 0 && !reporter ? load_word(reporter_tag) : 0ull;
     if (in_time) {
 #pragma unroll
-        for (int i = 0; i < kKeep; ++i)
-            if (begin + i * kWave < end)
-                assign_step(experts[i], begin + i * kWave + lane, end, lds.match[wave], lds.running[wave], route_to_row,
-                            row_to_route);
+        for (int i = 0; i < kSteps; ++i) {
+            const int route = begin + i * kWave + lane;
+            if (route < end) {
+                const int row = experts[i] >= 0 ? lds.running[wave][experts[i]] + rank[i] : -1;
+                route_to_row[route] = row;
+                if (row >= 0) row_to_route[row] = route;
+            }
+        }
     } else {
         // Some workgroup's histogram is missing: rows computed without it could lie anywhere.  No route gets a row
         // (and the counts above are all zero).
@@ -539,13 +573,116 @@ __global__ __launch_bounds__(kThreads) void layout_fused_kernel(
     }
 }
 
+// ---- one workgroup ---------------------------------------------------------------------------------------------------
+// Up to kSingleRoutes routes over up to kSingleExperts local experts: sixteen waves of ONE workgroup hold them all, and
+// nothing travels between workgroups (the exchange of the kernel above takes 2 us, whatever the size).  Every wave ranks
+// its routes within (wave, expert) as it counts them; after one scan over waves and experts a route's row is one LDS read away.
+// Bound by latencies (the ids 1 us, the scans, the stores) and by what one CU's LDS and store path take: 0.13 us per 256 routes.
+// row_to_route is scattered in LDS and leaves as whole lines: scattered stores cost a cycle per lane, 1.3 us at 4096 routes.
+// Measured on an MI355X, launches back to back, against the kernel above: 2400 routes over 256 experts 5.7 -> 3.8 us, 4096:
+// 5.9 -> 4.5, 4096 of which one in eight is local 5.5 -> 3.9; at 6144 routes both take 5.9 us, at 16 384 10.7 against 6.4.
+constexpr int kSingleWaves = 16;
+constexpr int kSingleThreads = kSingleWaves * kWave;
+constexpr int kSingleExperts = 256;
+constexpr int kSingleSteps = 4;  // 64-route steps per wave
+constexpr int kSingleRoutes = kSingleThreads * kSingleSteps;
+
+// kMega: as above; the workgroups behind the first prepare rows.
+template <typename IdxT, bool kMega>
+__global__ __launch_bounds__(kSingleThreads) void layout_single_kernel(
+    const IdxT* __restrict__ idx, int n_routes, int num_experts, int expert_begin, int num_local, int* __restrict__ counts,
+    int* __restrict__ psum, int* __restrict__ offsets, int* __restrict__ num_rows, int* __restrict__ route_to_row,
+    int* __restrict__ row_to_route, IdxT* __restrict__ idx_copy, SendCounts send, uint32_t* __restrict__ mailbox, uint32_t sequence,
+    MegaFront front)
+{
+    __shared__ int rows_of[kSingleWaves][kSingleExperts];  // routes per wave and expert, later the wave's first row
+    __shared__ unsigned long long match[kSingleWaves][kSingleExperts];
+    __shared__ int totals[kSingleExperts];
+    __shared__ int wave_sums[kSingleWaves];
+    __shared__ int route_of[kSingleSteps * kSingleThreads];  // row_to_route: scattered here, copied out in order
+    if (kMega && blockIdx.x > 0) {
+        prepare_rows<kSingleThreads>(front, blockIdx.x - 1, reinterpret_cast<uint8_t*>(match));
+        return;
+    }
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int steps = (n_routes + kSingleThreads - 1) / kSingleThreads;  // the routes are dealt out evenly
+    const int begin = min(wave * steps * kWave, n_routes), end = min(begin + steps * kWave, n_routes);
+    int experts[kSingleSteps], rank[kSingleSteps];
+    fetch_experts(experts, idx, begin, end, n_routes, num_experts, expert_begin, num_local, idx_copy);
+    for (int e = lane; e < num_local; e += kWave) {
+        rows_of[wave][e] = 0;
+        match[wave][e] = 0ull;
+    }
+    wave_sync();
+#pragma unroll
+    for (int i = 0; i < kSingleSteps; ++i)
+        if (begin + i * kWave < end) rank[i] = rank_step(experts[i], match[wave], rows_of[wave]);
+    __syncthreads();
+    int own[kSingleWaves], total = 0;
+    if (tid < num_local) {
+#pragma unroll
+        for (int w = 0; w < kSingleWaves; ++w) {
+            own[w] = rows_of[w][tid];
+            total += own[w];
+        }
+    }
+    const int incl = wave_scan(total);
+    if (lane == kWave - 1) wave_sums[wave] = incl;
+    if (tid < kSingleExperts) totals[tid] = total;
+    __syncthreads();
+    int sums[kSingleExperts / kWave], all = 0, offset = incl - total;
+#pragma unroll
+    for (int w = 0; w < kSingleExperts / kWave; ++w) {
+        sums[w] = wave_sums[w];
+        if (w < wave) offset += sums[w];
+        all += sums[w];
+    }
+    if (tid < num_local) {
+        int next = offset;
+#pragma unroll
+        for (int w = 0; w < kSingleWaves; ++w) {
+            rows_of[w][tid] = next;
+            next += own[w];
+        }
+        counts[tid] = total;
+        psum[tid] = next;
+        offsets[tid + 1] = next;
+        if (send.counts != nullptr) send.counts[send.expert_begin + tid] = next;
+    }
+    if (tid == 0) {
+        offsets[0] = 0;
+        num_rows[0] = all;
+    }
+    if (mailbox != nullptr) {
+        if (tid * 4 < num_local) {
+            const int four[4] = {totals[tid * 4], totals[tid * 4 + 1], totals[tid * 4 + 2], totals[tid * 4 + 3]};
+            mailbox_store_counts(mailbox, tid * 4, four, sequence, mailbox_narrow(n_routes));
+        }
+        if (tid == 0) mailbox_store_rows(mailbox, all, sequence);
+    }
+    send_counts_of_others(send, num_local, all, tid, kSingleThreads);
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < kSingleSteps; ++i) {
+        const int route = begin + i * kWave + lane;
+        if (route < end) {
+            const int row = experts[i] >= 0 ? rows_of[wave][experts[i]] + rank[i] : -1;
+            route_to_row[route] = row;
+            if (row >= 0) route_of[row] = route;
+        }
+    }
+    __syncthreads();
+    for (int row = tid; row < all; row += kSingleThreads) row_to_route[row] = route_of[row];
+    if (kMega && front.num_shared > 0) shared_rows(front, all, num_local, offsets, row_to_route, tid, kSingleThreads);
+}
+
 // The same preparation behind a layout that took two launches.
 __global__ __launch_bounds__(kFrontThreads) void mega_front_kernel(MegaFront front, const int* __restrict__ num_rows, int num_local,
                                                                    int* __restrict__ offsets, int* __restrict__ row_to_route)
 {
     __shared__ __attribute__((aligned(16))) uint8_t staged[kFrontThreads / 2];
-    const unsigned blocks = (front.units + kFrontThreads - 1) / kFrontThreads;
-    if (blockIdx.x < blocks) prepare_rows(front, blockIdx.x, staged);
+    const unsigned blocks = front_blocks(front, kFrontThreads);
+    if (blockIdx.x < blocks) prepare_rows<kFrontThreads>(front, blockIdx.x, staged);
     else shared_rows(front, num_rows[0], num_local, offsets, row_to_route, (blockIdx.x - blocks) * kFrontThreads + threadIdx.x,
                      (gridDim.x - blocks) * kFrontThreads);
 }
@@ -650,6 +787,17 @@ int launch_layout(void* ws, const IdxT* idx, int num_tokens, int num_topk, int n
         w->mailbox_narrow = mailbox_narrow(n_routes);
     }
     uint32_t* mailbox = report_to_host ? w->mailbox_device : nullptr;
+    // (a test that wants the exchange to run out of time gets the kernel that has one)
+    if (one_launch && n_routes <= kSingleRoutes && num_local <= kSingleExperts && w->exchange_extra_rows == 0) {
+        auto launch = [&](auto kernel, unsigned more, const MegaFront& f) {
+            hipLaunchKernelGGL(kernel, dim3(1 + more), dim3(kSingleThreads), 0, stream, idx, n_routes, num_experts, expert_begin,
+                               num_local, counts, psum, offsets, num_rows, route_to_row, row_to_route, idx_copy, send, mailbox,
+                               w->sequence, f);
+        };
+        if (front != nullptr) launch(layout_single_kernel<IdxT, true>, front_blocks(*front, kSingleThreads), *front);
+        else launch(layout_single_kernel<IdxT, false>, 0u, MegaFront{});
+        return launch_status("layout_single");
+    }
     if (one_launch) {
         char* sync = static_cast<char*>(w->sync);
         auto launch = [&](auto kernel, unsigned more, const MegaFront& f) {
@@ -659,8 +807,14 @@ int launch_layout(void* ws, const IdxT* idx, int num_tokens, int num_topk, int n
                                reinterpret_cast<unsigned long long*>(sync + kSyncTagged), blocks, blocks + w->exchange_extra_rows,
                                w->exchange_ticks, w->mailbox_device + kMailboxTimeout, w->layout_launches, f);
         };
-        if (front != nullptr) launch(layout_fused_kernel<IdxT, true>, front_blocks(*front), *front);
-        else launch(layout_fused_kernel<IdxT, false>, 0u, MegaFront{});
+        auto launch_steps = [&](auto steps_constant) {
+            constexpr int kSteps = decltype(steps_constant)::value;
+            if (front != nullptr) launch(layout_fused_kernel<IdxT, true, kSteps>, front_blocks(*front, kFrontThreads), *front);
+            else launch(layout_fused_kernel<IdxT, false, kSteps>, 0u, MegaFront{});
+        };
+        if (chunk <= 4 * kWave) launch_steps(std::integral_constant<int, 4>{});
+        else if (chunk <= 8 * kWave) launch_steps(std::integral_constant<int, 8>{});
+        else launch_steps(std::integral_constant<int, kKeep>{});
         return launch_status("layout_fused");
     }
     if (int rc = enqueue_count_and_assign<IdxT>(idx, n_routes, num_experts, expert_begin, num_local, padded, chunk, num_chunks,
@@ -669,7 +823,7 @@ int launch_layout(void* ws, const IdxT* idx, int num_tokens, int num_topk, int n
         return rc;
     if (front != nullptr && (front->units > 0 || front->num_shared > 0)) {
         const unsigned rows_blocks = (static_cast<unsigned>(front->num_shared) * front->num_tokens + kFrontThreads - 1) / kFrontThreads;
-        hipLaunchKernelGGL(mega_front_kernel, dim3(front_blocks(*front) + rows_blocks), dim3(kFrontThreads), 0, stream, *front, num_rows,
+        hipLaunchKernelGGL(mega_front_kernel, dim3(front_blocks(*front, kFrontThreads) + rows_blocks), dim3(kFrontThreads), 0, stream, *front, num_rows,
                            num_local, offsets, row_to_route);
         return launch_status("mega_front");
     }

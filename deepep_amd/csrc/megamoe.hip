@@ -1055,13 +1055,8 @@ __global__ __launch_bounds__(64 * kWaves, 2) void grouped_gemm_few_rows_kernel(G
         const int e = lane + 64 * h;
         tiles_through[h] = 0;
         if (64 * h >= p.num_local) continue;
-        int sum = e < p.num_local ? (p.offsets[e + 1] - p.offsets[e] + kRows - 1) / kRows : 0;
-#pragma unroll
-        for (int d = 1; d < 64; d *= 2) {
-            const int below = __shfl_up(sum, d);
-            if (lane >= d) sum += below;
-        }
-        tiles_through[h] = total + sum;
+        const int sum = e < p.num_local ? (p.offsets[e + 1] - p.offsets[e] + kRows - 1) / kRows : 0;
+        tiles_through[h] = total + wave_scan(sum);
         total = __builtin_amdgcn_readlane(tiles_through[h], 63);
     }
 

@@ -69,13 +69,14 @@ struct MegaFront {
     int num_shared, num_tokens, num_topk;
 };
 constexpr int kFrontThreads = 256;
-inline unsigned front_blocks(const MegaFront& f) { return (f.units + kFrontThreads - 1) / kFrontThreads; }
+inline __host__ __device__ unsigned front_blocks(const MegaFront& f, int threads) { return (f.units + threads - 1) / threads; }
 
-// One workgroup's piece of the input rows.  staged: 128 bytes of LDS, 16-byte aligned (the workgroup's scale bytes leave as
+// One workgroup's piece of the input rows.  staged: kThreads / 2 bytes of LDS, 16-byte aligned (the workgroup's scale bytes leave as
 // 16-byte stores).  Called by all threads.
+template <int kThreads>
 __device__ __forceinline__ void prepare_rows(const MegaFront& f, unsigned block, uint8_t* staged)
 {
-    const unsigned unit = block * kFrontThreads + threadIdx.x, per_row = f.hp / 16;
+    const unsigned unit = block * kThreads + threadIdx.x, per_row = f.hp / 16;
     const bool live = unit < f.units;
     const unsigned row = unit / per_row, at = unit - row * per_row;
     const bool real = live && at * 16 < static_cast<unsigned>(f.h);  // (h is a multiple of 32: both lanes of a block agree)
@@ -98,11 +99,11 @@ __device__ __forceinline__ void prepare_rows(const MegaFront& f, unsigned block,
     if (live) f.codes_out[unit] = codes;  // (cached: the GEMM gathers these rows next)
     if ((threadIdx.x & 1) == 0) staged[threadIdx.x >> 1] = static_cast<uint8_t>(byte);
     __syncthreads();
-    const unsigned first = block * (kFrontThreads / 2), blocks = f.units >> 1;
-    if (first + kFrontThreads / 2 <= blocks) {
-        if (threadIdx.x < kFrontThreads / 32)
+    const unsigned first = block * (kThreads / 2), blocks = f.units >> 1;
+    if (first + kThreads / 2 <= blocks) {
+        if (threadIdx.x < kThreads / 32)
             *reinterpret_cast<u32x4*>(f.scales_out + first + threadIdx.x * 16) = *reinterpret_cast<const u32x4*>(staged + threadIdx.x * 16);
-    } else if (threadIdx.x < blocks - first && threadIdx.x < kFrontThreads / 2) {
+    } else if (threadIdx.x < blocks - first && threadIdx.x < kThreads / 2) {
         f.scales_out[first + threadIdx.x] = staged[threadIdx.x];
     }
 }

@@ -109,3 +109,16 @@ def test_layout_at_the_largest_expert_counts(ops, ws, experts, begin, local, tok
     finally:
         ws.tune("layout_one_launch", 1)
     _compare(_layout_static(_lib.load(), idx, experts, begin, local), want, case)
+
+
+@pytest.mark.parametrize("local", [1, 63, 255, 256, 257])
+@pytest.mark.parametrize("tokens", [1, 64, 1023, 1024, 1025, 4095, 4096, 4097, 16384, 16385, 65537])
+def test_layout_where_its_one_launch_kernels_change(ops, ws, tokens, local):
+    """One workgroup up to 4096 routes and 256 local experts, several beyond, of four, eight or sixteen steps per wave."""
+    rng = np.random.default_rng(tokens * 7 + local)
+    ids = rng.integers(0, local + 3, size=(tokens, 1)).astype(np.int64)
+    want = olayout.layout(ids, local + 3, 1, local)
+    got = ops.layout(ws, torch.from_numpy(ids).cuda(), local + 3, 1, local)
+    host_counts, host_rows = ops.layout_wait(ws, local)
+    assert host_rows == want["num_rows"] and host_counts == want["counts"].tolist()
+    _compare(got, want, (tokens, local))
