@@ -30,6 +30,7 @@ SIGNATURES = {
     "dpep_layout_static": (_I, (_P, _I, _I, _I, _I, _I, _P, _P, _P, _P, _P, _P, _P)),
     "dpep_layout_wait": (_I, (_P, _P, _I, ctypes.POINTER(ctypes.c_int32), ctypes.c_longlong)),
     "dpep_layout_ready": (_I, (_P,)),
+    "dpep_stream_raise": (_I, (_P, ctypes.c_uint64, _P)),
     "dpep_dispatch_fresh": (_I, (_P, _P, _P)),
     "dpep_dispatch_store_policy": (_I, (_I,)),
     "dpep_dispatch_copy": (_I, (_P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P, _P, _P, _P)),

@@ -166,7 +166,7 @@ struct EventPool {
     }
 };
 
-// A counter that one stream raises and other streams wait for (hipStreamWriteValue64 / hipStreamWaitValue64): the cheaper way to
+// A counter that one stream raises and other streams wait for (dpep_stream_raise / hipStreamWaitValue64): the cheaper way to
 // order two streams.  A recorded event plus a wait costs 8 us of host time and 7 of the GPU's when the event is still
 // pending, this 4.5 and 5 (two streams passing the turn back and forth).  Only one stream at a time may raise a counter,
 // or a later value could be seen before an earlier one was written; values only grow, so a counter may go from owner to owner.
@@ -311,8 +311,8 @@ Marker* marker_new(const std::shared_ptr<EventPool>& pool, Counter* counter, con
             pool->give_back(e);
             return reinterpret_cast<Marker*>(raise_hip("hipEventRecord", err));
         }
-    } else if (hipError_t err = hipStreamWriteValue64(stream.raw, counter->word, ++counter->raised, 0); err != hipSuccess) {
-        return reinterpret_cast<Marker*>(raise_hip("hipStreamWriteValue64", err));
+    } else if (int rc = dpep_stream_raise(counter->word, ++counter->raised, stream.raw); rc != DPEP_OK) {
+        return reinterpret_cast<Marker*>(raise_native(rc));
     }
     Marker* m = reinterpret_cast<Marker*>(MarkerType.tp_alloc(&MarkerType, 0));
     if (m == nullptr) {
@@ -558,8 +558,8 @@ bool join_caller(Exchange* e, const Stream& caller)
     Counter* c = e->caller_counter;
     if (c != nullptr && (e->counted == caller || c->reached(c->raised)) && !capturing(caller.raw)) {
         e->counted = caller;
-        hipError_t err = hipStreamWriteValue64(caller.raw, c->word, ++c->raised, 0);
-        if (err == hipSuccess) err = hipStreamWaitValue64(e->comm.raw, c->word, c->raised, hipStreamWaitValueGte, ~0ull);
+        if (int rc = dpep_stream_raise(c->word, ++c->raised, caller.raw); rc != DPEP_OK) return raise_native(rc) != nullptr;
+        const hipError_t err = hipStreamWaitValue64(e->comm.raw, c->word, c->raised, hipStreamWaitValueGte, ~0ull);
         return err == hipSuccess ? true : raise_hip("ordering two streams", err) != nullptr;
     }
     return wait_for_stream(e, e->comm.raw, caller.raw);

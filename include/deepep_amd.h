@@ -97,6 +97,9 @@ int dpep_layout_static(const int64_t* topk_idx, int num_tokens, int num_topk, in
 int dpep_layout_wait(void* ws, int32_t* counts_host, int num_local, int32_t* num_rows_host, long long timeout_us);
 /* 1 if the most recent layout launched on ws has reported (dpep_layout_wait would not have to wait), else 0. */
 int dpep_layout_ready(void* ws);
+/* Stores value in *word (8-byte aligned, GPU-accessible memory such as hipMallocSignalMemory's) behind everything the stream was
+ * given before: what other streams' hipStreamWaitValue64 wait for. */
+int dpep_stream_raise(void* word, uint64_t value, void* stream);
 
 /* Expand-permute payload dispatch: out[row(t,s)] = x[t] for every route with a row.
  * Replaces dispatch() (csrc/ops/dispatch.cpp:82-211 -> dispatch_kernel, csrc/kernels/dispatch/dispatch.cpp:628)

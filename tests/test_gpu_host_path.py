@@ -266,3 +266,16 @@ def test_asynchronous_cached_calls_in_a_hip_graph():
     finally:
         torch.cuda.synchronize()
         buffer.destroy()
+
+
+def test_stream_raise_stores_behind_earlier_work_and_refuses_bad_words():
+    from deepep_amd import _lib
+
+    lib = _lib.load()
+    word = torch.zeros(2, dtype=torch.int64, device="cuda")
+    stream = torch.cuda.current_stream().cuda_stream
+    word.fill_(3)
+    assert lib.dpep_stream_raise(word.data_ptr(), 5_000_000_000, stream) == 0
+    assert word.tolist() == [5_000_000_000, 3]
+    for bad in (0, word.data_ptr() + 4):
+        assert lib.dpep_stream_raise(bad, 1, stream) != 0
