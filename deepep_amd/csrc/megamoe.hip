@@ -11,6 +11,7 @@
 //   B: lane l holds column l%32; 4 VGPRs = 32 nibbles k in [32g, 32g+32), low nibble first
 //   scales: lane l supplies the e8m0 byte of (row or column l%32, 32-wide k block l/32)
 //   D: acc[j] is row (j/4)*8 + (l/32)*4 + j%4, column l%32
+#include <algorithm>
 #include <atomic>
 #include <type_traits>
 #include <utility>
@@ -1629,6 +1630,11 @@ int allow_lds(Kernel kernel, int bytes, std::atomic<bool>* configured, int max_d
     return DPEP_OK;
 }
 
+// Two workgroups on a CU each run at about half speed: worth it where that does not add rounds (512 tiles on 256 CUs: one
+// round of 512 instead of two of 256, with twice the requests in flight; 700 tiles: two slow rounds would replace three
+// fast ones).
+bool two_workgroups_pay(double tiles, int cus) { return 2.0 * ceil(tiles / (2.0 * cus)) <= ceil(tiles / cus); }
+
 template <int RT, bool kGateUp>
 int launch_gemm_rt(const GemmParams& p, double expected_tiles, hipStream_t stream, const char* what)
 {
@@ -1637,12 +1643,8 @@ int launch_gemm_rt(const GemmParams& p, double expected_tiles, hipStream_t strea
         constexpr int kLds = ColCfg<RT>::kLdsBytes;
         static std::atomic<bool> configured[kMaxDevices];
         if (int rc = allow_lds(&grouped_gemm_colwave_kernel<RT, kGateUp>, kLds, configured, kMaxDevices)) return rc;
-        // Two workgroups on a CU each run at about half speed: worth it where that does not add rounds (512 tiles on
-        // 256 CUs: one round of 512 instead of two of 256, with twice the requests in flight; 700 tiles: two slow rounds
-        // would replace three fast ones).
         const int cus = gemm_grid();
-        int per_cu = 1;
-        if (ColCfg<RT>::kWorkgroupsPerCu == 2 && 2.0 * ceil(expected_tiles / (2.0 * cus)) <= ceil(expected_tiles / cus)) per_cu = 2;
+        const int per_cu = ColCfg<RT>::kWorkgroupsPerCu == 2 && two_workgroups_pay(expected_tiles, cus) ? 2 : 1;
         hipLaunchKernelGGL((grouped_gemm_colwave_kernel<RT, kGateUp>), dim3(cus * per_cu), dim3(kGemmThreads), kLds, stream, p);
         return launch_status(what);
     }
@@ -1653,14 +1655,21 @@ int launch_gemm_rt(const GemmParams& p, double expected_tiles, hipStream_t strea
     return launch_status(what);
 }
 
+// How many rows an expert is expected to have (the true counts stay on the device).
+struct ExpectedRows {
+    int average;    // over routed and shared experts
+    double routed;  // of a routed expert
+    double spread;  // standard deviation of that: a token goes to a given expert or not
+    int shared;     // of a shared expert: every token
+};
+
 // Row-tile height: the cheapest of 64 / 128 / 192 rows by a small cost model, judged from the expected rows per expert (the true counts
-// stay on the device).  Routing scatters the counts around that mean (about +-sqrt(mean)), and one expert a few
-// rows over a multiple of the tile height costs a whole extra row tile each: the tile count is therefore the
-// expectation of ceil(rows / height) under a normal spread, not ceil(mean / height).  (Mean 256 over 8 experts:
-// 128-row tiles need 2.5 row tiles per expert on average = 320 tiles = two rounds on 256 CUs, 192-row tiles need
-// 2 = one round; measured 103 vs 80 us.)
+// stay on the device).  Routing scatters the counts around that mean, and one expert a few rows over a multiple of the tile
+// height costs a whole extra row tile each: the tile count is therefore the expectation of ceil(rows / height) under a
+// normal spread, not ceil(mean / height); an expert without rows has no tile.  (Mean 256 over 8 experts: 128-row tiles need 2.5
+// row tiles per expert on average = 320 tiles = two rounds on 256 CUs, 192-row tiles need 2 = one round; measured 94 vs 67 us.)
 template <bool kGateUp>
-int launch_gemm(const GemmParams& p, int expected_rows_per_expert, hipStream_t stream, const char* what)
+int launch_gemm(const GemmParams& p, const ExpectedRows& expected, hipStream_t stream, const char* what)
 {
     const int cus = gemm_grid();
     const int n_tiles = p.n / kBN;
@@ -1668,7 +1677,7 @@ int launch_gemm(const GemmParams& p, int expected_rows_per_expert, hipStream_t s
     // line lies where a tile of 32 still holds nearly all experts.  (7168 x 2048, 32 of 256 experts, whole forward, 64-row
     // tiles -> few rows: mean 16: 153 -> 137 us, 20: 149 -> 138, 24: 148 -> 160, 32: 152 -> 208.)
     // Source rows are addressed with 32 bits here.
-    if (expected_rows_per_expert <= 20 && p.column_waves && p.forced_rt == 0 &&
+    if (expected.average <= 20 && p.column_waves && p.forced_rt == 0 &&
         (!kGateUp || static_cast<long long>(p.a_rows) * p.k < (1LL << 32))) {
         const int tiles = p.num_local * n_tiles;
         // One workgroup per column tile fills half the CUs or fewer: a CU draws no more than about 50 GB/s from memory, so
@@ -1680,29 +1689,33 @@ int launch_gemm(const GemmParams& p, int expected_rows_per_expert, hipStream_t s
             hipLaunchKernelGGL((grouped_gemm_few_rows_kernel<kGemmWaves, kGateUp>), dim3(tiles), dim3(kGemmThreads), 0, stream, p);
         return launch_status(what);
     }
-    const double mean = expected_rows_per_expert > 1 ? expected_rows_per_expert : 1;
-    const double sigma = sqrt(mean);
+    const double mean = expected.routed;
+    const int num_shared = p.num_local - p.num_routed;
+    const int kind = p.column_waves && p.k % 512 == 0 ? 0 : 1;  // the kernel that launch_gemm_rt takes
     int best = 2;
     double best_cost = 1e30, tiles_of[4] = {0.0, 0.0, 0.0, 0.0};
     for (int rt = 1; rt <= 3; ++rt) {
         const int bm = 64 * rt;
-        double m_tiles = 1.0;  // E[ceil(X / bm)] = sum over j >= 0 of P(X > j * bm)
-        for (int j = 1; j * bm < mean + 6.0 * sigma; ++j) m_tiles += 0.5 * erfc((j * bm - mean) / (sigma * 1.4142135623730951));
-        const double tiles = p.num_local * m_tiles * n_tiles;
+        double m_tiles = 1.0 - exp(-mean);  // E[ceil(X / bm)] = sum over j >= 0 of P(X > j * bm)
+        for (int j = 1; j * bm < mean + 6.0 * expected.spread; ++j)
+            m_tiles += 0.5 * erfc((j * bm + 0.5 - mean) / (expected.spread * 1.4142135623730951));
+        const double row_tiles = p.num_routed * m_tiles + static_cast<double>(num_shared) * ((expected.shared + bm - 1) / bm);
+        const double tiles = row_tiles * n_tiles;
         tiles_of[rt] = tiles;
-        const double rounds = ceil(tiles / cus - 0.02);  // a stray tile in one launch out of fifty does not count
-        // Microseconds, fitted to kernel traces on an MI355X over shares from 32 to 2048 rows per expert, 4 to 32
-        // experts and two problem sizes (it reproduced the measured order of the three heights in 14 of 16 small cases,
-        // was within 7 % in the other two, and in the many-round cases of a large batch): once per launch the part of the
-        // first tile that nothing overlaps (the 192-row kernel's three-stage ring starts slowly), per tile its epilogue
-        // and switch, per k tile the main loop; an expert with a single row tile streams its weight tile from HBM with
-        // nobody to share it with, which adds about 0.3 us per k tile whatever the height.
-        // (These figures are the column-wave kernel's; how to refit them: force each height with the workspace setting
-        // "gemm_tile_rows" on a many-round launch, take a kernel trace, and solve time = rounds * (per tile + k tiles * per
-        // item) over two k lengths: the two GEMMs of one forward give them.)
-        constexpr double kFirst[3] = {0.0, 0.0, 4.7}, kPerTile[3] = {4.0, 3.0, 3.4}, kPerItem[3] = {0.50, 0.83, 1.15};
-        const double per_item = kPerItem[rt - 1] + (m_tiles <= 1.2 ? 0.3 : 0.0);
-        const double cost = kFirst[rt - 1] + (rounds < 1.0 ? 1.0 : rounds) * (kPerTile[rt - 1] + (p.k / kBK) * per_item);
+        // Rounds of one workgroup per CU; a stray tile in one launch out of a hundred does not count.
+        const bool in_pairs = rt == 1 && kind == 0 && two_workgroups_pay(tiles, cus);
+        const double rounds = in_pairs ? 2.0 * ceil(tiles / (2.0 * cus) - 0.01) : ceil(tiles / cus - 0.01);
+        // Microseconds, fitted to kernel traces of both GEMMs on an MI355X at 285 shapes (2 to 64 experts, up to 5000 rows each,
+        // k from 512 to 8192), [column waves, 2 x 2][height]: once per launch, per tile its epilogue and switch, per k tile the
+        // main loop, and per k tile what it costs to stream the weights from memory, shared by the row tiles of an expert.
+        // Over them the height it picks is 0.3 % slower than the best on average and 11 % at worst.  (64 experts of
+        // 7168 x 2048, whole forward with the heights it picks / with 64 rows throughout: 64 rows each 355 / 414 us; 80:
+        // 373 / 535; 128: 485 / 661.)
+        // How to refit: force each height with the workspace setting "gemm_tile_rows" and take a kernel trace.
+        constexpr double kFirst[2][3] = {{1.8, 0.3, 0.8}, {1.4, 0.9, 1.0}}, kPerTile[2][3] = {{4.5, 6.0, 7.9}, {5.0, 6.4, 8.7}};
+        constexpr double kPerItem[2][3] = {{0.46, 0.74, 1.02}, {0.46, 0.75, 0.99}}, kWeights[2][3] = {{0.09, 0.04, 0.09}, {0.12, 0.07, 0.10}};
+        const double per_item = kPerItem[kind][rt - 1] + kWeights[kind][rt - 1] * p.num_local / std::max(row_tiles, 1e-3);
+        const double cost = kFirst[kind][rt - 1] + (rounds < 1.0 ? 1.0 : rounds) * (kPerTile[kind][rt - 1] + (p.k / kBK) * per_item);
         if (cost < best_cost - 1e-9) {
             best_cost = cost;
             best = rt;
@@ -1903,17 +1916,17 @@ bool replay_column_waves(int my_tiles, int ktiles, int epilogue_stores, int slac
     return ok;
 }
 
-int launch_gemm1(const GemmParams& p, int expected_rows_per_expert, hipStream_t stream)
+int launch_gemm1(const GemmParams& p, const ExpectedRows& expected, hipStream_t stream)
 {
     if (int rc = check_gemm("gemm1", p.n, p.k, p.num_local)) return rc;
     DPEP_REQUIRE(p.row_to_route != nullptr && p.topk >= 1, "gemm1: needs the row -> route map");
-    return launch_gemm<true>(p, expected_rows_per_expert, stream, "grouped_gemm1");
+    return launch_gemm<true>(p, expected, stream, "grouped_gemm1");
 }
 
-int launch_gemm2(const GemmParams& p, int expected_rows_per_expert, hipStream_t stream)
+int launch_gemm2(const GemmParams& p, const ExpectedRows& expected, hipStream_t stream)
 {
     if (int rc = check_gemm("gemm2", p.n, p.k, p.num_local)) return rc;
-    return launch_gemm<false>(p, expected_rows_per_expert, stream, "grouped_gemm2");
+    return launch_gemm<false>(p, expected, stream, "grouped_gemm2");
 }
 
 }  // namespace dpep
@@ -2182,7 +2195,9 @@ int dpep_megamoe_run(void* ws, const dpep_megamoe_call* call, void* stream)
     // token for a shared one.
     const long long expected_routed = static_cast<long long>(num_tokens) * num_topk * num_local / num_experts;
     const long long expected_rows = expected_routed + static_cast<long long>(num_tokens) * num_shared;
-    const int per_expert = static_cast<int>((expected_rows + g1.num_local - 1) / g1.num_local);
+    const double routed = static_cast<double>(num_tokens) * num_topk / num_experts;
+    const ExpectedRows expected = {static_cast<int>((expected_rows + g1.num_local - 1) / g1.num_local),
+                                   routed, sqrt(routed * std::max(0.0, 1.0 - static_cast<double>(num_topk) / num_experts)) + 1e-3, num_tokens};
     // Without shared experts most tokens of a share have no row: workgroups of the first GEMM that get no tile
     // zero those rows of y meanwhile, and the weighted reduce skips what they got through.
     int* fill_state = reinterpret_cast<int*>(base + l.fill_state);
@@ -2202,7 +2217,7 @@ int dpep_megamoe_run(void* ws, const dpep_megamoe_call* call, void* stream)
         g1.fill_stop = fill_stop;
     }
     g1.fill_state = fill_state;  // written even when nothing fills (then as "no fillers")
-    if (int rc = launch_gemm1(g1, per_expert, s)) return rc;
+    if (int rc = launch_gemm1(g1, expected, s)) return rc;
     GemmParams g2{};
     g2.a_codes = base + l.act_codes;
     g2.a_scales = base + l.act_scales;
@@ -2221,7 +2236,7 @@ int dpep_megamoe_run(void* ws, const dpep_megamoe_call* call, void* stream)
     g2.out_cols = hidden;
     g2.forced_rt = g1.forced_rt;
     g2.column_waves = g1.column_waves;
-    if (int rc = launch_gemm2(g2, per_expert, s)) return rc;
+    if (int rc = launch_gemm2(g2, expected, s)) return rc;
     return combine_routes(base + l.out2, topk_weights, route_to_row, num_tokens, num_topk,
                           static_cast<int>(expected_rows),
                           hidden, y, num_shared > 0 ? num_rows : nullptr, num_shared, fill ? fill_state : nullptr,
