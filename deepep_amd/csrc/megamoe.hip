@@ -370,6 +370,44 @@ __device__ __forceinline__ void settle_accumulators() { asm volatile("s_nop 15\n
 // an accumulator at the end of a branch, 18 states and an s_waitcnt behind the MFMA, read the last two registers stale.
 __device__ __forceinline__ void settle_accumulators(v16f (&acc)[2]) { asm volatile("s_nop 15\n\ts_nop 7" : "+v"(acc[0]), "+v"(acc[1])); }
 
+// The lane's number, worked out on the spot (two instructions) instead of kept in a register: the code that runs once
+// per tile or span (tile switches, scale requests, the epilogue) takes its lane-dependent addresses from this, so that the
+// item loop does not have to carry them.
+__device__ __forceinline__ int lane_now()
+{
+    int lane;
+    asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(lane));
+    return lane;
+}
+
+// Tiles before each expert: tile_base[0 .. kMaxMoeExperts], the entries past the last expert hold the total.  One wave, two experts
+// per lane: a walk over the experts, here and at every tile switch (where the matrix pipe waits for it), cost a dependent LDS
+// read each.  Without the walks: 64 experts of 1024 x 512, 64 rows each, whole forward 47.9 -> 35.1 us, 100 of 2048 x 768,
+// 330 rows each 291 -> 246, 32 of 7168 x 2048, 2048 rows each 2466 -> 2402.
+template <int kBM>
+__device__ __forceinline__ void number_tiles(const int* row_offsets, int num_local, int n_tiles, int lane, int* tile_base)
+{
+    static_assert(kMaxMoeExperts <= 128, "two experts per lane");
+    int before = 0;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        const int e = lane + 64 * h;
+        const int rows = e < num_local ? row_offsets[e + 1] - row_offsets[e] : 0;
+        const int through = before + wave_scan((rows + kBM - 1) / kBM * n_tiles);
+        tile_base[e + 1] = through;
+        before = __builtin_amdgcn_readlane(through, 63);
+    }
+    if (lane == 0) tile_base[0] = 0;
+}
+// The expert that a tile (below the total) belongs to: how many experts end at or before it, asked of 64 at a time.
+__device__ __forceinline__ int expert_of_tile(int tile, const int* tile_base, int num_local)
+{
+    const int lane = lane_now();
+    int e = __popcll(__ballot(tile >= tile_base[lane + 1]));
+    if (num_local > 64) e += __popcll(__ballot(tile >= tile_base[lane + 65]));
+    return e;
+}
+
 struct TileInfo {
     int expert, nt, row0, valid;  // row0 = first row of the tile in the expanded layout; valid rows <= kBM
 };
@@ -398,15 +436,7 @@ __global__ __launch_bounds__(kGemmThreads, 1) void grouped_gemm_kernel(GemmParam
     // (The offsets are fetched by one thread each, in parallel; only the tiny scan is serial.)
     if (tid <= p.num_local) row_offsets[tid] = p.offsets[tid];
     __syncthreads();
-    if (tid == 0) {
-        int total = 0;
-        for (int e = 0; e < p.num_local; ++e) {
-            tile_base[e] = total;
-            const int rows = row_offsets[e + 1] - row_offsets[e];
-            total += (rows + kBM - 1) / kBM * n_tiles;
-        }
-        tile_base[p.num_local] = total;
-    }
+    if (wave == 0) number_tiles<kBM>(row_offsets, p.num_local, n_tiles, lane, tile_base);
     __syncthreads();
     const int total_tiles = tile_base[p.num_local];
 
@@ -443,11 +473,10 @@ __global__ __launch_bounds__(kGemmThreads, 1) void grouped_gemm_kernel(GemmParam
     const int my_tiles = one_round ? 1 : (total_tiles - first + stride - 1) / stride;
 
     auto decode = [&](int tile) {
-        int e = 0;
-        while (tile >= tile_base[e + 1]) ++e;
-        const int row_begin = row_offsets[e], rows = row_offsets[e + 1] - row_begin;
+        const int e = expert_of_tile(tile, tile_base, p.num_local);
+        const int row_begin = __builtin_amdgcn_readfirstlane(row_offsets[e]), rows = __builtin_amdgcn_readfirstlane(row_offsets[e + 1]) - row_begin;
         const int m_tiles = (rows + kBM - 1) / kBM;
-        const int local = tile - tile_base[e];
+        const int local = tile - __builtin_amdgcn_readfirstlane(tile_base[e]);
         TileInfo info;
         info.expert = e;
         info.nt = local / m_tiles;
@@ -943,16 +972,6 @@ __device__ __forceinline__ void mfma_fp4_fp8_regs(v16f& acc, const v8i& x, int s
                        "n"(kReg), "n"(kReg + 3));
 }
 
-// The lane's number, worked out on the spot (two instructions) instead of kept in a register: the code that runs once
-// per tile or span (tile switches, scale requests, the epilogue) takes its lane-dependent addresses from this, so that the
-// item loop does not have to carry them.
-__device__ __forceinline__ int lane_now()
-{
-    int lane;
-    asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(lane));
-    return lane;
-}
-
 // ---- epilogue pieces: a 32-row tile straight from the accumulators -------------------------------------------------------
 // With the weights as the instruction's A operand a lane holds, for its row, columns q*8 + g*4 .. + 3 (q = 0..3) of a column
 // tile, its partner lane (l ^ 32) the four columns in between.  Two register swaps between the lane halves give the lower lane
@@ -1237,15 +1256,7 @@ __global__ __launch_bounds__(kGemmThreads, ColCfg<RT>::kWorkgroupsPerCu) void gr
 
     if (tid <= p.num_local) row_offsets[tid] = p.offsets[tid];
     __syncthreads();
-    if (tid == 0) {
-        int total = 0;
-        for (int e = 0; e < p.num_local; ++e) {
-            tile_base[e] = total;
-            const int rows = row_offsets[e + 1] - row_offsets[e];
-            total += (rows + kBM - 1) / kBM * n_tiles;
-        }
-        tile_base[p.num_local] = total;
-    }
+    if (wave == 0) number_tiles<kBM>(row_offsets, p.num_local, n_tiles, lane, tile_base);
     __syncthreads();
     const int total_tiles = tile_base[p.num_local];
 
@@ -1277,11 +1288,10 @@ __global__ __launch_bounds__(kGemmThreads, ColCfg<RT>::kWorkgroupsPerCu) void gr
     const int my_tiles = one_round ? 1 : (total_tiles - first + stride - 1) / stride;
 
     auto decode = [&](int tile) {
-        int e = 0;
-        while (tile >= tile_base[e + 1]) ++e;
-        const int row_begin = row_offsets[e], rows = row_offsets[e + 1] - row_begin;
+        const int e = expert_of_tile(tile, tile_base, p.num_local);
+        const int row_begin = __builtin_amdgcn_readfirstlane(row_offsets[e]), rows = __builtin_amdgcn_readfirstlane(row_offsets[e + 1]) - row_begin;
         const int m_tiles = (rows + kBM - 1) / kBM;
-        const int local = tile - tile_base[e];
+        const int local = tile - __builtin_amdgcn_readfirstlane(tile_base[e]);
         // Inside an expert the tiles are numbered panel by panel: kPanel column tiles wide (the last panel may be
         // narrower), all row tiles high, row by row.  The 32 consecutive tiles an XCD works on at a time are then a block of
         // about 4 row tiles x 8 column tiles, whose activation rows and weight columns that XCD's L2 fetches once, instead
