@@ -1667,68 +1667,88 @@ int launch_gemm_rt(const GemmParams& p, double expected_tiles, hipStream_t strea
 
 // How many rows an expert is expected to have (the true counts stay on the device).
 struct ExpectedRows {
-    int average;    // over routed and shared experts
     double routed;  // of a routed expert
     double spread;  // standard deviation of that: a token goes to a given expert or not
     int shared;     // of a shared expert: every token
 };
 
-// Row-tile height: the cheapest of 64 / 128 / 192 rows by a small cost model, judged from the expected rows per expert (the true counts
-// stay on the device).  Routing scatters the counts around that mean, and one expert a few rows over a multiple of the tile
-// height costs a whole extra row tile each: the tile count is therefore the expectation of ceil(rows / height) under a
-// normal spread, not ceil(mean / height); an expert without rows has no tile.  (Mean 256 over 8 experts: 128-row tiles need 2.5
-// row tiles per expert on average = 320 tiles = two rounds on 256 CUs, 192-row tiles need 2 = one round; measured 94 vs 67 us.)
+// Kernel and row-tile height, by a small cost model: 64, 128 or 192 rows, or the few-rows kernel's 32 with one or four waves per
+// workgroup.  Judged from the expected rows per expert (the true counts stay on the device).  Routing scatters the counts
+// around that mean, and one expert a few rows over a multiple of the tile height costs a whole extra row tile each: the tile
+// count is therefore the expectation of ceil(rows / height) under a normal spread, not ceil(mean / height); an expert
+// without rows has no tile.  (Mean 256 over 8 experts: 128-row tiles need 2.5 row tiles per expert on average = 320 tiles = two
+// rounds on 256 CUs, 192-row tiles need 2 = one round; measured 94 vs 67 us.)
+// Times are in microseconds, fitted to kernel traces of both GEMMs on an MI355X at 263 shapes (2 to 100 experts, k from 512 to
+// 8192): once per launch; per round of one tile per CU its epilogue and switch, and per k tile the main loop and the weights'
+// way from memory, which the row tiles of an expert share; nothing below the time to read the weights once.  What it picks is 1.1 %
+// slower than the best on average.  How to refit: force each height with the workspace setting "gemm_tile_rows" and
+// take a kernel trace.
+// The few-rows kernel is the better one for small launches whatever the rows: a CU draws no more than about 50 GB/s from
+// memory, and with up to 64 tiles one-wave workgroups spread the columns over four times as many CUs (2 experts of
+// 7168 x 2048, 24 rows each: first GEMM 27 us with 64-row tiles, 24 with four waves, 17.5 with one; 192 rows: 35, 23, 34; 16 of
+// 1024 x 512, 24 rows: 12.7, 7.7, 6.6).  Large ones it streams as well as the 64-row kernel up to about 20 rows, where a
+// tile of 32 still holds nearly all experts (64 of 7168 x 2048, 20 rows: 148 against 154 us; 28 rows: 168 against 159).
 template <bool kGateUp>
 int launch_gemm(const GemmParams& p, const ExpectedRows& expected, hipStream_t stream, const char* what)
 {
     const int cus = gemm_grid();
-    const int n_tiles = p.n / kBN;
-    // Few rows: the counts scatter by about sqrt(mean), and every expert beyond 32 rows streams its weights once more, so the
-    // line lies where a tile of 32 still holds nearly all experts.  (7168 x 2048, 32 of 256 experts, whole forward, 64-row
-    // tiles -> few rows: mean 16: 153 -> 137 us, 20: 149 -> 138, 24: 148 -> 160, 32: 152 -> 208.)
-    // Source rows are addressed with 32 bits here.
-    if (expected.average <= 20 && p.column_waves && p.forced_rt == 0 &&
-        (!kGateUp || static_cast<long long>(p.a_rows) * p.k < (1LL << 32))) {
-        const int tiles = p.num_local * n_tiles;
-        // One workgroup per column tile fills half the CUs or fewer: a CU draws no more than about 50 GB/s from memory, so
-        // the columns are spread over four times as many (16 experts of 2048 x 768, 8 rows each: 96 + 128 tiles, 26.4 ->
-        // 24.7 us; at 7168 x 2048, 512 + 896 tiles, it costs 15 us: every wave then fetches the activations for itself).
-        if (tiles <= cus / 2)
-            hipLaunchKernelGGL((grouped_gemm_few_rows_kernel<1, kGateUp>), dim3(kGemmWaves * tiles), dim3(64), 0, stream, p);
-        else
-            hipLaunchKernelGGL((grouped_gemm_few_rows_kernel<kGemmWaves, kGateUp>), dim3(tiles), dim3(kGemmThreads), 0, stream, p);
-        return launch_status(what);
-    }
-    const double mean = expected.routed;
+    const int n_tiles = p.n / kBN, ktiles = p.k / kBK;
     const int num_shared = p.num_local - p.num_routed;
-    const int kind = p.column_waves && p.k % 512 == 0 ? 0 : 1;  // the kernel that launch_gemm_rt takes
+    const double mean = expected.routed;
+    const double routed_with_rows = 1.0 - exp(-mean);
+    auto expected_row_tiles = [&](int bm) {
+        double m_tiles = routed_with_rows;  // E[ceil(X / bm)] = sum over j >= 0 of P(X > j * bm)
+        for (int j = 1; j * bm < mean + 6.0 * expected.spread; ++j)
+            m_tiles += 0.5 * erfc((j * bm + 0.5 - mean) / (expected.spread * 1.4142135623730951));
+        return p.num_routed * m_tiles + static_cast<double>(num_shared) * ((expected.shared + bm - 1) / bm);
+    };
+    // Rounds of `unit` workgroups; a stray tile in one launch out of a hundred does not count.
+    auto rounds_of = [](double tiles, double unit) { return std::max(1.0, ceil(tiles / unit - 0.01)); };
+    const double weight_bytes = (p.num_routed * routed_with_rows + num_shared) * n_tiles * ktiles * 16896.0;
+    // Nothing ends before the weights are read; where that decides, the one that would be done first otherwise is still better.
+    auto bounded = [&](double t) { return std::max(2.0 + weight_bytes / 6.3e6, t) + 0.05 * t; };
+    const int kind = p.column_waves && p.k % 512 == 0 ? 0 : 1;  // the kernel that launch_gemm_rt takes: column waves, 2 x 2
     int best = 2;
     double best_cost = 1e30, tiles_of[4] = {0.0, 0.0, 0.0, 0.0};
     for (int rt = 1; rt <= 3; ++rt) {
-        const int bm = 64 * rt;
-        double m_tiles = 1.0 - exp(-mean);  // E[ceil(X / bm)] = sum over j >= 0 of P(X > j * bm)
-        for (int j = 1; j * bm < mean + 6.0 * expected.spread; ++j)
-            m_tiles += 0.5 * erfc((j * bm + 0.5 - mean) / (expected.spread * 1.4142135623730951));
-        const double row_tiles = p.num_routed * m_tiles + static_cast<double>(num_shared) * ((expected.shared + bm - 1) / bm);
+        const double row_tiles = expected_row_tiles(64 * rt);
         const double tiles = row_tiles * n_tiles;
         tiles_of[rt] = tiles;
-        // Rounds of one workgroup per CU; a stray tile in one launch out of a hundred does not count.
         const bool in_pairs = rt == 1 && kind == 0 && two_workgroups_pay(tiles, cus);
-        const double rounds = in_pairs ? 2.0 * ceil(tiles / (2.0 * cus) - 0.01) : ceil(tiles / cus - 0.01);
-        // Microseconds, fitted to kernel traces of both GEMMs on an MI355X at 285 shapes (2 to 64 experts, up to 5000 rows each,
-        // k from 512 to 8192), [column waves, 2 x 2][height]: once per launch, per tile its epilogue and switch, per k tile the
-        // main loop, and per k tile what it costs to stream the weights from memory, shared by the row tiles of an expert.
-        // Over them the height it picks is 0.3 % slower than the best on average and 11 % at worst.  (64 experts of
-        // 7168 x 2048, whole forward with the heights it picks / with 64 rows throughout: 64 rows each 355 / 414 us; 80:
-        // 373 / 535; 128: 485 / 661.)
-        // How to refit: force each height with the workspace setting "gemm_tile_rows" and take a kernel trace.
-        constexpr double kFirst[2][3] = {{1.8, 0.3, 0.8}, {1.4, 0.9, 1.0}}, kPerTile[2][3] = {{4.5, 6.0, 7.9}, {5.0, 6.4, 8.7}};
-        constexpr double kPerItem[2][3] = {{0.46, 0.74, 1.02}, {0.46, 0.75, 0.99}}, kWeights[2][3] = {{0.09, 0.04, 0.09}, {0.12, 0.07, 0.10}};
+        const double rounds = in_pairs ? 2.0 * rounds_of(tiles, 2.0 * cus) : rounds_of(tiles, cus);
+        constexpr double kFirst[2][3] = {{1.7, 0.4, 0.3}, {5.3, 3.1, 1.2}}, kPerTile[2][3] = {{3.7, 4.4, 8.7}, {3.2, 4.5, 6.5}};
+        constexpr double kPerItem[2][3] = {{0.61, 0.77, 0.99}, {0.52, 0.85, 1.10}}, kWeights[2][3] = {{0.0, 0.01, 0.10}, {0.02, 0.03, 0.06}};
         const double per_item = kPerItem[kind][rt - 1] + kWeights[kind][rt - 1] * p.num_local / std::max(row_tiles, 1e-3);
-        const double cost = kFirst[kind][rt - 1] + (rounds < 1.0 ? 1.0 : rounds) * (kPerTile[kind][rt - 1] + (p.k / kBK) * per_item);
+        const double cost = bounded(kFirst[kind][rt - 1] + rounds * (kPerTile[kind][rt - 1] + ktiles * per_item));
         if (cost < best_cost - 1e-9) {
             best_cost = cost;
             best = rt;
+        }
+    }
+    // Source rows are addressed with 32 bits in the few-rows kernel.  A share with more than one 64-row tile per expert has so many
+    // tokens without a row that its first GEMM's idle workgroups are better used for their zero rows.
+    if (p.column_waves && p.forced_rt == 0 && (p.fill_out == nullptr || mean <= 64.0) && (!kGateUp || static_cast<long long>(p.a_rows) * p.k < (1LL << 32))) {
+        const double tiles = expected_row_tiles(32) * n_tiles;
+        const double one = bounded(3.0 + 0.30 * ktiles + (rounds_of(kGemmWaves * tiles, cus) - 1.0) * (1.1 + 0.17 * ktiles));
+        const double four = bounded(1.5 + rounds_of(tiles, cus) * (2.7 + 0.50 * ktiles));
+        // Zero rows of the output that this launch's idle workgroups would have written (at about 30 GB/s each): the few-rows
+        // kernel leaves them to the reduce, which writes them at 8 TB/s, and the GEMM is faster without the company: 4300 zero
+        // rows of 5120 columns beside 31 experts of 5120 x 512 cost the forward 57 us filled and 49 not.
+        double unfilled = 0.0;
+        if (p.fill_out != nullptr && tiles_of[best] < cus) {
+            const double zeros = p.fill_tokens * exp(-mean * p.num_routed / p.fill_tokens) * p.fill_vec * 16.0;
+            unfilled = std::min(zeros, (cus - tiles_of[best]) * 30e3 * best_cost) / 11e6;
+        }
+        if (std::min(one, four) + unfilled < best_cost) {
+            // Workgroups for more rows than expected (those without a tile end at once, while one with two doubles the time).
+            const long long row_tiles = static_cast<long long>(p.num_routed) * static_cast<long long>(ceil(std::max(1.0, mean + 3.0 * expected.spread) / 32.0)) +
+                                        static_cast<long long>(num_shared) * ((expected.shared + 31) / 32);
+            const unsigned grid = static_cast<unsigned>(row_tiles * n_tiles);
+            if (one < four)
+                hipLaunchKernelGGL((grouped_gemm_few_rows_kernel<1, kGateUp>), dim3(kGemmWaves * grid), dim3(64), 0, stream, p);
+            else
+                hipLaunchKernelGGL((grouped_gemm_few_rows_kernel<kGemmWaves, kGateUp>), dim3(grid), dim3(kGemmThreads), 0, stream, p);
+            return launch_status(what);
         }
     }
     if (p.forced_rt >= 1 && p.forced_rt <= 3) best = p.forced_rt;
@@ -2206,8 +2226,7 @@ int dpep_megamoe_run(void* ws, const dpep_megamoe_call* call, void* stream)
     const long long expected_routed = static_cast<long long>(num_tokens) * num_topk * num_local / num_experts;
     const long long expected_rows = expected_routed + static_cast<long long>(num_tokens) * num_shared;
     const double routed = static_cast<double>(num_tokens) * num_topk / num_experts;
-    const ExpectedRows expected = {static_cast<int>((expected_rows + g1.num_local - 1) / g1.num_local),
-                                   routed, sqrt(routed * std::max(0.0, 1.0 - static_cast<double>(num_topk) / num_experts)) + 1e-3, num_tokens};
+    const ExpectedRows expected = {routed, sqrt(routed * std::max(0.0, 1.0 - static_cast<double>(num_topk) / num_experts)) + 1e-3, num_tokens};
     // Without shared experts most tokens of a share have no row: workgroups of the first GEMM that get no tile
     // zero those rows of y meanwhile, and the weighted reduce skips what they got through.
     int* fill_state = reinterpret_cast<int*>(base + l.fill_state);

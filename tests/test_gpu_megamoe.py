@@ -232,6 +232,26 @@ def test_few_rows_per_expert(ops, hidden, inter, local, rows):
     np.testing.assert_array_equal(y, tall)
 
 
+@pytest.mark.parametrize("hidden,inter,rows", [
+    (2048, 384, [24, 40, 33, 31]),    # about one row tile of 32 each
+    (1088, 384, [65, 0, 64, 63]),     # two, k = 1280 ends in half a span of scales
+    (1024, 512, [97, 223]),           # three and seven
+    (512, 256, [150, 10, 90, 4, 1, 33, 300, 2]),
+])
+def test_small_launches_take_the_few_rows_kernel(ops, hidden, inter, rows):
+    """All experts here and the routing uneven: more row tiles than workgroups were launched for, and fewer.  Against the oracle,
+    and bit for bit against the kernel with 64-row tiles."""
+    experts = len(rows)
+    x_codes, x_scales, l1, l2, idx, weights = _make_problem(sum(rows), hidden, inter, experts, 0, experts, 1, seed=experts)
+    idx[:, 0] = np.random.default_rng(experts).permutation(np.repeat(np.arange(experts), rows)).astype(np.int32)
+    y, counts = _run(ops, x_codes, x_scales, l1, l2, idx, weights, experts, 0, experts)
+    np.testing.assert_array_equal(counts, rows)
+    ref = _oracle(x_codes, x_scales, l1, l2, idx, weights, 0)
+    assert np.linalg.norm(y - ref) <= 2e-2 * np.linalg.norm(ref)
+    tall, _ = _run(ops, x_codes, x_scales, l1, l2, idx, weights, experts, 0, experts, tile_rows=64)
+    np.testing.assert_array_equal(y, tall)
+
+
 @pytest.mark.parametrize("tokens,hidden,inter,tile_rows", [
     (1000, 2304, 1280, 64),   # 320 + 288 tiles of 18 and 10 k tiles on 256 workgroups
     (1700, 1280, 768, 64),    # 10 and 6 k tiles: the shortest tile that still switches without letting the copies land
