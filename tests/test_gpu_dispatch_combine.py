@@ -821,3 +821,33 @@ def test_combine_and_cast_back_on_infinities_and_nans(ops):
         scales[0, 0], scales[1, 1], scales[2, 0], scales[3, 1], scales[4, 0], scales[5, 0] = np.inf, np.nan, 0, -1, 3e38, 1e-42
         got = ops.cast_back(torch.from_numpy(codes).cuda().view(torch.float8_e4m3fn), torch.from_numpy(scales).cuda())
         _same_but_for_nan_encoding(bf16_bits(got), oquant.cast_back(codes, scales))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("tokens,topk,hidden,rows", [
+    (3, 1, 8, 1), (5, 32, 2048, 2), (130, 7, 2056, 60), (1500, 3, 264, 0), (2049, 8, 1032, 700), (4099, 2, 72, 2049), (4200, 6, 16, 300)])
+def test_combine_of_a_share_where_most_tokens_own_no_row(ops, tokens, topk, hidden, rows, dtype):
+    """Fewer rows than half the tokens: one to 64 / top-k tokens to a workgroup, widths around a wave's quarter of a row, tokens with
+    several rows and with none, unserved tokens zeroed or left alone.  The same bits as fp32 sums in slot order."""
+    gen = torch.Generator().manual_seed(tokens)
+    route_to_row = torch.full((tokens * topk,), -1, dtype=torch.int32)
+    route_to_row[torch.randperm(tokens * topk, generator=gen)[:rows]] = torch.randperm(rows, generator=gen).int()
+    route_to_row = route_to_row.view(tokens, topk)
+    y = torch.randn(rows, hidden, generator=gen).to(dtype)
+    weights, back = torch.rand(rows, generator=gen), torch.randn(rows, generator=gen)
+    owned = route_to_row >= 0
+    at = route_to_row.clamp(min=0).long()
+    for w in (None, weights):
+        want = torch.zeros(tokens, hidden)
+        for slot in range(topk if rows else 0):
+            term = y[at[:, slot]].float()
+            if w is not None:
+                term = term * w[at[:, slot], None]
+            want = torch.where(owned[:, slot, None], want + term, want)
+        got, returned = ops.combine(y.cuda(), route_to_row.cuda(), None if w is None else w.cuda(), return_values=back.cuda())
+        assert torch.equal(got.cpu(), want.to(dtype))
+        assert torch.equal(returned.cpu(), torch.where(owned, back[at] if rows else torch.zeros(at.shape), torch.zeros(())))
+        if dtype == torch.bfloat16:
+            out = torch.full((tokens, hidden), 3.0, dtype=dtype, device="cuda")
+            ops.combine(y.cuda(), route_to_row.cuda(), None if w is None else w.cuda(), out=out, served_only=True)
+            assert torch.equal(out.cpu(), torch.where(owned.any(dim=1, keepdim=True), want.to(dtype), torch.tensor(3.0, dtype=dtype)))
