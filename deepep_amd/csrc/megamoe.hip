@@ -1697,8 +1697,10 @@ int launch_gemm(const GemmParams& p, const ExpectedRows& expected, hipStream_t s
     const double mean = expected.routed;
     const double routed_with_rows = 1.0 - exp(-mean);
     auto expected_row_tiles = [&](int bm) {
-        double m_tiles = routed_with_rows;  // E[ceil(X / bm)] = sum over j >= 0 of P(X > j * bm)
-        for (int j = 1; j * bm < mean + 6.0 * expected.spread; ++j)
+        // E[ceil(X / bm)] = sum over j >= 0 of P(X > j * bm), which is 1 up to six deviations below the mean
+        const int sure = std::max(0, static_cast<int>((mean - 6.0 * expected.spread) / bm));
+        double m_tiles = routed_with_rows + sure;
+        for (int j = sure + 1; j * bm < mean + 6.0 * expected.spread; ++j)
             m_tiles += 0.5 * erfc((j * bm + 0.5 - mean) / (expected.spread * 1.4142135623730951));
         return p.num_routed * m_tiles + static_cast<double>(num_shared) * ((expected.shared + bm - 1) / bm);
     };
