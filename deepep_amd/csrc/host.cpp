@@ -624,6 +624,44 @@ PyObject* event_of(Exchange* e, const Target& t, std::initializer_list<const at:
     return overlap.release();
 }
 
+// Answers for the tensors of a call from its first launch until the call has an event (event_of), whatever way the call ends.
+// On the communication stream a launch may still be pending when a tensor is let go, and memory that was allocated on the
+// caller's stream is handed out again in that stream's order alone: so it is declared to the allocator first, where an output
+// is replaced (replace) and where a launch, a wait or an allocation fails behind a launch.  In the latter case the buffer
+// takes no further calls either.
+struct Pending {
+    Exchange* e;
+    const Target& t;
+    const at::Tensor* used[8];
+    int count = 0;
+    bool launched = false;
+    Pending(Exchange* exchange, const Target& target, std::initializer_list<const at::Tensor*> tensors) : e(exchange), t(target)
+    {
+        for (const at::Tensor* x : tensors)
+            if (x != nullptr) used[count++] = x;
+    }
+    void declare(const at::Tensor& x) const
+    {
+        if (x.defined() && t.asynchronous && !(t.stream == t.caller)) x.record_stream(t.stream.torch(e->device));
+    }
+    void replace(at::Tensor* x, at::IntArrayRef sizes, at::ScalarType type) const
+    {
+        declare(*x);
+        *x = allocate(sizes, type, e->device);
+    }
+    ~Pending()
+    {
+        if (!launched) return;
+        e->failed = true;
+        for (int i = 0; i < count; ++i) {
+            try {
+                declare(*used[i]);
+            } catch (...) {  // (nothing can be reported from here)
+            }
+        }
+    }
+};
+
 // A dispatch's payload, checked as far as it can be without knowing which path it takes.
 struct Payload {
     const at::Tensor* x = nullptr;
@@ -749,6 +787,8 @@ PyObject* run_fresh(Exchange* e, const FreshCall& c, const Target& t, PyObject* 
     call.quantize = c.quantize;
     call.capacity_rows = static_cast<int32_t>(capacity);
     call.report_to_host = !c.low_latency;
+    Pending pending(e, t, {&out, &scales, &weights, &routing, c.in.x, c.in.scales, c.weights, c.idx});
+    pending.launched = true;
     if (const int status = dpep_dispatch_fresh(e->workspace, &call, t.stream.raw)) return raise_native(status);
 
     // ---- while the GPU works: everything that does not depend on R -----------------------------------------------------
@@ -819,8 +859,8 @@ PyObject* run_fresh(Exchange* e, const FreshCall& c, const Target& t, PyObject* 
         plan->rows = rows;
         e->share = static_cast<double>(rows) / static_cast<double>(routes);
         if (rows > capacity) {  // more rows than the share suggested: once more, into outputs of the right size
-            out = allocate({rows, width}, out_type, device);
-            if (scales.defined()) scales = allocate({rows, scale_cols}, scale_type, device);
+            pending.replace(&out, {rows, width}, out_type);
+            if (scales.defined()) pending.replace(&scales, {rows, scale_cols}, scale_type);
             if (weights.defined()) weights = allocate({rows}, at::kFloat, device);
             float* s_out = scales.defined() ? static_cast<float*>(scales.data_ptr()) : nullptr;
             float* w_out = weights.defined() ? static_cast<float*>(weights.data_ptr()) : nullptr;
@@ -853,6 +893,7 @@ PyObject* run_fresh(Exchange* e, const FreshCall& c, const Target& t, PyObject* 
     if (PyObject_SetAttr(handle.p, N.__dict__, d) < 0) return nullptr;
 
     Ref event(event_of(e, t, {&out, &scales, &weights, &routing}, {c.in.x, c.in.scales, c.weights, c.idx}));
+    pending.launched = !event;
     Ref payload(wrap(out));
     if (!event || !payload) return nullptr;
     if (scales.defined()) {
@@ -878,6 +919,8 @@ PyObject* run_cached(Exchange* e, const Payload& in, bool quantize, const at::Te
     const float* w_in = weights_in != nullptr ? static_cast<const float*>(weights_in->data_ptr()) : nullptr;
     float* s_out = scales.defined() ? static_cast<float*>(scales.data_ptr()) : nullptr;
     float* w_out = weights.defined() ? static_cast<float*>(weights.data_ptr()) : nullptr;
+    Pending pending(e, t, {&out, &scales, &weights, in.x, in.scales, weights_in, plan->routing});
+    pending.launched = true;
     const int status = quantize ? dpep_dispatch_quant_fp8(in.x->data_ptr(), w_in, plan->route_to_row, plan->row_to_route, plan->tokens,
                                                           plan->topk, static_cast<int>(rows), static_cast<int>(width), out.data_ptr(), s_out,
                                                           w_out, t.stream.raw)
@@ -888,6 +931,7 @@ PyObject* run_cached(Exchange* e, const Payload& in, bool quantize, const at::Te
     if (status) return raise_native(status);
     if (!set_int(dict, N.num_compute_units, fp8 ? 64 : 32)) return nullptr;
     Ref event(event_of(e, t, {&out, &scales, &weights}, {in.x, in.scales, weights_in, plan->routing}));
+    pending.launched = !event;
     Ref payload(wrap(out));
     if (!event || !payload) return nullptr;
     if (scales.defined()) {
@@ -1045,12 +1089,15 @@ PyObject* Exchange_combine(PyObject* self, PyObject* const* a, Py_ssize_t n)
         if (values != nullptr) returned = allocate({plan->tokens, plan->topk}, at::kFloat, e->device);
         const float* row_weights = plan->low_latency ? static_cast<const float*>(plan->weights->data_ptr()) : nullptr;
         const int expected = plan->low_latency ? static_cast<int>(static_cast<long long>(plan->tokens) * plan->topk / e->world) : static_cast<int>(plan->rows);
+        Pending pending(e, t, {&out, &returned, rows, values, plan->routing, plan->weights});
+        pending.launched = true;
         if (const int status = dpep_combine_expecting(rows->data_ptr(), type == at::kHalf, row_weights, plan->route_to_row, plan->tokens, plan->topk,
                                                       static_cast<int>(plan->rows), expected, plan->hidden, out.data_ptr(),
                                                       values != nullptr ? static_cast<const float*>(values->data_ptr()) : nullptr,
                                                       returned.defined() ? static_cast<float*>(returned.data_ptr()) : nullptr, t.stream.raw))
             return raise_native(status);
         Ref event(event_of(e, t, {&out, &returned}, {rows, values, plan->routing, plan->weights}));
+        pending.launched = !event;
         Ref first(wrap(out)), second(returned.defined() ? wrap(returned) : new_ref(Py_None));
         return event && first && second ? PyTuple_Pack(3, first.p, second.p, event.p) : nullptr;
     };

@@ -183,6 +183,69 @@ def test_memory_of_asynchronous_calls_is_not_handed_out_too_early(wait):
         buffer.destroy()
 
 
+@pytest.mark.parametrize("fp8", [False, True])
+def test_memory_of_an_outgrown_asynchronous_dispatch_is_not_handed_out_too_early(fp8):
+    """A share several times the expected one, on the communication stream: the outputs it outgrew are let go inside the call,
+    and the caller asks for memory of their size at once, on its own stream and without waiting for the event."""
+    world, rank, experts, topk, tokens, hidden = 4, 1, 16, 4, 8192, 2048
+    rng = np.random.default_rng(6)
+    ids = np.stack([rank * 4 + rng.permutation(4)[:topk] for _ in range(tokens)]).astype(np.int64)
+    x, w = _batch(tokens, hidden, topk, 6)
+    want = olayout.layout(ids, experts, rank * 4, 4)
+    rows = want["num_rows"]
+    order = torch.from_numpy(want["row_to_route"]).cuda().long()
+    xd, wd, idx = x.cuda(), w.cuda(), torch.from_numpy(ids).cuda()
+    expected = (xd if not fp8 else oquant.cast_to_fp8_torch(x)[0].cuda().view(torch.uint8))[order // topk]
+    for _ in range(4):
+        # a new buffer each time: with the batch before as its guide the share would fit
+        buffer = _buffer(num_bytes=4 << 20, rank=rank, world_size=world, use_fp8_dispatch=fp8)
+        try:
+            torch.cuda.synchronize()
+            recv, _, recv_w, handle, event = buffer.dispatch(xd, topk_idx=idx, topk_weights=wd, num_experts=experts,
+                                                             async_with_compute_stream=True)
+            noise = [torch.full((n, hidden), 7.0, dtype=torch.bfloat16, device="cuda")
+                     for n in (rows // 4, rows // 4 + rows // 16, rows // 3, rows // 8, rows // 8)]
+            event.current_stream_wait()
+            torch.cuda.synchronize()
+            assert handle.num_expanded_tokens == rows == tokens * topk
+            assert torch.equal(recv[0].view(torch.uint8) if fp8 else recv, expected)
+            assert torch.equal(recv_w, wd.view(-1)[order])
+            for block in noise:
+                assert bool((block == 7.0).all())
+            del recv, recv_w, handle, event, noise
+        finally:
+            torch.cuda.synchronize()
+            buffer.destroy()
+
+
+def test_a_call_that_fails_behind_its_launch_leaves_its_buffer_closed():
+    """The layout gives up waiting (forced by its own bound, every kernel ends normally): the asynchronous call raises with its
+    payload queued on the communication stream, the caller's tensors go at once, and the buffer takes no further calls."""
+    from deepep_amd import _lib
+
+    tokens, hidden, topk, experts = 4096, 1024, 4, 16
+    x, w = _batch(tokens, hidden, topk, 7)
+    idx = torch.stack([torch.randperm(experts)[:topk] for _ in range(tokens)]).cuda()
+    buffer = _buffer(num_bytes=4 << 20)
+    try:
+        workspace = buffer._runtime.workspace
+        workspace.tune("layout_exchange_extra_rows", 1)
+        workspace.tune("layout_exchange_ticks", 10_000)
+        payload = x.cuda()
+        with pytest.raises(_lib.NativeError, match="ran out of time"):
+            buffer.dispatch(payload, topk_idx=idx, topk_weights=w.cuda(), num_experts=experts, async_with_compute_stream=True)
+        del payload
+        noise = [torch.full((tokens * topk, hidden), 7.0, dtype=torch.bfloat16, device="cuda") for _ in range(2)]
+        buffer.get_comm_stream().synchronize()
+        torch.cuda.synchronize()
+        assert all(bool((block == 7.0).all()) for block in noise)
+        with pytest.raises(RuntimeError, match="previous communication launch failed"):
+            buffer.dispatch(x.cuda(), topk_idx=idx, num_experts=experts)
+    finally:
+        torch.cuda.synchronize()
+        buffer.destroy()
+
+
 def test_event_of_an_asynchronous_call_stands_in_for_torchs():
     x, _ = _batch(64, 256, 2, 3)
     idx = torch.stack([torch.randperm(8)[:2] for _ in range(64)]).cuda()
