@@ -345,7 +345,7 @@ PyObject* Marker_hold_current_stream(PyObject* o, PyObject*)
         PyErr_SetString(PyExc_RuntimeError, "Cannot wait for an event from another GPU");
         return nullptr;
     }
-    return marker_wait(m, current_stream(m->device).raw);  // (None: a Lease asks for the current stream itself)
+    return marker_wait(m, current_stream(m->device).raw);  // (None: a lease asks for the current stream itself)
     END_HANDLE_TH_ERRORS
 }
 // torch.cuda.Event's methods, the stream given as a torch stream object or not at all.

@@ -53,14 +53,17 @@ class _Lease:
     on every stream that ``touch`` names, so that their memory is not handed out again while a stream still works
     on it."""
 
-    __slots__ = ("objects", "tensors")
+    __slots__ = ("objects", "tensors", "gpu")
 
     def __init__(self, objects, gpu: int):
-        self.objects = objects
+        self.objects, self.gpu = objects, gpu
         flat = objects if isinstance(objects, (tuple, list)) else (objects,)
         self.tensors = [t for t in flat if isinstance(t, torch.Tensor) and t.device.type != "cpu" and t.device.index == gpu]
 
     def touch(self, stream) -> None:
+        """None: the current stream (markers of the native host path do not make an object of it)."""
+        if stream is None and self.tensors:
+            stream = gpu_api().current_stream(self.gpu)
         for tensor in self.tensors:
             tensor.record_stream(stream)
 

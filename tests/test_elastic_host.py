@@ -268,6 +268,27 @@ def test_keyword_aliases(host):
     assert handle.num_compute_units == 5
 
 
+def test_lease_without_a_stream_uses_the_current_one(host, monkeypatch):
+    """A marker may return no stream object from its wait; what the overlap keeps is then declared to the current stream."""
+    make, calls = host
+    declared = []
+
+    class DeviceTensor(torch.Tensor):
+        device = SimpleNamespace(type="cuda", index=0)
+
+        def record_stream(self, stream):
+            assert stream is not None
+            declared.append(stream)
+
+    handle = event.EventHandle()
+    wait = handle._marker.hold_current_stream
+    handle._marker = SimpleNamespace(gpu=0, stream="producer", hold_current_stream=lambda: wait() and None)
+    tensor = torch.zeros(2).as_subclass(DeviceTensor)
+    overlap = event.EventOverlap(handle, extra_tensors=(tensor,))
+    overlap.current_stream_wait()
+    assert calls["event_wait"] == 1 and declared == ["producer", event.gpu_api().current_stream(0)]
+
+
 def test_constructor_gates():
     with pytest.raises(NotImplementedError, match="explicitly_destroy"):
         elastic.ElasticBuffer(num_bytes=1 << 21)

@@ -267,6 +267,38 @@ def test_event_of_an_asynchronous_call_stands_in_for_torchs():
         buffer.destroy()
 
 
+@pytest.mark.parametrize("on_side_stream", [False, True])
+def test_an_overlap_made_from_the_event_of_an_asynchronous_call_keeps_its_tensors(on_side_stream):
+    """EventOverlap's public constructor with the event of a call: the given tensors are kept for the work and declared to
+    whichever stream waits."""
+    from deepep_amd.event import EventOverlap
+
+    x, _ = _batch(64, 256, 2, 3)
+    idx = torch.stack([torch.randperm(8)[:2] for _ in range(64)]).cuda()
+    buffer = _buffer(num_bytes=4 << 20)
+    try:
+        xd = x.cuda()
+        recv, _, _, handle, made = buffer.dispatch(xd, topk_idx=idx, num_experts=8, async_with_compute_stream=True)
+        extra = torch.full((1 << 20,), 3.0, device="cuda")
+        overlap = EventOverlap(made.event, extra_tensors=(extra,))
+        calls = []
+        overlap.register_hook_after_wait(lambda: calls.append(1) or "done")
+        with torch.cuda.stream(torch.cuda.Stream() if on_side_stream else torch.cuda.current_stream()):
+            assert overlap.current_stream_wait() == "done" and calls == [1]
+            twice = recv.float() * 2
+            total = extra.sum()
+        del extra
+        with overlap(release_handle=True):
+            pass
+        assert overlap.event is None and overlap._lease is None
+        torch.cuda.synchronize()
+        assert total.item() == 3.0 * (1 << 20)
+        assert torch.equal(twice, xd.float()[handle.weight_return_meta.long() // 2] * 2)
+    finally:
+        torch.cuda.synchronize()
+        buffer.destroy()
+
+
 def test_asynchronous_calls_from_changing_streams_keep_their_order():
     """The caller's stream changes from call to call while the one before is still busy: every asynchronous call has to see
     its own caller's input, whichever stream raised the buffer's counter last."""
