@@ -170,7 +170,7 @@ struct EventPool {
 // order two streams.  A recorded event plus a wait costs 8 us of host time and 7 of the GPU's when the event is still
 // pending, this 4.5 and 5 (two streams passing the turn back and forth).  Only one stream at a time may raise a counter,
 // or a later value could be seen before an earlier one was written; values only grow, so a counter may go from owner to owner.
-// Counters are kept for the life of the process and reused, as many as there were buffers at work at once.
+// Counters are kept for the life of the process and reused, two for each buffer that lived at the same time as others.
 struct Counter {
     uint64_t* word = nullptr;
     uint64_t raised = 0;
@@ -582,9 +582,6 @@ bool choose_target(Exchange* e, bool asynchronous, PyObject* previous_event, Tar
     if (asynchronous && !e->has_comm) {
         if (!stream_from(e->comm_object, &e->comm)) return false;
         e->has_comm = true;
-        e->comm_counter = take_counter(e->device);
-        e->caller_counter = e->comm_counter != nullptr ? take_counter(e->device) : nullptr;
-        e->counted = t->caller;
     }
     t->stream = asynchronous ? e->comm : t->caller;
     if (asynchronous && !(e->comm == t->caller) && !join_caller(e, t->caller)) return false;
@@ -1136,6 +1133,10 @@ PyObject* Exchange_new(PyTypeObject* type, PyObject* args, PyObject*)
     e->comm_object = new_ref(comm);
     e->share = 0.0;
     e->order = nullptr;
+    // (taken with the buffer, whose workspace is allocated now as well: the first asynchronous call may be under capture, where
+    // nothing may be allocated)
+    e->comm_counter = take_counter(device);
+    e->caller_counter = e->comm_counter != nullptr ? take_counter(device) : nullptr;
     return reinterpret_cast<PyObject*>(e);
     END_HANDLE_TH_ERRORS
 }

@@ -328,9 +328,11 @@ def test_asynchronous_calls_from_changing_streams_keep_their_order():
         buffer.destroy()
 
 
-def test_asynchronous_cached_calls_in_a_hip_graph():
+@pytest.mark.parametrize("first_in_the_graph", [False, True])
+def test_asynchronous_cached_calls_in_a_hip_graph(first_in_the_graph):
     """Under capture streams are ordered by events: a cached dispatch and a combine on the communication stream, captured once
-    and replayed on new payloads, with the program's own work between the replays."""
+    and replayed on new payloads, with the program's own work between the replays.  With and without an asynchronous call of
+    the buffer before the capture: what such calls need is there from the start, none of it is allocated under capture."""
     tokens, hidden, topk, experts = 96, 512, 3, 8
     gen = torch.Generator().manual_seed(4)
     idx = torch.stack([torch.randperm(experts, generator=gen)[:topk] for _ in range(tokens)]).cuda()
@@ -338,8 +340,9 @@ def test_asynchronous_cached_calls_in_a_hip_graph():
     buffer = _buffer(num_bytes=4 << 20)
     try:
         _, _, _, handle, _ = buffer.dispatch(x, topk_idx=idx, num_experts=experts)
-        _, _, _, _, event = buffer.dispatch(x, handle=handle, async_with_compute_stream=True)
-        event.current_stream_wait()
+        if not first_in_the_graph:
+            _, _, _, _, event = buffer.dispatch(x, handle=handle, async_with_compute_stream=True)
+            event.current_stream_wait()
         torch.cuda.synchronize()
         side = torch.cuda.Stream()
         with torch.cuda.stream(side):
@@ -358,6 +361,9 @@ def test_asynchronous_cached_calls_in_a_hip_graph():
             eager_rows, _, _, _, _ = buffer.dispatch(x, handle=handle)
             assert torch.equal(recv, eager_rows)
             assert torch.equal(out, buffer.combine(eager_rows, handle)[0])
+            rows, _, _, _, event = buffer.dispatch(x, handle=handle, async_with_compute_stream=True)  # by the counters again
+            event.current_stream_wait()
+            assert torch.equal(rows, eager_rows)
     finally:
         torch.cuda.synchronize()
         buffer.destroy()
