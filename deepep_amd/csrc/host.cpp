@@ -14,7 +14,6 @@
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
-#include <memory>
 #include <vector>
 
 #include <ATen/core/Tensor.h>
@@ -135,34 +134,23 @@ at::Tensor over(const c10::Storage& storage, int64_t offset, at::ScalarType type
 inline PyObject* wrap(at::Tensor t) { return THPVariable_Wrap(std::move(t)); }
 inline uint32_t version_of(const at::Tensor& t) { return t.unsafeGetTensorImpl()->version_counter().current_version(); }
 
-// ---- events and what has to outlive them ---------------------------------------------------------------------------------
-// Events order streams of one GPU, so they carry no system-scope fence (hipEventDisableSystemFence): behind a fenced one
-// a wait of another stream took 8-15 us of host time and 10 us of the GPU's, without the fence 7 and 7.
-// Recorded events are reused: a wait that has been queued refers to the recording it saw, so an event may be recorded
-// again as soon as nobody can ask for its old state any more.  Bounded; lives as long as a buffer or one of its markers.
-struct EventPool {
-    static constexpr size_t kMost = 32;
-    std::vector<hipEvent_t> idle;
-    hipEvent_t take()
+// ---- stream order and what has to outlive it ------------------------------------------------------------------------------
+// The event a buffer orders two streams with: recorded anew each time (a wait that has been queued refers to the recording it
+// saw), so one suffices.  It orders streams of one GPU, so it carries no system-scope fence (hipEventDisableSystemFence):
+// behind a fenced one a wait of another stream took 8-15 us of host time and 10 us of the GPU's, without the fence 7 and 7.
+struct OrderEvent {
+    hipEvent_t event;
+    // `waits` waits for everything that `on` has been given so far.
+    hipError_t order(hipStream_t waits, hipStream_t on)
     {
-        hipEvent_t e = nullptr;
-        if (!idle.empty()) {
-            e = idle.back();
-            idle.pop_back();
-        } else if (hipEventCreateWithFlags(&e, hipEventDisableTiming | hipEventDisableSystemFence) != hipSuccess) {
-            (void)hipGetLastError();
-            e = nullptr;
-        }
-        return e;
+        hipError_t err = event != nullptr ? hipSuccess : hipEventCreateWithFlags(&event, hipEventDisableTiming | hipEventDisableSystemFence);
+        if (err == hipSuccess) err = hipEventRecord(event, on);
+        return err == hipSuccess ? hipStreamWaitEvent(waits, event, 0) : err;
     }
-    void give_back(hipEvent_t e)
+    void release()
     {
-        if (idle.size() < kMost) idle.push_back(e);
-        else (void)hipEventDestroy(e);
-    }
-    ~EventPool()
-    {
-        for (hipEvent_t e : idle) (void)hipEventDestroy(e);
+        if (event != nullptr) (void)hipEventDestroy(event);
+        event = nullptr;
     }
 };
 
@@ -236,12 +224,11 @@ PyObject* stream_object(const Stream& s, int device)
     return kwargs ? PyObject_Call(type.p, g_empty_tuple, kwargs.p) : nullptr;
 }
 
-// One event recorded on a stream (what deepep_amd.event._Marker is for events recorded through torch).  It stands in for
-// torch's event object too: wait / query / synchronize / record.
+// A value of a stream's counter, reached when the stream has done what it was given before: what deepep_amd.event._Marker is for
+// a torch event, with the methods that EventHandle and EventOverlap use.  Who asks the handle for its event gets one of torch's
+// (deepep_amd.event.EventHandle.event).
 struct Marker {
     PyObject_HEAD
-    std::shared_ptr<EventPool> pool;
-    hipEvent_t event;   // nullptr: the marker is a value of the counter
     Counter* counter;
     uint64_t value;
     Stream stream;
@@ -293,48 +280,23 @@ PyObject* Lease_touch(PyObject* o, PyObject*)
 PyMethodDef lease_methods[] = {{"touch", Lease_touch, METH_O, nullptr}, {nullptr, nullptr, 0, nullptr}};
 PyTypeObject LeaseType = {PyVarObject_HEAD_INIT(nullptr, 0) "deepep_amd._host.Lease", sizeof(Lease)};
 
-void Marker_dealloc(PyObject* o)
+// Marks what `stream` has been given so far; `stream` alone raises `counter`.
+Marker* marker_new(Counter* counter, const Stream& stream, int device)
 {
-    Marker* m = reinterpret_cast<Marker*>(o);
-    if (m->event != nullptr) m->pool->give_back(m->event);
-    m->pool.~shared_ptr();
-    Py_TYPE(o)->tp_free(o);
-}
-// A marker of what `stream` has been given so far: a value of `counter` (which this stream alone raises), or an event.
-Marker* marker_new(const std::shared_ptr<EventPool>& pool, Counter* counter, const Stream& stream, int device)
-{
-    hipEvent_t e = nullptr;
-    if (counter == nullptr) {
-        e = pool->take();
-        if (e == nullptr) return reinterpret_cast<Marker*>(raise_hip("hipEventCreate", hipErrorUnknown));
-        if (hipError_t err = hipEventRecord(e, stream.raw); err != hipSuccess) {
-            pool->give_back(e);
-            return reinterpret_cast<Marker*>(raise_hip("hipEventRecord", err));
-        }
-    } else if (int rc = dpep_stream_raise(counter->word, ++counter->raised, stream.raw); rc != DPEP_OK) {
-        return reinterpret_cast<Marker*>(raise_native(rc));
-    }
+    if (int rc = dpep_stream_raise(counter->word, ++counter->raised, stream.raw); rc != DPEP_OK) return reinterpret_cast<Marker*>(raise_native(rc));
     Marker* m = reinterpret_cast<Marker*>(MarkerType.tp_alloc(&MarkerType, 0));
-    if (m == nullptr) {
-        if (e != nullptr) pool->give_back(e);
-        return nullptr;
-    }
-    new (&m->pool) std::shared_ptr<EventPool>(pool);
-    m->event = e;
+    if (m == nullptr) return nullptr;
     m->counter = counter;
-    m->value = counter != nullptr ? counter->raised : 0;
+    m->value = counter->raised;
     m->stream = stream;
     m->device = device;
     return m;
 }
 PyObject* marker_wait(Marker* m, hipStream_t s)
 {
-    if (m->event != nullptr) {
-        if (hipError_t err = hipStreamWaitEvent(s, m->event, 0); err != hipSuccess) return raise_hip("hipStreamWaitEvent", err);
-    } else if (!m->counter->reached(m->value)) {
+    if (!m->counter->reached(m->value))
         if (hipError_t err = hipStreamWaitValue64(s, m->counter->word, m->value, hipStreamWaitValueGte, ~0ull); err != hipSuccess)
             return raise_hip("hipStreamWaitValue64", err);
-    }
     Py_RETURN_NONE;
 }
 PyObject* Marker_hold_current_stream(PyObject* o, PyObject*)
@@ -348,70 +310,21 @@ PyObject* Marker_hold_current_stream(PyObject* o, PyObject*)
     return marker_wait(m, current_stream(m->device).raw);  // (None: a lease asks for the current stream itself)
     END_HANDLE_TH_ERRORS
 }
-// torch.cuda.Event's methods, the stream given as a torch stream object or not at all.
-bool optional_stream(PyObject* args, int device, Stream* s)
+PyObject* Marker_wait(PyObject* o, PyObject* stream)
 {
-    PyObject* given = Py_None;
-    if (!PyArg_ParseTuple(args, "|O", &given)) return false;
-    if (given != Py_None) return stream_from(given, s);
-    *s = current_stream(device);
-    return true;
-}
-PyObject* Marker_wait(PyObject* o, PyObject* args)
-{
-    HANDLE_TH_ERRORS
-    Marker* m = reinterpret_cast<Marker*>(o);
     Stream s;
-    if (!optional_stream(args, m->device, &s)) return nullptr;
-    return marker_wait(m, s.raw);
-    END_HANDLE_TH_ERRORS
-}
-PyObject* Marker_record(PyObject* o, PyObject* args)
-{
-    HANDLE_TH_ERRORS
-    Marker* m = reinterpret_cast<Marker*>(o);
-    Stream s;
-    if (!optional_stream(args, m->device, &s)) return nullptr;
-    if (m->event == nullptr && (m->event = m->pool->take()) == nullptr) return raise_hip("hipEventCreate", hipErrorUnknown);
-    if (hipError_t err = hipEventRecord(m->event, s.raw); err != hipSuccess) return raise_hip("hipEventRecord", err);
-    Py_RETURN_NONE;
-    END_HANDLE_TH_ERRORS
-}
-PyObject* Marker_query(PyObject* o, PyObject*)
-{
-    Marker* m = reinterpret_cast<Marker*>(o);
-    if (m->event == nullptr) return PyBool_FromLong(m->counter->reached(m->value));
-    const hipError_t err = hipEventQuery(reinterpret_cast<Marker*>(o)->event);
-    if (err == hipErrorNotReady) (void)hipGetLastError();
-    else if (err != hipSuccess) return raise_hip("hipEventQuery", err);
-    return PyBool_FromLong(err == hipSuccess);
-}
-PyObject* Marker_synchronize(PyObject* o, PyObject*)
-{
-    Marker* m = reinterpret_cast<Marker*>(o);
-    hipError_t err;
-    Py_BEGIN_ALLOW_THREADS;
-    // (a counter's value is behind everything its stream was given before, so waiting for that stream suffices)
-    err = m->event != nullptr ? hipEventSynchronize(m->event) : m->counter->reached(m->value) ? hipSuccess : hipStreamSynchronize(m->stream.raw);
-    Py_END_ALLOW_THREADS;
-    if (err != hipSuccess) return raise_hip("hipEventSynchronize", err);
-    Py_RETURN_NONE;
+    return stream_from(stream, &s) ? marker_wait(reinterpret_cast<Marker*>(o), s.raw) : nullptr;
 }
 PyObject* Marker_get_gpu(PyObject* o, void*) { return PyLong_FromLong(reinterpret_cast<Marker*>(o)->device); }
-PyObject* Marker_get_event(PyObject* o, void*) { return new_ref(o); }
 PyObject* Marker_get_stream(PyObject* o, void*)
 {
     Marker* m = reinterpret_cast<Marker*>(o);
     return stream_object(m->stream, m->device);
 }
 PyMethodDef marker_methods[] = {{"hold_current_stream", Marker_hold_current_stream, METH_NOARGS, nullptr},
-                                {"wait", Marker_wait, METH_VARARGS, nullptr},
-                                {"record", Marker_record, METH_VARARGS, nullptr},
-                                {"query", Marker_query, METH_NOARGS, nullptr},
-                                {"synchronize", Marker_synchronize, METH_NOARGS, nullptr},
+                                {"wait", Marker_wait, METH_O, nullptr},
                                 {nullptr, nullptr, 0, nullptr}};
 PyGetSetDef marker_getset[] = {{"gpu", Marker_get_gpu, nullptr, nullptr, nullptr},
-                               {"event", Marker_get_event, nullptr, nullptr, nullptr},
                                {"stream", Marker_get_stream, nullptr, nullptr, nullptr},
                                {nullptr, nullptr, nullptr, nullptr, nullptr}};
 PyTypeObject MarkerType = {PyVarObject_HEAD_INIT(nullptr, 0) "deepep_amd._host.Marker", sizeof(Marker)};
@@ -504,7 +417,6 @@ Plan* intact_plan(PyObject* handle, PyObject* owner, PyObject** dict)
 // ---- the exchange of one buffer -------------------------------------------------------------------------------------------
 struct Exchange {
     PyObject_HEAD
-    std::shared_ptr<EventPool> pool;
     void* workspace;
     PyObject* token;  // the buffer's handle token
     PyObject* lock;   // the buffer's lock (a threading.RLock)
@@ -515,7 +427,7 @@ struct Exchange {
     Stream comm, last;      // call only (torch makes a pooled stream when its handle is first read, 0.25 ms)
     bool has_comm, has_last;
     double share;     // rows per route of the most recent fresh dispatch: sizes the next one's outputs, see capacity_for
-    hipEvent_t order; // for waits between two streams, recorded anew each time
+    OrderEvent order;
     // asynchronous calls: the communication stream's counter, and the one that the callers' stream raises (one stream at a
     // time: another takes it over when everything it was told to reach has been reached); nullptr: events instead
     Counter *comm_counter, *caller_counter;
@@ -546,9 +458,7 @@ struct Locked {  // the buffer's lock, held
 
 bool wait_for_stream(Exchange* e, hipStream_t waits, hipStream_t on)
 {
-    if (e->order == nullptr && (e->order = e->pool->take()) == nullptr) return raise_hip("hipEventCreate", hipErrorUnknown) != nullptr;
-    hipError_t err = hipEventRecord(e->order, on);
-    if (err == hipSuccess) err = hipStreamWaitEvent(waits, e->order, 0);
+    const hipError_t err = e->order.order(waits, on);
     return err == hipSuccess ? true : raise_hip("ordering two streams", err) != nullptr;
 }
 
@@ -597,11 +507,16 @@ PyObject* event_of(Exchange* e, const Target& t, std::initializer_list<const at:
 {
     Ref overlap(g_overlap_type->tp_new(g_overlap_type, g_empty_tuple, nullptr));
     if (!overlap || !t.asynchronous) return overlap.release();
-    Ref marker(reinterpret_cast<PyObject*>(marker_new(e->pool, e->comm_counter != nullptr && !capturing(e->comm.raw) ? e->comm_counter : nullptr,
-                                                      e->comm, e->device)));
-    if (!marker) return nullptr;
-    Ref event(g_event_type->tp_new(g_event_type, g_empty_tuple, nullptr));
-    if (!event || PyObject_SetAttr(event.p, N._marker, marker.p) < 0) return nullptr;
+    Ref event;
+    if (e->comm_counter != nullptr && !capturing(e->comm.raw)) {
+        Ref marker(reinterpret_cast<PyObject*>(marker_new(e->comm_counter, e->comm, e->device)));
+        if (!marker) return nullptr;
+        event = Ref(g_event_type->tp_new(g_event_type, g_empty_tuple, nullptr));
+        if (!event || PyObject_SetAttr(event.p, N._marker, marker.p) < 0) return nullptr;
+    } else {  // (under capture a value would be frozen into the graph) EventHandle(stream): a torch event
+        event = Ref(PyObject_CallOneArg(reinterpret_cast<PyObject*>(g_event_type), e->comm_object));
+        if (!event) return nullptr;
+    }
     Lease* lease = reinterpret_cast<Lease*>(LeaseType.tp_alloc(&LeaseType, 0));
     if (lease == nullptr) return nullptr;
     Ref owned(reinterpret_cast<PyObject*>(lease));
@@ -1116,7 +1031,6 @@ PyObject* Exchange_new(PyTypeObject* type, PyObject* args, PyObject*)
     if (ws == nullptr && PyErr_Occurred()) return nullptr;
     Exchange* e = reinterpret_cast<Exchange*>(type->tp_alloc(type, 0));
     if (e == nullptr) return nullptr;
-    new (&e->pool) std::shared_ptr<EventPool>(std::make_shared<EventPool>());
     e->workspace = ws;
     e->token = new_ref(token);
     e->lock = new_ref(lock);
@@ -1132,7 +1046,6 @@ PyObject* Exchange_new(PyTypeObject* type, PyObject* args, PyObject*)
     e->failed = e->closed = e->has_comm = e->has_last = false;
     e->comm_object = new_ref(comm);
     e->share = 0.0;
-    e->order = nullptr;
     // (taken with the buffer, whose workspace is allocated now as well: the first asynchronous call may be under capture, where
     // nothing may be allocated)
     e->comm_counter = take_counter(device);
@@ -1143,13 +1056,12 @@ PyObject* Exchange_new(PyTypeObject* type, PyObject* args, PyObject*)
 void Exchange_dealloc(PyObject* o)
 {
     Exchange* e = reinterpret_cast<Exchange*>(o);
-    if (e->order != nullptr) e->pool->give_back(e->order);
+    e->order.release();
     for (Counter* c : {e->comm_counter, e->caller_counter})
         if (c != nullptr && c->reached(c->raised)) g_idle_counters.push_back(c);  // (one still pending is not used again)
     Py_XDECREF(e->token);
     Py_XDECREF(e->lock);
     Py_XDECREF(e->comm_object);
-    e->pool.~shared_ptr();
     Py_TYPE(o)->tp_free(o);
 }
 PyObject* Exchange_get_failed(PyObject* o, void*) { return PyBool_FromLong(reinterpret_cast<Exchange*>(o)->failed); }
@@ -1191,7 +1103,6 @@ PyTypeObject ExchangeType = {PyVarObject_HEAD_INIT(nullptr, 0) "deepep_amd._host
 // One SymmBuffer's forward (deepep_amd.megamoe.api._run), and the FP8 casts.
 struct Mega {
     PyObject_HEAD
-    std::shared_ptr<EventPool> pool;
     PyObject* lock;      // the buffer's lock (a threading.Lock)
     PyObject *logical1, *logical2, *shared1, *shared2;  // (experts, N, K) that l1 / l2 / shared l1 / shared l2 must have
     void* workspace;     // of batches of `batch` rows; nullptr before the first
@@ -1199,7 +1110,7 @@ struct Mega {
     int device, experts, first_expert, local, topk, hidden, inter, shared, capacity, padded;
     Stream last;
     bool has_last, closed;
-    hipEvent_t order;
+    OrderEvent order;
 };
 extern PyTypeObject MegaType;
 PyTypeObject* g_pair_type;  // deepep_amd.megamoe.api._PreparedPair
@@ -1273,12 +1184,8 @@ PyObject* Mega_forward(PyObject* self, PyObject* const* a, Py_ssize_t n)
     if (!held.held) return nullptr;
     if (m->closed || m->workspace == nullptr || rows != m->batch) Py_RETURN_NONE;
     const Stream stream = current_stream(m->device);
-    if (m->has_last && !(m->last == stream)) {
-        if (m->order == nullptr && (m->order = m->pool->take()) == nullptr) return raise_hip("hipEventCreate", hipErrorUnknown);
-        hipError_t err = hipEventRecord(m->order, m->last.raw);
-        if (err == hipSuccess) err = hipStreamWaitEvent(stream.raw, m->order, 0);
-        if (err != hipSuccess) return raise_hip("ordering two streams", err);
-    }
+    if (m->has_last && !(m->last == stream))
+        if (const hipError_t err = m->order.order(stream.raw, m->last.raw); err != hipSuccess) return raise_hip("ordering two streams", err);
     m->last = stream;
     m->has_last = true;
     at::Tensor y = out != nullptr ? *out : allocate({rows, m->hidden}, at::kBFloat16, m->device);
@@ -1326,7 +1233,6 @@ PyObject* Mega_new(PyTypeObject* type, PyObject* args, PyObject*)
     if (!PyArg_ParseTuple(args, "Oiiiiiiiii", &lock, &device, &experts, &first, &local, &topk, &hidden, &inter, &shared, &capacity)) return nullptr;
     Mega* m = reinterpret_cast<Mega*>(type->tp_alloc(type, 0));
     if (m == nullptr) return nullptr;
-    new (&m->pool) std::shared_ptr<EventPool>(std::make_shared<EventPool>());
     m->lock = new_ref(lock);
     m->device = device;
     m->experts = experts;
@@ -1347,9 +1253,8 @@ PyObject* Mega_new(PyTypeObject* type, PyObject* args, PyObject*)
 void Mega_dealloc(PyObject* o)
 {
     Mega* m = reinterpret_cast<Mega*>(o);
-    if (m->order != nullptr) m->pool->give_back(m->order);
+    m->order.release();
     for (PyObject* p : {m->lock, m->logical1, m->logical2, m->shared1, m->shared2}) Py_XDECREF(p);
-    m->pool.~shared_ptr();
     Py_TYPE(o)->tp_free(o);
 }
 // use(workspace handle, batch): the workspace of the batches to come; use(0, 0): none.
@@ -1479,7 +1384,6 @@ PyMODINIT_FUNC PyInit__host()
     if ((g_empty_tuple = PyTuple_New(0)) == nullptr) return nullptr;
     LeaseType.tp_dealloc = Lease_dealloc;
     LeaseType.tp_methods = lease_methods;
-    MarkerType.tp_dealloc = Marker_dealloc;
     MarkerType.tp_methods = marker_methods;
     MarkerType.tp_getset = marker_getset;
     PlanType.tp_dealloc = Plan_dealloc;

@@ -4,8 +4,8 @@ protocol), over HIP events through ``torch.cuda``.
 
 How it is put together here: a ``_Marker`` is one recorded HIP event plus where it was recorded; a ``_Lease`` keeps
 objects alive and tells torch's caching allocator which streams use which tensors.  ``EventHandle`` is a marker with
-a public face, ``EventOverlap`` a marker, a lease and an optional hook.  The native host path makes markers and leases of
-its own (``_host.Marker``, ``_host.Lease``) with the same methods.
+a public face, ``EventOverlap`` a marker, a lease and an optional hook.  The native host path makes leases of its own
+(``_host.Lease``) and marks a stream by the value of a counter (``_host.Marker``), with the same methods but no event.
 """
 
 from __future__ import annotations
@@ -37,6 +37,18 @@ class _Marker:
             raise RuntimeError("Cannot record an event on another GPU")
         self.event = api.Event()
         self.event.record(self.stream)
+
+    @classmethod
+    def _of(cls, counted):
+        """A HIP event that completes when the counter value of ``_host.Marker`` ``counted`` is reached, neither earlier nor
+        later: recorded on a stream of its own that waits for the value and for nothing else."""
+        api = gpu_api()
+        marker = cls.__new__(cls)
+        marker.gpu, marker.stream, marker.event = counted.gpu, counted.stream, api.Event()
+        side = api.Stream(device=marker.gpu)
+        counted.wait(side)
+        marker.event.record(side)
+        return marker
 
     def hold_current_stream(self):
         """Makes the current stream of the marker's GPU wait for the event; returns that stream."""
@@ -76,6 +88,9 @@ class EventHandle:
 
     @property
     def event(self) -> Any:
+        """The event itself, one of torch's.  From then on the handle goes by it (so recording it again counts)."""
+        if not isinstance(self._marker, _Marker):
+            self._marker = _Marker._of(self._marker)
         return self._marker.event
 
     @property

@@ -267,6 +267,40 @@ def test_event_of_an_asynchronous_call_stands_in_for_torchs():
         buffer.destroy()
 
 
+def test_event_of_an_asynchronous_call_is_torchs_own_and_marks_that_call_only():
+    x, _ = _batch(64, 256, 2, 3)
+    idx = torch.stack([torch.randperm(8)[:2] for _ in range(64)]).cuda()
+    buffer = _buffer(num_bytes=4 << 20)
+    try:
+        comm = buffer.get_comm_stream()
+        for sleep_first in (False, True):  # the value is still to come when the event is asked for, or is there already
+            if sleep_first:
+                with torch.cuda.stream(comm):
+                    torch.cuda._sleep(2_000_000)
+            recv, _, _, handle, overlap = buffer.dispatch(x.cuda(), topk_idx=idx, num_experts=8, async_with_compute_stream=True)
+            event = overlap.event.event
+            assert isinstance(event, torch.cuda.Event) and event is overlap.event.event and event.cuda_event != 0
+            with torch.cuda.stream(comm):
+                torch.cuda._sleep(200_000_000)  # about 0.1 s: what the stream is given later is not waited for
+            event.synchronize()
+            assert event.query() and not comm.query()
+            torch.cuda.synchronize()
+            # recorded again, it stands for what that stream has been given by then
+            late = torch.zeros(4, device="cuda")
+            torch.cuda.synchronize()
+            with torch.cuda.stream(comm):
+                torch.cuda._sleep(20_000_000)
+                late.add_(1)
+                event.record(comm)
+            overlap.current_stream_wait()
+            assert (late * 1).tolist() == [1.0] * 4
+        with pytest.raises(Exception):
+            event.elapsed_time(event)  # (made without timing, as before)
+    finally:
+        torch.cuda.synchronize()
+        buffer.destroy()
+
+
 @pytest.mark.parametrize("on_side_stream", [False, True])
 def test_an_overlap_made_from_the_event_of_an_asynchronous_call_keeps_its_tensors(on_side_stream):
     """EventOverlap's public constructor with the event of a call: the given tensors are kept for the work and declared to
