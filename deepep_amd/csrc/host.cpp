@@ -32,6 +32,7 @@ namespace {
 constexpr int kMaxTokens = 16384, kMaxHidden = 7168, kMaxTopk = 16, kMaxExperts = 1024;
 constexpr int kLowLatencyMaxTokens = 256;
 constexpr long long kWaitTimeoutUs = 100LL * 1000 * 1000;
+constexpr int64_t kSmallBlock = 64 << 10;
 constexpr int kSpinsWithGil = 4096;  // about 100 us of polling before other Python threads get their turn
 
 // ---- small helpers ---------------------------------------------------------------------------------------------------
@@ -654,12 +655,17 @@ PyObject* run_fresh(Exchange* e, const FreshCall& c, const Target& t, PyObject* 
     const bool small = routes <= 2048;
     const long long capacity = c.low_latency ? c.capacity_rows : capacity_for(e, routes, local, c.experts, small);
 
-    // One block for all of the routing: [ids 8 B][route_to_row][row_to_route][counts][psum][offsets][num_rows][send_counts]
-    // [row weights], and one for the payload, which holds the scales too where both are small (an allocation takes 1 us).
-    const int64_t at_forward = c.copy_idx ? routes * 8 : 0, at_rows = at_forward + routes * 4, at_counts = at_rows + routes * 4;
+    // One block for all of the routing: [ids 8 B][route_to_row][row_to_route][counts][psum][offsets][num_rows][send_counts], with
+    // the row weights behind it where both are small, and one for the payload, which holds the scales too where both are
+    // small (an allocation takes 1 us).  Maps and weights start at multiples of 256 bytes, as tensors of their own would; a
+    // caller that keeps the received weights for longer than the handle keeps no more than kSmallBlock with them.
+    auto aligned = [](int64_t bytes) { return (bytes + 255) / 256 * 256; };
+    const int64_t at_forward = c.copy_idx ? aligned(routes * 8) : 0, at_rows = at_forward + aligned(routes * 4);
+    const int64_t at_counts = at_rows + aligned(routes * 4);
     const int64_t at_psum = at_counts + local * 4, at_offsets = at_psum + local * 4, at_num = at_offsets + (local + 1) * 4;
-    const int64_t at_send = at_num + 4, at_weights = at_send + (c.low_latency ? c.experts * 4 : 0);
-    at::Tensor routing = allocate({at_weights + (c.weights != nullptr ? capacity * 4 : 0)}, at::kByte, device), out, scales, weights;
+    const int64_t at_send = at_num + 4, at_weights = aligned(at_send + (c.low_latency ? c.experts * 4 : 0));
+    const bool weights_inside = c.weights != nullptr && at_weights + capacity * 4 <= kSmallBlock;
+    at::Tensor routing = allocate({at_weights + (weights_inside ? capacity * 4 : 0)}, at::kByte, device), out, scales, weights;
     const at::ScalarType scale_type = c.quantize || c.in.scales == nullptr ? at::kFloat : c.in.scales->scalar_type();
     const int64_t code_bytes = capacity * width, scale_bytes = capacity * scale_cols * 4;
     if (scale_cols > 0 && code_bytes <= (1 << 20)) {  // (codes of one byte; width is a multiple of 16)
@@ -670,7 +676,8 @@ PyObject* run_fresh(Exchange* e, const FreshCall& c, const Target& t, PyObject* 
         out = allocate({capacity, width}, out_type, device);
         if (scale_cols > 0) scales = allocate({capacity, scale_cols}, scale_type, device);
     }
-    if (c.weights != nullptr) weights = over(routing.storage(), at_weights, at::kFloat, {capacity});
+    if (c.weights != nullptr)
+        weights = weights_inside ? over(routing.storage(), at_weights, at::kFloat, {capacity}) : allocate({capacity}, at::kFloat, device);
     char* base = static_cast<char*>(routing.data_ptr());
 
     dpep_fresh_dispatch call = {};
@@ -773,7 +780,7 @@ PyObject* run_fresh(Exchange* e, const FreshCall& c, const Target& t, PyObject* 
         if (rows > capacity) {  // more rows than the share suggested: once more, into outputs of the right size
             pending.replace(&out, {rows, width}, out_type);
             if (scales.defined()) pending.replace(&scales, {rows, scale_cols}, scale_type);
-            if (weights.defined()) weights = allocate({rows}, at::kFloat, device);
+            if (weights.defined()) pending.replace(&weights, {rows}, at::kFloat);
             float* s_out = scales.defined() ? static_cast<float*>(scales.data_ptr()) : nullptr;
             float* w_out = weights.defined() ? static_cast<float*>(weights.data_ptr()) : nullptr;
             status = c.quantize ? dpep_dispatch_quant_fp8(call.x, call.topk_weights, call.route_to_row, call.row_to_route, call.num_tokens,
@@ -784,7 +791,7 @@ PyObject* run_fresh(Exchange* e, const FreshCall& c, const Target& t, PyObject* 
         } else if (rows < capacity) {
             out = over(out.storage(), 0, out_type, {rows, width});
             if (scales.defined()) scales = over(scales.storage(), scales.storage_offset() * 4, scale_type, {rows, scale_cols});
-            if (weights.defined()) weights = over(storage, at_weights, at::kFloat, {rows});
+            if (weights.defined()) weights = over(weights.storage(), weights.storage_offset() * 4, at::kFloat, {rows});
         }
         Ref list(PyList_New(local));
         if (!list) return nullptr;

@@ -106,6 +106,33 @@ def test_low_latency_ids_and_send_counts(per_rank, skewed):
         buffer.destroy()
 
 
+@pytest.mark.parametrize("world,tokens,experts,topk", [(1, 1, 1, 1), (1, 31, 8, 2), (1, 1000, 160, 6), (8, 2048, 256, 8), (16, 37, 496, 3),
+                                                       (16, 256, 512, 5)])
+def test_received_weights_and_maps_are_aligned_and_keep_little_else_alive(world, tokens, experts, topk):
+    """Whatever they share an allocation with: addresses as a tensor of its own would have them, and no more than 64 KiB
+    held through the weights beyond their own rows."""
+    hidden, per_rank = 256, tokens if world < 16 else -(-tokens // world)
+    x, w = _batch(per_rank * world if world >= 16 else tokens, hidden, topk, 8)
+    idx = torch.stack([torch.randperm(experts)[:topk] for _ in range(x.shape[0])]).cuda()
+    buffer = _buffer(num_bytes=8 << 30, rank=world - 1, world_size=world)
+    try:
+        recv, _, recv_w, handle, _ = buffer.dispatch(x.cuda(), topk_idx=idx, topk_weights=w.cuda(), num_experts=experts)
+        assert handle.is_low_latency == (world == 16)
+        weights = handle.source_weights if handle.is_low_latency else recv_w
+        maps = [handle.topk_idx, handle.route_to_row] + ([] if handle.is_low_latency else [handle.weight_return_meta])
+        for t in (weights, *maps):
+            assert t.data_ptr() % 256 == 0
+        held = weights.untyped_storage().nbytes()
+        assert held <= 65536 or held <= 4 * recv.untyped_storage().nbytes() // (hidden * 2)
+        if not handle.is_low_latency:
+            want = olayout.layout(idx.cpu().numpy(), experts, (world - 1) * experts // world, experts // world)
+            np.testing.assert_array_equal(f32_bits(weights), olayout.expand_weights(w.numpy(), want["row_to_route"]).view(np.uint32))
+            np.testing.assert_array_equal(handle.weight_return_meta.cpu().numpy(), want["row_to_route"])
+            np.testing.assert_array_equal(handle.expert_offsets.cpu().numpy(), want["offsets"])
+    finally:
+        buffer.destroy()
+
+
 def test_changed_handles_and_unusual_tensors_take_the_slow_path():
     x, w = _batch(40, 256, 2, 1)
     idx = torch.stack([torch.randperm(8)[:2] for _ in range(40)]).cuda()
