@@ -540,7 +540,7 @@ PyObject* event_of(Exchange* e, const Target& t, std::initializer_list<const at:
 // Answers for the tensors of a call from its first launch until the call has an event (event_of), whatever way the call ends.
 // On the communication stream a launch may still be pending when a tensor is let go, and memory that was allocated on the
 // caller's stream is handed out again in that stream's order alone: so it is declared to the allocator first, where an output
-// is replaced (replace) and where a launch, a wait or an allocation fails behind a launch.  In the latter case the buffer
+// is replaced (replace; a small batch's launch writes what fits) and where a launch, a wait or an allocation fails behind a launch.  In the latter case the buffer
 // takes no further calls either.
 struct Pending {
     Exchange* e;
@@ -560,6 +560,7 @@ struct Pending {
     void replace(at::Tensor* x, at::IntArrayRef sizes, at::ScalarType type) const
     {
         declare(*x);
+        *x = at::Tensor();  // (first, so that its memory can be had again)
         *x = allocate(sizes, type, e->device);
     }
     ~Pending()
@@ -626,8 +627,9 @@ bool keep_same(Plan* plan, PyObject* dict, std::initializer_list<PyObject*> name
 // Rows to allocate for a fresh dispatch's payload before R is known.  Where at least half of the experts are local (or the
 // batch is small) all T*K routes, as the payload kernel then runs at once and the surplus is small.  Otherwise a quarter more
 // than the share that the expert range or the previous batch suggests: the payload can then be queued behind the layout as
-// well, instead of after the host has read R (which left the GPU idle for the length of a host round trip); a batch with
-// more rows than that is dispatched again into outputs of the right size.
+// well, instead of after the host has read R (which left the GPU idle for the length of a host round trip).  A batch with
+// more rows than that is moved once the host knows R, into outputs of that size: the payload that is queued already finds the
+// count on the device and ends without moving anything.
 long long capacity_for(const Exchange* e, long long routes, long long local, long long experts, bool small)
 {
     if (small || 2 * local >= experts) return routes;
@@ -705,7 +707,7 @@ PyObject* run_fresh(Exchange* e, const FreshCall& c, const Target& t, PyObject* 
     call.scale_cols = static_cast<int32_t>(c.quantize ? 0 : scale_cols);
     call.quantize = c.quantize;
     call.capacity_rows = static_cast<int32_t>(capacity);
-    call.report_to_host = !c.low_latency;
+    call.report_to_host = c.low_latency ? 0 : DPEP_REPORT_ALL_OR_NONE;
     Pending pending(e, t, {&out, &scales, &weights, &routing, c.in.x, c.in.scales, c.weights, c.idx});
     pending.launched = true;
     if (const int status = dpep_dispatch_fresh(e->workspace, &call, t.stream.raw)) return raise_native(status);
@@ -777,7 +779,7 @@ PyObject* run_fresh(Exchange* e, const FreshCall& c, const Target& t, PyObject* 
         rows = reported;
         plan->rows = rows;
         e->share = static_cast<double>(rows) / static_cast<double>(routes);
-        if (rows > capacity) {  // more rows than the share suggested: once more, into outputs of the right size
+        if (rows > capacity) {  // more rows than the share suggested: into outputs of the right size
             pending.replace(&out, {rows, width}, out_type);
             if (scales.defined()) pending.replace(&scales, {rows, scale_cols}, scale_type);
             if (weights.defined()) pending.replace(&weights, {rows}, at::kFloat);

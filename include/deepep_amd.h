@@ -159,7 +159,10 @@ int dpep_layout_dispatch_small(void* ws, const int64_t* topk_idx, const void* x,
 /* One fresh dispatch as ElasticBuffer makes it (notify + dispatch, deep_ep/backends/mesh_clos/elastic.py:648-1008): the layout
  * and, queued behind it before the host knows R, the payload; for a small batch both in one launch (see above).  The
  * payload outputs hold capacity_rows rows, of which the first min(R, capacity_rows) are written: a caller that finds
- * R > capacity_rows allocates R rows and calls dpep_dispatch_copy / dpep_dispatch_quant_fp8 with the same maps. */
+ * R > capacity_rows allocates R rows and calls dpep_dispatch_copy / dpep_dispatch_quant_fp8 with the same maps.  One that always
+ * does so sets report_to_host to DPEP_REPORT_ALL_OR_NONE: if R > capacity_rows the outputs are then left as they are (a small
+ * batch may write part of them), and the launch ends at once. */
+#define DPEP_REPORT_ALL_OR_NONE 2
 typedef struct dpep_fresh_dispatch {
     const int64_t* topk_idx;    /* [T,K] */
     int64_t* topk_idx_copy;     /* [T,K] receives a copy of topk_idx (the handle's own), or NULL */
@@ -180,7 +183,7 @@ typedef struct dpep_fresh_dispatch {
     int32_t row_bytes, scale_cols;
     int32_t quantize;           /* != 0: x is BF16 and is quantised per 128 columns (scales NULL, out FP8, out_scales [.,H/128]) */
     int32_t capacity_rows;
-    int32_t report_to_host;     /* != 0: counts and R also go to the host mailbox (dpep_layout_wait) */
+    int32_t report_to_host;     /* != 0: counts and R also go to the host mailbox (dpep_layout_wait); see above for 2 */
 } dpep_fresh_dispatch;
 int dpep_dispatch_fresh(void* ws, const dpep_fresh_dispatch* call, void* stream);
 

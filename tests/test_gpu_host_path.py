@@ -2,6 +2,8 @@
 and outgrown by it, row-major payloads that walk past their grid, the routing copy, ids per rank of the low-latency path,
 handles that leave the native path, and memory that is handed out again behind asynchronous calls."""
 
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -441,3 +443,80 @@ def test_stream_raise_stores_behind_earlier_work_and_refuses_bad_words():
     assert word.tolist() == [5_000_000_000, 3]
     for bad in (0, word.data_ptr() + 4):
         assert lib.dpep_stream_raise(bad, 1, stream) != 0
+
+
+class _FreshDispatch(ctypes.Structure):
+    _fields_ = [(name, ctypes.c_void_p) for name in (
+        "topk_idx", "topk_idx_copy", "x", "scales", "topk_weights", "counts", "psum", "offsets", "route_to_row", "row_to_route", "num_rows",
+        "send_counts", "out", "out_scales", "out_weights")] + [(name, ctypes.c_int32) for name in (
+            "num_tokens", "num_topk", "num_experts", "expert_begin", "num_local", "row_bytes", "scale_cols", "quantize", "capacity_rows",
+            "report_to_host")]
+
+
+@pytest.mark.parametrize("report,short_by", [(2, 0), (2, 1), (2, 3000), (1, 1), (1, 3000)])
+@pytest.mark.parametrize("quantize", [False, True])
+@pytest.mark.parametrize("tokens,topk,experts,local", [(1000, 8, 32, 8), (4001, 1, 16, 4)])  # token-major and row-major payloads
+def test_fresh_dispatch_into_outputs_that_are_too_small(tokens, topk, experts, local, quantize, report, short_by):
+    """dpep_dispatch_fresh with capacities around the number of rows: all rows, the first ones, or (all or none) nothing."""
+    from deepep_amd import _lib, ops
+
+    hidden, begin = 256, local
+    rng = np.random.default_rng(tokens)
+    popularity = np.where((np.arange(experts) >= begin) & (np.arange(experts) < begin + local), 20.0, 1.0)
+    ids = np.stack([rng.choice(experts, topk, replace=False, p=popularity / popularity.sum()) for _ in range(tokens)]).astype(np.int64)
+    want = olayout.layout(ids, experts, begin, local)
+    rows = want["num_rows"]
+    capacity = max(rows - short_by, 0)
+    moved = rows if short_by == 0 else capacity if report == 1 else 0
+    x, w = _batch(tokens, hidden, topk, 9)
+    device = dict(device="cuda")
+    idx, xd, wd = torch.from_numpy(ids).cuda(), x.cuda(), w.cuda()
+    meta = torch.zeros(3 * local + 2, dtype=torch.int32, **device)
+    forward = torch.zeros(tokens * topk, dtype=torch.int32, **device)
+    back = torch.zeros(tokens * topk, dtype=torch.int32, **device)
+    out = torch.full((rows, hidden * (1 if quantize else 2)), 0x55, dtype=torch.uint8, **device)
+    scales = torch.full((rows, hidden // 128), 5.0, **device) if quantize else None
+    weights = torch.full((rows,), 5.0, **device)
+    call = _FreshDispatch(
+        idx.data_ptr(), None, xd.data_ptr(), None, wd.data_ptr(), meta.data_ptr(), meta[local:].data_ptr(), meta[2 * local :].data_ptr(),
+        forward.data_ptr(), back.data_ptr(), meta[3 * local + 1 :].data_ptr(), None, out.data_ptr(),
+        scales.data_ptr() if quantize else None, weights.data_ptr(), tokens, topk, experts, begin, local, hidden * 2, 0, int(quantize),
+        capacity, report)
+    workspace = ops.Workspace(1 << 20)
+    try:
+        stream = torch.cuda.current_stream().cuda_stream
+        _lib.check(_lib.load().dpep_dispatch_fresh(workspace.handle, ctypes.byref(call), stream), "dispatch_fresh")
+        assert ops.layout_wait(workspace) == (None, rows)
+        torch.cuda.synchronize()
+    finally:
+        workspace.destroy()
+    np.testing.assert_array_equal(forward.cpu().numpy().reshape(tokens, topk), want["route_to_row"])
+    if quantize:
+        codes, factors = oquant.cast_to_fp8_torch(x)
+        np.testing.assert_array_equal(f32_bits(scales[:moved]), olayout.expand_rows(f32_bits(factors), want["row_to_route"], topk)[:moved])
+        assert bool((scales[moved:] == 5.0).all())
+        payload = fp8_bits(codes)
+    else:
+        payload = x.view(torch.uint8).numpy()
+    np.testing.assert_array_equal(out[:moved].cpu().numpy(), olayout.expand_rows(payload, want["row_to_route"], topk)[:moved])
+    np.testing.assert_array_equal(f32_bits(weights[:moved]), olayout.expand_weights(w.numpy(), want["row_to_route"]).view(np.uint32)[:moved])
+    assert bool((out[moved:] == 0x55).all()) and bool((weights[moved:] == 5.0).all())
+
+
+def test_outputs_that_a_share_outgrows_are_given_back_first():
+    """A hot batch behind a cold one: the outputs made for the cold one's share are gone when those of the right size are made."""
+    world, experts, topk, tokens, hidden = 4, 16, 4, 8192, 2048
+    hot = torch.stack([torch.randperm(4)[:topk] for _ in range(tokens)]).cuda()
+    x = torch.randn(tokens, hidden, device="cuda").bfloat16()
+    buffer = _buffer(num_bytes=4 << 20, rank=0, world_size=world)
+    try:
+        torch.cuda.synchronize()
+        before = torch.cuda.memory_allocated()
+        torch.cuda.reset_peak_memory_stats()
+        recv, _, _, handle, _ = buffer.dispatch(x, topk_idx=hot, num_experts=experts)
+        peak = torch.cuda.max_memory_allocated() - before
+        assert handle.num_expanded_tokens == tokens * topk
+        payload = tokens * topk * hidden * 2
+        assert payload <= recv.untyped_storage().nbytes() == payload and peak <= payload + (2 << 20)
+    finally:
+        buffer.destroy()
