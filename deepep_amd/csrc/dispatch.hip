@@ -49,7 +49,7 @@ void with_store_policy(Launch&& launch)
 }
 
 // ---- token-major copy: one workgroup per (token, column part); read once, write K times -----------
-// Rows at or beyond `capacity` are dropped; with all_rows (the layout's count) nothing is moved unless all rows fit.
+// Rows at or beyond `capacity` are dropped; with all_rows (the layout's count) nothing is moved unless DPEP_ROWS_KEPT.
 template <int kPolicy>
 __global__ __launch_bounds__(kMaxThreads) void dispatch_copy_token_kernel(
     const u32x4* __restrict__ x, const float* __restrict__ scales, const float* __restrict__ weights,
@@ -60,7 +60,7 @@ __global__ __launch_bounds__(kMaxThreads) void dispatch_copy_token_kernel(
     __shared__ int rows[DPEP_MAX_TOPK];
     __shared__ int any_valid;
     const int token = blockIdx.x / parts, part = blockIdx.x % parts;
-    const bool fits = all_rows == nullptr || *all_rows <= capacity;  // (travels with the values and the routes)
+    const int all = all_rows != nullptr ? *all_rows : capacity;  // (travels with the values and the routes)
     const int v_begin = part * vec_per_part;
     const int v_end = min(v_begin + vec_per_part, vec_per_row);
     const u32x4* src = x + static_cast<size_t>(token) * vec_per_row;
@@ -72,7 +72,7 @@ __global__ __launch_bounds__(kMaxThreads) void dispatch_copy_token_kernel(
     __syncthreads();
     if (threadIdx.x < num_topk) {
         int row = route_to_row[static_cast<size_t>(token) * num_topk + threadIdx.x];
-        if (row >= capacity || !fits) row = -1;  // outputs allocated before R was known
+        if (row >= capacity || !DPEP_ROWS_KEPT(all, capacity)) row = -1;  // outputs allocated before R was known
         rows[threadIdx.x] = row;
         if (row >= 0) any_valid = 1;
     }
@@ -102,19 +102,19 @@ __global__ __launch_bounds__(kMaxThreads) void dispatch_copy_token_kernel(
 
 // ---- row-major: one workgroup per (output row, column part); for sparse receive shares -------------
 // Rows [0, rows): `rows` from the host, or, rows_on_device, the smaller of that bound and the count the layout left on the
-// device (a payload queued before the host knows R); all_or_none: no rows at all if the count is larger than the bound.
-// Such a launch has workgroups for about the expected number of rows;
+// device (a payload queued before the host knows R); all_or_none, the outputs' capacity: no rows at all unless DPEP_ROWS_KEPT
+// (0: the first rows in any case).  Such a launch has workgroups for about the expected number of rows;
 // they walk on by the grid's rows until the real count is reached, and the first row's route is asked for together with
 // the count (row_to_route has an entry for every row of the grid, so the load is in bounds whatever the count says).
 struct RowRange {
     int rows;
     const int* rows_on_device;
-    bool all_or_none;
+    int all_or_none;
     __device__ __forceinline__ int count() const
     {
         if (rows_on_device == nullptr) return rows;
         const int all = *rows_on_device;
-        return all <= rows ? all : all_or_none ? 0 : rows;
+        return all_or_none == 0 || DPEP_ROWS_KEPT(all, all_or_none) ? min(all, rows) : 0;
     }
 };
 
@@ -222,7 +222,7 @@ __global__ __launch_bounds__(kMaxThreads) void dispatch_quant_token_kernel(
     __shared__ int any_valid;
     __shared__ float part_scales[kMaxScaleCols];
     const int token = blockIdx.x / parts, part = blockIdx.x % parts;
-    const bool fits = all_rows == nullptr || *all_rows <= capacity;  // (travels with the values and the routes)
+    const int all = all_rows != nullptr ? *all_rows : capacity;  // (travels with the values and the routes)
     const int u_begin = part * units_per_part;
     const int u_end = min(u_begin + units_per_part, units_per_row);
     const u32x4* src = x + static_cast<size_t>(token) * units_per_row * 2;
@@ -243,7 +243,7 @@ __global__ __launch_bounds__(kMaxThreads) void dispatch_quant_token_kernel(
     __syncthreads();
     if (threadIdx.x < num_topk) {
         int row = route_to_row[static_cast<size_t>(token) * num_topk + threadIdx.x];
-        if (row >= capacity || !fits) row = -1;  // outputs allocated before R was known
+        if (row >= capacity || !DPEP_ROWS_KEPT(all, capacity)) row = -1;  // outputs allocated before R was known
         rows[threadIdx.x] = row;
         if (row >= 0) any_valid = 1;
     }
@@ -598,7 +598,7 @@ struct Payload {
     float* out_weights;
 };
 
-// token-major: the grid does not depend on R; rows at or beyond `capacity` are dropped, all of them if the count at all_rows is larger.
+// token-major: the grid does not depend on R; rows at or beyond `capacity` are dropped; all_rows: all of them unless DPEP_ROWS_KEPT.
 int launch_token_major(const Payload& p, const int32_t* route_to_row, int capacity, const int32_t* all_rows, hipStream_t s)
 {
     const Split sp = choose_split(p.num_tokens, p.units, p.quantize ? 8 : 1);
@@ -642,7 +642,7 @@ int launch_payload(const Payload& p, const int32_t* route_to_row, const int32_t*
 {
     if (num_rows < 0 || static_cast<long long>(num_rows) > static_cast<long long>(kRowMajorRatio) * p.num_tokens)
         return launch_token_major(p, route_to_row, 0x7fffffff, nullptr, s);
-    return launch_row_major(p, row_to_route, RowRange{num_rows, nullptr, false}, num_rows, s);
+    return launch_row_major(p, row_to_route, RowRange{num_rows, nullptr, 0}, num_rows, s);
 }
 
 int launch_small(Workspace* w, const dpep_fresh_dispatch& c, int units, hipStream_t s)
@@ -782,14 +782,14 @@ int dpep_dispatch_fresh(void* ws, const dpep_fresh_dispatch* call, void* stream)
         // row-major over the rows that the layout finds: a token-major grid is mostly workgroups of tokens without a row
         // (6144 tokens of which 560 own a row: 10.5 us).
         const long long expected = n_routes * c.num_local / c.num_experts;
-        const bool all_or_none = c.report_to_host == DPEP_REPORT_ALL_OR_NONE && c.capacity_rows < n_routes;
+        const bool all_or_none = c.report_to_host == DPEP_REPORT_ALL_OR_NONE;
         if (expected > static_cast<long long>(kRowMajorRatio) * c.num_tokens)
             return launch_token_major(p, c.route_to_row, c.capacity_rows, all_or_none ? c.num_rows : nullptr, s);
         long long grid_rows = expected + expected / 8 + 64;
         if (grid_rows > c.capacity_rows) grid_rows = c.capacity_rows;
         if (grid_rows > n_routes) grid_rows = n_routes;
         const int bound = n_routes < c.capacity_rows ? static_cast<int>(n_routes) : c.capacity_rows;
-        return launch_row_major(p, c.row_to_route, RowRange{bound, c.num_rows, all_or_none}, static_cast<int>(grid_rows), s);
+        return launch_row_major(p, c.row_to_route, RowRange{bound, c.num_rows, all_or_none ? c.capacity_rows : 0}, static_cast<int>(grid_rows), s);
     }
     return fresh_in_one_launch(w, c, s);
 }
@@ -830,7 +830,7 @@ int dpep_cast_to_fp8(const void* x, int num_tokens, int hidden, void* out, float
     auto launch = [&](auto policy) {
         hipLaunchKernelGGL(dispatch_quant_row_kernel<decltype(policy)::value>, dim3(num_tokens * sp.parts),
                            dim3(sp.threads), 0, static_cast<hipStream_t>(stream), static_cast<const u32x4*>(x), nullptr,
-                           nullptr, RowRange{num_tokens, nullptr, false}, num_tokens, 1, units, sp.per_part, sp.parts,
+                           nullptr, RowRange{num_tokens, nullptr, 0}, num_tokens, 1, units, sp.per_part, sp.parts,
                            static_cast<u32x4*>(out), out_scales, nullptr);
     };
     // (codes that the memory-side cache takes are written through, whatever the dispatch's policy: the quantiser's reader is next.

@@ -427,7 +427,7 @@ struct Exchange {
     PyObject* comm_object;  // the communication stream as torch's object; its raw stream is asked for by the first asynchronous
     Stream comm, last;      // call only (torch makes a pooled stream when its handle is first read, 0.25 ms)
     bool has_comm, has_last;
-    double share;     // rows per route of the most recent fresh dispatch: sizes the next one's outputs, see capacity_for
+    double share;     // rows per route of the most recent fresh dispatch (negative: none yet), see capacity_for
     OrderEvent order;
     // asynchronous calls: the communication stream's counter, and the one that the callers' stream raises (one stream at a
     // time: another takes it over when everything it was told to reach has been reached); nullptr: events instead
@@ -540,7 +540,7 @@ PyObject* event_of(Exchange* e, const Target& t, std::initializer_list<const at:
 // Answers for the tensors of a call from its first launch until the call has an event (event_of), whatever way the call ends.
 // On the communication stream a launch may still be pending when a tensor is let go, and memory that was allocated on the
 // caller's stream is handed out again in that stream's order alone: so it is declared to the allocator first, where an output
-// is replaced (replace; a small batch's launch writes what fits) and where a launch, a wait or an allocation fails behind a launch.  In the latter case the buffer
+// is replaced (replace) and where a launch, a wait or an allocation fails behind a launch.  In the latter case the buffer
 // takes no further calls either.
 struct Pending {
     Exchange* e;
@@ -624,18 +624,18 @@ bool keep_same(Plan* plan, PyObject* dict, std::initializer_list<PyObject*> name
     return true;
 }
 
-// Rows to allocate for a fresh dispatch's payload before R is known.  Where at least half of the experts are local (or the
-// batch is small) all T*K routes, as the payload kernel then runs at once and the surplus is small.  Otherwise a quarter more
-// than the share that the expert range or the previous batch suggests: the payload can then be queued behind the layout as
-// well, instead of after the host has read R (which left the GPU idle for the length of a host round trip).  A batch with
-// more rows than that is moved once the host knows R, into outputs of that size: the payload that is queued already finds the
-// count on the device and ends without moving anything.
-long long capacity_for(const Exchange* e, long long routes, long long local, long long experts, bool small)
+// Rows to allocate for a fresh dispatch's payload before R is known.  Where at least half of the experts are local, or the batch is
+// small (one launch, at most 2048 rows), all T*K routes: the surplus is small.  Otherwise an eighth and 256 rows more than the previous batch's share of the routes suggests
+// (the first batch: than the expert range does), so that the payload can be queued behind the layout as well, instead of
+// after the host has read R, which left the GPU idle for the length of a host round trip.  (Random routes spread around an
+// even share of 16 384 rows by 128.)  A batch that jumps out of these bounds, up or down (DPEP_ROWS_KEPT: a received tensor keeps its
+// whole storage for as long as it lives), is moved once the host knows R, into outputs of that size: the payload that is
+// queued already finds the count on the device and ends without moving anything.  (Cold and hot batches in turn, us a dispatch,
+// against moving what fits and then everything: 16 384 tokens of 7168 columns, EP8, 173 -> 136; 4096 of 4096, EP4, 41 -> 37.)
+long long capacity_for(const Exchange* e, long long routes, long long local, long long experts)
 {
-    if (small || 2 * local >= experts) return routes;
-    const double share = std::max(static_cast<double>(local) / static_cast<double>(experts), e->share);
-    const long long rows = static_cast<long long>(share * 1.25 * static_cast<double>(routes)) + 256;
-    return std::min(rows, routes);
+    const double share = e->share >= 0.0 ? e->share : static_cast<double>(local) / static_cast<double>(experts);
+    return std::min(static_cast<long long>(share * 1.125 * static_cast<double>(routes)) + 256, routes);
 }
 
 struct FreshCall {
@@ -654,8 +654,8 @@ PyObject* run_fresh(Exchange* e, const FreshCall& c, const Target& t, PyObject* 
     const bool fp8_out = c.quantize || c.in.x->scalar_type() == at::kFloat8_e4m3fn;
     const at::ScalarType out_type = c.quantize ? at::kFloat8_e4m3fn : c.in.x->scalar_type();
     const long long scale_cols = c.quantize ? width / 128 : c.in.scales != nullptr ? c.in.scales->size(1) : 0;
-    const bool small = routes <= 2048;
-    const long long capacity = c.low_latency ? c.capacity_rows : capacity_for(e, routes, local, c.experts, small);
+    const bool all_routes = 2 * local >= c.experts || routes <= 2048;
+    const long long capacity = c.low_latency ? c.capacity_rows : all_routes ? routes : capacity_for(e, routes, local, c.experts);
 
     // One block for all of the routing: [ids 8 B][route_to_row][row_to_route][counts][psum][offsets][num_rows][send_counts], with
     // the row weights behind it where both are small, and one for the payload, which holds the scales too where both are
@@ -707,7 +707,7 @@ PyObject* run_fresh(Exchange* e, const FreshCall& c, const Target& t, PyObject* 
     call.scale_cols = static_cast<int32_t>(c.quantize ? 0 : scale_cols);
     call.quantize = c.quantize;
     call.capacity_rows = static_cast<int32_t>(capacity);
-    call.report_to_host = c.low_latency ? 0 : DPEP_REPORT_ALL_OR_NONE;
+    call.report_to_host = c.low_latency ? 0 : all_routes ? 1 : DPEP_REPORT_ALL_OR_NONE;
     Pending pending(e, t, {&out, &scales, &weights, &routing, c.in.x, c.in.scales, c.weights, c.idx});
     pending.launched = true;
     if (const int status = dpep_dispatch_fresh(e->workspace, &call, t.stream.raw)) return raise_native(status);
@@ -779,7 +779,7 @@ PyObject* run_fresh(Exchange* e, const FreshCall& c, const Target& t, PyObject* 
         rows = reported;
         plan->rows = rows;
         e->share = static_cast<double>(rows) / static_cast<double>(routes);
-        if (rows > capacity) {  // more rows than the share suggested: into outputs of the right size
+        if (!all_routes && !DPEP_ROWS_KEPT(rows, capacity)) {  // far from what the share suggested
             pending.replace(&out, {rows, width}, out_type);
             if (scales.defined()) pending.replace(&scales, {rows, scale_cols}, scale_type);
             if (weights.defined()) pending.replace(&weights, {rows}, at::kFloat);
@@ -1054,7 +1054,7 @@ PyObject* Exchange_new(PyTypeObject* type, PyObject* args, PyObject*)
     e->low_latency_workspace = low_latency;
     e->failed = e->closed = e->has_comm = e->has_last = false;
     e->comm_object = new_ref(comm);
-    e->share = 0.0;
+    e->share = -1.0;
     // (taken with the buffer, whose workspace is allocated now as well: the first asynchronous call may be under capture, where
     // nothing may be allocated)
     e->comm_counter = take_counter(device);

@@ -159,10 +159,12 @@ int dpep_layout_dispatch_small(void* ws, const int64_t* topk_idx, const void* x,
 /* One fresh dispatch as ElasticBuffer makes it (notify + dispatch, deep_ep/backends/mesh_clos/elastic.py:648-1008): the layout
  * and, queued behind it before the host knows R, the payload; for a small batch both in one launch (see above).  The
  * payload outputs hold capacity_rows rows, of which the first min(R, capacity_rows) are written: a caller that finds
- * R > capacity_rows allocates R rows and calls dpep_dispatch_copy / dpep_dispatch_quant_fp8 with the same maps.  One that always
- * does so sets report_to_host to DPEP_REPORT_ALL_OR_NONE: if R > capacity_rows the outputs are then left as they are (a small
- * batch may write part of them), and the launch ends at once. */
+ * R > capacity_rows allocates R rows and calls dpep_dispatch_copy / dpep_dispatch_quant_fp8 with the same maps.  One that does
+ * so whenever DPEP_ROWS_KEPT says that the outputs are too small, or mostly unused, sets report_to_host to
+ * DPEP_REPORT_ALL_OR_NONE: the outputs are then left as they are in these cases (a small batch may write part of them), and the
+ * launch ends at once. */
 #define DPEP_REPORT_ALL_OR_NONE 2
+#define DPEP_ROWS_KEPT(rows, capacity) ((rows) <= (capacity) && (capacity) - (rows) <= (rows) / 2 + 1024)
 typedef struct dpep_fresh_dispatch {
     const int64_t* topk_idx;    /* [T,K] */
     int64_t* topk_idx_copy;     /* [T,K] receives a copy of topk_idx (the handle's own), or NULL */

@@ -453,11 +453,13 @@ class _FreshDispatch(ctypes.Structure):
             "report_to_host")]
 
 
-@pytest.mark.parametrize("report,short_by", [(2, 0), (2, 1), (2, 3000), (1, 1), (1, 3000)])
+@pytest.mark.parametrize("report,short_by", [(2, 0), (2, 1), (2, 3000), (2, -2000), (2, "most unused"), (2, "just kept"), (1, 1), (1, 3000),
+                                             (1, -5000)])
 @pytest.mark.parametrize("quantize", [False, True])
 @pytest.mark.parametrize("tokens,topk,experts,local", [(1000, 8, 32, 8), (4001, 1, 16, 4)])  # token-major and row-major payloads
 def test_fresh_dispatch_into_outputs_that_are_too_small(tokens, topk, experts, local, quantize, report, short_by):
-    """dpep_dispatch_fresh with capacities around the number of rows: all rows, the first ones, or (all or none) nothing."""
+    """dpep_dispatch_fresh with capacities around the number of rows: all rows, the first ones, or (all or none: outputs too
+    small or mostly unused) nothing."""
     from deepep_amd import _lib, ops
 
     hidden, begin = 256, local
@@ -466,17 +468,20 @@ def test_fresh_dispatch_into_outputs_that_are_too_small(tokens, topk, experts, l
     ids = np.stack([rng.choice(experts, topk, replace=False, p=popularity / popularity.sum()) for _ in range(tokens)]).astype(np.int64)
     want = olayout.layout(ids, experts, begin, local)
     rows = want["num_rows"]
+    if isinstance(short_by, str):
+        short_by = -(rows // 2 + 1024 + (short_by == "most unused"))
     capacity = max(rows - short_by, 0)
-    moved = rows if short_by == 0 else capacity if report == 1 else 0
+    moved = min(capacity, rows) if report == 1 or capacity >= rows and capacity - rows <= rows // 2 + 1024 else 0
     x, w = _batch(tokens, hidden, topk, 9)
     device = dict(device="cuda")
     idx, xd, wd = torch.from_numpy(ids).cuda(), x.cuda(), w.cuda()
     meta = torch.zeros(3 * local + 2, dtype=torch.int32, **device)
     forward = torch.zeros(tokens * topk, dtype=torch.int32, **device)
     back = torch.zeros(tokens * topk, dtype=torch.int32, **device)
-    out = torch.full((rows, hidden * (1 if quantize else 2)), 0x55, dtype=torch.uint8, **device)
-    scales = torch.full((rows, hidden // 128), 5.0, **device) if quantize else None
-    weights = torch.full((rows,), 5.0, **device)
+    size = max(rows, capacity)
+    out = torch.full((size, hidden * (1 if quantize else 2)), 0x55, dtype=torch.uint8, **device)
+    scales = torch.full((size, hidden // 128), 5.0, **device) if quantize else None
+    weights = torch.full((size,), 5.0, **device)
     call = _FreshDispatch(
         idx.data_ptr(), None, xd.data_ptr(), None, wd.data_ptr(), meta.data_ptr(), meta[local:].data_ptr(), meta[2 * local :].data_ptr(),
         forward.data_ptr(), back.data_ptr(), meta[3 * local + 1 :].data_ptr(), None, out.data_ptr(),
@@ -501,6 +506,30 @@ def test_fresh_dispatch_into_outputs_that_are_too_small(tokens, topk, experts, l
     np.testing.assert_array_equal(out[:moved].cpu().numpy(), olayout.expand_rows(payload, want["row_to_route"], topk)[:moved])
     np.testing.assert_array_equal(f32_bits(weights[:moved]), olayout.expand_weights(w.numpy(), want["row_to_route"]).view(np.uint32)[:moved])
     assert bool((out[moved:] == 0x55).all()) and bool((weights[moved:] == 5.0).all())
+
+
+@pytest.mark.parametrize("world,tokens", [(8, 6000), (8, 240), (2, 3000)])
+def test_storage_of_a_share_stays_close_to_its_rows(world, tokens):
+    """Batches whose share jumps up and down: what a received tensor keeps alive follows its own number of rows."""
+    experts, topk, hidden, local = world * 8, 4, 512, 8
+    rng = np.random.default_rng(12)
+    x, w = _batch(tokens, hidden, topk, 12)
+    xd, wd = x.cuda(), w.cuda()
+    buffer = _buffer(num_bytes=4 << 20, rank=0, world_size=world)
+    try:
+        for step, share in enumerate((1.0, 1.0, 0.02, 0.02, 10.0, 0.0, 0.5, 1.0, 300.0, 0.3)):
+            popularity = np.where(np.arange(experts) < local, share + 1e-12, 1.0)
+            ids = np.stack([rng.choice(experts, topk, replace=False, p=popularity / popularity.sum()) for _ in range(tokens)]).astype(np.int64)
+            want = olayout.layout(ids, experts, 0, local)
+            rows = want["num_rows"]
+            recv, _, recv_w, handle, _ = buffer.dispatch(xd, topk_idx=torch.from_numpy(ids).cuda(), topk_weights=wd, num_experts=experts)
+            kept = recv.untyped_storage().nbytes() / (hidden * 2)
+            assert handle.num_expanded_tokens == rows == recv.shape[0] == recv_w.shape[0]
+            assert kept <= (tokens * topk if world == 2 else rows * 1.5 + 1024 if tokens * topk > 2048 else 2048), (step, rows, kept)
+            np.testing.assert_array_equal(bf16_bits(recv), olayout.expand_rows(bf16_bits(x), want["row_to_route"], topk))
+            np.testing.assert_array_equal(f32_bits(recv_w), olayout.expand_weights(w.numpy(), want["row_to_route"]).view(np.uint32))
+    finally:
+        buffer.destroy()
 
 
 def test_outputs_that_a_share_outgrows_are_given_back_first():
