@@ -33,7 +33,6 @@ constexpr int kMaxTokens = 16384, kMaxHidden = 7168, kMaxTopk = 16, kMaxExperts 
 constexpr int kLowLatencyMaxTokens = 256;
 constexpr long long kWaitTimeoutUs = 100LL * 1000 * 1000;
 constexpr int64_t kSmallBlock = 64 << 10;
-constexpr int kSpinsWithGil = 4096;  // about 100 us of polling before other Python threads get their turn
 
 // ---- small helpers ---------------------------------------------------------------------------------------------------
 struct Ref {  // an owned reference
@@ -766,7 +765,6 @@ PyObject* run_fresh(Exchange* e, const FreshCall& c, const Target& t, PyObject* 
     if (!c.low_latency) {
         // ---- the one host synchronisation -------------------------------------------------------------------------------
         int32_t counts[DPEP_MAX_LOCAL_EXPERTS], reported = 0;
-        for (int spin = 0; spin < kSpinsWithGil && !dpep_layout_ready(e->workspace); ++spin) __builtin_ia32_pause();
         int status;
         if (dpep_layout_ready(e->workspace)) {
             status = dpep_layout_wait(e->workspace, counts, static_cast<int>(local), &reported, kWaitTimeoutUs);

@@ -3,6 +3,7 @@ and outgrown by it, row-major payloads that walk past their grid, the routing co
 handles that leave the native path, and memory that is handed out again behind asynchronous calls."""
 
 import ctypes
+import threading
 
 import numpy as np
 import pytest
@@ -529,6 +530,36 @@ def test_storage_of_a_share_stays_close_to_its_rows(world, tokens):
             np.testing.assert_array_equal(bf16_bits(recv), olayout.expand_rows(bf16_bits(x), want["row_to_route"], topk))
             np.testing.assert_array_equal(f32_bits(recv_w), olayout.expand_weights(w.numpy(), want["row_to_route"]).view(np.uint32))
     finally:
+        buffer.destroy()
+
+
+def test_other_python_threads_run_while_a_dispatch_waits_for_its_row_count():
+    """A wait as short as a busy stream's few ten microseconds is made without the GIL too."""
+    x, _ = _batch(64, 256, 2, 3)
+    idx = torch.stack([torch.randperm(8)[:2] for _ in range(64)]).cuda()
+    xd = x.cuda()
+    buffer = _buffer(num_bytes=4 << 20)
+    turns, stop = [0], threading.Event()
+
+    def other():
+        while not stop.is_set():
+            turns[0] += 1
+
+    thread = threading.Thread(target=other)
+    try:
+        buffer.dispatch(xd, topk_idx=idx, num_experts=8)
+        thread.start()
+        let_in = 0
+        for _ in range(20):
+            torch.cuda.synchronize()
+            torch.cuda._sleep(40_000)  # about 20 us
+            before = turns[0]
+            buffer.dispatch(xd, topk_idx=idx, num_experts=8)
+            let_in += turns[0] > before
+        assert let_in >= 15
+    finally:
+        stop.set()
+        thread.join(timeout=60)
         buffer.destroy()
 
 
