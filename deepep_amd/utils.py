@@ -15,7 +15,7 @@ def per_token_cast_to_fp8(x: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]:
     Bit-identical to the reference's torch expression on CPU.  ``x`` is a BF16 [T, H] GPU tensor of any width: a last
     block shorter than 128 is quantised as if padded with zeros, as in the reference (the kernel takes widths that
     are multiples of 16; other widths are padded to the next one here and the codes cut back to H)."""
-    done = _lib.host().cast_to_fp8(x)  # the ordinary call, made natively
+    done = _lib.host().cast_to_fp8(x) if x.is_cuda else None  # the ordinary call, made natively
     if done is not None:
         return done
     if x.dim() != 2:
@@ -31,7 +31,7 @@ def per_token_cast_back(x_fp8: torch.Tensor, x_scales: torch.Tensor) -> torch.Te
     """bf16(fp32(q) * scale) per block of 128 columns (deep_ep/utils/math.py:64-79); an int32 scale holds the e8m0
     exponent bytes of four consecutive blocks.  Device tensors go through the HIP kernel (``dpep_cast_back``); host
     tensors are evaluated with torch, as the reference does on any device."""
-    done = _lib.host().cast_back(x_fp8, x_scales)  # the ordinary call, made natively
+    done = _lib.host().cast_back(x_fp8, x_scales) if x_fp8.is_cuda else None  # the ordinary call, made natively
     if done is not None:
         return done
     if x_fp8.numel() == 0:
