@@ -29,8 +29,8 @@
 
 namespace {
 
-constexpr int kMaxTokens = 16384, kMaxHidden = 7168, kMaxTopk = 16, kMaxExperts = 1024;
-constexpr int kLowLatencyMaxTokens = 256;
+// Bounds of the arguments, given by the Python layer, which has them for its own checks (configure).
+int g_max_tokens, g_max_hidden, g_max_topk, g_max_experts, g_low_latency_max_tokens;
 constexpr long long kWaitTimeoutUs = 100LL * 1000 * 1000;
 constexpr int64_t kSmallBlock = 64 << 10;
 
@@ -347,7 +347,6 @@ struct Plan {
     const int32_t* route_to_row;
     const int32_t* row_to_route;
     PyObject* owner;                // owned: the buffer's token
-    Stream home;                    // stream the routing storage was allocated on
     long long rows;                 // rows of the payload outputs (low latency: the capacity)
     int tokens, topk, hidden, experts;
     bool low_latency;
@@ -722,7 +721,6 @@ PyObject* run_fresh(Exchange* e, const FreshCall& c, const Target& t, PyObject* 
     plan->route_to_row = call.route_to_row;
     plan->row_to_route = call.row_to_route;
     plan->owner = new_ref(e->token);
-    plan->home = t.caller;
     plan->tokens = call.num_tokens;
     plan->topk = call.num_topk;
     plan->hidden = static_cast<int>(width);
@@ -908,8 +906,8 @@ PyObject* Exchange_dispatch(PyObject* self, PyObject* const* a, Py_ssize_t n)
     }
     const long long per_rank = (in.tokens + e->world - 1) / e->world;
     long long capacity = e->bound != 0 ? e->bound : per_rank;
-    if (max_tokens != Py_None && (capacity = exact_int(max_tokens, 0, kMaxTokens)) < 0) Py_RETURN_NONE;
-    if (capacity < per_rank || capacity > kMaxTokens || (e->bound != 0 && capacity > e->bound)) Py_RETURN_NONE;
+    if (max_tokens != Py_None && (capacity = exact_int(max_tokens, 0, g_max_tokens)) < 0) Py_RETURN_NONE;
+    if (capacity < per_rank || capacity > g_max_tokens || (e->bound != 0 && capacity > e->bound)) Py_RETURN_NONE;
     if (e->hidden != 0 && in.width != e->hidden) Py_RETURN_NONE;
 
     Plan* plan = nullptr;
@@ -924,7 +922,7 @@ PyObject* Exchange_dispatch(PyObject* self, PyObject* const* a, Py_ssize_t n)
         c.copy_idx = handle_copy == Py_True;
         if (!c.copy_idx && c.idx->is_inference()) Py_RETURN_NONE;
         c.topk = c.idx->size(1);
-        c.experts = exact_int(num_experts, e->world, kMaxExperts);
+        c.experts = exact_int(num_experts, e->world, g_max_experts);
         if (c.experts < 0 || c.experts % e->world != 0) Py_RETURN_NONE;
     } else {
         if (topk_idx != Py_None || (plan = intact_plan(handle, e->token, &dict)) == nullptr || plan->low_latency) Py_RETURN_NONE;
@@ -936,7 +934,7 @@ PyObject* Exchange_dispatch(PyObject* self, PyObject* const* a, Py_ssize_t n)
     if (c.topk < 1 || (e->topk != 0 && e->topk != c.topk) || (weights != nullptr && !has_shape(*weights, in.tokens, c.topk))) Py_RETURN_NONE;
 
     // Path selection as in ElasticBuffer._choose_low_latency: small batches of EP16-EP256 jobs with weights and default options.
-    if (handle == Py_None && e->world >= 16 && e->world <= 256 && capacity <= kLowLatencyMaxTokens && weights != nullptr && sms == 0 && qps == 0 &&
+    if (handle == Py_None && e->world >= 16 && e->world <= 256 && capacity <= g_low_latency_max_tokens && weights != nullptr && sms == 0 && qps == 0 &&
         previous == Py_None && asynchronous == Py_False && (type == at::kBFloat16 || type == at::kHalf || type == at::kFloat8_e4m3fn) &&
         !(e->fp8 && type != at::kFloat8_e4m3fn) && in.width * in.x->element_size() % 16 == 0 && c.topk <= DPEP_MAX_TOPK &&
         (type == at::kFloat8_e4m3fn
@@ -953,8 +951,8 @@ PyObject* Exchange_dispatch(PyObject* self, PyObject* const* a, Py_ssize_t n)
             Py_RETURN_NONE;
         c.quantize = e->fp8 && !in.tuple;
         const bool fp8 = c.quantize || in.tuple;
-        if (in.width > kMaxHidden || in.width % (fp8 ? 128 : 16) != 0 || (sms != 0 && sms != (fp8 ? 64 : 32)) || c.topk > kMaxTopk ||
-            in.tokens > static_cast<long long>(kMaxTokens) * e->world || (handle == Py_None && cpu_sync == Py_False))
+        if (in.width > g_max_hidden || in.width % (fp8 ? 128 : 16) != 0 || (sms != 0 && sms != (fp8 ? 64 : 32)) || c.topk > g_max_topk ||
+            in.tokens > static_cast<long long>(g_max_tokens) * e->world || (handle == Py_None && cpu_sync == Py_False))
             Py_RETURN_NONE;
     }
     Locked held(e->lock);
@@ -1358,11 +1356,13 @@ PyObject* configure_mega(PyObject*, PyObject* args)
     Py_RETURN_NONE;
 }
 
-// configure(EPHandle, template dict, EventOverlap, EventHandle, NativeError): the Python classes whose objects are made here.
+// configure(EPHandle, template dict, EventOverlap, EventHandle, NativeError, (most tokens, hidden, top-k, experts, low-latency
+// tokens)): the Python classes whose objects are made here, and the bounds.
 PyObject* configure(PyObject*, PyObject* args)
 {
     PyObject *handle, *form, *overlap, *event, *error;
-    if (!PyArg_ParseTuple(args, "O!O!O!O!O", &PyType_Type, &handle, &PyDict_Type, &form, &PyType_Type, &overlap, &PyType_Type, &event, &error))
+    if (!PyArg_ParseTuple(args, "O!O!O!O!O(iiiii)", &PyType_Type, &handle, &PyDict_Type, &form, &PyType_Type, &overlap, &PyType_Type, &event,
+                          &error, &g_max_tokens, &g_max_hidden, &g_max_topk, &g_max_experts, &g_low_latency_max_tokens))
         return nullptr;
     g_handle_type = reinterpret_cast<PyTypeObject*>(new_ref(handle));
     g_handle_template = PyDict_Copy(form);

@@ -90,7 +90,8 @@ def _load_host():
 
     host = _lib.host()
     form = EPHandle(True, 0, 1, 0, 0, None, None, 0, [], None, None, None, None, None, None, None)
-    host.configure(EPHandle, vars(form), EventOverlap, EventHandle, _lib.NativeError)
+    host.configure(EPHandle, vars(form), EventOverlap, EventHandle, _lib.NativeError,
+                   (MAX_TOKENS, MAX_HIDDEN, MAX_TOPK, MAX_EXPERTS, LOW_LATENCY_MAX_TOKENS))
     return host
 
 
