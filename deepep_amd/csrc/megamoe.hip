@@ -244,7 +244,8 @@ struct GemmParams {
     int fill_tokens, fill_vec, fill_topk;
     int* fill_state;
     int* fill_stop;
-    int forced_rt;                  // 1..3: tile height 64 * forced_rt whatever the cost model says (tests); 0: the model decides
+    int forced_rows;                // 64 / 128 / 192: that tile height whatever the cost model says (tests); 32: the few-rows kernel
+    int forced_waves;               //   with so many waves per workgroup (1, 4); 0: the model decides
     int column_waves;               // 1: the kernel whose waves split the tile's columns and load their weights straight into registers
 };
 
@@ -1688,10 +1689,14 @@ struct ExpectedRows {
 // 7168 x 2048, 24 rows each: first GEMM 27 us with 64-row tiles, 24 with four waves, 17.5 with one; 192 rows: 35, 23, 34; 16 of
 // 1024 x 512, 24 rows: 12.7, 7.7, 6.6).  Large ones it streams as well as the 64-row kernel up to about 20 rows, where a
 // tile of 32 still holds nearly all experts (64 of 7168 x 2048, 20 rows: 148 against 154 us; 28 rows: 168 against 159).
+struct GemmChoice {
+    int rows;      // row-tile height: 64, 128, 192; 32: the few-rows kernel
+    int waves;     // per workgroup (4 but for the few-rows kernel's small launches)
+    double tiles;  // expected, of that height
+};
 template <bool kGateUp>
-int launch_gemm(const GemmParams& p, const ExpectedRows& expected, hipStream_t stream, const char* what)
+GemmChoice choose_gemm(const GemmParams& p, const ExpectedRows& expected, int cus)
 {
-    const int cus = gemm_grid();
     const int n_tiles = p.n / kBN, ktiles = p.k / kBK;
     const int num_shared = p.num_local - p.num_routed;
     const double mean = expected.routed;
@@ -1729,34 +1734,81 @@ int launch_gemm(const GemmParams& p, const ExpectedRows& expected, hipStream_t s
     }
     // Source rows are addressed with 32 bits in the few-rows kernel.  A share with more than one 64-row tile per expert has so many
     // tokens without a row that its first GEMM's idle workgroups are better used for their zero rows.
-    if (p.column_waves && p.forced_rt == 0 && (p.fill_out == nullptr || mean <= 64.0) && (!kGateUp || static_cast<long long>(p.a_rows) * p.k < (1LL << 32))) {
-        const double tiles = expected_row_tiles(32) * n_tiles;
+    const double tiles = expected_row_tiles(32) * n_tiles;
+    if (p.column_waves && p.forced_rows == 0 && (p.fill_tokens == 0 || mean <= 64.0) && (!kGateUp || static_cast<long long>(p.a_rows) * p.k < (1LL << 32))) {
         const double one = bounded(3.0 + 0.30 * ktiles + (rounds_of(kGemmWaves * tiles, cus) - 1.0) * (1.1 + 0.17 * ktiles));
         const double four = bounded(1.5 + rounds_of(tiles, cus) * (2.7 + 0.50 * ktiles));
         // Zero rows of the output that this launch's idle workgroups would have written (at about 30 GB/s each): the few-rows
         // kernel leaves them to the reduce, which writes them at 8 TB/s, and the GEMM is faster without the company: 4300 zero
         // rows of 5120 columns beside 31 experts of 5120 x 512 cost the forward 57 us filled and 49 not.
         double unfilled = 0.0;
-        if (p.fill_out != nullptr && tiles_of[best] < cus) {
+        if (p.fill_tokens > 0 && tiles_of[best] < cus) {
             const double zeros = p.fill_tokens * exp(-mean * p.num_routed / p.fill_tokens) * p.fill_vec * 16.0;
             unfilled = std::min(zeros, (cus - tiles_of[best]) * 30e3 * best_cost) / 11e6;
         }
-        if (std::min(one, four) + unfilled < best_cost) {
-            // Workgroups for more rows than expected (those without a tile end at once, while one with two doubles the time).
-            const long long row_tiles = static_cast<long long>(p.num_routed) * static_cast<long long>(ceil(std::max(1.0, mean + 3.0 * expected.spread) / 32.0)) +
-                                        static_cast<long long>(num_shared) * ((expected.shared + 31) / 32);
-            const unsigned grid = static_cast<unsigned>(row_tiles * n_tiles);
-            if (one < four)
-                hipLaunchKernelGGL((grouped_gemm_few_rows_kernel<1, kGateUp>), dim3(kGemmWaves * grid), dim3(64), 0, stream, p);
-            else
-                hipLaunchKernelGGL((grouped_gemm_few_rows_kernel<kGemmWaves, kGateUp>), dim3(grid), dim3(kGemmThreads), 0, stream, p);
-            return launch_status(what);
-        }
+        if (std::min(one, four) + unfilled < best_cost) return {32, one < four ? 1 : kGemmWaves, tiles};
     }
-    if (p.forced_rt >= 1 && p.forced_rt <= 3) best = p.forced_rt;
-    if (best == 1) return launch_gemm_rt<1, kGateUp>(p, tiles_of[1], stream, what);
-    if (best == 2) return launch_gemm_rt<2, kGateUp>(p, tiles_of[2], stream, what);
-    return launch_gemm_rt<3, kGateUp>(p, tiles_of[3], stream, what);
+    if (p.forced_rows == 32) return {32, p.forced_waves, tiles};
+    if (p.forced_rows != 0) best = p.forced_rows / 64;
+    return {64 * best, kGemmWaves, tiles_of[best]};
+}
+
+template <bool kGateUp>
+int launch_gemm(const GemmParams& p, const ExpectedRows& expected, hipStream_t stream, const char* what)
+{
+    const GemmChoice choice = choose_gemm<kGateUp>(p, expected, gemm_grid());
+    if (choice.rows == 32) {
+        DPEP_REQUIRE(!kGateUp || static_cast<long long>(p.a_rows) * p.k < (1LL << 32), "%s: 32-row tiles address at most 4 GiB of input rows", what);
+        // Workgroups for more rows than expected (those without a tile end at once, while one with two doubles the time).
+        const int num_shared = p.num_local - p.num_routed;
+        const long long row_tiles =
+            static_cast<long long>(p.num_routed) * static_cast<long long>(ceil(std::max(1.0, expected.routed + 3.0 * expected.spread) / 32.0)) +
+            static_cast<long long>(num_shared) * ((expected.shared + 31) / 32);
+        const unsigned grid = static_cast<unsigned>(row_tiles * (p.n / kBN));
+        if (choice.waves == 1)
+            hipLaunchKernelGGL((grouped_gemm_few_rows_kernel<1, kGateUp>), dim3(kGemmWaves * grid), dim3(64), 0, stream, p);
+        else
+            hipLaunchKernelGGL((grouped_gemm_few_rows_kernel<kGemmWaves, kGateUp>), dim3(grid), dim3(kGemmThreads), 0, stream, p);
+        return launch_status(what);
+    }
+    if (choice.rows == 64) return launch_gemm_rt<1, kGateUp>(p, choice.tiles, stream, what);
+    if (choice.rows == 128) return launch_gemm_rt<2, kGateUp>(p, choice.tiles, stream, what);
+    return launch_gemm_rt<3, kGateUp>(p, choice.tiles, stream, what);
+}
+
+// The sizes of one of the two GEMMs of a forward, and the workspace's settings for it (ws == nullptr: the defaults).
+struct MegaSizes {
+    int num_tokens, hidden, intermediate, num_topk, num_experts, num_local, num_shared;
+};
+GemmParams gemm_of(const MegaSizes& m, const Workspace* w, bool second)
+{
+    const int hp = padded_dim(m.hidden), ip = padded_dim(m.intermediate);
+    GemmParams p{};
+    p.topk = second ? 1 : m.num_topk;
+    p.a_rows = second ? 0 : m.num_tokens;
+    p.num_local = m.num_local + m.num_shared;
+    p.num_routed = m.num_local;
+    p.n = second ? hp : 2 * ip;
+    p.k = second ? ip : hp;
+    p.forced_rows = w != nullptr ? w->gemm_tile_rows : 0;
+    p.forced_waves = w != nullptr ? w->gemm_few_rows_waves : 0;
+    p.column_waves = w != nullptr ? w->gemm_column_waves : 1;
+    // Without shared experts most tokens of a share have no row: workgroups of the first GEMM that get no tile
+    // zero those rows of y meanwhile, and the weighted reduce skips what they got through.  (Served-only: rows of y whose
+    // token no local expert serves are nobody's business, neither the fillers' nor the reduce's; with shared experts every
+    // token is served.)
+    if (!second && m.num_shared == 0 && (w == nullptr || (w->gemm_zero_fill && !w->megamoe_served_only))) {
+        p.fill_tokens = m.num_tokens;
+        p.fill_vec = m.hidden / 8;
+        p.fill_topk = m.num_topk;
+    }
+    return p;
+}
+// Expected rows (the true counts stay on the device): tokens * topk / experts per routed expert, every token for a shared one.
+ExpectedRows expected_rows_of(const MegaSizes& m)
+{
+    const double routed = static_cast<double>(m.num_tokens) * m.num_topk / m.num_experts;
+    return {routed, sqrt(routed * std::max(0.0, 1.0 - static_cast<double>(m.num_topk) / m.num_experts)) + 1e-3, m.num_tokens};
 }
 
 }  // namespace
@@ -2095,6 +2147,23 @@ size_t dpep_megamoe_workspace_bytes(int num_tokens, int num_topk, int hidden, in
     return mega_layout(num_tokens, num_topk, hidden, intermediate, num_local, num_shared).total;
 }
 
+int dpep_megamoe_gemm_choice(void* ws, int num_tokens, int hidden, int intermediate, int num_topk, int num_experts, int num_local,
+                             int num_shared, int second, int32_t* tile_rows, int32_t* waves)
+{
+    using namespace dpep;
+    const Workspace* w = as_workspace(ws);
+    DPEP_REQUIRE(ws == nullptr || w != nullptr, "megamoe_gemm_choice: not a live workspace");
+    DPEP_REQUIRE(tile_rows != nullptr && waves != nullptr, "megamoe_gemm_choice: NULL output");
+    DPEP_REQUIRE(num_tokens >= 1 && hidden >= 1 && intermediate >= 1 && num_topk >= 1 && num_experts >= num_local && num_local >= 1 && num_shared >= 0,
+                 "megamoe_gemm_choice: bad sizes");
+    const MegaSizes sizes = {num_tokens, hidden, intermediate, num_topk, num_experts, num_local, num_shared};
+    const GemmParams p = gemm_of(sizes, w, second != 0);
+    const GemmChoice choice = second != 0 ? choose_gemm<false>(p, expected_rows_of(sizes), gemm_grid()) : choose_gemm<true>(p, expected_rows_of(sizes), gemm_grid());
+    *tile_rows = choice.rows;
+    *waves = choice.waves;
+    return DPEP_OK;
+}
+
 int dpep_megamoe_fill_report(void* ws, int num_tokens, int num_topk, int hidden, int intermediate, int num_local,
                              int num_shared, int32_t* fillers_host, int64_t* tokens_filled_host, void* stream)
 {
@@ -2206,67 +2275,43 @@ int dpep_megamoe_run(void* ws, const dpep_megamoe_call* call, void* stream)
     if (int rc = layout_i32(ws, topk_idx, num_tokens, num_topk, num_experts, expert_begin, num_local, expert_token_nums,
                             psum, offsets, route_to_row, row_to_route, num_rows, front, s))
         return rc;
-    GemmParams g1{};
+    const MegaSizes sizes = {num_tokens, hidden, intermediate, num_topk, num_experts, num_local, num_shared};
+    GemmParams g1 = gemm_of(sizes, w, false);
     g1.a_codes = codes;
     g1.a_scales = scales;
     g1.row_to_route = row_to_route;
-    g1.topk = num_topk;
-    g1.a_rows = num_tokens;
     g1.offsets = offsets;
-    g1.num_local = num_local + num_shared;
-    g1.num_routed = num_local;
     g1.w = w1;
     g1.ws = s1;
     g1.w_shared = shared_w1;
     g1.ws_shared = shared_s1;
-    g1.n = 2 * ip;
-    g1.k = hp;
     g1.act_codes = base + l.act_codes;
     g1.act_scales = base + l.act_scales;
-    // Expected rows (the true counts stay on the device): tokens * topk / experts per routed expert, every
-    // token for a shared one.
     const long long expected_routed = static_cast<long long>(num_tokens) * num_topk * num_local / num_experts;
     const long long expected_rows = expected_routed + static_cast<long long>(num_tokens) * num_shared;
-    const double routed = static_cast<double>(num_tokens) * num_topk / num_experts;
-    const ExpectedRows expected = {routed, sqrt(routed * std::max(0.0, 1.0 - static_cast<double>(num_topk) / num_experts)) + 1e-3, num_tokens};
-    // Without shared experts most tokens of a share have no row: workgroups of the first GEMM that get no tile
-    // zero those rows of y meanwhile, and the weighted reduce skips what they got through.
+    const ExpectedRows expected = expected_rows_of(sizes);
     int* fill_state = reinterpret_cast<int*>(base + l.fill_state);
     int* fill_stop = reinterpret_cast<int*>(static_cast<char*>(w->sync) + kSyncFillStop);
-    g1.forced_rt = w->gemm_tile_rows / 64;
-    g1.column_waves = w->gemm_column_waves;
-    // (served-only: rows of y whose token no local expert serves are nobody's business, neither the fillers' nor the
-    // reduce's; with shared experts every token is served)
     const bool served_only = num_shared == 0 && w->megamoe_served_only;
-    const bool fill = num_shared == 0 && w->gemm_zero_fill && !served_only;
+    const bool fill = g1.fill_tokens > 0;
     if (fill) {
         g1.fill_out = static_cast<u32x4*>(y);
         g1.fill_route_to_row = route_to_row;
-        g1.fill_tokens = num_tokens;
-        g1.fill_vec = hidden / 8;
-        g1.fill_topk = num_topk;
         g1.fill_stop = fill_stop;
     }
     g1.fill_state = fill_state;  // written even when nothing fills (then as "no fillers")
     if (int rc = launch_gemm1(g1, expected, s)) return rc;
-    GemmParams g2{};
+    GemmParams g2 = gemm_of(sizes, w, true);
     g2.a_codes = base + l.act_codes;
     g2.a_scales = base + l.act_scales;
     g2.row_to_route = nullptr;
-    g2.topk = 1;
     g2.offsets = offsets;
-    g2.num_local = num_local + num_shared;
-    g2.num_routed = num_local;
     g2.w = w2;
     g2.ws = s2;
     g2.w_shared = shared_w2;
     g2.ws_shared = shared_s2;
-    g2.n = hp;
-    g2.k = ip;
     g2.out = reinterpret_cast<uint16_t*>(base + l.out2);
     g2.out_cols = hidden;
-    g2.forced_rt = g1.forced_rt;
-    g2.column_waves = g1.column_waves;
     if (int rc = launch_gemm2(g2, expected, s)) return rc;
     return combine_routes(base + l.out2, topk_weights, route_to_row, num_tokens, num_topk,
                           static_cast<int>(expected_rows),

@@ -89,6 +89,7 @@ int dpep_workspace_create(size_t bytes, void** ws)
     w->exchange_extra_rows = 0;
     w->layout_one_launch = 1;
     w->gemm_tile_rows = 0;
+    w->gemm_few_rows_waves = 4;
     w->gemm_column_waves = 1;
     w->gemm_zero_fill = 1;
     w->megamoe_served_only = 0;
@@ -191,9 +192,12 @@ int dpep_workspace_tune(void* ws, const char* key, long long value)
     } else if (strcmp(key, "gemm_column_waves") == 0) {
         w->gemm_column_waves = value != 0;
     } else if (strcmp(key, "gemm_tile_rows") == 0) {
-        DPEP_REQUIRE(value == 0 || value == 64 || value == 128 || value == 192,
-                     "workspace_tune: gemm_tile_rows is 0 (automatic), 64, 128 or 192");
+        DPEP_REQUIRE(value == 0 || value == 32 || value == 64 || value == 128 || value == 192,
+                     "workspace_tune: gemm_tile_rows is 0 (automatic), 32, 64, 128 or 192");
         w->gemm_tile_rows = static_cast<int>(value);
+    } else if (strcmp(key, "gemm_few_rows_waves") == 0) {
+        DPEP_REQUIRE(value == 1 || value == 4, "workspace_tune: gemm_few_rows_waves is 1 or 4");
+        w->gemm_few_rows_waves = static_cast<int>(value);
     } else {
         return dpep::fail(DPEP_EINVAL, "workspace_tune: unknown key '%s'", key);
     }

@@ -453,6 +453,20 @@ def megamoe_prepare_weights(w_packed, w_scales, gate_up: bool):
     return out_w, out_s
 
 
+def megamoe_gemm_choice(num_tokens: int, hidden: int, intermediate: int, num_topk: int, num_experts: int, num_local: int,
+                        num_shared: int = 0, ws: Optional[Workspace] = None):
+    """``((tile rows, waves per workgroup) of the first GEMM, the same of the second)`` that a forward of these sizes takes;
+    32 rows: the kernel for few rows per expert.  Host arithmetic only."""
+    chosen = []
+    for second in (0, 1):
+        rows, waves = ctypes.c_int32(), ctypes.c_int32()
+        status = _lib.load().dpep_megamoe_gemm_choice(None if ws is None else ws.handle, num_tokens, hidden, intermediate, num_topk, num_experts,
+                                                      num_local, num_shared, second, ctypes.byref(rows), ctypes.byref(waves))
+        _lib.check(status, "megamoe_gemm_choice")
+        chosen.append((rows.value, waves.value))
+    return tuple(chosen)
+
+
 def megamoe_fill_report(ws, num_tokens, num_topk, hidden, intermediate, num_local, num_shared: int = 0):
     """(filler waves, tokens they looked at) of the most recent forward on ``ws``; waits for the current stream."""
     fillers, filled = ctypes.c_int32(0), ctypes.c_int64(0)

@@ -51,7 +51,11 @@ int dpep_workspace_capacity(void* ws, size_t* bytes);
  *                                   untouched (one rank's share of an EP job, where other ranks produce those rows);
  *                                   0 (default): they are zeroed
  *   "gemm_tile_rows"                0 (default): dpep_megamoe_forward chooses the row-tile height of its grouped GEMMs
- *                                   from the expected rows per expert; 64, 128 or 192: that height for both */
+ *                                   from the expected rows per expert; 64, 128 or 192: that height for both, 32: the
+ *                                   kernel for few rows per expert for both
+ *   "gemm_few_rows_waves"           its waves per workgroup when forced: 4 (default) or 1
+ *   "gemm_column_waves"             1 (default): the GEMM whose waves split a tile's columns, where it takes the sizes;
+ *                                   0: always the 2 x 2 form */
 int dpep_workspace_tune(void* ws, const char* key, long long value);
 /* Scratch bytes dpep_layout needs for T*K routes and L local experts
  * (notify_layout() workspace_bytes, csrc/ops/notify.cpp:98-110). */
@@ -255,6 +259,12 @@ int dpep_megamoe_schedule_check(int tile_rows, int tiles_per_workgroup, int ktil
  * weights straight into registers; k tiles come in fours).  slack = operations the replayed wait allows in flight beyond
  * the kernel's own count: with slack > 0 the check has to fail, which is how the tests know that it can. */
 int dpep_megamoe_schedule_check_column_waves(int tile_rows, int tiles_per_workgroup, int ktiles, int epilogue_stores, int slack);
+
+/* Which grouped GEMM kernel a forward of these sizes takes on this workspace (NULL: one with default settings), for the
+ * first or (second != 0) the second GEMM: its row-tile height (64, 128, 192, or 32 for the kernel for few rows per expert)
+ * and its waves per workgroup.  Host arithmetic only; no counterpart in the reference. */
+int dpep_megamoe_gemm_choice(void* ws, int num_tokens, int hidden, int intermediate, int num_topk, int num_experts, int num_local,
+                             int num_shared, int second, int32_t* tile_rows, int32_t* waves);
 
 /* Bytes of workspace dpep_megamoe_forward needs (buffer_size(), experiments/megamoe/csrc/forward.cpp:480).
  * num_shared = number of shared experts (0..8) whose rows (every token, each) are held next to the routed ones. */

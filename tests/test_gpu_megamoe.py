@@ -88,7 +88,7 @@ def _oracle(x_codes, x_scales, l1, l2, idx, weights, begin):
     return mm.round_bf16(mm.local_reference(xq, idx, weights, d1, d2, begin))
 
 
-def _run(ops, x_codes, x_scales, l1, l2, idx, weights, experts, begin, local, tile_rows=0, column_waves=1):
+def _run(ops, x_codes, x_scales, l1, l2, idx, weights, experts, begin, local, tile_rows=0, column_waves=1, few_rows_waves=4):
     tokens, hidden = x_codes.shape
     inter = l2[0].shape[2] * 2
     dev = "cuda"
@@ -97,6 +97,11 @@ def _run(ops, x_codes, x_scales, l1, l2, idx, weights, experts, begin, local, ti
     ws = ops.Workspace(ops.megamoe_workspace_bytes(tokens, idx.shape[1], hidden, inter, local))
     ws.tune("gemm_tile_rows", tile_rows)
     ws.tune("gemm_column_waves", column_waves)
+    ws.tune("gemm_few_rows_waves", few_rows_waves)
+    if tile_rows:
+        sizes = (tokens, hidden, inter, idx.shape[1], experts, local)
+        taken = (tile_rows, few_rows_waves if tile_rows == 32 else 4)
+        assert ops.megamoe_gemm_choice(*sizes, ws=ws) == (taken, taken)
     y = torch.full((tokens, hidden), float("nan"), dtype=torch.bfloat16, device=dev)
     counts = torch.empty((local,), dtype=torch.int32, device=dev)
     ops.megamoe_forward(
@@ -212,12 +217,12 @@ def test_both_grouped_gemm_kernels_agree_bit_for_bit(ops, tokens, hidden, inter,
     (1024, 256, 3, [33, 1, 0]),              # a wave per workgroup; k = 1024 and 512
     (1088, 384, 6, [0, 31, 32, 0, 64, 5]),   # k = 1280 ends in half a span of scales
     (1280, 1536, 6, [7, 40, 1, 0, 32, 2]),   # three whole spans
-    (1088, 384, 40, [1, 0, 32, 33, 2] * 8),  # four waves per workgroup
+    (1088, 384, 40, [1, 0, 32, 33, 2] * 8),  # more column tiles than CUs
     (512, 640, 70, [0, 3, 7] + [0] * 60 + [1, 0, 97, 32, 2, 0, 4]),  # more experts than a wave has lanes, one far over the mean
 ])
 def test_few_rows_per_expert(ops, hidden, inter, local, rows):
-    """Expected rows per expert below a row tile, actual ones from none to several tiles: against the oracle, and bit for bit
-    against the kernel with 64-row tiles."""
+    """Expected rows per expert below a row tile, actual ones from none to several tiles: against the oracle, and with one and
+    with four waves per workgroup bit for bit against the kernel with 64-row tiles."""
     begin, experts, remote = 2, 16 * local, 40
     tokens = sum(rows) + remote
     x_codes, x_scales, l1, l2, idx, weights = _make_problem(tokens, hidden, inter, experts, begin, local, 1, seed=local)
@@ -228,8 +233,12 @@ def test_few_rows_per_expert(ops, hidden, inter, local, rows):
     np.testing.assert_array_equal(counts, rows)
     ref = _oracle(x_codes, x_scales, l1, l2, idx, weights, begin)
     assert np.linalg.norm(y - ref) <= 2e-2 * np.linalg.norm(ref)
+    assert all(height == 32 for height, _ in ops.megamoe_gemm_choice(tokens, hidden, inter, 1, experts, local))
     tall, _ = _run(ops, x_codes, x_scales, l1, l2, idx, weights, experts, begin, local, tile_rows=64)
     np.testing.assert_array_equal(y, tall)
+    for waves in (1, 4):
+        few, _ = _run(ops, x_codes, x_scales, l1, l2, idx, weights, experts, begin, local, tile_rows=32, few_rows_waves=waves)
+        np.testing.assert_array_equal(few, tall)
 
 
 @pytest.mark.parametrize("hidden,inter,rows", [
@@ -240,7 +249,8 @@ def test_few_rows_per_expert(ops, hidden, inter, local, rows):
 ])
 def test_small_launches_take_the_few_rows_kernel(ops, hidden, inter, rows):
     """All experts here and the routing uneven: more row tiles than workgroups were launched for, and fewer.  Against the oracle,
-    and bit for bit against the kernel with 64-row tiles."""
+    and bit for bit against the kernel with 64-row tiles, as chosen (at least the second GEMM) and forced with one and with
+    four waves per workgroup."""
     experts = len(rows)
     x_codes, x_scales, l1, l2, idx, weights = _make_problem(sum(rows), hidden, inter, experts, 0, experts, 1, seed=experts)
     idx[:, 0] = np.random.default_rng(experts).permutation(np.repeat(np.arange(experts), rows)).astype(np.int32)
@@ -248,8 +258,12 @@ def test_small_launches_take_the_few_rows_kernel(ops, hidden, inter, rows):
     np.testing.assert_array_equal(counts, rows)
     ref = _oracle(x_codes, x_scales, l1, l2, idx, weights, 0)
     assert np.linalg.norm(y - ref) <= 2e-2 * np.linalg.norm(ref)
+    assert ops.megamoe_gemm_choice(sum(rows), hidden, inter, 1, experts, experts)[1][0] == 32
     tall, _ = _run(ops, x_codes, x_scales, l1, l2, idx, weights, experts, 0, experts, tile_rows=64)
     np.testing.assert_array_equal(y, tall)
+    for waves in (1, 4):
+        few, _ = _run(ops, x_codes, x_scales, l1, l2, idx, weights, experts, 0, experts, tile_rows=32, few_rows_waves=waves)
+        np.testing.assert_array_equal(few, tall)
 
 
 @pytest.mark.parametrize("tokens,hidden,inter,tile_rows", [

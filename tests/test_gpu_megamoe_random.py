@@ -208,7 +208,7 @@ def test_tile_heights_and_kernels_agree_at_large_random_shapes(ops, seed):
     """Sizes the oracle cannot follow (up to 16 384 tokens, hidden up to 8192, intermediate up to 4096, 32 local experts,
     masked routes in a third of the draws): a k sum is taken in the same order whatever the tile height and whichever
     grouped GEMM kernel runs, so the forward must give the same bits at 64, 128 and 192 rows, through the column-wave
-    kernel and the 2 x 2 kernel, and again on a second run; counts against a bincount, every served token written."""
+    kernel and the 2 x 2 kernel, through the few-rows kernel, and again on a second run; counts against a bincount, every served token written."""
     _agreement_case(ops, seed, *_draw_large(seed))
 
 
@@ -254,13 +254,15 @@ def _agreement_case(ops, seed, tokens, hidden, inter, experts, begin, local, top
     route_weights = torch.rand((tokens, topk), device=dev, generator=g, dtype=torch.float32)
     sentinel = 3.0
     first = None
-    for column_waves, tile_rows in [(1, 0), (1, 64), (1, 128), (1, 192), (0, 64), (0, 128), (0, 192), (1, 0)]:
+    for column_waves, tile_rows, few_rows_waves in [(1, 0, 4), (1, 64, 4), (1, 128, 4), (1, 192, 4), (0, 64, 4), (0, 128, 4), (0, 192, 4),
+                                                    (1, 32, 1), (1, 32, 4), (1, 0, 4)]:
         ws = ops.Workspace(ops.megamoe_workspace_bytes(tokens, topk, hidden, inter, local, shared))
         y = torch.full((tokens, hidden), sentinel, dtype=torch.bfloat16, device=dev)
         counts = torch.empty((local,), dtype=torch.int32, device=dev)
         try:
             ws.tune("gemm_tile_rows", tile_rows)
             ws.tune("gemm_column_waves", column_waves)
+            ws.tune("gemm_few_rows_waves", few_rows_waves)
             ws.tune("gemm_zero_fill", zero_fill)
             ws.tune("megamoe_served_only", served_only)
             ops.megamoe_forward(ws, x.view(torch.float8_e4m3fn), x_scales, idx, route_weights, w1, s1, w2, s2, experts, begin, local, y,
