@@ -345,7 +345,7 @@ def megamoe_bench(torch, ops, timer, with_cpu):
     weight_bytes = 32 * (2 * inter * hidden + hidden * inter) // 2
     result["decode_share"] = {
         "workload": "512 tokens x top-8, 32 of 256 experts local (about 16 rows per expert): the GEMMs are bound by streaming "
-        "their 705 MB of FP4 weights (64-row tiles, non-temporal weight copies); whole forward",
+        "their 705 MB of FP4 weights (the kernel for few rows per expert); whole forward",
         "rows": rows, "us_forward": us, "flushed_us": cold, "weight_bytes": weight_bytes,
         "weights_GBps_forward": weight_bytes / us / 1e3, "frac_of_8TBps": weight_bytes / us / 1e3 / HBM_PEAK_GBS,
     }
