@@ -779,6 +779,9 @@ PyObject* run_fresh(Exchange* e, const FreshCall& c, const Target& t, PyObject* 
             pending.replace(&out, {rows, width}, out_type);
             if (scales.defined()) pending.replace(&scales, {rows, scale_cols}, scale_type);
             if (weights.defined()) pending.replace(&weights, {rows}, at::kFloat);
+            // (the wait was made without the GIL: what another thread has queued on the caller's stream since may still work
+            // on the memory that these tensors got in that stream's order)
+            if (t.asynchronous && !(t.stream == t.caller) && !join_caller(e, t.caller)) return nullptr;
             float* s_out = scales.defined() ? static_cast<float*>(scales.data_ptr()) : nullptr;
             float* w_out = weights.defined() ? static_cast<float*>(weights.data_ptr()) : nullptr;
             status = c.quantize ? dpep_dispatch_quant_fp8(call.x, call.topk_weights, call.route_to_row, call.row_to_route, call.num_tokens,

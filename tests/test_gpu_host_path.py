@@ -4,6 +4,7 @@ handles that leave the native path, and memory that is handed out again behind a
 
 import ctypes
 import threading
+import time
 
 import numpy as np
 import pytest
@@ -244,6 +245,48 @@ def test_memory_of_an_outgrown_asynchronous_dispatch_is_not_handed_out_too_early
                 assert bool((block == 7.0).all())
             del recv, recv_w, handle, event, noise
         finally:
+            torch.cuda.synchronize()
+            buffer.destroy()
+
+
+def test_outputs_made_after_the_wait_are_free_of_other_threads_work():
+    """While an asynchronous dispatch waits for its row count, another thread uses the caller's stream: it fills memory of the size
+    that the outputs turn out to need, late, and lets it go.  The outputs may well get that memory; the payload comes behind."""
+    world, experts, topk, tokens, hidden = 4, 16, 4, 4096, 2048
+    x, _ = _batch(tokens, hidden, topk, 10)
+    ids = np.stack([np.random.default_rng(10).permutation(4)[:topk] for _ in range(tokens)]).astype(np.int64)
+    want = olayout.layout(ids, experts, 0, 4)
+    xd, idx = x.cuda(), torch.from_numpy(ids).cuda()
+    expected = xd[torch.from_numpy(want["row_to_route"]).cuda().long() // topk]
+    torch.empty((tokens * topk, hidden), dtype=torch.bfloat16, device="cuda")  # (so that the allocator has such a block)
+    for _ in range(3):
+        buffer = _buffer(num_bytes=4 << 20, rank=0, world_size=world)
+        ready, queued = threading.Event(), []
+
+        def other():
+            ready.wait(30)
+            time.sleep(0.005)
+            block = torch.empty((tokens * topk, hidden), dtype=torch.bfloat16, device="cuda")
+            torch.cuda._sleep(20_000_000)
+            block.fill_(7.0)
+            queued.append(time.perf_counter())
+
+        thread = threading.Thread(target=other)
+        try:
+            torch.cuda.synchronize()
+            thread.start()
+            torch.cuda._sleep(200_000_000)  # about 90 ms: the layout, behind the caller's stream, waits for it
+            ready.set()
+            recv, _, _, handle, event = buffer.dispatch(xd, topk_idx=idx, num_experts=experts, async_with_compute_stream=True)
+            returned = time.perf_counter()
+            event.current_stream_wait()
+            thread.join(timeout=60)
+            torch.cuda.synchronize()
+            assert handle.num_expanded_tokens == tokens * topk and queued and queued[0] < returned
+            assert torch.equal(recv, expected)
+            del recv, handle, event
+        finally:
+            thread.join(timeout=60)
             torch.cuda.synchronize()
             buffer.destroy()
 
