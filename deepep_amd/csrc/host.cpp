@@ -424,7 +424,7 @@ struct Exchange {
     bool fp8, combine_only, low_latency_workspace, failed, closed;
     PyObject* comm_object;  // the communication stream as torch's object; its raw stream is asked for by the first asynchronous
     Stream comm, last;      // call only (torch makes a pooled stream when its handle is first read, 0.25 ms)
-    bool has_comm, has_last;
+    bool has_comm, has_last, has_counters;
     double share;     // rows per route of the most recent fresh dispatch (negative: none yet), see capacity_for
     OrderEvent order;
     // asynchronous calls: the communication stream's counter, and the one that the callers' stream raises (one stream at a
@@ -491,6 +491,13 @@ bool choose_target(Exchange* e, bool asynchronous, PyObject* previous_event, Tar
     if (asynchronous && !e->has_comm) {
         if (!stream_from(e->comm_object, &e->comm)) return false;
         e->has_comm = true;
+    }
+    // By the first asynchronous call outside capture, where nothing may be allocated: under capture events do without them.
+    // (Not with the buffer: one that makes no such call would pay 70 us for them.)
+    if (asynchronous && !e->has_counters && !capturing(t->caller.raw)) {
+        e->has_counters = true;
+        e->comm_counter = take_counter(e->device);
+        e->caller_counter = e->comm_counter != nullptr ? take_counter(e->device) : nullptr;
     }
     t->stream = asynchronous ? e->comm : t->caller;
     if (asynchronous && !(e->comm == t->caller) && !join_caller(e, t->caller)) return false;
@@ -1051,13 +1058,9 @@ PyObject* Exchange_new(PyTypeObject* type, PyObject* args, PyObject*)
     e->fp8 = fp8;
     e->combine_only = combine_only;
     e->low_latency_workspace = low_latency;
-    e->failed = e->closed = e->has_comm = e->has_last = false;
+    e->failed = e->closed = e->has_comm = e->has_last = e->has_counters = false;
     e->comm_object = new_ref(comm);
     e->share = -1.0;
-    // (taken with the buffer, whose workspace is allocated now as well: the first asynchronous call may be under capture, where
-    // nothing may be allocated)
-    e->comm_counter = take_counter(device);
-    e->caller_counter = e->comm_counter != nullptr ? take_counter(device) : nullptr;
     return reinterpret_cast<PyObject*>(e);
     END_HANDLE_TH_ERRORS
 }

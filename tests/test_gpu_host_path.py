@@ -439,7 +439,7 @@ def test_asynchronous_calls_from_changing_streams_keep_their_order():
 def test_asynchronous_cached_calls_in_a_hip_graph(first_in_the_graph):
     """Under capture streams are ordered by events: a cached dispatch and a combine on the communication stream, captured once
     and replayed on new payloads, with the program's own work between the replays.  With and without an asynchronous call of
-    the buffer before the capture: what such calls need is there from the start, none of it is allocated under capture."""
+    the buffer before the capture: counters are not taken under capture, where nothing may be allocated, but by the first call after."""
     tokens, hidden, topk, experts = 96, 512, 3, 8
     gen = torch.Generator().manual_seed(4)
     idx = torch.stack([torch.randperm(experts, generator=gen)[:topk] for _ in range(tokens)]).cuda()
