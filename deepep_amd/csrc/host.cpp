@@ -493,7 +493,7 @@ bool choose_target(Exchange* e, bool asynchronous, PyObject* previous_event, Tar
         e->has_comm = true;
     }
     // By the first asynchronous call outside capture, where nothing may be allocated: under capture events do without them.
-    // (Not with the buffer: one that makes no such call would pay 70 us for them.)
+    // (A buffer that makes no such call takes none; two cost 2 us, the process's first allocation of the kind 39.)
     if (asynchronous && !e->has_counters && !capturing(t->caller.raw)) {
         e->has_counters = true;
         e->comm_counter = take_counter(e->device);
