@@ -778,11 +778,14 @@ int dpep_dispatch_fresh(void* ws, const dpep_fresh_dispatch* call, void* stream)
         if (c.capacity_rows == 0) return DPEP_OK;
         const Payload p = {c.x, c.scales, c.topk_weights, c.num_tokens, c.num_topk, units, c.quantize ? 0 : c.scale_cols,
                            c.quantize != 0, c.out, c.out_scales, c.out_weights};
-        // Expected rows of this rank's share.  Many rows per token: token-major, which reads every token once.  Otherwise
-        // row-major over the rows that the layout finds: a token-major grid is mostly workgroups of tokens without a row
-        // (6144 tokens of which 560 own a row: 10.5 us).
-        const long long expected = n_routes * c.num_local / c.num_experts;
+        // Expected rows of this rank's share: what the caller made its outputs for, or the even share.  Many rows per token:
+        // token-major, which reads every token once.  Otherwise row-major over the rows that the layout finds: a token-major
+        // grid is mostly workgroups of tokens without a row (6144 tokens of which 560 own a row: 10.5 us).  16 384 BF16
+        // tokens of 7168 columns, row-major / token-major: 0.5 rows per token 36.8 / 39.6 us, 1: 67.5 / 61.6, 1.5: 102 / 83, 4:
+        // 268 / 175; FP8 20.3 / 24.7, 35.4 / 35.0, 53.3 / 45.2, 138 / 90.
         const bool all_or_none = c.report_to_host == DPEP_REPORT_ALL_OR_NONE;
+        const long long expected =
+            all_or_none ? (c.capacity_rows > 256 ? (c.capacity_rows - 256LL) * 8 / 9 : 0) : n_routes * c.num_local / c.num_experts;
         if (expected > static_cast<long long>(kRowMajorRatio) * c.num_tokens)
             return launch_token_major(p, c.route_to_row, c.capacity_rows, all_or_none ? c.num_rows : nullptr, s);
         long long grid_rows = expected + expected / 8 + 64;

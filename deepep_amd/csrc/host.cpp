@@ -640,7 +640,8 @@ bool keep_same(Plan* plan, PyObject* dict, std::initializer_list<PyObject*> name
 long long capacity_for(const Exchange* e, long long routes, long long local, long long experts)
 {
     const double share = e->share >= 0.0 ? e->share : static_cast<double>(local) / static_cast<double>(experts);
-    return std::min(static_cast<long long>(share * 1.125 * static_cast<double>(routes)) + 256, routes);
+    const long long rows = static_cast<long long>(share * static_cast<double>(routes) + 0.5);
+    return std::min(DPEP_CAPACITY(rows), routes);
 }
 
 struct FreshCall {

@@ -166,8 +166,10 @@ int dpep_layout_dispatch_small(void* ws, const int64_t* topk_idx, const void* x,
  * R > capacity_rows allocates R rows and calls dpep_dispatch_copy / dpep_dispatch_quant_fp8 with the same maps.  One that does
  * so whenever DPEP_ROWS_KEPT says that the outputs are too small, or mostly unused, sets report_to_host to
  * DPEP_REPORT_ALL_OR_NONE: the outputs are then left as they are in these cases (a small batch may write part of them), and the
- * launch ends at once. */
+ * launch ends at once.  capacity_rows is then taken for DPEP_CAPACITY of the rows that the caller expects (with other values
+ * the even share of the routes is what is expected); the expectation decides how the work is split, never what is computed. */
 #define DPEP_REPORT_ALL_OR_NONE 2
+#define DPEP_CAPACITY(rows) ((rows) + (rows) / 8 + 256)
 #define DPEP_ROWS_KEPT(rows, capacity) ((rows) <= (capacity) && (capacity) - (rows) <= (rows) / 2 + 1024)
 typedef struct dpep_fresh_dispatch {
     const int64_t* topk_idx;    /* [T,K] */

@@ -561,7 +561,7 @@ def test_storage_of_a_share_stays_close_to_its_rows(world, tokens):
     xd, wd = x.cuda(), w.cuda()
     buffer = _buffer(num_bytes=4 << 20, rank=0, world_size=world)
     try:
-        for step, share in enumerate((1.0, 1.0, 0.02, 0.02, 10.0, 0.0, 0.5, 1.0, 300.0, 0.3)):
+        for step, share in enumerate((1.0, 1.0, 0.02, 0.02, 10.0, 10.0, 0.0, 0.5, 1.0, 300.0, 300.0, 0.3)):
             popularity = np.where(np.arange(experts) < local, share + 1e-12, 1.0)
             ids = np.stack([rng.choice(experts, topk, replace=False, p=popularity / popularity.sum()) for _ in range(tokens)]).astype(np.int64)
             want = olayout.layout(ids, experts, 0, local)
