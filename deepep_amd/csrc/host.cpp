@@ -19,6 +19,7 @@
 #include <ATen/core/Tensor.h>
 #include <ATen/hip/EmptyTensor.h>
 #include <c10/core/InferenceMode.h>
+#include <c10/core/StreamGuard.h>
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
 #include <hip/hip_runtime_api.h>
@@ -544,9 +545,8 @@ PyObject* event_of(Exchange* e, const Target& t, std::initializer_list<const at:
 
 // Answers for the tensors of a call from its first launch until the call has an event (event_of), whatever way the call ends.
 // On the communication stream a launch may still be pending when a tensor is let go, and memory that was allocated on the
-// caller's stream is handed out again in that stream's order alone: so it is declared to the allocator first, where an output
-// is replaced (replace) and where a launch, a wait or an allocation fails behind a launch.  In the latter case the buffer
-// takes no further calls either.
+// caller's stream is handed out again in that stream's order alone: so it is declared to the allocator first, where a launch, a
+// wait or an allocation fails behind a launch.  The buffer takes no further calls then either.
 struct Pending {
     Exchange* e;
     const Target& t;
@@ -560,13 +560,23 @@ struct Pending {
     }
     void declare(const at::Tensor& x) const
     {
-        if (x.defined() && t.asynchronous && !(t.stream == t.caller)) x.record_stream(t.stream.torch(e->device));
+        if (x.defined() && crosses()) x.record_stream(t.stream.torch(e->device));
     }
+    bool crosses() const { return t.asynchronous && !(t.stream == t.caller); }
+    // For an output that the queued launch leaves alone (DPEP_REPORT_ALL_OR_NONE): nothing to declare, its memory can be had again.
+    // The new one is allocated on the stream that writes it: the host has waited since without the GIL, and what another thread
+    // has queued on the caller's stream meanwhile may still work on memory that is free in that stream's order.  (The
+    // communication stream waiting for the caller's once more instead: 5 us more where shares jump from batch to batch.)
     void replace(at::Tensor* x, at::IntArrayRef sizes, at::ScalarType type) const
     {
-        declare(*x);
-        *x = at::Tensor();  // (first, so that its memory can be had again)
+        *x = at::Tensor();
+        if (!crosses()) {
+            *x = allocate(sizes, type, e->device);
+            return;
+        }
+        const c10::StreamGuard on_its_stream(t.stream.torch(e->device));
         *x = allocate(sizes, type, e->device);
+        x->record_stream(t.caller.torch(e->device));
     }
     ~Pending()
     {
@@ -768,6 +778,7 @@ PyObject* run_fresh(Exchange* e, const FreshCall& c, const Target& t, PyObject* 
     if (!ok || !handle) return nullptr;
 
     long long rows = capacity;
+    bool replaced = false;  // the outputs belong to the communication stream
     if (!c.low_latency) {
         // ---- the one host synchronisation -------------------------------------------------------------------------------
         int32_t counts[DPEP_MAX_LOCAL_EXPERTS], reported = 0;
@@ -787,9 +798,7 @@ PyObject* run_fresh(Exchange* e, const FreshCall& c, const Target& t, PyObject* 
             pending.replace(&out, {rows, width}, out_type);
             if (scales.defined()) pending.replace(&scales, {rows, scale_cols}, scale_type);
             if (weights.defined()) pending.replace(&weights, {rows}, at::kFloat);
-            // (the wait was made without the GIL: what another thread has queued on the caller's stream since may still work
-            // on the memory that these tensors got in that stream's order)
-            if (t.asynchronous && !(t.stream == t.caller) && !join_caller(e, t.caller)) return nullptr;
+            replaced = pending.crosses();
             float* s_out = scales.defined() ? static_cast<float*>(scales.data_ptr()) : nullptr;
             float* w_out = weights.defined() ? static_cast<float*>(weights.data_ptr()) : nullptr;
             status = c.quantize ? dpep_dispatch_quant_fp8(call.x, call.topk_weights, call.route_to_row, call.row_to_route, call.num_tokens,
@@ -820,7 +829,8 @@ PyObject* run_fresh(Exchange* e, const FreshCall& c, const Target& t, PyObject* 
     if (!c.low_latency && !keep_same(plan, d, {N._row_to_route_full})) return nullptr;
     if (PyObject_SetAttr(handle.p, N.__dict__, d) < 0) return nullptr;
 
-    Ref event(event_of(e, t, {&out, &scales, &weights, &routing}, {c.in.x, c.in.scales, c.weights, c.idx}));
+    Ref event(replaced ? event_of(e, t, {&routing}, {&out, &scales, &weights, c.in.x, c.in.scales, c.weights, c.idx})
+                       : event_of(e, t, {&out, &scales, &weights, &routing}, {c.in.x, c.in.scales, c.weights, c.idx}));
     pending.launched = !event;
     Ref payload(wrap(out));
     if (!event || !payload) return nullptr;

@@ -214,6 +214,40 @@ def test_memory_of_asynchronous_calls_is_not_handed_out_too_early(wait):
         buffer.destroy()
 
 
+@pytest.mark.parametrize("wait", ["caller", "other", "never"])
+def test_rows_of_an_outgrown_asynchronous_dispatch_outlive_their_tensor_while_they_are_read(wait):
+    """The outputs made once the row count is known belong to the communication stream: dropped right behind their last use
+    (queued, not run yet), their memory must not go to what that stream is given next."""
+    world, experts, topk, tokens, hidden = 4, 16, 4, 4096, 1024
+    x, _ = _batch(tokens, hidden, topk, 13)
+    ids = np.stack([np.random.default_rng(13).permutation(4)[:topk] for _ in range(tokens)]).astype(np.int64)
+    want = olayout.layout(ids, experts, 0, 4)
+    xd, idx = x.cuda(), torch.from_numpy(ids).cuda()
+    expected = xd[torch.from_numpy(want["row_to_route"]).cuda().long() // topk]
+    side = torch.cuda.Stream()
+    for _ in range(3):
+        buffer = _buffer(num_bytes=4 << 20, rank=0, world_size=world)
+        try:
+            torch.cuda.synchronize()
+            recv, _, _, _, event = buffer.dispatch(xd, topk_idx=idx, num_experts=experts, async_with_compute_stream=True)
+            if wait == "never":
+                kept = recv
+            else:
+                with torch.cuda.stream(side if wait == "other" else torch.cuda.current_stream()):
+                    event.current_stream_wait()
+                    torch.cuda._sleep(20_000_000)
+                    kept = recv.clone()
+            del recv, event
+            with torch.cuda.stream(buffer.get_comm_stream()):
+                noise = [torch.full((tokens * topk, hidden), 7.0, dtype=torch.bfloat16, device="cuda") for _ in range(3)]
+            torch.cuda.synchronize()
+            assert torch.equal(kept, expected)
+            del noise, kept
+        finally:
+            torch.cuda.synchronize()
+            buffer.destroy()
+
+
 @pytest.mark.parametrize("fp8", [False, True])
 def test_memory_of_an_outgrown_asynchronous_dispatch_is_not_handed_out_too_early(fp8):
     """A share several times the expected one, on the communication stream: the outputs it outgrew are let go inside the call,
