@@ -244,8 +244,8 @@ struct GemmParams {
     int fill_tokens, fill_vec, fill_topk;
     int* fill_state;
     int* fill_stop;
-    int forced_rows;                // 64 / 128 / 192: that tile height whatever the cost model says (tests); 32: the few-rows kernel
-    int forced_waves;               //   with so many waves per workgroup (1, 4); 0: the model decides
+    int forced;                     // 64 / 128 / 192: that tile height whatever the cost model says (tests); 32: the few-rows kernel
+                                    //   with (1, 4) << 8 waves per workgroup; 0: the model decides
     int column_waves;               // 1: the kernel whose waves split the tile's columns and load their weights straight into registers
 };
 
@@ -1735,7 +1735,7 @@ GemmChoice choose_gemm(const GemmParams& p, const ExpectedRows& expected, int cu
     // Source rows are addressed with 32 bits in the few-rows kernel.  A share with more than one 64-row tile per expert has so many
     // tokens without a row that its first GEMM's idle workgroups are better used for their zero rows.
     const double tiles = expected_row_tiles(32) * n_tiles;
-    if (p.column_waves && p.forced_rows == 0 && (p.fill_tokens == 0 || mean <= 64.0) && (!kGateUp || static_cast<long long>(p.a_rows) * p.k < (1LL << 32))) {
+    if (p.column_waves && p.forced == 0 && (p.fill_tokens == 0 || mean <= 64.0) && (!kGateUp || static_cast<long long>(p.a_rows) * p.k < (1LL << 32))) {
         const double one = bounded(3.0 + 0.30 * ktiles + (rounds_of(kGemmWaves * tiles, cus) - 1.0) * (1.1 + 0.17 * ktiles));
         const double four = bounded(1.5 + rounds_of(tiles, cus) * (2.7 + 0.50 * ktiles));
         // Zero rows of the output that this launch's idle workgroups would have written (at about 30 GB/s each): the few-rows
@@ -1748,8 +1748,8 @@ GemmChoice choose_gemm(const GemmParams& p, const ExpectedRows& expected, int cu
         }
         if (std::min(one, four) + unfilled < best_cost) return {32, one < four ? 1 : kGemmWaves, tiles};
     }
-    if (p.forced_rows == 32) return {32, p.forced_waves, tiles};
-    if (p.forced_rows != 0) best = p.forced_rows / 64;
+    if ((p.forced & 0xff) == 32) return {32, p.forced >> 8, tiles};
+    if (p.forced != 0) best = p.forced / 64;
     return {64 * best, kGemmWaves, tiles_of[best]};
 }
 
@@ -1790,8 +1790,7 @@ GemmParams gemm_of(const MegaSizes& m, const Workspace* w, bool second)
     p.num_routed = m.num_local;
     p.n = second ? hp : 2 * ip;
     p.k = second ? ip : hp;
-    p.forced_rows = w != nullptr ? w->gemm_tile_rows : 0;
-    p.forced_waves = w != nullptr ? w->gemm_few_rows_waves : 0;
+    p.forced = w == nullptr ? 0 : w->gemm_tile_rows == 32 ? 32 | w->gemm_few_rows_waves << 8 : w->gemm_tile_rows;
     p.column_waves = w != nullptr ? w->gemm_column_waves : 1;
     // Without shared experts most tokens of a share have no row: workgroups of the first GEMM that get no tile
     // zero those rows of y meanwhile, and the weighted reduce skips what they got through.  (Served-only: rows of y whose
