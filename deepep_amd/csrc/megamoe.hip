@@ -223,7 +223,9 @@ struct GemmParams {
     int num_routed;            // experts >= num_routed are shared experts with weights of their own:
     const uint8_t* w_shared;   //   expert e reads w_shared / ws_shared at index e - num_routed
     const uint8_t* ws_shared;
-    int n, k;
+    int n, k;                  // padded sizes: the strides of the operands
+    int n_real, k_real;        // what is not padding of them (first GEMM: n counts gate and up)
+    int live_n_tiles;          // column tiles that the 128-row paired kernel works on (first GEMM: all, unless the second reads no padding)
     uint8_t* act_codes;        // first GEMM: [rows, N/2] e4m3
     uint8_t* act_scales;       //             [rows, N/64] e8m0
     uint16_t* out;             // second GEMM: [rows, out_cols] bf16
@@ -984,20 +986,23 @@ __device__ __forceinline__ void swap_halves(uint32_t lower_q, uint32_t upper_q, 
     out[0] = swapped[0];
     out[1] = swapped[1];
 }
-// First GEMM: gate and up columns act_col .. act_col + 31 of one row -> SwiGLU -> one MXFP8 block.
-__device__ __forceinline__ void store_gate_up(const GemmParams& p, const v16f& gates, const v16f& ups, size_t row, bool row_exists, int act_col, int g)
+// First GEMM: gate and up columns act_col .. act_col + 31 of one row -> SwiGLU -> one MXFP8 block.  pairs(j): columns j and j + 1 of
+// both as BF16 pairs.
+template <typename Pairs>
+__device__ __forceinline__ void store_gate_up_pairs(const GemmParams& p, Pairs&& pairs, size_t row, bool row_exists, int act_col, int g)
 {
     float v[16];
     float amax = 0.0f;
-#pragma unroll
-    for (int j = 0; j < 16; j += 2) {
-        const uint32_t gate = pack_bf16x2(gates[j], gates[j + 1]), up = pack_bf16x2(ups[j], ups[j + 1]);
+    static_for<8>([&](auto pair_constant) {
+        constexpr int j = 2 * decltype(pair_constant)::value;
+        const u32x2 both = pairs(std::integral_constant<int, j>{});
+        const uint32_t gate = both[0], up = both[1];
         const uint32_t act = pack_bf16x2(silu_mul(__uint_as_float(gate << 16), __uint_as_float(up << 16)),
                                          silu_mul(__uint_as_float(gate & 0xffff0000u), __uint_as_float(up & 0xffff0000u)));
         v[j] = bf16_to_f32(act & 0xffffu);
         v[j + 1] = bf16_to_f32(act >> 16);
         amax = fmaxf(amax, fmaxf(fabsf(v[j]), fabsf(v[j + 1])));
-    }
+    });
     amax = fmaxf(amax, __shfl_xor(amax, 32));  // the row's other sixteen columns
     const int byte = mx_scale_byte(amax);
     uint32_t code[4];
@@ -1013,6 +1018,13 @@ __device__ __forceinline__ void store_gate_up(const GemmParams& p, const v16f& g
         *reinterpret_cast<u32x4*>(p.act_codes + row * act_width + act_col + g * 16) = codes;
         if (g == 0) p.act_scales[row * (act_width / 32) + (act_col >> 5)] = static_cast<uint8_t>(byte);
     }
+}
+__device__ __forceinline__ void store_gate_up(const GemmParams& p, const v16f& gates, const v16f& ups, size_t row, bool row_exists, int act_col, int g)
+{
+    store_gate_up_pairs(p, [&](auto at) {
+        constexpr int j = decltype(at)::value;
+        return u32x2{pack_bf16x2(gates[j], gates[j + 1]), pack_bf16x2(ups[j], ups[j + 1])};
+    }, row, row_exists, act_col, g);
 }
 // Second GEMM: columns col0 .. col0 + 31 of one row as BF16.
 __device__ __forceinline__ void store_output(const GemmParams& p, const v16f& acc, size_t row, bool row_exists, int col0, int g)
@@ -1602,6 +1614,425 @@ __global__ __launch_bounds__(kGemmThreads, ColCfg<RT>::kWorkgroupsPerCu) void gr
     wait_copies_then_barrier<0>();
 }
 
+// =====================================================================================================
+// Grouped GEMM, column-wave form with two workgroups to a CU: 128-row tiles that skip what is padding
+// =====================================================================================================
+// The column-wave kernel above owns its CU, so nothing runs on the matrix pipes while a tile starts or ends, and it works on whole
+// tiles: 97 rows cost as much as 128, 2880 columns of k as much as 3072, and k must come in multiples of 512.  This one leaves
+// room for a second workgroup on the CU (two waves per SIMD, 256 registers and half of the LDS each), whose MFMAs fill those gaps, and
+// jumps over every MFMA of a row tile without rows, of a k step behind the end of k, and of a wave whose columns are only
+// padding; column tiles of nothing but padding are not even numbered where the second GEMM does not read them.
+// Bound by the matrix pipes (their clock falls with the work in flight: large batches take as long at 192 rows on one
+// workgroup), by streaming the weights where an expert has about one row tile, and by a tile's start and end where a launch is
+// a single round.  Measured on an MI355X against the best of the other heights, whole forwards, us: 4584 tokens over 29 + 2 experts of
+// 1600 x 2944 243 -> 198, 8512 over 3 + 2 of 3264 x 3840 672 -> 565, 4560 x top-8 over 59 + 2 of 1088 x 384 77 -> 63, 777 x top-4 over
+// 32 + 1 of 2880 x 1408 97 -> 91; 8192 x top-8 over 32 of 7168 x 2048: 2336 with 192 rows, 2408 with this.
+//
+// Accumulators and weight fragments live in registers that only the assembly statements name (a0..a127, v96..v127): with two
+// workgroups to a CU the accumulators are all the accumulation registers there are, and the register allocator, which may not
+// spill one, put all of them on the stack.  tests/test_gemm_registers.py checks that the compiler's own values stay out of them;
+// the jumps are harmless to it for the same reason.
+//
+// Requests: the activation copies (and a span's scales, a tile's gather indices) run four items ahead, an LDS stage each, the
+// weights two items ahead, 16 registers each (four ahead were 1 to 3 % slower).  Every item asks, in this order, for its first k step's weights of
+// the item two ahead (2 loads, behind its own first step, whose registers are then free), its LDS stage's next
+// activations (4 copies, behind the barrier), its second k step's weights (2 loads, behind its second step); a span's first
+// item also for the scales of the span after this one, in front of the copies.  With that, an item's first weights have
+// arrived when at most 6 + 8 later requests are in flight (kWaitFirst), its second ones when at most 8 + 2 are (kWaitSecond).  The wait
+// for an item's second weights also covers everything that the items before the one two back asked for, which includes
+// the next item's activations and scales, and, at a tile's last item, the gather indices asked for at its first; the barrier
+// behind it makes them everybody's.  Requests of skipped work are issued all the same (for the last real k tile again), so the counts hold.
+struct PairCfg {
+    static constexpr int kStages = 4;                  // LDS stages = items the activation copies run ahead = unroll of the item loop
+    static constexpr int kRing = 2;                    // items the weights run ahead
+    static constexpr int kBM = 128;
+    static constexpr int kRowTiles = 4, kColTiles = 2;  // 32 x 32 MFMA tiles per wave
+    static constexpr int kStageBytes = kBM * kBK;
+    static constexpr int kRowScaleSlot = kBM * 16;
+    static constexpr int kOffRowScales = kStages * kStageBytes;
+    static constexpr int kColScaleSlot = 4096;
+    static constexpr int kOffColScales = kOffRowScales + 2 * kRowScaleSlot;
+    static constexpr int kLdsBytes = kOffColScales + 2 * kColScaleSlot;
+    static constexpr int kWeightRegs = 96;  // first of the ordinary registers that hold weight fragments (v96..v127)
+    static constexpr int kRequests = kRowTiles + 2 * kColTiles;  // per thread and item
+    static constexpr int kWaitFirst = (kRing - 1) * kRequests + kRowTiles + kColTiles;
+    static constexpr int kWaitSecond = (kRing - 1) * kRequests + kColTiles;
+};
+#define DPEP_PAIR_ACC_REGS \
+    "a0", "a1", "a2", "a3", "a4", "a5", "a6", "a7", "a8", "a9", "a10", "a11", "a12", "a13", "a14", "a15", \
+        "a16", "a17", "a18", "a19", "a20", "a21", "a22", "a23", "a24", "a25", "a26", "a27", "a28", "a29", "a30", "a31", \
+        "a32", "a33", "a34", "a35", "a36", "a37", "a38", "a39", "a40", "a41", "a42", "a43", "a44", "a45", "a46", "a47", \
+        "a48", "a49", "a50", "a51", "a52", "a53", "a54", "a55", "a56", "a57", "a58", "a59", "a60", "a61", "a62", "a63", \
+        "a64", "a65", "a66", "a67", "a68", "a69", "a70", "a71", "a72", "a73", "a74", "a75", "a76", "a77", "a78", "a79", \
+        "a80", "a81", "a82", "a83", "a84", "a85", "a86", "a87", "a88", "a89", "a90", "a91", "a92", "a93", "a94", "a95", \
+        "a96", "a97", "a98", "a99", "a100", "a101", "a102", "a103", "a104", "a105", "a106", "a107", "a108", "a109", "a110", "a111", \
+        "a112", "a113", "a114", "a115", "a116", "a117", "a118", "a119", "a120", "a121", "a122", "a123", "a124", "a125", "a126", "a127"
+#define DPEP_PAIR_WEIGHT_REGS \
+    "v96", "v97", "v98", "v99", "v100", "v101", "v102", "v103", "v104", "v105", "v106", "v107", "v108", "v109", "v110", "v111", \
+        "v112", "v113", "v114", "v115", "v116", "v117", "v118", "v119", "v120", "v121", "v122", "v123", "v124", "v125", "v126", "v127"
+// kStreamed: weights past the caches, where each is read by about one row tile and the memory-side cache does not hold them all (55
+// experts of 57 rows, 409 MB: 106 -> 96.5 us; up to 250 MB it is 5 % slower on average, with several row tiles 10 to 20 %).
+template <int kReg, int kImm, bool kStreamed>
+__device__ __forceinline__ void load16_to_paired_weight_regs(const void* uniform_base, uint32_t lane_offset)
+{
+    static_assert(kReg >= PairCfg::kWeightRegs && kReg + 3 < 128, "not one of the kernel's weight registers");
+    if constexpr (kStreamed)
+        asm volatile("global_load_dwordx4 v[%3:%4], %0, %1 offset:%2 nt" ::"v"(lane_offset), "s"(uniform_base), "n"(kImm), "n"(kReg), "n"(kReg + 3)
+                     : "memory", DPEP_PAIR_WEIGHT_REGS);
+    else
+        asm volatile("global_load_dwordx4 v[%3:%4], %0, %1 offset:%2 sc1" ::"v"(lane_offset), "s"(uniform_base), "n"(kImm), "n"(kReg), "n"(kReg + 3)
+                     : "memory", DPEP_PAIR_WEIGHT_REGS);
+}
+// The MFMAs of row tile kI (both column tiles, accumulators a[32 kI : 32 kI + 31]; weights v[kReg : kReg + 3] and the four behind), jumped over
+// unless kI < row_tiles.  Operands the other way round, as in mfma_fp4_fp8_regs.
+template <int kI, int kReg, int kByteW, int kByteX>
+__device__ __forceinline__ void mfma_row_tile(const v8i& x, int scale_w0, int scale_w1, int scale_x, int row_tiles)
+{
+    asm volatile("s_cmp_le_i32 %14, %15\n\ts_cbranch_scc1 .Lskip_mfma_%=\n\t"
+                 "v_mfma_scale_f32_32x32x64_f8f6f4 a[%10:%11], v[%8:%9], %0, a[%10:%11], %1, %3 op_sel:[%4,%5,0] op_sel_hi:[%6,%7,0] cbsz:4\n\t"
+                 "v_mfma_scale_f32_32x32x64_f8f6f4 a[%12:%13], v[%8+4:%9+4], %0, a[%12:%13], %2, %3 op_sel:[%4,%5,0] op_sel_hi:[%6,%7,0] cbsz:4\n"
+                 ".Lskip_mfma_%=:" ::"v"(x),
+                 "v"(scale_w0), "v"(scale_w1), "v"(scale_x), "n"(kByteW & 1), "n"(kByteX & 1), "n"(kByteW >> 1), "n"(kByteX >> 1), "n"(kReg), "n"(kReg + 3),
+                 "n"(32 * kI), "n"(32 * kI + 15), "n"(32 * kI + 16), "n"(32 * kI + 31), "s"(row_tiles), "n"(kI)
+                 : "scc", DPEP_PAIR_ACC_REGS);
+}
+template <int kAcc>
+__device__ __forceinline__ void clear_acc_tile()
+{
+    asm volatile(".irp r, 0, 1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15\n\tv_accvgpr_write_b32 a[%0+\\r], 0\n\t.endr" ::"n"(kAcc) : DPEP_PAIR_ACC_REGS);
+}
+template <int kAcc>
+__device__ __forceinline__ float read_acc()
+{
+    float v;
+    asm volatile("v_accvgpr_read_b32 %0, a[%1]" : "=v"(v) : "n"(kAcc) : "memory");
+    return v;
+}
+template <int kAcc>
+__device__ __forceinline__ v16f read_acc_tile()
+{
+    v16f v;
+    static_for<16>([&](auto j) { v[decltype(j)::value] = read_acc<kAcc + decltype(j)::value>(); });
+    return v;
+}
+template <int kOutstanding>
+__device__ __forceinline__ void wait_requests()
+{
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kOutstanding) : "memory");
+}
+
+template <bool kStreamed, bool kGateUp>
+__global__ __launch_bounds__(kGemmThreads, 2) void grouped_gemm_paired_kernel(GemmParams p)
+{
+    constexpr bool kGather = kGateUp;
+    using Cfg = PairCfg;
+    constexpr int kBM = Cfg::kBM, kStageBytes = Cfg::kStageBytes, kRowTiles = Cfg::kRowTiles, kCols = Cfg::kColTiles;
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+    __shared__ int tile_base[kMaxMoeExperts + 1];
+    __shared__ int row_offsets[kMaxMoeExperts + 1];
+    __shared__ int tile_index[2][kBM];   // row_to_route of a tile's rows; slots alternate per tile
+    __shared__ uint32_t row_from[2][kBM];  // byte offset from a_codes of each row of the tile under the request cursor; slots alternate per tile
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int g = lane >> 5, lr = lane & 31;
+    const int n_tiles = p.n / kBN;
+    const int live_n_tiles = p.live_n_tiles;  // (column tiles of nothing but padding are left out)
+    // The matrix is stored and addressed with its padded k (p.k); what is computed ends with the last k step that holds any of it.  An
+    // item behind that keeps its place in the rings (the last real k tile is asked for again), without MFMAs.
+    const int stored_ktiles = p.k / kBK, steps = (p.k_real + 63) / 64, last_kt = (steps - 1) / 2, ktiles = (last_kt + 4) & ~3;
+    const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(lds));
+    const uint32_t lds_index = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(&tile_index[0][0]));
+    const uint32_t wave_lds = __builtin_amdgcn_readfirstlane(lds0 + wave * 1024);
+
+    if (tid <= p.num_local) row_offsets[tid] = p.offsets[tid];
+    __syncthreads();
+    if (wave == 0) number_tiles<kBM>(row_offsets, p.num_local, live_n_tiles, lane, tile_base);
+    __syncthreads();
+    const int total_tiles = __builtin_amdgcn_readfirstlane(tile_base[p.num_local]);
+
+    // Workgroups are dealt round-robin over the 8 XCDs.  A full round's tiles are dealt out in 8 contiguous ranges, one per XCD (consecutive
+    // tiles share weights and rows: an XCD's L2 sees them from one place, and the ranges that share some are at work at the
+    // same time).  So are those of the last round, which may not be full: it then leaves one tile, at full speed, to each of some
+    // CUs on every XCD.
+    const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3, grid = gridDim.x;
+    const int full_rounds = total_tiles / grid, rest = total_tiles - full_rounds * grid, rest_first = rest * xcd / 8;
+    const int my_tiles = full_rounds + (rest_first + slot < rest * (xcd + 1) / 8 ? 1 : 0);
+    if (blockIdx.x == 0 && tid == 0 && p.fill_state != nullptr) p.fill_state[0] = 0;
+    if (my_tiles == 0) return;
+    auto tile_of = [&](int round) __attribute__((always_inline)) {
+        return round * grid + slot + (round < full_rounds ? xcd * (grid >> 3) : rest_first);
+    };
+
+    auto decode = [&](int tile) __attribute__((always_inline)) {  // panels of eight column tiles: as in the column-wave kernel
+        const int e = expert_of_tile(tile, tile_base, p.num_local);
+        const int row_begin = __builtin_amdgcn_readfirstlane(row_offsets[e]), rows = __builtin_amdgcn_readfirstlane(row_offsets[e + 1]) - row_begin;
+        const int m_tiles = (rows + kBM - 1) / kBM;
+        const int local = tile - __builtin_amdgcn_readfirstlane(tile_base[e]);
+        constexpr int kPanel = 8;
+        const int panel = local / (m_tiles * kPanel), in_panel = local - panel * (m_tiles * kPanel);
+        const int width = min(kPanel, live_n_tiles - panel * kPanel);
+        TileInfo info;
+        info.expert = e;
+        info.nt = panel * kPanel + in_panel % width;
+        const int m0 = (in_panel / width) * kBM;
+        info.row0 = row_begin + m0;
+        info.valid = min(kBM, rows - m0);
+        return info;
+    };
+
+    // ---- request cursors ---------------------------------------------------------------------------------------------------
+    const uint32_t b_lane = static_cast<uint32_t>(wave * 4096 + lane * 16);
+    const uint8_t* b_next = p.w;   // first weight fragment of the tile under the activation cursor
+    const uint8_t* b_at = p.w;     // of the item under the weight cursor
+    int b_kt = 0;
+    const uint8_t* sb_base = p.ws;
+    int index_row0 = 0, index_valid = 1;
+    int copy_kt = 0, copy_span = -1, copy_ordinal = 0;
+    const int scale_bytes = p.k / 32, spans = (stored_ktiles + 3) / 4;
+    TileInfo next_info = decode(tile_of(0));
+
+    auto point_at_tile = [&](const TileInfo& info) __attribute__((always_inline)) {
+        const int* index = tile_index[copy_ordinal & 1];
+        const int r = min(wave * 64 + lane_now(), kBM - 1), from = min(r, info.valid - 1);  // rows past the tile's end repeat its last row
+        const int src = kGather ? min(max(index[from] / p.topk, 0), p.a_rows - 1) : info.row0 + from;
+        row_from[copy_ordinal & 1][r] = static_cast<uint32_t>(src) * static_cast<uint32_t>(p.k);
+        const bool shared = info.expert >= p.num_routed;
+        const size_t weight_index = shared ? info.expert - p.num_routed : info.expert;
+
+        b_next = (shared ? p.w_shared : p.w) + weight_index * p.n * (p.k / 2) + static_cast<size_t>(info.nt) * stored_ktiles * 16384;
+        sb_base = (shared ? p.ws_shared : p.ws) + (weight_index * n_tiles + info.nt) * spans * Cfg::kColScaleSlot;
+    };
+    auto aim_index_prefetch = [&](const TileInfo& info) __attribute__((always_inline)) {
+        index_row0 = info.row0;
+        index_valid = info.valid;
+    };
+    auto index_offset = [&]() __attribute__((always_inline)) { return static_cast<uint32_t>(index_row0 + min((wave & 1) * 64 + lane_now(), index_valid - 1)) * 4u; };
+
+    u32x2 bscale_now[kCols], bscale_next[kCols];
+
+    // activation copy c of wave w fills LDS rows c*32 + w*8 + lane/8; chunk (lane%8) ^ ((row>>1)&7) of the 128-byte row
+    const uint32_t a_chunk = static_cast<uint32_t>(((lane & 7) ^ ((wave * 4 + (lane >> 4)) & 7)) * 16);
+    const uint32_t* my_rows = &row_from[0][wave * 8 + (lane >> 3)];  // + kBM for the other slot
+    auto request_activations_at = [&](auto pos, auto piece, uint32_t row_offset) __attribute__((always_inline)) {
+        constexpr int kPos = decltype(pos)::value, kPiece = decltype(piece)::value;
+        copy16_to_lds_at<kPos * kStageBytes + kPiece * 4096>(p.a_codes + static_cast<size_t>(min(copy_kt, last_kt)) * kBK, row_offset + a_chunk, wave_lds);
+    };
+    auto request_weights = [&](auto slot, auto step) __attribute__((always_inline)) {
+        constexpr int kSlot = decltype(slot)::value, kStep = decltype(step)::value;
+        constexpr int kReg = Cfg::kWeightRegs + 16 * kSlot + 8 * kStep;
+        load16_to_paired_weight_regs<kReg, kStep * 1024, kStreamed>(b_at, b_lane);
+        load16_to_paired_weight_regs<kReg + 4, 2048 + kStep * 1024, kStreamed>(b_at, b_lane);
+    };
+    auto request_span = [&]() __attribute__((always_inline)) {
+        ++copy_span;
+        const int window = min(copy_kt * 4, scale_bytes - 16);  // (a last span of two k tiles: its bytes sit two words up)
+        const int t = wave * 64 + lane_now();
+        copy16_to_lds(p.a_scales + window, row_from[copy_ordinal & 1][t % kBM] >> 5, lds0 + Cfg::kOffRowScales + (copy_span & 1) * Cfg::kRowScaleSlot + (wave & 1) * 1024);
+        copy16_to_lds(sb_base + static_cast<size_t>(copy_kt >> 2) * Cfg::kColScaleSlot, static_cast<uint32_t>(t * 16),
+                      lds0 + Cfg::kOffColScales + (copy_span & 1) * Cfg::kColScaleSlot + wave * 1024);
+        if (kGather)
+            copy4_to_lds_unless(p.row_to_route, index_offset(), lds_index + ((copy_ordinal + 1) & 1) * (kBM * 4) + (wave & 1) * 256, copy_kt);
+    };
+    auto advance_activations = [&](bool in_prologue, bool last_of_four) __attribute__((always_inline)) {
+        ++copy_kt;
+        if (last_of_four && copy_kt == ktiles) {
+            if (copy_ordinal + 1 < my_tiles) {
+                if (kGather && switch_needs_drain(in_prologue, ktiles, Cfg::kStages)) wait_copies_then_barrier<0>();
+                copy_kt = 0;
+                ++copy_ordinal;
+                point_at_tile(next_info);
+                if (copy_ordinal + 1 < my_tiles) next_info = decode(tile_of(copy_ordinal + 1));
+                aim_index_prefetch(next_info);
+            } else {
+                copy_kt = ktiles - 4;  // past the last tile: keep asking for its last span (never used)
+            }
+        }
+    };
+    // The weight cursor enters a tile two items behind the activation cursor, which by then points at that tile and at no later one yet (a tile
+    // has at least four items; past the last tile: at the same tile still, whose first items are asked for again and never used).
+    auto advance_weights = [&](bool last_of_four) __attribute__((always_inline)) {
+        if (b_kt < last_kt) b_at += 16384;
+        ++b_kt;
+        if (last_of_four && b_kt == ktiles) {
+            b_kt = 0;
+            b_at = b_next;
+        }
+    };
+
+    if (kGather) {
+        aim_index_prefetch(next_info);
+        copy4_to_lds(p.row_to_route, index_offset(), lds_index + (wave & 1) * 256);
+        wait_copies_then_barrier<0>();
+    }
+    point_at_tile(next_info);
+    b_at = b_next;
+    if (my_tiles > 1) next_info = decode(tile_of(1));
+    aim_index_prefetch(next_info);
+    __syncthreads();  // row_from
+
+    int a_addr[2][2];  // [k step][lo/hi 16 bytes] of row tile 0; row tile i lies i * 4096 bytes further (same swizzle)
+    {
+        const int sw = (lr >> 1) & 7;
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb) {
+            a_addr[kb][0] = lr * kBK + (((kb * 4 + g) ^ sw) << 4);
+            a_addr[kb][1] = lr * kBK + (((kb * 4 + 2 + g) ^ sw) << 4);
+        }
+    }
+    // LDS address of this lane's row-scale entry in the slot of the span that begins with k tile `from`
+    auto row_scales_of = [&](int slot, int from) __attribute__((always_inline)) {
+        return Cfg::kOffRowScales + lr * 16 + slot * Cfg::kRowScaleSlot + (from * 4 > scale_bytes - 16 ? 8 : 0);
+    };
+    int row_scale_at = row_scales_of(0, 0);
+    int col_scale_slot = 0;
+    v8i afrag[kRowTiles];  // of the k step at work, overwritten row tile by row tile with the next one's
+    int ascale[kRowTiles];
+    auto read_fragment = [&](int stage, int kb, int i) __attribute__((always_inline)) {
+        const uint8_t* at = lds + stage * kStageBytes + i * 4096;
+        const u32x4 lo = *reinterpret_cast<const u32x4*>(at + a_addr[kb][0]);
+        const u32x4 hi = *reinterpret_cast<const u32x4*>(at + a_addr[kb][1]);
+        afrag[i] = v8i{(int)lo[0], (int)lo[1], (int)lo[2], (int)lo[3], (int)hi[0], (int)hi[1], (int)hi[2], (int)hi[3]};
+    };
+    auto read_row_scale = [&](int pos, int i) __attribute__((always_inline)) {
+        ascale[i] = static_cast<int>(*reinterpret_cast<const uint32_t*>(lds + row_scale_at + (i * 512 + pos * 4)));
+    };
+    auto read_col_scales = [&]() __attribute__((always_inline)) {
+        const int sb_addr = Cfg::kOffColScales + wave * 1024 + lane_now() * 8;
+#pragma unroll
+        for (int c = 0; c < kCols; ++c) bscale_next[c] = *reinterpret_cast<const u32x2*>(lds + sb_addr + c * 512 + col_scale_slot);
+    };
+
+    auto clear_acc = [&]() __attribute__((always_inline)) { static_for<kRowTiles * kCols>([&](auto n) __attribute__((always_inline)) { clear_acc_tile<16 * decltype(n)::value>(); }); };
+    auto epilogue = [&](const TileInfo& info) __attribute__((always_inline)) {
+        const int lane = lane_now(), g = lane >> 5, lr = lane & 31;
+        static_for<kRowTiles>([&](auto i_constant) __attribute__((always_inline)) {
+            constexpr int i = decltype(i_constant)::value;
+            const bool row_exists = lr < info.valid - 32 * i;
+            const size_t row = static_cast<size_t>(info.row0) + 32 * i + lr;
+            if constexpr (kGateUp) {
+                store_gate_up_pairs(p, [&](auto at) __attribute__((always_inline)) {
+                    constexpr int gate = 32 * i + decltype(at)::value, up = gate + 16;
+                    const uint32_t gates = pack_bf16x2(read_acc<gate>(), read_acc<gate + 1>());
+                    return u32x2{gates, pack_bf16x2(read_acc<up>(), read_acc<up + 1>())};
+                }, row, row_exists, (info.nt * (kBN / 64) + wave) * 32, g);
+            } else {
+                store_output(p, read_acc_tile<32 * i>(), row, row_exists, info.nt * kBN + wave * kCols * 32, g);
+                store_output(p, read_acc_tile<32 * i + 16>(), row, row_exists, info.nt * kBN + (wave * kCols + 1) * 32, g);
+            }
+        });
+    };
+
+    // ---- prologue: activations and scales of items 0..3, weights of items 0 and 1; all of it arrives before item 0, which the counted waits build on -----------------------------------------
+    static_for<4>([&](auto pos) __attribute__((always_inline)) {
+        if (decltype(pos)::value == 0) request_span();
+        static_for<kRowTiles>([&](auto piece) __attribute__((always_inline)) { request_activations_at(pos, piece, my_rows[(copy_ordinal & 1) * kBM + decltype(piece)::value * 32]); });
+        advance_activations(true, decltype(pos)::value == 3);
+    });
+    static_for<Cfg::kRing>([&](auto slot) __attribute__((always_inline)) {
+        request_weights(slot, std::integral_constant<int, 0>{});
+        request_weights(slot, std::integral_constant<int, 1>{});
+        advance_weights(false);
+    });
+    wait_copies_then_barrier<0>();
+    int read_span = 0;
+    read_col_scales();
+#pragma unroll
+    for (int i = 0; i < kRowTiles; ++i) {
+        read_row_scale(0, i);
+        read_fragment(0, 0, i);
+    }
+    clear_acc();
+    asm volatile("s_nop 3");
+    int ordinal = 0, kt = 0;
+    // Row tiles that hold a row; none for a wave whose columns are only padding.
+    auto live_row_tiles = [&](const TileInfo& tile_info) __attribute__((always_inline)) {
+        return __builtin_amdgcn_readfirstlane(tile_info.nt * kBN + wave * 64 < p.n_real ? (tile_info.valid + 31) / 32 : 0);
+    };
+    TileInfo info = decode(tile_of(0));
+    int row_tiles = live_row_tiles(info);
+    long long items_left = static_cast<long long>(my_tiles) * ktiles;
+    constexpr int kMfmas = kRowTiles * kCols;
+
+    auto item_body = [&](auto pos) __attribute__((always_inline)) {
+        constexpr int kPos = decltype(pos)::value, kSlot = kPos % Cfg::kRing;
+        constexpr std::integral_constant<int, kSlot> slot{};
+        if (kPos == 0) {
+#pragma unroll
+            for (int c = 0; c < kCols; ++c) bscale_now[c] = bscale_next[c];
+        }
+        const int scale_b0 = static_cast<int>(bscale_now[0][kPos >> 1]), scale_b1 = static_cast<int>(bscale_now[1][kPos >> 1]);
+        int shifted[kRowTiles];
+#pragma unroll
+        for (int i = 0; i < kRowTiles; ++i) shifted[i] = ascale[i] >> (8 * g);
+        const int first_step = 2 * (kt + kPos);
+        const int live0 = first_step < steps ? row_tiles : 0, live1 = first_step + 1 < steps ? row_tiles : 0;
+        auto mfma = [&](auto step, auto n) __attribute__((always_inline)) {
+            constexpr int kStep = decltype(step)::value, kN = decltype(n)::value, kI = kN / kCols, kC = kN % kCols;
+            if constexpr (kC == 0)
+                mfma_row_tile<kI, Cfg::kWeightRegs + 16 * kSlot + 8 * kStep, 2 * (kPos & 1) + kStep, 2 * kStep>(
+                    afrag[kI], scale_b0, scale_b1, shifted[kI], kStep == 0 ? live0 : live1);
+        };
+        wait_requests<Cfg::kWaitFirst>();
+        static_for<kMfmas>([&](auto n) __attribute__((always_inline)) {
+            constexpr int kN = decltype(n)::value;
+            mfma(std::integral_constant<int, 0>{}, n);
+            if constexpr (kN % kCols == kCols - 1) read_fragment(kPos, 1, kN / kCols);
+        });
+        request_weights(slot, std::integral_constant<int, 0>{});
+        wait_requests<Cfg::kWaitSecond>();
+        if (kPos == 3) {
+            ++read_span;
+            row_scale_at = row_scales_of(read_span & 1, kt + 4 == ktiles ? 0 : kt + 4);
+            col_scale_slot = (read_span & 1) * Cfg::kColScaleSlot;
+            read_col_scales();
+        }
+        uint32_t copy_from[kRowTiles];
+        static_for<kMfmas>([&](auto n) __attribute__((always_inline)) {
+            constexpr int kN = decltype(n)::value;
+            mfma(std::integral_constant<int, 1>{}, n);
+            if constexpr (kN == kCols - 1) {
+                asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+#pragma unroll
+                for (int i = 0; i < kRowTiles; ++i) copy_from[i] = my_rows[(copy_ordinal & 1) * kBM + i * 32];
+                if (kPos == 0) request_span();
+            }
+            if constexpr (kN >= 3 && kN < 3 + kRowTiles) request_activations_at(pos, std::integral_constant<int, kN - 3>{}, copy_from[kN - 3]);
+            if constexpr (kN % kCols == kCols - 1) {
+                read_row_scale((kPos + 1) & 3, kN / kCols);
+                read_fragment((kPos + 1) & 3, 0, kN / kCols);
+            }
+        });
+        request_weights(slot, std::integral_constant<int, 1>{});
+        advance_activations(false, kPos == 3);
+        advance_weights(((kPos + Cfg::kRing) & 3) == 3);
+    };
+
+    for (; items_left > 0; items_left -= 4) {
+        static_for<4>(item_body);
+        kt += 4;
+        if (__builtin_expect(kt == ktiles, 0)) {
+            settle_accumulators();
+            epilogue(info);
+            clear_acc();
+            // (read once more: kept across the epilogue, the next item's fragments and row scales would cost it 36 registers)
+#pragma unroll
+            for (int i = 0; i < kRowTiles; ++i) {
+                read_row_scale(0, i);
+                read_fragment(0, 0, i);
+            }
+            asm volatile("s_nop 3");
+            kt = 0;
+            if (++ordinal < my_tiles) {
+                info = decode(tile_of(ordinal));
+                row_tiles = live_row_tiles(info);
+            }
+        }
+    }
+    // Nothing may still be in flight into this workgroup's LDS or registers when it retires.
+    wait_copies_then_barrier<0>();
+}
+
 // What the GEMM works on for a logical dimension (hidden or intermediate): whole 256-column tiles and whole spans of
 // scales, at least 512 (a row's scale bytes fill one 16-byte copy).  Weights are padded when they are prepared,
 // activations by a copy of their own before the first GEMM; padding multiplies zero codes.
@@ -1645,6 +2076,16 @@ int allow_lds(Kernel kernel, int bytes, std::atomic<bool>* configured, int max_d
 // round of 512 instead of two of 256, with twice the requests in flight; 700 tiles: two slow rounds would replace three
 // fast ones).
 bool two_workgroups_pay(double tiles, int cus) { return 2.0 * ceil(tiles / (2.0 * cus)) <= ceil(tiles / cus); }
+
+template <bool kStreamed, bool kGateUp>
+int launch_paired(const GemmParams& p, hipStream_t stream, const char* what)
+{
+    constexpr int kMaxDevices = 64;
+    static std::atomic<bool> configured[kMaxDevices];
+    if (int rc = allow_lds(&grouped_gemm_paired_kernel<kStreamed, kGateUp>, PairCfg::kLdsBytes, configured, kMaxDevices)) return rc;
+    hipLaunchKernelGGL((grouped_gemm_paired_kernel<kStreamed, kGateUp>), dim3(2 * gemm_grid()), dim3(kGemmThreads), PairCfg::kLdsBytes, stream, p);
+    return launch_status(what);
+}
 
 template <int RT, bool kGateUp>
 int launch_gemm_rt(const GemmParams& p, double expected_tiles, hipStream_t stream, const char* what)
@@ -1693,6 +2134,7 @@ struct GemmChoice {
     int rows;      // row-tile height: 64, 128, 192; 32: the few-rows kernel
     int waves;     // per workgroup (4 but for the few-rows kernel's small launches)
     double tiles;  // expected, of that height
+    bool paired, streamed;  // 128 rows: the kernel with two workgroups to a CU; its weights past the caches
 };
 template <bool kGateUp>
 GemmChoice choose_gemm(const GemmParams& p, const ExpectedRows& expected, int cus)
@@ -1732,31 +2174,64 @@ GemmChoice choose_gemm(const GemmParams& p, const ExpectedRows& expected, int cu
             best = rt;
         }
     }
-    // Source rows are addressed with 32 bits in the few-rows kernel.  A share with more than one 64-row tile per expert has so many
-    // tokens without a row that its first GEMM's idle workgroups are better used for their zero rows.
+    // The 128-row paired kernel: full rounds of two tiles per CU, then a last one that is a pair or, with at most one tile per CU, a
+    // single tile; per tile its start and end, per item a part that grows with the 32-row tiles that hold rows and one for weights that
+    // few row tiles share.  It counts only what is not padding.  Fitted to kernel traces of both GEMMs at 240 shapes (8 to 10 000 rows for
+    // each of 2 to 64 experts), three sets of inputs in turn: 7 % off on average; with it among the candidates the chosen kernels
+    // are 5.6 % faster on average (1.2 % slower than the best ones, 6.8 % without it).
+    double paired = 1e30, paired_row_tiles = 0.0;
+    bool streamed = false;
+    const double experts_with_rows = p.num_routed * routed_with_rows + num_shared;
+    if (p.column_waves) {
+        const int steps = (p.k_real + 63) / 64, items = ((steps - 1) / 2 + 4) / 4 * 4, slots = 2 * cus;
+        paired_row_tiles = expected_row_tiles(128);
+        const double live_row_tiles = expected_row_tiles(32), live = live_row_tiles / std::max(paired_row_tiles, 1e-3);
+        const double share = experts_with_rows / std::max(paired_row_tiles, 1e-3);
+        const double tiles = paired_row_tiles * p.live_n_tiles, full = floor(std::max(0.0, tiles / slots - 0.01)), rest = (tiles - full * slots) / cus;
+        const double pair = 5.0 + items * (0.652 + 0.147 * live + 0.269 * share), single = 3.37 + items * (0.236 + 0.112 * live + 0.135 * share);
+        const double t = 2.94 + full * pair + (rest > 1.01 ? pair : rest > 0.0 ? single : 0.0);
+        const double live_bytes = experts_with_rows * p.live_n_tiles * ((steps + 1) / 2) * 16896.0;
+        // A long launch runs at the power limit, and where it has nothing to jump over, 192-row tiles win by moving a third fewer
+        // weights: of nine launches of 8 and more rounds with less than 6 % of padding in those tiles they were 1.6 % faster on average
+        // (8192 x top-8 over 32 experts of 7168 x 2048: first GEMM 1343 us against 1375, second 803 against 840).
+        const double tall_work = tiles_of[3] * 6.0 * ktiles * 2.0, live_work = live_row_tiles * p.live_n_tiles * steps;
+        const bool power_limited = kind == 0 && best == 3 && full >= 8.0 && tall_work < 1.06 * live_work;
+        if (!power_limited) paired = std::max(2.0 + live_bytes / 5.32e6, t) + 0.05 * t;
+        // Weights that the memory-side cache does not hold, each read by about one row tile: past the caches.
+        streamed = live_bytes > 256e6 && paired_row_tiles < 1.3 * experts_with_rows;
+    }
+    const GemmChoice pair_choice = {128, kGemmWaves, paired_row_tiles * p.live_n_tiles, true, streamed};
+    // A share with more than one 64-row tile per expert has so many tokens without a row that its first GEMM's idle workgroups are
+    // better used for their zero rows: kernels that do not fill are no candidates there.
+    const bool fills = p.fill_tokens > 0 && tiles_of[best] < cus;
+    const bool unfilled_allowed = !fills || mean <= 64.0;
+    // Source rows are addressed with 32 bits in the few-rows kernel.
     const double tiles = expected_row_tiles(32) * n_tiles;
-    if (p.column_waves && p.forced == 0 && (p.fill_tokens == 0 || mean <= 64.0) && (!kGateUp || static_cast<long long>(p.a_rows) * p.k < (1LL << 32))) {
-        const double one = bounded(3.0 + 0.30 * ktiles + (rounds_of(kGemmWaves * tiles, cus) - 1.0) * (1.1 + 0.17 * ktiles));
-        const double four = bounded(1.5 + rounds_of(tiles, cus) * (2.7 + 0.50 * ktiles));
-        // Zero rows of the output that this launch's idle workgroups would have written (at about 30 GB/s each): the few-rows
-        // kernel leaves them to the reduce, which writes them at 8 TB/s, and the GEMM is faster without the company: 4300 zero
+    if (p.column_waves && p.forced == 0) {
+        const bool few_allowed = (p.fill_tokens == 0 || mean <= 64.0) && (!kGateUp || static_cast<long long>(p.a_rows) * p.k < (1LL << 32));
+        const double one = few_allowed ? bounded(3.0 + 0.30 * ktiles + (rounds_of(kGemmWaves * tiles, cus) - 1.0) * (1.1 + 0.17 * ktiles)) : 1e30;
+        const double four = few_allowed ? bounded(1.5 + rounds_of(tiles, cus) * (2.7 + 0.50 * ktiles)) : 1e30;
+        // Zero rows of the output that this launch's idle workgroups would have written (at about 30 GB/s each): these two
+        // kernels leave them to the reduce, which writes them at 8 TB/s, and the GEMM is faster without the company: 4300 zero
         // rows of 5120 columns beside 31 experts of 5120 x 512 cost the forward 57 us filled and 49 not.
         double unfilled = 0.0;
-        if (p.fill_tokens > 0 && tiles_of[best] < cus) {
+        if (fills) {
             const double zeros = p.fill_tokens * exp(-mean * p.num_routed / p.fill_tokens) * p.fill_vec * 16.0;
             unfilled = std::min(zeros, (cus - tiles_of[best]) * 30e3 * best_cost) / 11e6;
         }
-        if (std::min(one, four) + unfilled < best_cost) return {32, one < four ? 1 : kGemmWaves, tiles};
+        const double few = std::min(one, four);
+        if (unfilled_allowed && paired < few && paired + unfilled < best_cost) return pair_choice;
+        if (few + unfilled < best_cost) return {32, one < four ? 1 : kGemmWaves, tiles, false, false};
     }
-    if ((p.forced & 0xff) == 32) return {32, p.forced >> 8, tiles};
+    if ((p.forced & 0xff) == 32) return {32, p.forced >> 8, tiles, false, false};
+    if (p.forced == 128 && p.column_waves && (p.fill_tokens == 0 || tiles_of[2] >= cus)) return pair_choice;
     if (p.forced != 0) best = p.forced / 64;
-    return {64 * best, kGemmWaves, tiles_of[best]};
+    return {64 * best, kGemmWaves, tiles_of[best], false, false};
 }
 
 template <bool kGateUp>
-int launch_gemm(const GemmParams& p, const ExpectedRows& expected, hipStream_t stream, const char* what)
+int launch_gemm(const GemmParams& p, const GemmChoice& choice, const ExpectedRows& expected, hipStream_t stream, const char* what)
 {
-    const GemmChoice choice = choose_gemm<kGateUp>(p, expected, gemm_grid());
     if (choice.rows == 32) {
         DPEP_REQUIRE(!kGateUp || static_cast<long long>(p.a_rows) * p.k < (1LL << 32), "%s: 32-row tiles address at most 4 GiB of input rows", what);
         // Workgroups for more rows than expected (those without a tile end at once, while one with two doubles the time).
@@ -1771,6 +2246,7 @@ int launch_gemm(const GemmParams& p, const ExpectedRows& expected, hipStream_t s
             hipLaunchKernelGGL((grouped_gemm_few_rows_kernel<kGemmWaves, kGateUp>), dim3(grid), dim3(kGemmThreads), 0, stream, p);
         return launch_status(what);
     }
+    if (choice.paired) return choice.streamed ? launch_paired<true, kGateUp>(p, stream, what) : launch_paired<false, kGateUp>(p, stream, what);
     if (choice.rows == 64) return launch_gemm_rt<1, kGateUp>(p, choice.tiles, stream, what);
     if (choice.rows == 128) return launch_gemm_rt<2, kGateUp>(p, choice.tiles, stream, what);
     return launch_gemm_rt<3, kGateUp>(p, choice.tiles, stream, what);
@@ -1790,6 +2266,9 @@ GemmParams gemm_of(const MegaSizes& m, const Workspace* w, bool second)
     p.num_routed = m.num_local;
     p.n = second ? hp : 2 * ip;
     p.k = second ? ip : hp;
+    p.n_real = second ? m.hidden : 2 * m.intermediate;
+    p.k_real = second ? m.intermediate : m.hidden;
+    p.live_n_tiles = second ? (m.hidden + kBN - 1) / kBN : p.n / kBN;
     p.forced = w == nullptr ? 0 : w->gemm_tile_rows == 32 ? 32 | w->gemm_few_rows_waves << 8 : w->gemm_tile_rows;
     p.column_waves = w != nullptr ? w->gemm_column_waves : 1;
     // Without shared experts most tokens of a share have no row: workgroups of the first GEMM that get no tile
@@ -1808,6 +2287,20 @@ ExpectedRows expected_rows_of(const MegaSizes& m)
 {
     const double routed = static_cast<double>(m.num_tokens) * m.num_topk / m.num_experts;
     return {routed, sqrt(routed * std::max(0.0, 1.0 - static_cast<double>(m.num_topk) / m.num_experts)) + 1e-3, m.num_tokens};
+}
+// Kernels of both GEMMs.  The second one first: the paired kernel reads no padding of the activations, so that the first GEMM, if it
+// is that kernel too, leaves out the column tiles that would only write some.
+struct GemmChoices {
+    GemmChoice first, second;
+};
+GemmChoices choose_gemms(const MegaSizes& m, GemmParams& g1, const GemmParams& g2)
+{
+    const ExpectedRows expected = expected_rows_of(m);
+    GemmChoices c;
+    c.second = choose_gemm<false>(g2, expected, gemm_grid());
+    if (c.second.paired) g1.live_n_tiles = (g1.n_real + kBN - 1) / kBN;
+    c.first = choose_gemm<true>(g1, expected, gemm_grid());
+    return c;
 }
 
 }  // namespace
@@ -1999,17 +2492,17 @@ bool replay_column_waves(int my_tiles, int ktiles, int epilogue_stores, int slac
     return ok;
 }
 
-int launch_gemm1(const GemmParams& p, const ExpectedRows& expected, hipStream_t stream)
+int launch_gemm1(const GemmParams& p, const GemmChoice& choice, const ExpectedRows& expected, hipStream_t stream)
 {
     if (int rc = check_gemm("gemm1", p.n, p.k, p.num_local)) return rc;
     DPEP_REQUIRE(p.row_to_route != nullptr && p.topk >= 1, "gemm1: needs the row -> route map");
-    return launch_gemm<true>(p, expected, stream, "grouped_gemm1");
+    return launch_gemm<true>(p, choice, expected, stream, "grouped_gemm1");
 }
 
-int launch_gemm2(const GemmParams& p, const ExpectedRows& expected, hipStream_t stream)
+int launch_gemm2(const GemmParams& p, const GemmChoice& choice, const ExpectedRows& expected, hipStream_t stream)
 {
     if (int rc = check_gemm("gemm2", p.n, p.k, p.num_local)) return rc;
-    return launch_gemm<false>(p, expected, stream, "grouped_gemm2");
+    return launch_gemm<false>(p, choice, expected, stream, "grouped_gemm2");
 }
 
 }  // namespace dpep
@@ -2156,8 +2649,9 @@ int dpep_megamoe_gemm_choice(void* ws, int num_tokens, int hidden, int intermedi
     DPEP_REQUIRE(num_tokens >= 1 && hidden >= 1 && intermediate >= 1 && num_topk >= 1 && num_experts >= num_local && num_local >= 1 && num_shared >= 0,
                  "megamoe_gemm_choice: bad sizes");
     const MegaSizes sizes = {num_tokens, hidden, intermediate, num_topk, num_experts, num_local, num_shared};
-    const GemmParams p = gemm_of(sizes, w, second != 0);
-    const GemmChoice choice = second != 0 ? choose_gemm<false>(p, expected_rows_of(sizes), gemm_grid()) : choose_gemm<true>(p, expected_rows_of(sizes), gemm_grid());
+    GemmParams g1 = gemm_of(sizes, w, false);
+    const GemmChoices choices = choose_gemms(sizes, g1, gemm_of(sizes, w, true));
+    const GemmChoice& choice = second != 0 ? choices.second : choices.first;
     *tile_rows = choice.rows;
     *waves = choice.waves;
     return DPEP_OK;
@@ -2275,7 +2769,8 @@ int dpep_megamoe_run(void* ws, const dpep_megamoe_call* call, void* stream)
                             psum, offsets, route_to_row, row_to_route, num_rows, front, s))
         return rc;
     const MegaSizes sizes = {num_tokens, hidden, intermediate, num_topk, num_experts, num_local, num_shared};
-    GemmParams g1 = gemm_of(sizes, w, false);
+    GemmParams g1 = gemm_of(sizes, w, false), g2 = gemm_of(sizes, w, true);
+    const GemmChoices choices = choose_gemms(sizes, g1, g2);
     g1.a_codes = codes;
     g1.a_scales = scales;
     g1.row_to_route = row_to_route;
@@ -2299,8 +2794,7 @@ int dpep_megamoe_run(void* ws, const dpep_megamoe_call* call, void* stream)
         g1.fill_stop = fill_stop;
     }
     g1.fill_state = fill_state;  // written even when nothing fills (then as "no fillers")
-    if (int rc = launch_gemm1(g1, expected, s)) return rc;
-    GemmParams g2 = gemm_of(sizes, w, true);
+    if (int rc = launch_gemm1(g1, choices.first, expected, s)) return rc;
     g2.a_codes = base + l.act_codes;
     g2.a_scales = base + l.act_scales;
     g2.row_to_route = nullptr;
@@ -2311,7 +2805,7 @@ int dpep_megamoe_run(void* ws, const dpep_megamoe_call* call, void* stream)
     g2.ws_shared = shared_s2;
     g2.out = reinterpret_cast<uint16_t*>(base + l.out2);
     g2.out_cols = hidden;
-    if (int rc = launch_gemm2(g2, expected, s)) return rc;
+    if (int rc = launch_gemm2(g2, choices.second, expected, s)) return rc;
     return combine_routes(base + l.out2, topk_weights, route_to_row, num_tokens, num_topk,
                           static_cast<int>(expected_rows),
                           hidden, y, num_shared > 0 ? num_rows : nullptr, num_shared, fill ? fill_state : nullptr,

@@ -157,3 +157,27 @@ def test_the_check_finds_an_accumulator_that_is_touched_too_early(assembly):
              ".LBB0_2:", "s_waitcnt vmcnt(0)", "v_mov_b32_e32 v40, v15"]
     assert [(found[1], found[2]) for found in _touched_too_early(piece)] == [("v_mov_b32_e32 v40, v15", 17)]
     assert not _touched_too_early(piece[:2] + ["s_nop 1"] + piece[2:])
+
+
+def test_registers_of_the_paired_kernel_belong_to_its_assembly_statements_alone(assembly):
+    """Accumulators (a0..a127, all there are with two workgroups to a CU) and weight fragments (v96..v127)."""
+    kernels = _kernels(assembly, "grouped_gemm_paired_kernel")
+    assert len(kernels) == 4  # {cached, streamed weights} x {first, second} GEMM
+    for name, (body, scratch) in kernels.items():
+        in_statement, outside, in_loads, accumulators = False, [], set(), set()
+        for line in body:
+            text = line.split(";")[0].strip() if not line.strip().startswith(";;#") else line.strip()
+            if text.startswith(";;#ASMSTART"):
+                in_statement = True
+            elif text.startswith(";;#ASMEND"):
+                in_statement = False
+            elif in_statement:
+                if text.startswith("global_load_dwordx4"):
+                    in_loads.update(_numbers(text.split(",")[0], "v"))
+                if text.startswith("v_mfma"):
+                    accumulators.update(_numbers(text.split(",")[0], "a"))
+            elif _numbers(text, "a") or any(r >= 96 for r in _numbers(text, "v")):
+                outside.append(text)
+        assert not outside, f"{name}: the compiler uses the kernel's own registers: {outside[:3]}"
+        assert min(in_loads) == 96 and max(in_loads) == 127 and min(accumulators) == 0 and max(accumulators) == 127
+        assert scratch == 0, f"{name}: {scratch} bytes of stack"

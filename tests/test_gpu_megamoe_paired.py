@@ -1,0 +1,68 @@
+"""The 128-row grouped GEMM with two workgroups to a CU, at the sizes where it can go wrong: row counts on both sides of its 32-row
+tiles, k that ends inside a span of four k tiles, inside a k tile and behind one MFMA step, column tiles and waves of nothing but
+padding, more tiles than workgroups.  A k sum is taken in the same order as in the few-rows kernel, so the two give the same bits; both
+against the fp32 oracle within the path's 2e-2."""
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import megamoe as mm
+
+pytestmark = pytest.mark.gpu
+
+EDGES = (1, 31, 32, 33, 0, 64, 65, 96, 97, 127, 128, 129, 160, 256, 257)
+
+
+def _forward(ops, x, l1, l2, shared, idx, weights, hidden, inter, local, tile_rows):
+    dev = "cuda"
+    num_shared = 0 if shared is None else shared[0][0].shape[0]
+
+    def prepared(l, n, gate_up):
+        return ops.megamoe_prepare_weights(torch.from_numpy(l[0]).to(dev), torch.from_numpy(l[1]).reshape(l[0].shape[0], n, -1).to(dev), gate_up)
+
+    w1, s1 = prepared(l1, 2 * inter, True)
+    w2, s2 = prepared(l2, hidden, False)
+    shared_weights = (*prepared(shared[0], 2 * inter, True), *prepared(shared[1], hidden, False)) if num_shared else None
+    ws = ops.Workspace(ops.megamoe_workspace_bytes(len(idx), idx.shape[1], hidden, inter, local, num_shared))
+    ws.tune("gemm_tile_rows", tile_rows)
+    ws.tune("gemm_zero_fill", 0)  # (a launch whose idle workgroups zero rows keeps the column-wave kernel)
+    y = torch.full((len(idx), hidden), float("nan"), dtype=torch.bfloat16, device=dev)
+    counts = torch.empty((local,), dtype=torch.int32, device=dev)
+    ops.megamoe_forward(ws, torch.from_numpy(x[0]).to(dev).view(torch.float8_e4m3fn), torch.from_numpy(x[1]).to(dev), torch.from_numpy(idx).to(dev),
+                        torch.from_numpy(weights).to(dev), w1, s1, w2, s2, local, 0, local, y, counts, shared=shared_weights, intermediate=inter)
+    torch.cuda.synchronize()
+    ws.destroy()
+    return y, counts.cpu().numpy()
+
+
+@pytest.mark.parametrize("hidden,inter,rows,num_shared", [
+    (64, 128, EDGES, 0),                # the smallest sizes: one k step in the first GEMM, one k tile in the second
+    (576, 384, EDGES, 0),               # k ends behind one step of a k tile; the first GEMM's fourth column tile is all padding
+    (1152, 1152, EDGES, 1),             # nine k tiles of ten: the last span holds one, its scale bytes sit two words up; a shared expert
+    (320, 640, EDGES[:8], 0),           # ten k tiles of 64 in the first GEMM, a last column tile with one live wave in the second
+    (2624, 1280, (40,) * 70, 0),        # 700 and 770 tiles for 512 workgroups
+    (512, 512, (2, 0, 700, 5), 2),      # experts of many and of few row tiles, every tile of exactly four items
+])
+def test_paired_kernel_at_its_edges(hidden, inter, rows, num_shared):
+    from deepep_amd import ops
+
+    rng = np.random.default_rng(hidden * 7 + inter)
+    local = len(rows)
+    idx = rng.permutation(np.repeat(np.arange(local, dtype=np.int32), rows))[:, None].copy()
+    x = mm.mx_quantize(rng.normal(size=(len(idx), hidden)).astype(np.float32))
+    weights = rng.random((len(idx), 1)).astype(np.float32)
+
+    def quantised(experts, n, k):  # (a few distinct matrices: quantising one takes the oracle a while)
+        few = mm.quantize_weight_mxfp4((rng.normal(size=(min(experts, 4), n, k)) * 0.02).astype(np.float32))
+        return tuple(np.ascontiguousarray(part[np.arange(experts) % len(part)]) for part in few)
+
+    l1, l2 = quantised(local, 2 * inter, hidden), quantised(local, hidden, inter)
+    shared = (quantised(num_shared, 2 * inter, hidden), quantised(num_shared, hidden, inter)) if num_shared else None
+    got, counts = _forward(ops, x, l1, l2, shared, idx, weights, hidden, inter, local, 128)
+    want, _ = _forward(ops, x, l1, l2, shared, idx, weights, hidden, inter, local, 32)
+    np.testing.assert_array_equal(counts, np.bincount(idx.ravel(), minlength=local))
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+    if len(idx) * hidden * inter < 2e9 and not num_shared:
+        oracle = mm.round_bf16(mm.local_reference(mm.mx_dequantize(*x), idx, weights, mm.unpack_weight(*l1), mm.unpack_weight(*l2), 0))
+        assert mm.relative_frobenius(got.float().cpu().numpy(), oracle) <= 2e-2
