@@ -223,9 +223,7 @@ struct GemmParams {
     int num_routed;            // experts >= num_routed are shared experts with weights of their own:
     const uint8_t* w_shared;   //   expert e reads w_shared / ws_shared at index e - num_routed
     const uint8_t* ws_shared;
-    int n, k;                  // padded sizes: the strides of the operands
-    int n_real, k_real;        // what is not padding of them (first GEMM: n counts gate and up)
-    int live_n_tiles;          // column tiles that the 128-row paired kernel works on (first GEMM: all, unless the second reads no padding)
+    int n, k;                  // padded sizes: the strides of the operands (what is not padding of them: n_real, k_real)
     uint8_t* act_codes;        // first GEMM: [rows, N/2] e4m3
     uint8_t* act_scales;       //             [rows, N/64] e8m0
     uint16_t* out;             // second GEMM: [rows, out_cols] bf16
@@ -249,6 +247,9 @@ struct GemmParams {
     int forced;                     // 64 / 128 / 192: that tile height whatever the cost model says (tests); 32: the few-rows kernel
                                     //   with (1, 4) << 8 waves per workgroup; 0: the model decides
     int column_waves;               // 1: the kernel whose waves split the tile's columns and load their weights straight into registers
+    int n_real, k_real;             // what is not padding of n and k (first GEMM: n counts gate and up)
+    int live_n_tiles;               // column tiles that the kernels that skip padding work on (first GEMM: all, unless the second reads none of it)
+    int numbered_n_tiles;           // few-rows kernels: column tiles that a row tile's numbers are given to, those behind live_n_tiles in vain
 };
 
 // gate / (1 + exp(-gate)) * up with the hardware exponential and reciprocal (v_exp_f32, v_rcp_f32: about 1 ulp each; the
@@ -1049,6 +1050,48 @@ __device__ __forceinline__ void store_output(const GemmParams& p, const v16f& ac
     }
 }
 
+// The 32-row tiles of the few-rows kernels.  They are numbered through the experts, so that the grid does not depend on how the
+// routes fell; every wave works the numbering out for itself (a lane has experts lane and lane + 64).
+struct FewRowsTiles {
+    static constexpr int kRows = 32;
+    int through[2], first_row[2], rows[2];
+    int total;
+    __device__ __forceinline__ FewRowsTiles(const GemmParams& p, int lane)
+    {
+        static_assert(kMaxMoeExperts <= 128, "two experts per lane");
+        total = 0;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const int e = lane + 64 * h;
+            through[h] = first_row[h] = rows[h] = 0;
+            if (64 * h >= p.num_local) continue;
+            if (e < p.num_local) {
+                first_row[h] = p.offsets[e];
+                rows[h] = p.offsets[e + 1] - first_row[h];
+            }
+            through[h] = total + wave_scan((rows[h] + kRows - 1) / kRows);
+            total = __builtin_amdgcn_readlane(through[h], 63);
+        }
+    }
+    // Expert, first row and number of rows of row tile `unit` (below the total), from the lane that has the expert: its offsets asked
+    // for again were a memory trip in front of everything else.
+    __device__ __forceinline__ void find(const GemmParams& p, int unit, int& expert, int& row0, int& valid) const
+    {
+        expert = __popcll(__ballot(through[0] <= unit));  // experts that end at or before this row tile
+        int before = 0;
+        if (expert == 64) {
+            expert += __popcll(__ballot(through[1] <= unit));
+            before = expert == 64 ? __builtin_amdgcn_readlane(through[0], 63) : __builtin_amdgcn_readlane(through[1], expert - 65);
+        } else if (expert > 0) {
+            before = __builtin_amdgcn_readlane(through[0], expert - 1);
+        }
+        expert = min(expert, p.num_local - 1);
+        const int in_expert = (unit - before) * kRows;
+        row0 = (expert < 64 ? __builtin_amdgcn_readlane(first_row[0], expert) : __builtin_amdgcn_readlane(first_row[1], expert - 64)) + in_expert;
+        valid = min(kRows, (expert < 64 ? __builtin_amdgcn_readlane(rows[0], expert) : __builtin_amdgcn_readlane(rows[1], expert - 64)) - in_expert);
+    }
+};
+
 // =====================================================================================================
 // Grouped GEMM for few rows per expert
 // =====================================================================================================
@@ -1065,6 +1108,7 @@ __device__ __forceinline__ void store_output(const GemmParams& p, const v16f& ac
 // included).  Whole forward: 0.5 rows per expert 92 -> 62 us, 2: 134 -> 106, 8: 144 -> 130, 16: 153 -> 137.
 // (Tried and not kept: eight k tiles ahead at one workgroup per CU, 143 us; 64-row tiles, 154 us.)
 // kWaves = 1 spreads a column tile over four workgroups of one wave each, for launches that would leave CUs idle (below).
+// k tiles and column tiles of nothing but padding are left out.
 typedef u32x4 u32x4_unaligned __attribute__((aligned(4)));
 template <int kWaves, bool kGateUp>
 __global__ __launch_bounds__(64 * kWaves, 2) void grouped_gemm_few_rows_kernel(GemmParams p)
@@ -1075,44 +1119,36 @@ __global__ __launch_bounds__(64 * kWaves, 2) void grouped_gemm_few_rows_kernel(G
     const int lane = threadIdx.x & 63, g = lane >> 5, lr = lane & 31;
     const int my_wave = kWaves == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     constexpr int kSplit = kGemmWaves / kWaves;  // workgroups per column tile
-    const int n_tiles = p.n / kBN, ktiles = p.k / kBK, spans = (ktiles + 3) / 4, scale_bytes = p.k / 32;
+    const int n_tiles = p.n / kBN, stored_ktiles = p.k / kBK, stored_spans = (stored_ktiles + 3) / 4, scale_bytes = p.k / 32;
+    // (k tiles and column tiles of nothing but padding are left out)
+    const int ktiles = (p.k_real + kBK - 1) / kBK, spans = (ktiles + 3) / 4, numbered_n_tiles = p.numbered_n_tiles;
     if (blockIdx.x == 0 && threadIdx.x == 0 && p.fill_state != nullptr) p.fill_state[0] = 0;
 
-    // Row tiles are numbered through the experts, so that the grid does not depend on how the routes fell; every wave works
-    // the numbering out for itself (a lane has experts lane and lane + 64).
-    static_assert(kMaxMoeExperts <= 128, "two experts per lane");
-    int tiles_through[2];
-    int total = 0;
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-        const int e = lane + 64 * h;
-        tiles_through[h] = 0;
-        if (64 * h >= p.num_local) continue;
-        const int sum = e < p.num_local ? (p.offsets[e + 1] - p.offsets[e] + kRows - 1) / kRows : 0;
-        tiles_through[h] = total + wave_scan(sum);
-        total = __builtin_amdgcn_readlane(tiles_through[h], 63);
-    }
-
-    for (int tile_id = blockIdx.x; tile_id < total * n_tiles * kSplit; tile_id += gridDim.x) {
-        const int unit = tile_id / (n_tiles * kSplit), piece = tile_id - unit * (n_tiles * kSplit);
+    const FewRowsTiles tiles(p, lane);
+    for (int tile_id = blockIdx.x; tile_id < tiles.total * numbered_n_tiles * kSplit; tile_id += gridDim.x) {
+        const int unit = tile_id / (numbered_n_tiles * kSplit), piece = tile_id - unit * (numbered_n_tiles * kSplit);
         const int nt = piece / kSplit, wave = kWaves == 1 ? piece % kSplit : my_wave;  // the column tile, the quarter of it
-        int expert = __popcll(__ballot(tiles_through[0] <= unit));  // experts that end at or before this row tile
-        int before = 0;
-        if (expert == 64) {
-            expert += __popcll(__ballot(tiles_through[1] <= unit));
-            before = expert == 64 ? __builtin_amdgcn_readlane(tiles_through[0], 63) : __builtin_amdgcn_readlane(tiles_through[1], expert - 65);
-        } else if (expert > 0) {
-            before = __builtin_amdgcn_readlane(tiles_through[0], expert - 1);
-        }
-        expert = min(expert, p.num_local - 1);
-        const int row0 = p.offsets[expert] + (unit - before) * kRows;
-        const int valid = min(kRows, p.offsets[expert + 1] - row0);
+        if (nt >= p.live_n_tiles) continue;
+        int expert, row0, valid;
+        tiles.find(p, unit, expert, row0, valid);
         const bool shared = expert >= p.num_routed;
         const size_t weight_index = shared ? expert - p.num_routed : expert;
-        const uint8_t* const w = (shared ? p.w_shared : p.w) + weight_index * p.n * (p.k / 2) + static_cast<size_t>(nt) * ktiles * 16384 +
+        const uint8_t* const w = (shared ? p.w_shared : p.w) + weight_index * p.n * (p.k / 2) + static_cast<size_t>(nt) * stored_ktiles * 16384 +
                                  wave * 4096 + lane * 16;
-        const uint8_t* const ws = (shared ? p.ws_shared : p.ws) + (weight_index * n_tiles + nt) * spans * 4096 + wave * 1024 + lane * 8;
+        const uint8_t* const ws = (shared ? p.ws_shared : p.ws) + (weight_index * n_tiles + nt) * stored_spans * 4096 + wave * 1024 + lane * 8;
 
+        v16f acc[2];
+#pragma unroll
+        for (int c = 0; c < 2; ++c)
+#pragma unroll
+            for (int j = 0; j < 16; ++j) acc[c][j] = 0.0f;
+        // (clamped: a map left incomplete by a layout launch that ran out of time must not become a wild address)
+        const uint8_t* const codes = kGather ? p.a_codes : p.a_codes + static_cast<size_t>(row0) * p.k;
+        const uint8_t* const row_scale_bytes = kGather ? p.a_scales : p.a_scales + static_cast<size_t>(row0) * scale_bytes;
+        auto source = [&](int r) {
+            r = min(r, valid - 1);
+            return static_cast<uint32_t>(kGather ? min(max(p.row_to_route[row0 + r] / p.topk, 0), p.a_rows - 1) : r);
+        };
         u32x4 wreg[4][4];  // [k tile of the span][column tile * 2 + k step]
         auto load_weights = [&](int slot, int kt) {
             const uint8_t* at = w + static_cast<size_t>(min(kt, ktiles - 1)) * 16384;  // (past the end: the last k tile again, never used)
@@ -1121,13 +1157,6 @@ __global__ __launch_bounds__(64 * kWaves, 2) void grouped_gemm_few_rows_kernel(G
         };
         // Activations: wave q fetches k tile q of a span for the whole workgroup.  Copy f: lane l asks for 16-byte chunk l % 8 of
         // row 8 f + l / 8, so that eight lanes read a row's 128 bytes.  Rows past the end repeat the last one.
-        // (clamped: a map left incomplete by a layout launch that ran out of time must not become a wild address)
-        const uint8_t* const codes = kGather ? p.a_codes : p.a_codes + static_cast<size_t>(row0) * p.k;
-        const uint8_t* const row_scale_bytes = kGather ? p.a_scales : p.a_scales + static_cast<size_t>(row0) * scale_bytes;
-        auto source = [&](int r) {
-            r = min(r, valid - 1);
-            return static_cast<uint32_t>(kGather ? min(max(p.row_to_route[row0 + r] / p.topk, 0), p.a_rows - 1) : r);
-        };
         uint32_t a_from[4];
 #pragma unroll
         for (int f = 0; f < 4; ++f) a_from[f] = source(8 * f + (lane >> 3)) * static_cast<uint32_t>(p.k) + (lane & 7) * 16;
@@ -1158,11 +1187,6 @@ __global__ __launch_bounds__(64 * kWaves, 2) void grouped_gemm_few_rows_kernel(G
             for (int c = 0; c < 2; ++c)
                 col_scales[parity][c] = *reinterpret_cast<const u32x2*>(ws + static_cast<size_t>(span) * 4096 + c * 512);
         };
-        v16f acc[2];
-#pragma unroll
-        for (int c = 0; c < 2; ++c)
-#pragma unroll
-            for (int j = 0; j < 16; ++j) acc[c][j] = 0.0f;
         load_activations(0);
         load_scales(0, 0);
         __builtin_amdgcn_sched_barrier(0);
@@ -1180,8 +1204,8 @@ __global__ __launch_bounds__(64 * kWaves, 2) void grouped_gemm_few_rows_kernel(G
             const bool shifted_window = span * 16 > scale_bytes - 16;  // (k % 512 = 256: the last span's bytes sit two words up)
             static_for<4>([&](auto q_constant) {
                 constexpr int q = decltype(q_constant)::value;
-                if (q < 2 || kMore || span * 4 + q < ktiles) {  // (k tiles come in twos)
-                    const uint32_t word = q < 2 && !kMore && shifted_window ? row_scales[kParity][q + 2] : row_scales[kParity][q];
+                if (q == 0 || kMore || span * 4 + q < ktiles) {
+                    const uint32_t word = q < 2 && !kMore && shifted_window ? row_scales[kParity][(q + 2) & 3] : row_scales[kParity][q];
                     const int x_scale = static_cast<int>(word >> (8 * g));
                     const uint8_t* const tile = &lds[kParity][q][lr * kBK];
                     static_for<2>([&](auto step_constant) {
@@ -1197,7 +1221,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void grouped_gemm_few_rows_kernel(G
                                                                                      static_cast<int>(col_scales[kParity][c][q >> 1]), 2 * step, x_scale);
                         }
                     });
-                    if constexpr (q > 0 && (q == 3 || !kMore)) settle_accumulators(acc);
+                    if constexpr (q == 3 || !kMore) settle_accumulators(acc);
                 }
                 if constexpr (kMore) load_weights(q, (span + 1) * 4 + q);
                 __builtin_amdgcn_sched_barrier(0);
@@ -1229,6 +1253,162 @@ __global__ __launch_bounds__(64 * kWaves, 2) void grouped_gemm_few_rows_kernel(G
         }
         // the next tile of this workgroup writes the LDS again
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        const bool row_exists = lr < valid;
+        const size_t row = static_cast<size_t>(row0) + lr;
+        if (kGateUp) {
+            store_gate_up(p, acc[0], acc[1], row, row_exists, (nt * (kBN / 64) + wave) * 32, g);
+        } else {
+#pragma unroll
+            for (int c = 0; c < 2; ++c) store_output(p, acc[c], row, row_exists, nt * kBN + (wave * 2 + c) * 32, g);
+        }
+    }
+}
+
+// The same with one wave per workgroup and no LDS, for launches that leave most SIMDs idle or whose tiles hold few rows.  Such a wave has
+// its SIMD to itself (up to 512 registers): activations go straight to registers as well, in the layout that the MFMA takes,
+// eight k tiles of everything are in flight, and no LDS, barrier or wait for either stands between the MFMAs, which then bound
+// the loop (0.13 us a k tile).  First GEMM, us: 40 tokens over 5 experts of 4032 x 640 12.9 -> 10.0, 2 x top-5 over 44 of 4864 x 1152
+// 18.9 -> 14.4, 1 x top-7 over 18 + 2 of 1216 x 1536 8.7 -> 7.3.  An activation load then touches one line per row instead of eight
+// rows' lines: with full tiles and several waves to a CU that is what bounds it (66 rows for each of 6 experts of 1280 x 1536 9.9 -> 12.1).
+template <bool kGateUp>
+__global__ __launch_bounds__(64, 1) void grouped_gemm_one_wave_kernel(GemmParams p)
+{
+    constexpr bool kGather = kGateUp;
+    const int lane = threadIdx.x, g = lane >> 5, lr = lane & 31;
+    constexpr int kSplit = kGemmWaves;  // workgroups per column tile
+    const int n_tiles = p.n / kBN, stored_ktiles = p.k / kBK, stored_spans = (stored_ktiles + 3) / 4, scale_bytes = p.k / 32;
+    // (k tiles and column tiles of nothing but padding are left out)
+    const int ktiles = (p.k_real + kBK - 1) / kBK, spans = (ktiles + 3) / 4, numbered_n_tiles = p.numbered_n_tiles;
+    if (blockIdx.x == 0 && threadIdx.x == 0 && p.fill_state != nullptr) p.fill_state[0] = 0;
+
+    const FewRowsTiles tiles(p, lane);
+    for (int tile_id = blockIdx.x; tile_id < tiles.total * numbered_n_tiles * kSplit; tile_id += gridDim.x) {
+        const int unit = tile_id / (numbered_n_tiles * kSplit), piece = tile_id - unit * (numbered_n_tiles * kSplit);
+        const int nt = piece / kSplit, wave = piece % kSplit;  // the column tile, the quarter of it
+        if (nt >= p.live_n_tiles) continue;
+        int expert, row0, valid;
+        tiles.find(p, unit, expert, row0, valid);
+        const bool shared = expert >= p.num_routed;
+        const size_t weight_index = shared ? expert - p.num_routed : expert;
+        const uint8_t* const w = (shared ? p.w_shared : p.w) + weight_index * p.n * (p.k / 2) + static_cast<size_t>(nt) * stored_ktiles * 16384 +
+                                 wave * 4096 + lane * 16;
+        const uint8_t* const ws = (shared ? p.ws_shared : p.ws) + (weight_index * n_tiles + nt) * stored_spans * 4096 + wave * 1024 + lane * 8;
+
+        v16f acc[2];
+#pragma unroll
+        for (int c = 0; c < 2; ++c)
+#pragma unroll
+            for (int j = 0; j < 16; ++j) acc[c][j] = 0.0f;
+        // (clamped: a map left incomplete by a layout launch that ran out of time must not become a wild address)
+        const uint8_t* const codes = kGather ? p.a_codes : p.a_codes + static_cast<size_t>(row0) * p.k;
+        const uint8_t* const row_scale_bytes = kGather ? p.a_scales : p.a_scales + static_cast<size_t>(row0) * scale_bytes;
+        // In the layout that the MFMA takes: lane l has row l % 32, two pieces of 16 bytes per k step.
+        constexpr int kSlots = 8;
+        u32x4 wreg[kSlots][4], areg[kSlots][4];  // [k tile % 8][column tile * 2 + k step], [k step * 2 + piece]
+        // The row's route is asked for first and the first weights behind it: they travel together.
+        const int my_row = min(lr, valid - 1);
+        const int route = kGather ? p.row_to_route[row0 + my_row] : 0;
+        __builtin_amdgcn_sched_barrier(0);
+        auto load_weights = [&](int slot, int kt) {
+            const uint8_t* const from = w + static_cast<size_t>(min(kt, ktiles - 1)) * 16384;  // (past the end: the last k tile again, never used)
+#pragma unroll
+            for (int f = 0; f < 4; ++f) wreg[slot][f] = load16_nt(from + f * 1024);
+        };
+        u32x4 row_scales[2];
+        u32x2 col_scales[2][2];  // [span parity][column tile]
+        auto load_col_scales = [&](int parity, int span) {
+            span = min(span, spans - 1);
+#pragma unroll
+            for (int c = 0; c < 2; ++c)
+                col_scales[parity][c] = *reinterpret_cast<const u32x2*>(ws + static_cast<size_t>(span) * 4096 + c * 512);
+        };
+        load_col_scales(0, 0);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) load_weights(q, q);
+        __builtin_amdgcn_sched_barrier(0);
+        const uint32_t from_row = static_cast<uint32_t>(kGather ? min(max(route / p.topk, 0), p.a_rows - 1) : my_row);
+        const uint8_t* const my_codes = codes + from_row * static_cast<uint32_t>(p.k) + g * 16;
+        const uint8_t* const my_scales = row_scale_bytes + from_row * static_cast<uint32_t>(scale_bytes);
+        auto load_activations = [&](int slot, int kt) {
+            const uint8_t* const row = my_codes + static_cast<size_t>(min(kt, ktiles - 1)) * kBK;
+#pragma unroll
+            for (int f = 0; f < 4; ++f) areg[slot][f] = load16(row + f * 32);
+        };
+        auto load_row_scales = [&](int parity, int span) {
+            row_scales[parity] = *reinterpret_cast<const u32x4_unaligned*>(my_scales + min(min(span, spans - 1) * 16, scale_bytes - 16));
+        };
+        load_row_scales(0, 0);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) load_activations(q, q);
+        __builtin_amdgcn_sched_barrier(0);
+        load_col_scales(1, 1);
+        load_row_scales(1, 1);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int q = 4; q < 8; ++q) {
+            load_weights(q, q);
+            load_activations(q, q);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        auto span_body = [&](auto parity_constant, auto ask_constant, auto whole_constant, int span) {
+            constexpr int kParity = decltype(parity_constant)::value;
+            constexpr bool kAsk = decltype(ask_constant)::value;      // the span after the next one exists
+            constexpr bool kWhole = decltype(whole_constant)::value;  // another span follows, so all four k tiles of this one are there
+            u32x4 rows_now = row_scales[kParity];
+            u32x2 cols_now[2] = {col_scales[kParity][0], col_scales[kParity][1]};
+            // (moved out of the way: the next scales of this parity are asked for in front of the weights that they go with)
+            asm volatile("" : "+v"(rows_now), "+v"(cols_now[0]), "+v"(cols_now[1]));
+            if constexpr (kAsk) {
+                load_col_scales(kParity, span + 2);
+                load_row_scales(kParity, span + 2);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            const bool shifted_window = span * 16 > scale_bytes - 16;  // (k % 512 = 256: the last span's bytes sit two words up)
+            static_for<4>([&](auto q_constant) {
+                constexpr int q = decltype(q_constant)::value, kSlot = 4 * kParity + q;
+                if (q == 0 || kWhole || span * 4 + q < ktiles) {
+                    const uint32_t word = q < 2 && !kWhole && shifted_window ? rows_now[(q + 2) & 3] : rows_now[q];
+                    const int x_scale = static_cast<int>(word >> (8 * g));
+                    static_for<2>([&](auto step_constant) {
+                        constexpr int step = decltype(step_constant)::value;
+                        const u32x4 lo = areg[kSlot][2 * step], hi = areg[kSlot][2 * step + 1];
+                        const v8i x = {(int)lo[0], (int)lo[1], (int)lo[2], (int)lo[3], (int)hi[0], (int)hi[1], (int)hi[2], (int)hi[3]};
+#pragma unroll
+                        for (int c = 0; c < 2; ++c) {
+                            const u32x4 f = wreg[kSlot][2 * c + step];
+                            const v8i m = {(int)f[0], (int)f[1], (int)f[2], (int)f[3], 0, 0, 0, 0};
+                            acc[c] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(m, x, acc[c], 4, 0, 2 * (q & 1) + step,
+                                                                                     static_cast<int>(cols_now[c][q >> 1]), 2 * step, x_scale);
+                        }
+                    });
+                    if constexpr (q == 3 || !kWhole) asm volatile("s_nop 15\n\ts_nop 7" : "+a"(acc[0]), "+a"(acc[1]));  // (settle_accumulators, where they are)
+                }
+                if constexpr (kAsk) {
+                    load_weights(kSlot, span * 4 + q + 8);
+                    load_activations(kSlot, span * 4 + q + 8);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            });
+        };
+        constexpr std::integral_constant<int, 0> even{};
+        constexpr std::integral_constant<int, 1> odd{};
+        constexpr std::integral_constant<bool, true> yes{};
+        constexpr std::integral_constant<bool, false> no{};
+        int span = 0;
+        for (; span + 3 < spans; span += 2) {
+            span_body(even, yes, yes, span);
+            span_body(odd, yes, yes, span + 1);
+        }
+        if (spans - span == 3) {
+            span_body(even, yes, yes, span);
+            span_body(odd, no, yes, span + 1);
+            span_body(even, no, no, span + 2);
+        } else if (spans - span == 2) {
+            span_body(even, no, yes, span);
+            span_body(odd, no, no, span + 1);
+        } else {
+            span_body(even, no, no, span);
+        }
         const bool row_exists = lr < valid;
         const size_t row = static_cast<size_t>(row0) + lr;
         if (kGateUp) {
@@ -2135,6 +2315,8 @@ struct GemmChoice {
     int waves;     // per workgroup (4 but for the few-rows kernel's small launches)
     double tiles;  // expected, of that height
     bool paired, streamed;  // 128 rows: the kernel with two workgroups to a CU; its weights past the caches
+    bool direct;            // 32 rows, one wave: the kernel without LDS
+    double row_tiles_per_expert;  // 32 rows: of the experts that have any
 };
 template <bool kGateUp>
 GemmChoice choose_gemm(const GemmParams& p, const ExpectedRows& expected, int cus)
@@ -2157,10 +2339,12 @@ GemmChoice choose_gemm(const GemmParams& p, const ExpectedRows& expected, int cu
     // Nothing ends before the weights are read; where that decides, the one that would be done first otherwise is still better.
     auto bounded = [&](double t) { return std::max(2.0 + weight_bytes / 6.3e6, t) + 0.05 * t; };
     const int kind = p.column_waves && p.k % 512 == 0 ? 0 : 1;  // the kernel that launch_gemm_rt takes: column waves, 2 x 2
+    double paired_row_tiles = 0.0;
     int best = 2;
     double best_cost = 1e30, tiles_of[4] = {0.0, 0.0, 0.0, 0.0};
     for (int rt = 1; rt <= 3; ++rt) {
         const double row_tiles = expected_row_tiles(64 * rt);
+        if (rt == 2) paired_row_tiles = row_tiles;
         const double tiles = row_tiles * n_tiles;
         tiles_of[rt] = tiles;
         const bool in_pairs = rt == 1 && kind == 0 && two_workgroups_pay(tiles, cus);
@@ -2179,13 +2363,12 @@ GemmChoice choose_gemm(const GemmParams& p, const ExpectedRows& expected, int cu
     // few row tiles share.  It counts only what is not padding.  Fitted to kernel traces of both GEMMs at 240 shapes (8 to 10 000 rows for
     // each of 2 to 64 experts), three sets of inputs in turn: 7 % off on average; with it among the candidates the chosen kernels
     // are 5.6 % faster on average (1.2 % slower than the best ones, 6.8 % without it).
-    double paired = 1e30, paired_row_tiles = 0.0;
+    double paired = 1e30;
     bool streamed = false;
-    const double experts_with_rows = p.num_routed * routed_with_rows + num_shared;
+    const double experts_with_rows = p.num_routed * routed_with_rows + num_shared, live_row_tiles = expected_row_tiles(32);
     if (p.column_waves) {
         const int steps = (p.k_real + 63) / 64, items = ((steps - 1) / 2 + 4) / 4 * 4, slots = 2 * cus;
-        paired_row_tiles = expected_row_tiles(128);
-        const double live_row_tiles = expected_row_tiles(32), live = live_row_tiles / std::max(paired_row_tiles, 1e-3);
+        const double live = live_row_tiles / std::max(paired_row_tiles, 1e-3);
         const double share = experts_with_rows / std::max(paired_row_tiles, 1e-3);
         const double tiles = paired_row_tiles * p.live_n_tiles, full = floor(std::max(0.0, tiles / slots - 0.01)), rest = (tiles - full * slots) / cus;
         const double pair = 5.0 + items * (0.652 + 0.147 * live + 0.269 * share), single = 3.37 + items * (0.236 + 0.112 * live + 0.135 * share);
@@ -2196,21 +2379,28 @@ GemmChoice choose_gemm(const GemmParams& p, const ExpectedRows& expected, int cu
         // (8192 x top-8 over 32 experts of 7168 x 2048: first GEMM 1343 us against 1375, second 803 against 840).
         const double tall_work = tiles_of[3] * 6.0 * ktiles * 2.0, live_work = live_row_tiles * p.live_n_tiles * steps;
         const bool power_limited = kind == 0 && best == 3 && full >= 8.0 && tall_work < 1.06 * live_work;
-        if (!power_limited) paired = std::max(2.0 + live_bytes / 5.32e6, t) + 0.05 * t;
+        // (the factor: a kernel as good by the model is the safer choice. It halves the launches that get slower, 28 of 920, at the same mean)
+        if (!power_limited) paired = 1.05 * (std::max(2.0 + live_bytes / 5.32e6, t) + 0.05 * t);
         // Weights that the memory-side cache does not hold, each read by about one row tile: past the caches.
         streamed = live_bytes > 256e6 && paired_row_tiles < 1.3 * experts_with_rows;
     }
-    const GemmChoice pair_choice = {128, kGemmWaves, paired_row_tiles * p.live_n_tiles, true, streamed};
+    const GemmChoice pair_choice = {128, kGemmWaves, paired_row_tiles * p.live_n_tiles, true, streamed, false, 0.0};
     // A share with more than one 64-row tile per expert has so many tokens without a row that its first GEMM's idle workgroups are
     // better used for their zero rows: kernels that do not fill are no candidates there.
     const bool fills = p.fill_tokens > 0 && tiles_of[best] < cus;
     const bool unfilled_allowed = !fills || mean <= 64.0;
     // Source rows are addressed with 32 bits in the few-rows kernel.
-    const double tiles = expected_row_tiles(32) * n_tiles;
+    const double tiles = live_row_tiles * p.live_n_tiles, row_tiles_per_expert = live_row_tiles / std::max(experts_with_rows, 1e-3);
+    // One-wave workgroups without LDS while there is at most one to a CU (16 % faster than with it over 167 launches, a tenth where tiles are
+    // full), or two with about half a dozen rows per tile (4 % over 67); with more of either they are 1 to 20 % slower.
+    const double waves = kGemmWaves * tiles, rows_per_tile = (p.num_routed * mean + static_cast<double>(num_shared) * expected.shared) * p.live_n_tiles / std::max(tiles, 1e-3);
+    const bool direct = waves <= cus || (waves <= 2.0 * cus && rows_per_tile <= 6.0);
     if (p.column_waves && p.forced == 0) {
+        // (by the padded sizes, as fitted: by the real ones these kernels look too good where little of a tile is real)
+        const double all_tiles = live_row_tiles * n_tiles;
         const bool few_allowed = (p.fill_tokens == 0 || mean <= 64.0) && (!kGateUp || static_cast<long long>(p.a_rows) * p.k < (1LL << 32));
-        const double one = few_allowed ? bounded(3.0 + 0.30 * ktiles + (rounds_of(kGemmWaves * tiles, cus) - 1.0) * (1.1 + 0.17 * ktiles)) : 1e30;
-        const double four = few_allowed ? bounded(1.5 + rounds_of(tiles, cus) * (2.7 + 0.50 * ktiles)) : 1e30;
+        const double one = few_allowed ? bounded(3.0 + 0.30 * ktiles + (rounds_of(kGemmWaves * all_tiles, cus) - 1.0) * (1.1 + 0.17 * ktiles)) : 1e30;
+        const double four = few_allowed ? bounded(1.5 + rounds_of(all_tiles, cus) * (2.7 + 0.50 * ktiles)) : 1e30;
         // Zero rows of the output that this launch's idle workgroups would have written (at about 30 GB/s each): these two
         // kernels leave them to the reduce, which writes them at 8 TB/s, and the GEMM is faster without the company: 4300 zero
         // rows of 5120 columns beside 31 experts of 5120 x 512 cost the forward 57 us filled and 49 not.
@@ -2221,12 +2411,12 @@ GemmChoice choose_gemm(const GemmParams& p, const ExpectedRows& expected, int cu
         }
         const double few = std::min(one, four);
         if (unfilled_allowed && paired < few && paired + unfilled < best_cost) return pair_choice;
-        if (few + unfilled < best_cost) return {32, one < four ? 1 : kGemmWaves, tiles, false, false};
+        if (few + unfilled < best_cost) return {32, one < four ? 1 : kGemmWaves, tiles, false, false, one < four && direct, row_tiles_per_expert};
     }
-    if ((p.forced & 0xff) == 32) return {32, p.forced >> 8, tiles, false, false};
+    if ((p.forced & 0xff) == 32) return {32, p.forced >> 8, tiles, false, false, (p.forced >> 8) == 1 && direct, row_tiles_per_expert};
     if (p.forced == 128 && p.column_waves && (p.fill_tokens == 0 || tiles_of[2] >= cus)) return pair_choice;
     if (p.forced != 0) best = p.forced / 64;
-    return {64 * best, kGemmWaves, tiles_of[best], false, false};
+    return {64 * best, kGemmWaves, tiles_of[best], false, false, false, 0.0};
 }
 
 template <bool kGateUp>
@@ -2239,11 +2429,18 @@ int launch_gemm(const GemmParams& p, const GemmChoice& choice, const ExpectedRow
         const long long row_tiles =
             static_cast<long long>(p.num_routed) * static_cast<long long>(ceil(std::max(1.0, expected.routed + 3.0 * expected.spread) / 32.0)) +
             static_cast<long long>(num_shared) * ((expected.shared + 31) / 32);
-        const unsigned grid = static_cast<unsigned>(row_tiles * (p.n / kBN));
-        if (choice.waves == 1)
-            hipLaunchKernelGGL((grouped_gemm_few_rows_kernel<1, kGateUp>), dim3(kGemmWaves * grid), dim3(64), 0, stream, p);
+        // One-wave workgroups whose expert has several row tiles: an even number of column tiles, so that a quarter of a column tile
+        // lands on the same XCD for every row tile (workgroups are dealt round-robin over the 8) and its weights are in that XCD's
+        // L2 (38 rows for each of 5 experts of 3904 x 1152, nine column tiles: 29.3 us, numbered as ten 27.8).
+        GemmParams numbered = p;
+        numbered.numbered_n_tiles = p.live_n_tiles + (choice.waves == 1 && choice.row_tiles_per_expert > 1.25 ? p.live_n_tiles & 1 : 0);
+        const unsigned grid = static_cast<unsigned>(row_tiles * numbered.numbered_n_tiles);
+        if (choice.direct)
+            hipLaunchKernelGGL(grouped_gemm_one_wave_kernel<kGateUp>, dim3(kGemmWaves * grid), dim3(64), 0, stream, numbered);
+        else if (choice.waves == 1)
+            hipLaunchKernelGGL((grouped_gemm_few_rows_kernel<1, kGateUp>), dim3(kGemmWaves * grid), dim3(64), 0, stream, numbered);
         else
-            hipLaunchKernelGGL((grouped_gemm_few_rows_kernel<kGemmWaves, kGateUp>), dim3(grid), dim3(kGemmThreads), 0, stream, p);
+            hipLaunchKernelGGL((grouped_gemm_few_rows_kernel<kGemmWaves, kGateUp>), dim3(grid), dim3(kGemmThreads), 0, stream, numbered);
         return launch_status(what);
     }
     if (choice.paired) return choice.streamed ? launch_paired<true, kGateUp>(p, stream, what) : launch_paired<false, kGateUp>(p, stream, what);
@@ -2288,8 +2485,8 @@ ExpectedRows expected_rows_of(const MegaSizes& m)
     const double routed = static_cast<double>(m.num_tokens) * m.num_topk / m.num_experts;
     return {routed, sqrt(routed * std::max(0.0, 1.0 - static_cast<double>(m.num_topk) / m.num_experts)) + 1e-3, m.num_tokens};
 }
-// Kernels of both GEMMs.  The second one first: the paired kernel reads no padding of the activations, so that the first GEMM, if it
-// is that kernel too, leaves out the column tiles that would only write some.
+// Kernels of both GEMMs.  The second one first: the paired and the few-rows kernel read no padding of the activations, so that the first
+// GEMM, if it is one of these too, leaves out the column tiles that would only write some.
 struct GemmChoices {
     GemmChoice first, second;
 };
@@ -2298,7 +2495,7 @@ GemmChoices choose_gemms(const MegaSizes& m, GemmParams& g1, const GemmParams& g
     const ExpectedRows expected = expected_rows_of(m);
     GemmChoices c;
     c.second = choose_gemm<false>(g2, expected, gemm_grid());
-    if (c.second.paired) g1.live_n_tiles = (g1.n_real + kBN - 1) / kBN;
+    if (c.second.paired || c.second.rows == 32) g1.live_n_tiles = (g1.n_real + kBN - 1) / kBN;
     c.first = choose_gemm<true>(g1, expected, gemm_grid());
     return c;
 }

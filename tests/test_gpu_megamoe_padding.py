@@ -1,4 +1,4 @@
-"""The 128-row grouped GEMM with two workgroups to a CU, at the sizes where it can go wrong: row counts on both sides of its 32-row
+"""The grouped GEMMs that leave out padding.  The 128-row one with two workgroups to a CU, at the sizes where it can go wrong: row counts on both sides of its 32-row
 tiles, k that ends inside a span of four k tiles, inside a k tile and behind one MFMA step, column tiles and waves of nothing but
 padding, more tiles than workgroups.  A k sum is taken in the same order as in the few-rows kernel, so the two give the same bits; both
 against the fp32 oracle within the path's 2e-2."""
@@ -14,7 +14,7 @@ pytestmark = pytest.mark.gpu
 EDGES = (1, 31, 32, 33, 0, 64, 65, 96, 97, 127, 128, 129, 160, 256, 257)
 
 
-def _forward(ops, x, l1, l2, shared, idx, weights, hidden, inter, local, tile_rows):
+def _forward(ops, x, l1, l2, shared, idx, weights, hidden, inter, local, tile_rows, few_rows_waves=4):
     dev = "cuda"
     num_shared = 0 if shared is None else shared[0][0].shape[0]
 
@@ -26,6 +26,7 @@ def _forward(ops, x, l1, l2, shared, idx, weights, hidden, inter, local, tile_ro
     shared_weights = (*prepared(shared[0], 2 * inter, True), *prepared(shared[1], hidden, False)) if num_shared else None
     ws = ops.Workspace(ops.megamoe_workspace_bytes(len(idx), idx.shape[1], hidden, inter, local, num_shared))
     ws.tune("gemm_tile_rows", tile_rows)
+    ws.tune("gemm_few_rows_waves", few_rows_waves)
     ws.tune("gemm_zero_fill", 0)  # (a launch whose idle workgroups zero rows keeps the column-wave kernel)
     y = torch.full((len(idx), hidden), float("nan"), dtype=torch.bfloat16, device=dev)
     counts = torch.empty((local,), dtype=torch.int32, device=dev)
@@ -66,3 +67,32 @@ def test_paired_kernel_at_its_edges(hidden, inter, rows, num_shared):
     if len(idx) * hidden * inter < 2e9 and not num_shared:
         oracle = mm.round_bf16(mm.local_reference(mm.mx_dequantize(*x), idx, weights, mm.unpack_weight(*l1), mm.unpack_weight(*l2), 0))
         assert mm.relative_frobenius(got.float().cpu().numpy(), oracle) <= 2e-2
+
+
+@pytest.mark.parametrize("hidden,inter,rows", [
+    (64, 128, (3, 1)),           # one k tile in both GEMMs
+    (960, 640, (5, 0, 2)),       # eight k tiles, the last half padding; five
+    (1664, 1152, (33, 1, 32)),   # 13 and nine: four and three spans of four
+    (2368, 3200, (5, 0, 33)),    # 19 and 25: five and seven spans
+    (2624, 2176, (1,) * 66),     # more experts than a wave has lanes
+])
+def test_few_rows_kernels_at_their_edges(hidden, inter, rows):
+    """k tiles of every number behind the last whole span, and a span loop of none, one and several rounds: one-wave workgroups (without
+    LDS where the launch is small) and four-wave ones against the 64-row kernel, bit for bit."""
+    from deepep_amd import ops
+
+    rng = np.random.default_rng(hidden)
+    local = len(rows)
+    idx = rng.permutation(np.repeat(np.arange(local, dtype=np.int32), rows))[:, None].copy()
+    x = mm.mx_quantize(rng.normal(size=(len(idx), hidden)).astype(np.float32))
+    weights = rng.random((len(idx), 1)).astype(np.float32)
+
+    def random_weights(n, k):  # (codes and scale bytes of any matrix will do: the kernels are held against each other)
+        return rng.integers(0, 256, (local, n, k // 2), dtype=np.uint8), rng.integers(118, 122, (local, n, k // 32), dtype=np.uint8)
+
+    l1, l2 = random_weights(2 * inter, hidden), random_weights(hidden, inter)
+    want, _ = _forward(ops, x, l1, l2, None, idx, weights, hidden, inter, local, 64)
+    for waves in (1, 4):
+        got, counts = _forward(ops, x, l1, l2, None, idx, weights, hidden, inter, local, 32, waves)
+        np.testing.assert_array_equal(counts, rows)
+        assert torch.equal(got.view(torch.int16), want.view(torch.int16)), waves
