@@ -231,12 +231,13 @@ struct GemmParams {
     // Zero rows of the final output.  When a launch has fewer tiles than workgroups, the workgroups left
     // without a tile stream zeros into the output rows of the tokens that no local expert serves (most tokens of a
     // rank's share), which the weighted reduce would otherwise have to write after the GEMMs: the stores cost the
-    // matrix pipes nothing.  Every wave of such a workgroup is a filler f and takes tokens f, f + fillers, ...
+    // matrix pipes nothing.  kFillWaves waves of such a workgroup are fillers f and take tokens f, f + fillers, ...
     // until a workgroup with a tile reaches its epilogue and raises *fill_stop.  The word is a counter that only ever
     // grows (device memory of the workspace): a filler remembers the value it found when it started and stops when
     // the word differs, so nothing has to clear it, no value comes from the host, and every replay of a captured
     // launch stops its own fillers.  (Launches on a workspace run one after the other, so a filler's first read sees
-    // every increment of the launches before it and none of its own launch: the first increment is a whole tile away.)
+    // every increment of the launches before it and none of its own launch: the first increment is a whole tile away.  One-wave launches
+    // have few_rows_fillers workgroups more for it.)
     // fill_state[0] = number of fillers, fill_state[1 + f] = tokens filler f got through.  All of it is null / zero in
     // launches that do not fill.
     u32x4* fill_out;                // [fill_tokens, fill_vec] or nullptr
@@ -250,6 +251,7 @@ struct GemmParams {
     int n_real, k_real;             // what is not padding of n and k (first GEMM: n counts gate and up)
     int live_n_tiles;               // column tiles that the kernels that skip padding work on (first GEMM: all, unless the second reads none of it)
     int numbered_n_tiles;           // few-rows kernels: column tiles that a row tile's numbers are given to, those behind live_n_tiles in vain
+    int few_rows_fillers;           // one-wave launches: workgroups in front of those with tiles that fill
 };
 
 // gate / (1 + exp(-gate)) * up with the hardware exponential and reciprocal (v_exp_f32, v_rcp_f32: about 1 ulp each; the
@@ -412,6 +414,26 @@ __device__ __forceinline__ int expert_of_tile(int tile, const int* tile_base, in
     return e;
 }
 
+// Wave number `filler` of `fillers`: zero rows of the output (see GemmParams).  Two waves of every workgroup without a tile: more of
+// them fill faster, but what they take from the GEMM grows faster still, and the reduce writes what is left at 6 TB/s (one EP64
+// rank's share of 16 384 tokens of 7168 columns, 64 idle workgroups, whole forward: four waves each 147.8 us, three 147.4, two 144.8, one
+// 149, none 154).
+constexpr int kFillWaves = 2;
+__device__ __forceinline__ void fill_zero_rows(const GemmParams& p, int filler, int fillers, int lane)
+{
+    const u32x4 zero = {0u, 0u, 0u, 0u};
+    int done = 0;
+    const int stop_at_start = __hip_atomic_load(p.fill_stop, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    for (int token = filler; token < p.fill_tokens; token += fillers, ++done) {
+        if (__hip_atomic_load(p.fill_stop, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != stop_at_start) break;
+        const bool mine = lane < p.fill_topk && p.fill_route_to_row[static_cast<size_t>(token) * p.fill_topk + lane] >= 0;
+        if (__ballot(mine) != 0ull) continue;  // some local expert serves the token: the reduce writes its row
+        u32x4* row = p.fill_out + static_cast<size_t>(token) * p.fill_vec;
+        for (int v = lane; v < p.fill_vec; v += 64) store16_nt(row + v, zero);
+    }
+    if (lane == 0) p.fill_state[1 + filler] = done;
+}
+
 struct TileInfo {
     int expert, nt, row0, valid;  // row0 = first row of the tile in the expanded layout; valid rows <= kBM
 };
@@ -451,7 +473,7 @@ __global__ __launch_bounds__(kGemmThreads, 1) void grouped_gemm_kernel(GemmParam
     // GEMM works from: fillers on every XCD fill faster but cost the GEMM three times as much); a launch that
     // does not fill shrinks the ranges evenly (about 4 % faster than leaving two XCDs idle).
     const bool one_round = total_tiles < static_cast<int>(gridDim.x);
-    const int fillers = one_round && p.fill_out != nullptr ? (static_cast<int>(gridDim.x) - total_tiles) * kGemmWaves : 0;
+    const int fillers = one_round && p.fill_out != nullptr ? (static_cast<int>(gridDim.x) - total_tiles) * kFillWaves : 0;
     const bool spread = one_round && fillers == 0 && (gridDim.x & 7) == 0;
     const int per_xcd = spread ? (total_tiles + 7) / 8 : (gridDim.x + 7) / 8;
     const int first = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
@@ -459,19 +481,7 @@ __global__ __launch_bounds__(kGemmThreads, 1) void grouped_gemm_kernel(GemmParam
     const bool has_tile = first < total_tiles && (!spread || static_cast<int>(blockIdx.x >> 3) < per_xcd);
     if (blockIdx.x == 0 && tid == 0 && p.fill_state != nullptr) p.fill_state[0] = fillers;  // workgroup 0 always has tile 0
     if (!has_tile) {
-        if (fillers == 0) return;
-        const int filler = (first - total_tiles) * kGemmWaves + wave;
-        const u32x4 zero = {0u, 0u, 0u, 0u};
-        int done = 0;
-        const int stop_at_start = __hip_atomic_load(p.fill_stop, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        for (int token = filler; token < p.fill_tokens; token += fillers, ++done) {
-            if (__hip_atomic_load(p.fill_stop, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != stop_at_start) break;
-            const bool mine = lane < p.fill_topk && p.fill_route_to_row[static_cast<size_t>(token) * p.fill_topk + lane] >= 0;
-            if (__ballot(mine) != 0ull) continue;  // some local expert serves the token: the reduce writes its row
-            u32x4* row = p.fill_out + static_cast<size_t>(token) * p.fill_vec;
-            for (int v = lane; v < p.fill_vec; v += 64) store16_nt(row + v, zero);
-        }
-        if (lane == 0) p.fill_state[1 + filler] = done;
+        if (fillers != 0 && wave < kFillWaves) fill_zero_rows(p, (first - total_tiles) * kFillWaves + wave, fillers, lane);
         return;
     }
     const int my_tiles = one_round ? 1 : (total_tiles - first + stride - 1) / stride;
@@ -1050,6 +1060,16 @@ __device__ __forceinline__ void store_output(const GemmParams& p, const v16f& ac
     }
 }
 
+// One-wave workgroups that fill stand in front of those with tiles: a filler has to start before a tile can end, or it would find the
+// counter raised already.  (A multiple of 8 of them, so that the tiles keep their XCDs.)
+__device__ __forceinline__ bool fill_of_few_rows(const GemmParams& p)
+{
+    if (blockIdx.x == 0 && threadIdx.x == 0 && p.fill_state != nullptr) p.fill_state[0] = p.few_rows_fillers;
+    if (static_cast<int>(blockIdx.x) >= p.few_rows_fillers) return false;
+    fill_zero_rows(p, static_cast<int>(blockIdx.x), p.few_rows_fillers, static_cast<int>(threadIdx.x));
+    return true;
+}
+
 // The 32-row tiles of the few-rows kernels.  They are numbered through the experts, so that the grid does not depend on how the
 // routes fell; every wave works the numbering out for itself (a lane has experts lane and lane + 64).
 struct FewRowsTiles {
@@ -1122,10 +1142,16 @@ __global__ __launch_bounds__(64 * kWaves, 2) void grouped_gemm_few_rows_kernel(G
     const int n_tiles = p.n / kBN, stored_ktiles = p.k / kBK, stored_spans = (stored_ktiles + 3) / 4, scale_bytes = p.k / 32;
     // (k tiles and column tiles of nothing but padding are left out)
     const int ktiles = (p.k_real + kBK - 1) / kBK, spans = (ktiles + 3) / 4, numbered_n_tiles = p.numbered_n_tiles;
-    if (blockIdx.x == 0 && threadIdx.x == 0 && p.fill_state != nullptr) p.fill_state[0] = 0;
 
+    if constexpr (kWaves == 1) {
+        if (fill_of_few_rows(p)) return;
+    } else if (blockIdx.x == 0 && threadIdx.x == 0 && p.fill_state != nullptr) {
+        p.fill_state[0] = 0;
+    }
     const FewRowsTiles tiles(p, lane);
-    for (int tile_id = blockIdx.x; tile_id < tiles.total * numbered_n_tiles * kSplit; tile_id += gridDim.x) {
+    const int fillers = kWaves == 1 ? p.few_rows_fillers : 0;
+    for (int tile_id = static_cast<int>(blockIdx.x) - fillers; tile_id < tiles.total * numbered_n_tiles * kSplit;
+         tile_id += static_cast<int>(gridDim.x) - fillers) {
         const int unit = tile_id / (numbered_n_tiles * kSplit), piece = tile_id - unit * (numbered_n_tiles * kSplit);
         const int nt = piece / kSplit, wave = kWaves == 1 ? piece % kSplit : my_wave;  // the column tile, the quarter of it
         if (nt >= p.live_n_tiles) continue;
@@ -1253,6 +1279,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void grouped_gemm_few_rows_kernel(G
         }
         // the next tile of this workgroup writes the LDS again
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        if (kWaves == 1 && fillers != 0 && tile_id == 0 && threadIdx.x == 0) __hip_atomic_fetch_add(p.fill_stop, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         const bool row_exists = lr < valid;
         const size_t row = static_cast<size_t>(row0) + lr;
         if (kGateUp) {
@@ -1279,10 +1306,12 @@ __global__ __launch_bounds__(64, 1) void grouped_gemm_one_wave_kernel(GemmParams
     const int n_tiles = p.n / kBN, stored_ktiles = p.k / kBK, stored_spans = (stored_ktiles + 3) / 4, scale_bytes = p.k / 32;
     // (k tiles and column tiles of nothing but padding are left out)
     const int ktiles = (p.k_real + kBK - 1) / kBK, spans = (ktiles + 3) / 4, numbered_n_tiles = p.numbered_n_tiles;
-    if (blockIdx.x == 0 && threadIdx.x == 0 && p.fill_state != nullptr) p.fill_state[0] = 0;
 
+    if (fill_of_few_rows(p)) return;
     const FewRowsTiles tiles(p, lane);
-    for (int tile_id = blockIdx.x; tile_id < tiles.total * numbered_n_tiles * kSplit; tile_id += gridDim.x) {
+    const int fillers = p.few_rows_fillers;
+    for (int tile_id = static_cast<int>(blockIdx.x) - fillers; tile_id < tiles.total * numbered_n_tiles * kSplit;
+         tile_id += static_cast<int>(gridDim.x) - fillers) {
         const int unit = tile_id / (numbered_n_tiles * kSplit), piece = tile_id - unit * (numbered_n_tiles * kSplit);
         const int nt = piece / kSplit, wave = piece % kSplit;  // the column tile, the quarter of it
         if (nt >= p.live_n_tiles) continue;
@@ -1409,6 +1438,7 @@ __global__ __launch_bounds__(64, 1) void grouped_gemm_one_wave_kernel(GemmParams
         } else {
             span_body(even, no, no, span);
         }
+        if (fillers != 0 && tile_id == 0 && threadIdx.x == 0) __hip_atomic_fetch_add(p.fill_stop, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         const bool row_exists = lr < valid;
         const size_t row = static_cast<size_t>(row0) + lr;
         if (kGateUp) {
@@ -1455,7 +1485,7 @@ __global__ __launch_bounds__(kGemmThreads, ColCfg<RT>::kWorkgroupsPerCu) void gr
 
     // Tiles to workgroups, and what the workgroups without a tile do: as in grouped_gemm_kernel.
     const bool one_round = total_tiles < static_cast<int>(gridDim.x);
-    const int fillers = one_round && p.fill_out != nullptr ? (static_cast<int>(gridDim.x) - total_tiles) * kGemmWaves : 0;
+    const int fillers = one_round && p.fill_out != nullptr ? (static_cast<int>(gridDim.x) - total_tiles) * kFillWaves : 0;
     const bool spread = one_round && fillers == 0 && (gridDim.x & 7) == 0;
     const int per_xcd = spread ? (total_tiles + 7) / 8 : (gridDim.x + 7) / 8;
     const int first = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
@@ -1463,19 +1493,7 @@ __global__ __launch_bounds__(kGemmThreads, ColCfg<RT>::kWorkgroupsPerCu) void gr
     const bool has_tile = first < total_tiles && (!spread || static_cast<int>(blockIdx.x >> 3) < per_xcd);
     if (blockIdx.x == 0 && tid == 0 && p.fill_state != nullptr) p.fill_state[0] = fillers;
     if (!has_tile) {
-        if (fillers == 0) return;
-        const int filler = (first - total_tiles) * kGemmWaves + wave;
-        const u32x4 zero = {0u, 0u, 0u, 0u};
-        int done = 0;
-        const int stop_at_start = __hip_atomic_load(p.fill_stop, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        for (int token = filler; token < p.fill_tokens; token += fillers, ++done) {
-            if (__hip_atomic_load(p.fill_stop, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != stop_at_start) break;
-            const bool mine = lane < p.fill_topk && p.fill_route_to_row[static_cast<size_t>(token) * p.fill_topk + lane] >= 0;
-            if (__ballot(mine) != 0ull) continue;
-            u32x4* row = p.fill_out + static_cast<size_t>(token) * p.fill_vec;
-            for (int v = lane; v < p.fill_vec; v += 64) store16_nt(row + v, zero);
-        }
-        if (lane == 0) p.fill_state[1 + filler] = done;
+        if (fillers != 0 && wave < kFillWaves) fill_zero_rows(p, (first - total_tiles) * kFillWaves + wave, fillers, lane);
         return;
     }
     const int my_tiles = one_round ? 1 : (total_tiles - first + stride - 1) / stride;
@@ -2385,10 +2403,6 @@ GemmChoice choose_gemm(const GemmParams& p, const ExpectedRows& expected, int cu
         streamed = live_bytes > 256e6 && paired_row_tiles < 1.3 * experts_with_rows;
     }
     const GemmChoice pair_choice = {128, kGemmWaves, paired_row_tiles * p.live_n_tiles, true, streamed, false, 0.0};
-    // A share with more than one 64-row tile per expert has so many tokens without a row that its first GEMM's idle workgroups are
-    // better used for their zero rows: kernels that do not fill are no candidates there.
-    const bool fills = p.fill_tokens > 0 && tiles_of[best] < cus;
-    const bool unfilled_allowed = !fills || mean <= 64.0;
     // Source rows are addressed with 32 bits in the few-rows kernel.
     const double tiles = live_row_tiles * p.live_n_tiles, row_tiles_per_expert = live_row_tiles / std::max(experts_with_rows, 1e-3);
     // One-wave workgroups without LDS while there is at most one to a CU (16 % faster than with it over 167 launches, a tenth where tiles are
@@ -2398,26 +2412,32 @@ GemmChoice choose_gemm(const GemmParams& p, const ExpectedRows& expected, int cu
     if (p.column_waves && p.forced == 0) {
         // (by the padded sizes, as fitted: by the real ones these kernels look too good where little of a tile is real)
         const double all_tiles = live_row_tiles * n_tiles;
-        const bool few_allowed = (p.fill_tokens == 0 || mean <= 64.0) && (!kGateUp || static_cast<long long>(p.a_rows) * p.k < (1LL << 32));
+        const bool few_allowed = !kGateUp || static_cast<long long>(p.a_rows) * p.k < (1LL << 32);
         const double one = few_allowed ? bounded(3.0 + 0.30 * ktiles + (rounds_of(kGemmWaves * all_tiles, cus) - 1.0) * (1.1 + 0.17 * ktiles)) : 1e30;
         const double four = few_allowed ? bounded(1.5 + rounds_of(all_tiles, cus) * (2.7 + 0.50 * ktiles)) : 1e30;
-        // Zero rows of the output that this launch's idle workgroups would have written (at about 30 GB/s each): these two
-        // kernels leave them to the reduce, which writes them at 8 TB/s, and the GEMM is faster without the company: 4300 zero
-        // rows of 5120 columns beside 31 experts of 5120 x 512 cost the forward 57 us filled and 49 not.
+        // Zero rows of the output that another kernel's idle workgroups write meanwhile (at about 30 GB/s each): the paired kernel leaves
+        // them to the reduce, which writes them at 8 TB/s. (Not held against the few-rows kernels: where the model prefers them they win by
+        // far more; 4300 zero rows of 6272 columns beside 3 experts of 6272 x 768, 95 rows each: 48 us with 64-row tiles and fillers, 36 without.)
         double unfilled = 0.0;
-        if (fills) {
+        if (p.fill_tokens > 0 && tiles_of[best] < cus) {
             const double zeros = p.fill_tokens * exp(-mean * p.num_routed / p.fill_tokens) * p.fill_vec * 16.0;
             unfilled = std::min(zeros, (cus - tiles_of[best]) * 30e3 * best_cost) / 11e6;
         }
         const double few = std::min(one, four);
-        if (unfilled_allowed && paired < few && paired + unfilled < best_cost) return pair_choice;
-        if (few + unfilled < best_cost) return {32, one < four ? 1 : kGemmWaves, tiles, false, false, one < four && direct, row_tiles_per_expert};
+        if (paired + unfilled < std::min(few, best_cost)) return pair_choice;
+        if (few < best_cost) return {32, one < four ? 1 : kGemmWaves, tiles, false, false, one < four && direct, row_tiles_per_expert};
     }
     if ((p.forced & 0xff) == 32) return {32, p.forced >> 8, tiles, false, false, (p.forced >> 8) == 1 && direct, row_tiles_per_expert};
     if (p.forced == 128 && p.column_waves && (p.fill_tokens == 0 || tiles_of[2] >= cus)) return pair_choice;
     if (p.forced != 0) best = p.forced / 64;
     return {64 * best, kGemmWaves, tiles_of[best], false, false, false, 0.0};
 }
+
+// A one-wave launch of a share with more than 64 rows per expert fills with this many waves: 16 to 60 MB of zeros beside 4 to 12 experts
+// cost the forward between 1 % more and 2.5 % less than in the reduce, nearly the same with 32 or 128 of them. With fewer rows, and beside
+// four-wave workgroups, whose CUs the fillers take, it costs more than it gives (3584 tokens of 2176 columns, 4 experts: first GEMM 15.7 us
+// alone, 16.9 with fillers, the reduce 4.5 either way).
+constexpr int kFewRowsFillers = 64;
 
 template <bool kGateUp>
 int launch_gemm(const GemmParams& p, const GemmChoice& choice, const ExpectedRows& expected, hipStream_t stream, const char* what)
@@ -2435,10 +2455,11 @@ int launch_gemm(const GemmParams& p, const GemmChoice& choice, const ExpectedRow
         GemmParams numbered = p;
         numbered.numbered_n_tiles = p.live_n_tiles + (choice.waves == 1 && choice.row_tiles_per_expert > 1.25 ? p.live_n_tiles & 1 : 0);
         const unsigned grid = static_cast<unsigned>(row_tiles * numbered.numbered_n_tiles);
+        if (choice.waves == 1 && p.fill_out != nullptr && expected.routed > 64.0) numbered.few_rows_fillers = kFewRowsFillers;
         if (choice.direct)
-            hipLaunchKernelGGL(grouped_gemm_one_wave_kernel<kGateUp>, dim3(kGemmWaves * grid), dim3(64), 0, stream, numbered);
+            hipLaunchKernelGGL(grouped_gemm_one_wave_kernel<kGateUp>, dim3(kGemmWaves * grid + numbered.few_rows_fillers), dim3(64), 0, stream, numbered);
         else if (choice.waves == 1)
-            hipLaunchKernelGGL((grouped_gemm_few_rows_kernel<1, kGateUp>), dim3(kGemmWaves * grid), dim3(64), 0, stream, numbered);
+            hipLaunchKernelGGL((grouped_gemm_few_rows_kernel<1, kGateUp>), dim3(kGemmWaves * grid + numbered.few_rows_fillers), dim3(64), 0, stream, numbered);
         else
             hipLaunchKernelGGL((grouped_gemm_few_rows_kernel<kGemmWaves, kGateUp>), dim3(grid), dim3(kGemmThreads), 0, stream, numbered);
         return launch_status(what);
@@ -2472,7 +2493,7 @@ GemmParams gemm_of(const MegaSizes& m, const Workspace* w, bool second)
     // zero those rows of y meanwhile, and the weighted reduce skips what they got through.  (Served-only: rows of y whose
     // token no local expert serves are nobody's business, neither the fillers' nor the reduce's; with shared experts every
     // token is served.)
-    if (!second && m.num_shared == 0 && (w == nullptr || (w->gemm_zero_fill && !w->megamoe_served_only))) {
+    if (!second && m.num_shared == 0 && m.num_local < m.num_experts && (w == nullptr || (w->gemm_zero_fill && !w->megamoe_served_only))) {
         p.fill_tokens = m.num_tokens;
         p.fill_vec = m.hidden / 8;
         p.fill_topk = m.num_topk;

@@ -14,7 +14,7 @@ pytestmark = pytest.mark.gpu
 EDGES = (1, 31, 32, 33, 0, 64, 65, 96, 97, 127, 128, 129, 160, 256, 257)
 
 
-def _forward(ops, x, l1, l2, shared, idx, weights, hidden, inter, local, tile_rows, few_rows_waves=4):
+def _forward(ops, x, l1, l2, shared, idx, weights, hidden, inter, local, tile_rows, few_rows_waves=4, experts=None, fill=0):
     dev = "cuda"
     num_shared = 0 if shared is None else shared[0][0].shape[0]
 
@@ -27,11 +27,11 @@ def _forward(ops, x, l1, l2, shared, idx, weights, hidden, inter, local, tile_ro
     ws = ops.Workspace(ops.megamoe_workspace_bytes(len(idx), idx.shape[1], hidden, inter, local, num_shared))
     ws.tune("gemm_tile_rows", tile_rows)
     ws.tune("gemm_few_rows_waves", few_rows_waves)
-    ws.tune("gemm_zero_fill", 0)  # (a launch whose idle workgroups zero rows keeps the column-wave kernel)
+    ws.tune("gemm_zero_fill", fill)  # (a launch whose idle workgroups zero rows keeps the column-wave kernel)
     y = torch.full((len(idx), hidden), float("nan"), dtype=torch.bfloat16, device=dev)
     counts = torch.empty((local,), dtype=torch.int32, device=dev)
     ops.megamoe_forward(ws, torch.from_numpy(x[0]).to(dev).view(torch.float8_e4m3fn), torch.from_numpy(x[1]).to(dev), torch.from_numpy(idx).to(dev),
-                        torch.from_numpy(weights).to(dev), w1, s1, w2, s2, local, 0, local, y, counts, shared=shared_weights, intermediate=inter)
+                        torch.from_numpy(weights).to(dev), w1, s1, w2, s2, experts or local, 0, local, y, counts, shared=shared_weights, intermediate=inter)
     torch.cuda.synchronize()
     ws.destroy()
     return y, counts.cpu().numpy()
@@ -96,3 +96,31 @@ def test_few_rows_kernels_at_their_edges(hidden, inter, rows):
         got, counts = _forward(ops, x, l1, l2, None, idx, weights, hidden, inter, local, 32, waves)
         np.testing.assert_array_equal(counts, rows)
         assert torch.equal(got.view(torch.int16), want.view(torch.int16)), waves
+
+
+@pytest.mark.parametrize("tokens,hidden,topk,experts", [
+    (70, 64, 4, 4),       # hardly more tokens than fillers; rows of 8 chunks, less than a lane each
+    (1000, 576, 2, 16),   # 72 chunks: a lane has one or two
+    (330, 1664, 4, 16),   # several tiles to a workgroup's XCD
+])
+def test_one_wave_launches_fill(tokens, hidden, topk, experts):
+    """Two of the experts are here, with more than 64 rows each: the launch has fillers, and the rows of the other tokens are zero whoever wrote them."""
+    from deepep_amd import ops
+
+    rng = np.random.default_rng(tokens)
+    inter, local = 256, 2
+    idx = np.argsort(rng.random((tokens, experts)), axis=1)[:, :topk].astype(np.int32)
+    if topk == experts:
+        idx[::3] = np.where(idx[::3] < local, -1, idx[::3])
+    x = mm.mx_quantize(rng.normal(size=(tokens, hidden)).astype(np.float32))
+    weights = rng.random((tokens, topk)).astype(np.float32)
+
+    def random_weights(n, k):
+        return rng.integers(0, 256, (local, n, k // 2), dtype=np.uint8), rng.integers(118, 122, (local, n, k // 32), dtype=np.uint8)
+
+    l1, l2 = random_weights(2 * inter, hidden), random_weights(hidden, inter)
+    want, _ = _forward(ops, x, l1, l2, None, idx, weights, hidden, inter, local, 32, 1, experts)
+    got, _ = _forward(ops, x, l1, l2, None, idx, weights, hidden, inter, local, 32, 1, experts, fill=1)
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+    unserved = ~((idx >= 0) & (idx < local)).any(1)
+    assert unserved.any() and not got.cpu()[torch.from_numpy(unserved)].any()
