@@ -2982,6 +2982,14 @@ int dpep_megamoe_run(void* ws, const dpep_megamoe_call* call, void* stream)
         front.codes_out = reinterpret_cast<u32x4*>(codes_out);
         codes = codes_out;
         scales = front.scales_out;
+        // Where most tokens are expected to have no row here, only those that have one are prepared: for 6976 tokens of 4160 columns
+        // that go to one of 64 ranks the forward took 80.6 us and takes 56.6, for 15 424 of 3456 (16 ranks, top-4) 105.0 and 97.4, and
+        // none of 29 shares from 8 to 16 192 tokens got slower.  (The look at the ids delays a row that is wanted.)
+        if (num_shared == 0 && pow(1.0 - static_cast<double>(num_local) / num_experts, num_topk) > 0.5) {
+            front.topk_idx = topk_idx;
+            front.expert_begin = expert_begin;
+            front.num_local = num_local;
+        }
     }
     if (int rc = layout_i32(ws, topk_idx, num_tokens, num_topk, num_experts, expert_begin, num_local, expert_token_nums,
                             psum, offsets, route_to_row, row_to_route, num_rows, front, s))

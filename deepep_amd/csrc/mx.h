@@ -67,9 +67,25 @@ struct MegaFront {
     u32x4* codes_out;
     uint8_t* scales_out;
     int num_shared, num_tokens, num_topk;
+    // Not null: rows whose token has no route to experts expert_begin .. + num_local are left as they are (nobody reads them).
+    const int32_t* topk_idx;
+    int expert_begin, num_local;
 };
 constexpr int kFrontThreads = 256;
 inline __host__ __device__ unsigned front_blocks(const MegaFront& f, int threads) { return (f.units + threads - 1) / threads; }
+
+// Whether row `row` has a route to a local expert.  The rows of a wave's lanes follow one another, so their ids are one piece of memory: one
+// load and a ballot.  (More than 64 ids, as with rows of 256 columns and 16 routes each: not looked at.)  Called by whole waves.
+__device__ __forceinline__ bool row_is_served(const MegaFront& f, unsigned row)
+{
+    const unsigned lane = threadIdx.x & 63, last = f.num_tokens - 1, mine = row < last ? row : last;
+    const unsigned first = __builtin_amdgcn_readfirstlane(mine), end = __builtin_amdgcn_readlane(mine, 63) + 1;
+    const unsigned ids = (end - first) * f.num_topk;
+    if (ids > 64) return true;
+    const int id = lane < ids ? f.topk_idx[static_cast<size_t>(first) * f.num_topk + lane] - f.expert_begin : -1;
+    const unsigned long long served = __ballot(id >= 0 && id < f.num_local) >> ((mine - first) * f.num_topk);
+    return (served & (~0ull >> (64 - f.num_topk))) != 0ull;
+}
 
 // One workgroup's piece of the input rows.  staged: kThreads / 2 bytes of LDS, 16-byte aligned (the workgroup's scale bytes leave as
 // 16-byte stores).  Called by all threads.
@@ -77,8 +93,8 @@ template <int kThreads>
 __device__ __forceinline__ void prepare_rows(const MegaFront& f, unsigned block, uint8_t* staged)
 {
     const unsigned unit = block * kThreads + threadIdx.x, per_row = f.hp / 16;
-    const bool live = unit < f.units;
     const unsigned row = unit / per_row, at = unit - row * per_row;
+    const bool wanted = f.topk_idx == nullptr || row_is_served(f, row), live = wanted && unit < f.units;
     const bool real = live && at * 16 < static_cast<unsigned>(f.h);  // (h is a multiple of 32: both lanes of a block agree)
     const u32x4 zero = {0u, 0u, 0u, 0u};
     u32x4 codes = zero;

@@ -124,3 +124,30 @@ def test_one_wave_launches_fill(tokens, hidden, topk, experts):
     assert torch.equal(got.view(torch.int16), want.view(torch.int16))
     unserved = ~((idx >= 0) & (idx < local)).any(1)
     assert unserved.any() and not got.cpu()[torch.from_numpy(unserved)].any()
+
+
+@pytest.mark.parametrize("tokens,hidden,topk,experts,local", [
+    (1, 64, 1, 8, 1),         # one row of sixteen pieces
+    (37, 192, 16, 64, 1),     # four rows to a wave: as many ids as it has lanes
+    (38, 192, 17, 64, 1),     # and more, which are not looked at
+    (333, 1088, 3, 16, 2),    # 80 pieces a row: waves with one row and with two; the last workgroup is not full
+    (1500, 576, 4, 64, 8),    # 48 pieces; a layout of several workgroups
+    (2500, 320, 4, 64, 3),    # two waves with the same rows; layout and preparation are neighbours in one grid
+])
+def test_rows_of_other_ranks_are_not_prepared(tokens, hidden, topk, experts, local):
+    """Padded rows, most tokens without a local expert: served rows against the oracle, the others zero."""
+    from deepep_amd import ops
+
+    rng = np.random.default_rng(tokens)
+    inter = 128
+    idx = np.argsort(rng.random((tokens, experts)), axis=1)[:, :topk].astype(np.int32)
+    idx[-1] = np.arange(topk)  # the last row is served
+    x = mm.mx_quantize(rng.normal(size=(tokens, hidden)).astype(np.float32))
+    weights = rng.random((tokens, topk)).astype(np.float32)
+    l1, l2 = (mm.quantize_weight_mxfp4((rng.normal(size=(local, n, k)) * 0.02).astype(np.float32)) for n, k in ((2 * inter, hidden), (hidden, inter)))
+    got, _ = _forward(ops, x, l1, l2, None, idx, weights, hidden, inter, local, 0, experts=experts)
+    oracle = mm.round_bf16(mm.local_reference(mm.mx_dequantize(*x), idx, weights, mm.unpack_weight(*l1), mm.unpack_weight(*l2), 0))
+    got, served = got.float().cpu().numpy(), (idx < local).any(1)
+    assert not got[~served].any()
+    for row in np.flatnonzero(served):
+        assert mm.relative_frobenius(got[row], oracle[row]) <= 2e-2, row
