@@ -64,12 +64,16 @@ struct Workspace {
 // kSyncFillStop the word through which the MegaMoE fillers are told to stop (a counter that only grows: a filler stops when
 // it differs from what the filler found at its start, so it needs no clearing and no value from the host); at kSyncReporterTag the tag the one-launch layout's reporter workgroup has settled on
 // (64 bits; it publishes no histogram, so this is how the others know that it has read the epoch); from kSyncTagged on the
-// tagged per-workgroup histograms of the one-launch layout.
+// tagged per-workgroup histograms of the one-launch layout; at kSyncTotal and from kSyncRows on the number of rows and the rows of the
+// routes (or the routes of the rows), for a payload in the layout's grid, tagged with the number of the launch.
 constexpr size_t kSyncFillStop = 64;
 constexpr size_t kSyncReporterTag = 128;
 constexpr size_t kSyncTagged = 256;
 constexpr size_t kSyncTaggedWords = 4096 + DPEP_MAX_LOCAL_EXPERTS;  // (workgroups + 1) * experts never exceeds this
-constexpr size_t kSyncBytes = kSyncTagged + kSyncTaggedWords * 8;
+constexpr size_t kSyncTotal = kSyncTagged + kSyncTaggedWords * 8;
+constexpr size_t kSyncRows = kSyncTotal + 256;
+constexpr int kSyncRowWords = 131072;
+constexpr size_t kSyncBytes = kSyncRows + static_cast<size_t>(kSyncRowWords) * 8;
 // The host mailbox (pinned memory, 32-bit words): word 0 = number of rows and word 1 = sequence number of the layout
 // that reported last (one 8-byte store); word kMailboxTimeout = launch number of a layout kernel whose wait for the
 // other workgroups' histograms ran out; from word kMailboxCounts on the per-expert counts, 16 bytes for experts 4i .. 4i + 3:

@@ -8,15 +8,14 @@
 #include <type_traits>
 
 #include "common.h"
+#include "payload.h"
 
 #pragma clang fp contract(off)
 
 namespace dpep {
 namespace {
 
-constexpr int kMaxThreads = 256;
 constexpr int kTargetBlocks = 8192;  // rows are split into column parts until a launch has about this many workgroups (4096 rows: two parts each measured 3-6 % faster than one, four no better)
-constexpr int kMaxScaleCols = 1024;  // hidden <= 131072 for the fused quantiser
 constexpr int kRowMajorRatio = 1;  // row-major kernels when rows <= ratio * tokens
 
 // Store policy of the payload rows.  Streaming (non-temporal, the default): the rows go to HBM past the caches at the
@@ -29,14 +28,6 @@ constexpr int kRowMajorRatio = 1;  // row-major kernels when rows <= ratio * tok
 // memory-side cache may still prefer write-through, hence the knob.
 int g_store_policy = DPEP_STORE_STREAMING;
 
-template <int kPolicy>
-__device__ __forceinline__ void store16_as(void* p, u32x4 v)
-{
-    if (kPolicy == DPEP_STORE_THROUGH) store16_through(p, v);
-    else if (kPolicy == DPEP_STORE_STREAMING) store16_nt(p, v);
-    else *reinterpret_cast<u32x4*>(p) = v;
-}
-
 // Calls launch(std::integral_constant<int, policy>) for the current policy.
 template <typename Launch>
 void with_store_policy(Launch&& launch)
@@ -48,277 +39,41 @@ void with_store_policy(Launch&& launch)
     }
 }
 
-// ---- token-major copy: one workgroup per (token, column part); read once, write K times -----------
-// Rows at or beyond `capacity` are dropped; with all_rows (the layout's count) nothing is moved unless DPEP_ROWS_KEPT.
 template <int kPolicy>
 __global__ __launch_bounds__(kMaxThreads) void dispatch_copy_token_kernel(
-    const u32x4* __restrict__ x, const float* __restrict__ scales, const float* __restrict__ weights,
-    const int* __restrict__ route_to_row, int num_topk, int vec_per_row, int vec_per_part, int parts, int scale_cols,
-    int capacity, const int* __restrict__ all_rows, u32x4* __restrict__ out, float* __restrict__ out_scales,
-    float* __restrict__ out_weights)
+    const u32x4* __restrict__ x, const float* __restrict__ scales, const float* __restrict__ weights, u32x4* __restrict__ out,
+    float* __restrict__ out_scales, float* __restrict__ out_weights, PayloadShape p, MappedTokens tokens)
 {
-    __shared__ int rows[DPEP_MAX_TOPK];
-    __shared__ int any_valid;
-    const int token = blockIdx.x / parts, part = blockIdx.x % parts;
-    const int all = all_rows != nullptr ? *all_rows : capacity;  // (travels with the values and the routes)
-    const int v_begin = part * vec_per_part;
-    const int v_end = min(v_begin + vec_per_part, vec_per_row);
-    const u32x4* src = x + static_cast<size_t>(token) * vec_per_row;
-    // The token's first values are asked for before its routes are known (see the quantising kernel below).
-    const int v_first = v_begin + threadIdx.x;
-    u32x4 first = {0u, 0u, 0u, 0u};
-    if (v_first < v_end) first = load16(src + v_first);
-    if (threadIdx.x == 0) any_valid = 0;
-    __syncthreads();
-    if (threadIdx.x < num_topk) {
-        int row = route_to_row[static_cast<size_t>(token) * num_topk + threadIdx.x];
-        if (row >= capacity || !DPEP_ROWS_KEPT(all, capacity)) row = -1;  // outputs allocated before R was known
-        rows[threadIdx.x] = row;
-        if (row >= 0) any_valid = 1;
-    }
-    __syncthreads();
-    if (!any_valid) return;
-    for (int v = v_first; v < v_end; v += blockDim.x) {
-        const u32x4 value = v == v_first ? first : load16(src + v);
-        for (int s = 0; s < num_topk; ++s) {
-            const int row = rows[s];
-            if (row >= 0) store16_as<kPolicy>(out + static_cast<size_t>(row) * vec_per_row + v, value);
-        }
-    }
-    if (part == 0) {
-        if (scales != nullptr) {
-            for (int c = threadIdx.x; c < scale_cols; c += blockDim.x) {
-                const float value = scales[static_cast<size_t>(token) * scale_cols + c];
-                for (int s = 0; s < num_topk; ++s) {
-                    const int row = rows[s];
-                    if (row >= 0) out_scales[static_cast<size_t>(row) * scale_cols + c] = value;
-                }
-            }
-        }
-        if (weights != nullptr && threadIdx.x < num_topk && rows[threadIdx.x] >= 0)
-            out_weights[rows[threadIdx.x]] = weights[static_cast<size_t>(token) * num_topk + threadIdx.x];
-    }
+    __shared__ TokenLds lds;
+    copy_token<kPolicy>(x, scales, weights, out, out_scales, out_weights, p, tokens, blockIdx.x, threadIdx.x, lds);
 }
-
-// ---- row-major: one workgroup per (output row, column part); for sparse receive shares -------------
-// Rows [0, rows): `rows` from the host, or, rows_on_device, the smaller of that bound and the count the layout left on the
-// device (a payload queued before the host knows R); all_or_none, the outputs' capacity: no rows at all unless DPEP_ROWS_KEPT
-// (0: the first rows in any case).  Such a launch has workgroups for about the expected number of rows;
-// they walk on by the grid's rows until the real count is reached, and the first row's route is asked for together with
-// the count (row_to_route has an entry for every row of the grid, so the load is in bounds whatever the count says).
-struct RowRange {
-    int rows;
-    const int* rows_on_device;
-    int all_or_none;
-    __device__ __forceinline__ int count() const
-    {
-        if (rows_on_device == nullptr) return rows;
-        const int all = *rows_on_device;
-        return all_or_none == 0 || DPEP_ROWS_KEPT(all, all_or_none) ? min(all, rows) : 0;
-    }
-};
 
 template <int kPolicy>
 __global__ __launch_bounds__(kMaxThreads) void dispatch_copy_row_kernel(
-    const u32x4* __restrict__ x, const float* __restrict__ scales, const float* __restrict__ weights,
-    const int* __restrict__ row_to_route, RowRange range, int num_tokens, int num_topk, int vec_per_row, int vec_per_part,
-    int parts, int scale_cols, u32x4* __restrict__ out, float* __restrict__ out_scales, float* __restrict__ out_weights)
+    const u32x4* __restrict__ x, const float* __restrict__ scales, const float* __restrict__ weights, u32x4* __restrict__ out,
+    float* __restrict__ out_scales, float* __restrict__ out_weights, PayloadShape p, const int* __restrict__ row_to_route,
+    RowRange range)
 {
-    const int part = blockIdx.x % parts, stride = gridDim.x / parts;
-    const int v_begin = part * vec_per_part;
-    const int v_end = min(v_begin + vec_per_part, vec_per_row);
-    int row = blockIdx.x / parts;
-    int next_route = row_to_route[row];
-    const int rows = range.count();
-    for (; row < rows; row += stride) {
-        // (clamped: a map left incomplete by a layout launch that reported a time-out must not become a wild address)
-        const int route = min(max(next_route, 0), num_tokens * num_topk - 1);
-        if (row + stride < rows) next_route = row_to_route[row + stride];
-        const int token = route / num_topk;
-        const u32x4* src = x + static_cast<size_t>(token) * vec_per_row;
-        u32x4* dst = out + static_cast<size_t>(row) * vec_per_row;
-        for (int v = v_begin + threadIdx.x; v < v_end; v += blockDim.x) store16_as<kPolicy>(dst + v, load16(src + v));
-        if (part == 0) {
-            if (scales != nullptr)
-                for (int c = threadIdx.x; c < scale_cols; c += blockDim.x)
-                    out_scales[static_cast<size_t>(row) * scale_cols + c] = scales[static_cast<size_t>(token) * scale_cols + c];
-            if (weights != nullptr && threadIdx.x == 0) out_weights[row] = weights[route];
-        }
-    }
+    copy_rows<kPolicy>(x, scales, weights, out, out_scales, out_weights, p, MappedRows<false>{row_to_route, range}, blockIdx.x, gridDim.x / p.parts, threadIdx.x);
 }
 
-// ---- per-128 FP8 quantiser ------------------------------------------------------------------------
-// One lane owns 16 consecutive BF16 values (two 16-byte loads), so 8 adjacent lanes own one
-// 128-element block.  amax is reduced over those 8 lanes with DPP-free xor shuffles inside the wave.
-struct Quant16 {
-    u32x4 codes;  // 16 e4m3fn bytes
-    float scale;  // amax / 448
-};
-
-// Largest of a value over the 8 lanes that share a 128-element block.
-__device__ __forceinline__ uint32_t max8(uint32_t v)
-{
-    v = max(v, static_cast<uint32_t>(__shfl_xor(static_cast<int>(v), 1)));
-    v = max(v, static_cast<uint32_t>(__shfl_xor(static_cast<int>(v), 2)));
-    v = max(v, static_cast<uint32_t>(__shfl_xor(static_cast<int>(v), 4)));
-    return v;
-}
-
-// fp32 -> e4m3fn byte pair, round-to-nearest-even, on the gfx950 converter (OCP FP8).
-__device__ __forceinline__ uint32_t pack4_e4m3(float a, float b, float c, float d)
-{
-    int packed = __builtin_amdgcn_cvt_pk_fp8_f32(a, b, 0, false);
-    packed = __builtin_amdgcn_cvt_pk_fp8_f32(c, d, packed, true);
-    return static_cast<uint32_t>(packed);
-}
-
-__device__ __forceinline__ Quant16 quantize16(u32x4 lo, u32x4 hi)
-{
-    float v[16];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        v[2 * i] = bf16_to_f32(lo[i] & 0xffffu);
-        v[2 * i + 1] = bf16_to_f32(lo[i] >> 16);
-        v[8 + 2 * i] = bf16_to_f32(hi[i] & 0xffffu);
-        v[8 + 2 * i + 1] = bf16_to_f32(hi[i] >> 16);
-    }
-    // amax as the largest magnitude BIT PATTERN (two BF16 magnitudes per word, v_pk_max_u16): for finite values that is
-    // the largest magnitude, and a NaN, whose pattern lies above infinity's, wins over everything, as it does in the
-    // reference's amax() and clamp() (torch propagates NaN through both, deep_ep/utils/math.py:52-53): a block that
-    // holds a NaN gets a NaN scale and the NaN code 0x7F for every value, whatever the others are.
-    typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
-    u16x2 both = {0, 0};
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        both = __builtin_elementwise_max(both, __builtin_bit_cast(u16x2, lo[i] & 0x7fff7fffu));
-        both = __builtin_elementwise_max(both, __builtin_bit_cast(u16x2, hi[i] & 0x7fff7fffu));
-    }
-    const uint32_t mine = max(static_cast<uint32_t>(both[0]), static_cast<uint32_t>(both[1]));
-    const uint32_t amax_bits = max(max8(mine) << 16, __float_as_uint(1e-4f));
-    const float amax = __uint_as_float(amax_bits);
-    const bool poisoned = amax_bits > 0x7f800000u;
-    // The reference writes 448.0 / amax, which torch evaluates as reciprocal(amax) * 448:
-    // two correctly rounded fp32 operations, reproduced here.
-    const float inv = __fmul_rn(__fdiv_rn(1.0f, amax), 448.0f);
-    Quant16 q;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const uint32_t codes = pack4_e4m3(__fmul_rn(v[4 * i], inv), __fmul_rn(v[4 * i + 1], inv), __fmul_rn(v[4 * i + 2], inv),
-                                          __fmul_rn(v[4 * i + 3], inv));
-        q.codes[i] = poisoned ? 0x7f7f7f7fu : codes;
-    }
-    q.scale = __fdiv_rn(amax, 448.0f);
-    return q;
-}
-
-// token-major: one workgroup per (token, column part); units = 16-element groups per row (H/16).
 template <int kPolicy>
 __global__ __launch_bounds__(kMaxThreads) void dispatch_quant_token_kernel(
-    const u32x4* __restrict__ x, const float* __restrict__ weights, const int* __restrict__ route_to_row, int num_topk,
-    int units_per_row, int units_per_part, int parts, int capacity, const int* __restrict__ all_rows, u32x4* __restrict__ out,
-    float* __restrict__ out_scales, float* __restrict__ out_weights)
+    const u32x4* __restrict__ x, const float* __restrict__ weights, u32x4* __restrict__ out, float* __restrict__ out_scales,
+    float* __restrict__ out_weights, PayloadShape p, MappedTokens tokens)
 {
-    __shared__ int rows[DPEP_MAX_TOPK];
-    __shared__ int any_valid;
+    __shared__ TokenLds lds;
     __shared__ float part_scales[kMaxScaleCols];
-    const int token = blockIdx.x / parts, part = blockIdx.x % parts;
-    const int all = all_rows != nullptr ? *all_rows : capacity;  // (travels with the values and the routes)
-    const int u_begin = part * units_per_part;
-    const int u_end = min(u_begin + units_per_part, units_per_row);
-    const u32x4* src = x + static_cast<size_t>(token) * units_per_row * 2;
-    // The token's first values are asked for before its routes are known: this grid is only used where most tokens own
-    // rows, and the row lookup and the payload then travel together instead of one after the other.
-    const int u_first = u_begin + threadIdx.x;
-    constexpr int kEarly = 2;  // units per thread fetched up front (all of a 7168-wide row with 256 threads)
-    u32x4 lo[kEarly], hi[kEarly];
-#pragma unroll
-    for (int j = 0; j < kEarly; ++j) {
-        const int u = u_first + j * static_cast<int>(blockDim.x);
-        if (u < u_end) {
-            lo[j] = load16(src + 2 * u);
-            hi[j] = load16(src + 2 * u + 1);
-        }
-    }
-    if (threadIdx.x == 0) any_valid = 0;
-    __syncthreads();
-    if (threadIdx.x < num_topk) {
-        int row = route_to_row[static_cast<size_t>(token) * num_topk + threadIdx.x];
-        if (row >= capacity || !DPEP_ROWS_KEPT(all, capacity)) row = -1;  // outputs allocated before R was known
-        rows[threadIdx.x] = row;
-        if (row >= 0) any_valid = 1;
-    }
-    __syncthreads();
-    if (!any_valid) return;
-    const int scale_cols = units_per_row / 8;
-    // units_per_part is a multiple of 8 and blockDim of 64, so the 8 lanes of a block stay together.
-    // Quantise first, then write row by row: at any moment the workgroup's stores run along ONE output row.
-    u32x4 codes[kEarly];
-#pragma unroll
-    for (int j = 0; j < kEarly; ++j) {
-        const int u = u_first + j * static_cast<int>(blockDim.x);
-        if (u < u_end) {
-            const Quant16 q = quantize16(lo[j], hi[j]);
-            codes[j] = q.codes;
-            if ((u & 7) == 0) part_scales[(u - u_begin) >> 3] = q.scale;
-        }
-    }
-    for (int s = 0; s < num_topk; ++s) {
-        const int row = rows[s];
-        if (row < 0) continue;
-#pragma unroll
-        for (int j = 0; j < kEarly; ++j) {
-            const int u = u_first + j * static_cast<int>(blockDim.x);
-            if (u < u_end) store16_as<kPolicy>(out + static_cast<size_t>(row) * units_per_row + u, codes[j]);
-        }
-    }
-    for (int u = u_first + kEarly * static_cast<int>(blockDim.x); u < u_end; u += blockDim.x) {  // rows wider than that
-        const Quant16 q = quantize16(load16(src + 2 * u), load16(src + 2 * u + 1));
-        for (int s = 0; s < num_topk; ++s) {
-            const int row = rows[s];
-            if (row >= 0) store16_as<kPolicy>(out + static_cast<size_t>(row) * units_per_row + u, q.codes);
-        }
-        if ((u & 7) == 0) part_scales[(u - u_begin) >> 3] = q.scale;
-    }
-    __syncthreads();
-    // The part's scales leave as contiguous runs (consecutive lanes, consecutive floats) instead of one
-    // 4-byte store per block of 128, which would turn every scale row into read-modify-write traffic.
-    const int part_cols = (u_end - u_begin) >> 3, col0 = u_begin >> 3;
-    for (int i = threadIdx.x; i < num_topk * part_cols; i += blockDim.x) {
-        const int s = i / part_cols, c = i - s * part_cols;
-        const int row = rows[s];
-        if (row >= 0) out_scales[static_cast<size_t>(row) * scale_cols + col0 + c] = part_scales[c];
-    }
-    if (part == 0 && weights != nullptr && threadIdx.x < num_topk && rows[threadIdx.x] >= 0)
-        out_weights[rows[threadIdx.x]] = weights[static_cast<size_t>(token) * num_topk + threadIdx.x];
+    quant_token<kPolicy>(x, weights, out, out_scales, out_weights, p, tokens, blockIdx.x, threadIdx.x, lds, part_scales);
 }
 
-// row-major: one workgroup per (output row, column part), rows as above; row_to_route == nullptr means identity
-// (row == token), which is the stand-alone quantiser.
 template <int kPolicy>
 __global__ __launch_bounds__(kMaxThreads) void dispatch_quant_row_kernel(
-    const u32x4* __restrict__ x, const float* __restrict__ weights, const int* __restrict__ row_to_route, RowRange range,
-    int num_tokens, int num_topk, int units_per_row, int units_per_part, int parts, u32x4* __restrict__ out,
-    float* __restrict__ out_scales, float* __restrict__ out_weights)
+    const u32x4* __restrict__ x, const float* __restrict__ weights, u32x4* __restrict__ out, float* __restrict__ out_scales,
+    float* __restrict__ out_weights, PayloadShape p, const int* __restrict__ row_to_route,
+    RowRange range)
 {
-    const int part = blockIdx.x % parts, stride = gridDim.x / parts;
-    const int u_begin = part * units_per_part;
-    const int u_end = min(u_begin + units_per_part, units_per_row);
-    const int scale_cols = units_per_row / 8;
-    int row = blockIdx.x / parts;
-    int next_route = row_to_route != nullptr ? row_to_route[row] : row;
-    const int rows = range.count();
-    for (; row < rows; row += stride) {
-        const int route = row_to_route != nullptr ? min(max(next_route, 0), num_tokens * num_topk - 1) : row;
-        if (row_to_route != nullptr && row + stride < rows) next_route = row_to_route[row + stride];
-        const int token = row_to_route != nullptr ? route / num_topk : row;
-        const u32x4* src = x + static_cast<size_t>(token) * units_per_row * 2;
-        for (int u = u_begin + threadIdx.x; u < u_end; u += blockDim.x) {
-            const Quant16 q = quantize16(load16(src + 2 * u), load16(src + 2 * u + 1));
-            store16_as<kPolicy>(out + static_cast<size_t>(row) * units_per_row + u, q.codes);
-            if ((u & 7) == 0) out_scales[static_cast<size_t>(row) * scale_cols + (u >> 3)] = q.scale;
-        }
-        if (part == 0 && weights != nullptr && threadIdx.x == 0) out_weights[row] = weights[route];
-    }
+    quant_rows<kPolicy>(x, weights, out, out_scales, out_weights, p, MappedRows<true>{row_to_route, range}, blockIdx.x, gridDim.x / p.parts, threadIdx.x);
 }
 
 // Stand-alone quantiser for rows whose width is not a multiple of 128: the last block of a row is short and is
@@ -588,31 +343,32 @@ int check_common(const char* what, int num_tokens, int num_topk, int num_rows, c
 
 // One payload launch.  units per row: 16-byte vectors (copy), or 16-value groups (quantise).
 struct Payload {
-    const void* x;
+    const u32x4* x;
     const float* scales;
     const float* weights;
     int num_tokens, num_topk, units, scale_cols;
     bool quantize;
-    void* out;
+    u32x4* out;
     float* out_scales;
     float* out_weights;
 };
+
+PayloadShape payload_shape(const Payload& p, const Split& sp)
+{
+    return {p.num_tokens, p.num_topk, p.units, sp.per_part, sp.parts, sp.threads, p.scale_cols};
+}
 
 // token-major: the grid does not depend on R; rows at or beyond `capacity` are dropped; all_rows: all of them unless DPEP_ROWS_KEPT.
 int launch_token_major(const Payload& p, const int32_t* route_to_row, int capacity, const int32_t* all_rows, hipStream_t s)
 {
     const Split sp = choose_split(p.num_tokens, p.units, p.quantize ? 8 : 1);
     const dim3 grid(p.num_tokens * sp.parts), block(sp.threads);
+    const MappedTokens tokens = {route_to_row, capacity, all_rows};
     with_store_policy([&](auto policy) {
         constexpr int kPolicy = decltype(policy)::value;
-        if (p.quantize)
-            hipLaunchKernelGGL(dispatch_quant_token_kernel<kPolicy>, grid, block, 0, s, static_cast<const u32x4*>(p.x), p.weights,
-                               route_to_row, p.num_topk, p.units, sp.per_part, sp.parts, capacity, all_rows,
-                               static_cast<u32x4*>(p.out), p.out_scales, p.out_weights);
-        else
-            hipLaunchKernelGGL(dispatch_copy_token_kernel<kPolicy>, grid, block, 0, s, static_cast<const u32x4*>(p.x), p.scales,
-                               p.weights, route_to_row, p.num_topk, p.units, sp.per_part, sp.parts, p.scale_cols, capacity, all_rows,
-                               static_cast<u32x4*>(p.out), p.out_scales, p.out_weights);
+        if (p.quantize) hipLaunchKernelGGL(dispatch_quant_token_kernel<kPolicy>, grid, block, 0, s, p.x, p.weights, p.out, p.out_scales, p.out_weights, payload_shape(p, sp), tokens);
+        else hipLaunchKernelGGL(dispatch_copy_token_kernel<kPolicy>, grid, block, 0, s, p.x, p.scales, p.weights, p.out, p.out_scales, p.out_weights,
+                                payload_shape(p, sp), tokens);
     });
     return launch_status("dispatch_token");
 }
@@ -624,14 +380,10 @@ int launch_row_major(const Payload& p, const int32_t* row_to_route, const RowRan
     const dim3 grid(grid_rows * sp.parts), block(sp.threads);
     with_store_policy([&](auto policy) {
         constexpr int kPolicy = decltype(policy)::value;
-        if (p.quantize)
-            hipLaunchKernelGGL(dispatch_quant_row_kernel<kPolicy>, grid, block, 0, s, static_cast<const u32x4*>(p.x), p.weights,
-                               row_to_route, range, p.num_tokens, p.num_topk, p.units, sp.per_part, sp.parts,
-                               static_cast<u32x4*>(p.out), p.out_scales, p.out_weights);
-        else
-            hipLaunchKernelGGL(dispatch_copy_row_kernel<kPolicy>, grid, block, 0, s, static_cast<const u32x4*>(p.x), p.scales,
-                               p.weights, row_to_route, range, p.num_tokens, p.num_topk, p.units, sp.per_part, sp.parts,
-                               p.scale_cols, static_cast<u32x4*>(p.out), p.out_scales, p.out_weights);
+        if (p.quantize) hipLaunchKernelGGL(dispatch_quant_row_kernel<kPolicy>, grid, block, 0, s, p.x, p.weights, p.out, p.out_scales, p.out_weights, payload_shape(p, sp),
+                               row_to_route, range);
+        else hipLaunchKernelGGL(dispatch_copy_row_kernel<kPolicy>, grid, block, 0, s, p.x, p.scales, p.weights, p.out, p.out_scales, p.out_weights,
+                                payload_shape(p, sp), row_to_route, range);
     });
     return launch_status("dispatch_row");
 }
@@ -710,7 +462,8 @@ int fresh_in_one_launch(Workspace* w, const dpep_fresh_dispatch& c, hipStream_t 
 
 }  // namespace
 
-int layout_of_fresh(void* ws, const dpep_fresh_dispatch& c, hipStream_t stream);
+// (layout.hip) *payload_launched: whether `payload` went along.
+int layout_of_fresh(void* ws, const dpep_fresh_dispatch& c, const LayoutPayload* payload, bool* payload_launched, hipStream_t stream);
 
 }  // namespace dpep
 
@@ -741,7 +494,8 @@ int dpep_dispatch_copy(const void* x, const float* scales, const float* topk_wei
     DPEP_REQUIRE(scales == nullptr || scale_cols > 0, "dispatch_copy: scale_cols must be positive with scales");
     DPEP_REQUIRE((topk_weights == nullptr) == (out_weights == nullptr), "dispatch_copy: weights and out_weights go together");
     DPEP_REQUIRE(x != nullptr && out != nullptr && aligned16(x) && aligned16(out), "dispatch_copy: x/out must be 16-byte aligned");
-    const Payload p = {x, scales, topk_weights, num_tokens, num_topk, row_bytes / 16, scale_cols, false, out, out_scales, out_weights};
+    const Payload p = {static_cast<const u32x4*>(x), scales, topk_weights, num_tokens, num_topk, row_bytes / 16, scale_cols, false, static_cast<u32x4*>(out),
+                       out_scales, out_weights};
     return launch_payload(p, route_to_row, row_to_route, num_rows, static_cast<hipStream_t>(stream));
 }
 
@@ -756,7 +510,8 @@ int dpep_dispatch_quant_fp8(const void* x, const float* topk_weights, const int3
     if (num_rows == 0 || num_tokens == 0) return DPEP_OK;  // (empty outputs may be null pointers)
     DPEP_REQUIRE((topk_weights == nullptr) == (out_weights == nullptr), "dispatch_quant_fp8: weights and out_weights go together");
     DPEP_REQUIRE(x && out && out_scales && aligned16(x) && aligned16(out), "dispatch_quant_fp8: x/out must be 16-byte aligned");
-    const Payload p = {x, nullptr, topk_weights, num_tokens, num_topk, hidden / 16, 0, true, out, out_scales, out_weights};
+    const Payload p = {static_cast<const u32x4*>(x), nullptr, topk_weights, num_tokens, num_topk, hidden / 16, 0, true, static_cast<u32x4*>(out),
+                       out_scales, out_weights};
     return launch_payload(p, route_to_row, row_to_route, num_rows, static_cast<hipStream_t>(stream));
 }
 
@@ -774,10 +529,8 @@ int dpep_dispatch_fresh(void* ws, const dpep_fresh_dispatch* call, void* stream)
         int units = 0;
         if (int rc = check_fresh_payload("dispatch_fresh", c, &units)) return rc;
         DPEP_REQUIRE(c.capacity_rows >= 0, "dispatch_fresh: capacity_rows=%d is negative", c.capacity_rows);
-        if (int rc = layout_of_fresh(ws, c, s)) return rc;  // (checks the routing arguments)
-        if (c.capacity_rows == 0) return DPEP_OK;
-        const Payload p = {c.x, c.scales, c.topk_weights, c.num_tokens, c.num_topk, units, c.quantize ? 0 : c.scale_cols,
-                           c.quantize != 0, c.out, c.out_scales, c.out_weights};
+        const Payload p = {static_cast<const u32x4*>(c.x), c.scales, c.topk_weights, c.num_tokens, c.num_topk, units, c.quantize ? 0 : c.scale_cols,
+                           c.quantize != 0, static_cast<u32x4*>(c.out), c.out_scales, c.out_weights};
         // Expected rows of this rank's share: what the caller made its outputs for, or the even share.  Many rows per token:
         // token-major, which reads every token once.  Otherwise row-major over the rows that the layout finds: a token-major
         // grid is mostly workgroups of tokens without a row (6144 tokens of which 560 own a row: 10.5 us).  16 384 BF16
@@ -786,12 +539,32 @@ int dpep_dispatch_fresh(void* ws, const dpep_fresh_dispatch* call, void* stream)
         const bool all_or_none = c.report_to_host == DPEP_REPORT_ALL_OR_NONE;
         const long long expected =
             all_or_none ? (c.capacity_rows > 256 ? (c.capacity_rows - 256LL) * 8 / 9 : 0) : n_routes * c.num_local / c.num_experts;
-        if (expected > static_cast<long long>(kRowMajorRatio) * c.num_tokens)
-            return launch_token_major(p, c.route_to_row, c.capacity_rows, all_or_none ? c.num_rows : nullptr, s);
+        const bool token_major = expected > static_cast<long long>(kRowMajorRatio) * c.num_tokens;
         long long grid_rows = expected + expected / 8 + 64;
         if (grid_rows > c.capacity_rows) grid_rows = c.capacity_rows;
         if (grid_rows > n_routes) grid_rows = n_routes;
         const int bound = n_routes < c.capacity_rows ? static_cast<int>(n_routes) : c.capacity_rows;
+        // In the layout's grid (launch_layout), where that is the better place.  A large token-major payload with several rows to a token ends
+        // 1 to 15 us sooner there; beside a small one the GPU waits for the host, and the layout reports to it 0.5 to 3 us later with a
+        // payload in its grid (dispatch and combine: 39 MB 33.0 -> 31.9 us, 43 MB 39.0 -> 34.6, 152 MB 91.8 -> 87.8, 18 MB 22.7 -> 23.5, 13 MB
+        // 25.2 -> 28.1; 1.25 rows per token, 41 MB 39.8 -> 46.8, 142 MB 197.5 and 196.7).  Row-major workgroups wait for their row before they
+        // can ask for its values, so it is only the launch that is saved, which counts where nothing is reported and the host is
+        // the one to wait for: 0.4 to 2 MB 17 -> 14 us, 4 MB 28.3 and 28.4, 10 MB 60.5 -> 63.1, 117 MB 124 -> 156.
+        LayoutPayload riding = {};
+        const long long payload_bytes = expected * (c.quantize ? c.row_bytes / 2 : c.row_bytes);
+        const bool worth_it = token_major ? payload_bytes >= (32LL << 20) && expected >= 5LL * c.num_tokens
+                                          : c.report_to_host == 0 && payload_bytes <= (3LL << 20);
+        const bool may_ride = worth_it && c.capacity_rows > 0 && dpep_dispatch_store_policy(DPEP_STORE_QUERY) == DPEP_STORE_STREAMING;
+        if (may_ride) {
+            const int lines = token_major ? c.num_tokens : static_cast<int>(grid_rows);
+            const Split sp = choose_split(lines, units, c.quantize ? 8 : 1);
+            riding = {p.x, p.scales, p.weights, p.out, p.out_scales, p.out_weights, payload_shape(p, sp), c.quantize != 0, !token_major, static_cast<unsigned>(lines) * sp.parts, bound, c.capacity_rows,
+                      all_or_none ? c.capacity_rows : 0};
+        }
+        bool launched = false;
+        if (int rc = layout_of_fresh(ws, c, may_ride ? &riding : nullptr, &launched, s)) return rc;  // (checks the routing arguments)
+        if (launched || c.capacity_rows == 0) return DPEP_OK;
+        if (token_major) return launch_token_major(p, c.route_to_row, c.capacity_rows, all_or_none ? c.num_rows : nullptr, s);
         return launch_row_major(p, c.row_to_route, RowRange{bound, c.num_rows, all_or_none ? c.capacity_rows : 0}, static_cast<int>(grid_rows), s);
     }
     return fresh_in_one_launch(w, c, s);
@@ -830,11 +603,11 @@ int dpep_cast_to_fp8(const void* x, int num_tokens, int hidden, void* out, float
         return launch_status("cast_to_fp8");
     }
     const Split sp = choose_split(num_tokens, units, 8);
+    const PayloadShape shape = {num_tokens, 1, units, sp.per_part, sp.parts, sp.threads, 0};
     auto launch = [&](auto policy) {
-        hipLaunchKernelGGL(dispatch_quant_row_kernel<decltype(policy)::value>, dim3(num_tokens * sp.parts),
-                           dim3(sp.threads), 0, static_cast<hipStream_t>(stream), static_cast<const u32x4*>(x), nullptr,
-                           nullptr, RowRange{num_tokens, nullptr, 0}, num_tokens, 1, units, sp.per_part, sp.parts,
-                           static_cast<u32x4*>(out), out_scales, nullptr);
+        hipLaunchKernelGGL(dispatch_quant_row_kernel<decltype(policy)::value>, dim3(num_tokens * sp.parts), dim3(sp.threads), 0,
+                           static_cast<hipStream_t>(stream), static_cast<const u32x4*>(x), nullptr, static_cast<u32x4*>(out), out_scales, nullptr, shape,
+                           nullptr, RowRange{num_tokens, nullptr, 0});
     };
     // (codes that the memory-side cache takes are written through, whatever the dispatch's policy: the quantiser's reader is next.
     // 10007 x 5120: quantise and dequantise 47.7 us instead of 53.2)

@@ -27,6 +27,7 @@
 
 #include "common.h"
 #include "mx.h"
+#include "payload.h"
 
 namespace dpep {
 namespace {
@@ -235,6 +236,11 @@ constexpr unsigned long long kCountMask = (1ull << kCountBits) - 1ull;
 __device__ __forceinline__ unsigned long long load_word(const unsigned long long* src)
 {
     return __hip_atomic_load(src, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+__device__ __forceinline__ void store_word(unsigned long long* dst, unsigned long long word)
+{
+    __hip_atomic_store(dst, word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // The workgroup's histogram (sum of its waves') out to its row of `tagged`.  Called by all threads, after a workgroup
@@ -481,21 +487,17 @@ __global__ __launch_bounds__(kThreads) void layout_assign_kernel(
 // (quantise or pad them), which does not depend on the routing, and every workgroup of the layout writes a piece of the shared
 // experts' rows once it knows R: up to three launches fewer (777 tokens of 2880 BF16 columns with a shared expert: layout 8.3 +
 // quantise 4.1 + pad 3.3 + shared rows 1.9 us as launches of their own).
-template <typename IdxT, bool kMega, int kSteps>
-__global__ __launch_bounds__(kThreads) void layout_fused_kernel(
-    const IdxT* __restrict__ idx, int n_routes, int num_experts, int expert_begin, int num_local, int padded_local,
+// What the layout's workgroups do.  kWords: a payload in the same grid waits for the rows of the routes (1) or the routes of the rows (2).
+template <typename IdxT, bool kMega, int kSteps, int kWords, typename Lds>
+__device__ __forceinline__ void fused_layout(
+    Lds& lds, const IdxT* __restrict__ idx, int n_routes, int num_experts, int expert_begin, int num_local, int padded_local,
     int chunk, int num_chunks, int* __restrict__ counts, int* __restrict__ psum, int* __restrict__ offsets,
     int* __restrict__ num_rows, int* __restrict__ route_to_row, int* __restrict__ row_to_route, IdxT* __restrict__ idx_copy,
     SendCounts send, uint32_t* __restrict__ mailbox, uint32_t sequence, unsigned long long* __restrict__ epoch,
     unsigned long long* __restrict__ tagged, int num_blocks, int rows, long long limit_ticks, uint32_t* __restrict__ timeouts,
-    uint32_t launch_id, MegaFront front)
+    uint32_t launch_id, const MegaFront& front,
+    unsigned long long* __restrict__ total_word = nullptr, unsigned long long* __restrict__ row_words = nullptr)
 {
-    __shared__ LayoutLds<kMega ? kMegaExperts : DPEP_MAX_LOCAL_EXPERTS, true> lds;
-    if (kMega && static_cast<int>(blockIdx.x) > num_blocks) {
-        __shared__ __attribute__((aligned(16))) uint8_t staged[kFrontThreads / 2];
-        prepare_rows<kFrontThreads>(front, blockIdx.x - num_blocks - 1, staged);
-        return;
-    }
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int g = blockIdx.x * kWaves + wave;
     const int begin = g < num_chunks ? g * chunk : 0;
@@ -533,6 +535,8 @@ __global__ __launch_bounds__(kThreads) void layout_fused_kernel(
     const TaggedSource source = {tagged, tag, rows, reporter ? limit_ticks : 2 * limit_ticks, timeouts, launch_id};
     const bool in_time = expert_bases<true>(lds, nullptr, nullptr, n_routes, num_local, padded_local, num_chunks, num_blocks, counts, psum,
                                             offsets, num_rows, send, mailbox, sequence, &source);
+    if (kWords != 0 && reporter && threadIdx.x == 0)  // (0 where the exchange ran out of time)
+        store_word(total_word, row_word(launch_id, lds.wave_sums[0] + lds.wave_sums[1] + lds.wave_sums[2] + lds.wave_sums[3]));
     // (asked for here, needed only at the very end: the load travels while the routes are assigned)
     unsigned long long reporter_seen = threadIdx.x == 0 && !reporter ? load_word(reporter_tag) : 0ull;
     if (in_time) {
@@ -543,12 +547,17 @@ __global__ __launch_bounds__(kThreads) void layout_fused_kernel(
                 const int row = experts[i] >= 0 ? lds.running[wave][experts[i]] + rank[i] : -1;
                 route_to_row[route] = row;
                 if (row >= 0) row_to_route[row] = route;
+                if (kWords == 1) store_word(row_words + route, row_word(launch_id, row));
+                if (kWords == 2 && row >= 0) store_word(row_words + row, row_word(launch_id, route));
             }
         }
     } else {
         // Some workgroup's histogram is missing: rows computed without it could lie anywhere.  No route gets a row
         // (and the counts above are all zero).
-        for (int route = begin + lane; route < end; route += kWave) route_to_row[route] = -1;
+        for (int route = begin + lane; route < end; route += kWave) {
+            route_to_row[route] = -1;
+            if (kWords == 1) store_word(row_words + route, row_word(launch_id, -1));
+        }
     }
     if (kMega && front.num_shared > 0)  // (R = 0 where the exchange ran out of time)
         shared_rows(front, lds.wave_sums[0] + lds.wave_sums[1] + lds.wave_sums[2] + lds.wave_sums[3], num_local, offsets, row_to_route,
@@ -570,6 +579,76 @@ __global__ __launch_bounds__(kThreads) void layout_fused_kernel(
             }
         }
         __hip_atomic_fetch_max(epoch, tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+}
+
+template <typename IdxT, bool kMega, int kSteps>
+__global__ __launch_bounds__(kThreads) void layout_fused_kernel(
+    const IdxT* __restrict__ idx, int n_routes, int num_experts, int expert_begin, int num_local, int padded_local,
+    int chunk, int num_chunks, int* __restrict__ counts, int* __restrict__ psum, int* __restrict__ offsets,
+    int* __restrict__ num_rows, int* __restrict__ route_to_row, int* __restrict__ row_to_route, IdxT* __restrict__ idx_copy,
+    SendCounts send, uint32_t* __restrict__ mailbox, uint32_t sequence, unsigned long long* __restrict__ epoch,
+    unsigned long long* __restrict__ tagged, int num_blocks, int rows, long long limit_ticks, uint32_t* __restrict__ timeouts,
+    uint32_t launch_id, MegaFront front)
+{
+    __shared__ LayoutLds<kMega ? kMegaExperts : DPEP_MAX_LOCAL_EXPERTS, true> lds;
+    if (kMega && static_cast<int>(blockIdx.x) > num_blocks) {
+        __shared__ __attribute__((aligned(16))) uint8_t staged[kFrontThreads / 2];
+        prepare_rows<kFrontThreads>(front, blockIdx.x - num_blocks - 1, staged);
+        return;
+    }
+    fused_layout<IdxT, kMega, kSteps, 0>(lds, idx, n_routes, num_experts, expert_begin, num_local, padded_local, chunk, num_chunks, counts, psum, offsets, num_rows, route_to_row, row_to_route, idx_copy, send, mailbox, sequence, epoch, tagged, num_blocks, rows, limit_ticks, timeouts, launch_id, front);
+}
+
+// ---- layout and payload in one grid ------------------------------------------------------------------------------------
+// The payload's workgroups, behind the layout's in the same grid, ask for their tokens at once and wait for the words that say where
+// these go: between the routes' ids and the first payload store there is no second launch, whose ramp and first loads would follow
+// the layout's last store.  A wait is short of a deadlock whatever else runs: the layout's workgroups come first in
+// the grid and wait for no payload, and every wait is bounded.  The words carry the number of the launch, which comes from the host, so a
+// captured launch (whose replays would repeat it) takes two.  128 registers, as the layout wants: four workgroups to a CU carry the payload
+// as fast as eight (with 64 the layout spills, and the kernel takes 7 us longer).
+// Bound by HBM once the words are there.  Dispatch and combine, launches back to back, one grid / two: 1000 tokens x top-6 of 5120 BF16 30.5 / 31.7 us,
+// 618 x 7 of 5824 28.8 / 32.7, 3407 x 6 of 1584 37.5 / 42.5, 4372 x 7 of 5840 169.5 / 177.2.  Up to kSingleRoutes routes the layout's
+// workgroup of its own is the better one (710 x 4 of 2672 20.1 / 18.7).
+constexpr int kRidingExperts = 256;
+template <int kSteps, bool kQuant, bool kRowMajor>
+__global__ __launch_bounds__(kThreads, 4) void layout_payload_kernel(
+    const int64_t* __restrict__ idx, int n_routes, int num_experts, int expert_begin, int num_local, int padded_local,
+    int chunk, int num_chunks, int* __restrict__ counts, int* __restrict__ psum, int* __restrict__ offsets,
+    int* __restrict__ num_rows, int* __restrict__ route_to_row, int* __restrict__ row_to_route, int64_t* __restrict__ idx_copy,
+    SendCounts send, uint32_t* __restrict__ mailbox, uint32_t sequence, unsigned long long* __restrict__ epoch,
+    unsigned long long* __restrict__ tagged, int num_blocks, int rows, long long limit_ticks, uint32_t* __restrict__ timeouts,
+    uint32_t launch_id,
+    unsigned long long* __restrict__ total_word, unsigned long long* __restrict__ row_words, LayoutPayload payload)
+{
+    using Lds = LayoutLds<kRidingExperts, true>;
+    struct Riding {
+        TokenLds tokens[kWaves];
+        float scales[kQuant && !kRowMajor ? kMaxScaleCols : 1];
+    };
+    __shared__ union Both {
+        Lds layout;
+        Riding riding;
+        __device__ Both() {}
+    } lds;
+    if (static_cast<int>(blockIdx.x) <= num_blocks) {
+        fused_layout<int64_t, false, kSteps, kRowMajor ? 2 : 1>(lds.layout, idx, n_routes, num_experts, expert_begin, num_local, padded_local, chunk, num_chunks, counts, psum, offsets, num_rows, route_to_row, row_to_route, idx_copy, send, mailbox, sequence, epoch, tagged, num_blocks, rows, limit_ticks, timeouts, launch_id, MegaFront{}, total_word, row_words);
+        return;
+    }
+    // Payload workgroups of fewer threads share one of these: `per` of them, each of whole waves.
+    const PayloadShape& p = payload.shape;
+    const int per = kThreads / p.threads, sub = threadIdx.x / p.threads, t = threadIdx.x - sub * p.threads;
+    const unsigned block = (blockIdx.x - num_blocks - 1) * per + sub;
+    if (sub >= per || block >= payload.blocks) return;  // (whole waves)
+    const AwaitedWords words = {row_words, total_word, launch_id, 4 * limit_ticks, timeouts, kRowMajor ? 16 : 8};
+    if (kRowMajor) {
+        const AwaitedRows rows = {words, payload.rows, payload.all_or_none};
+        if (kQuant) quant_rows<DPEP_STORE_STREAMING>(payload.x, payload.weights, payload.out, payload.out_scales, payload.out_weights, p, rows, block, payload.blocks / p.parts, t);
+        else copy_rows<DPEP_STORE_STREAMING>(payload.x, payload.scales, payload.weights, payload.out, payload.out_scales, payload.out_weights, p, rows, block, payload.blocks / p.parts, t);
+    } else {
+        const AwaitedTokens tokens = {words, payload.capacity, payload.all_or_none};
+        if (kQuant) quant_token<DPEP_STORE_STREAMING>(payload.x, payload.weights, payload.out, payload.out_scales, payload.out_weights, p, tokens, block, t, lds.riding.tokens[sub], lds.riding.scales + sub * (p.threads / 8));
+        else copy_token<DPEP_STORE_STREAMING>(payload.x, payload.scales, payload.weights, payload.out, payload.out_scales, payload.out_weights, p, tokens, block, t, lds.riding.tokens[sub]);
     }
 }
 
@@ -743,11 +822,17 @@ int enqueue_count_and_assign(const IdxT* idx, int n_routes, int num_experts, int
     return launch_status("layout_assign");
 }
 
+bool is_capturing(hipStream_t s)
+{
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(s, &status) != hipSuccess || status != hipStreamCaptureStatusNone;
+}
+
 template <typename IdxT>
 int launch_layout(void* ws, const IdxT* idx, int num_tokens, int num_topk, int num_experts, int expert_begin,
                   int num_local, int32_t* counts, int32_t* psum, int32_t* offsets, int32_t* route_to_row,
                   int32_t* row_to_route, int32_t* num_rows, IdxT* idx_copy, const SendCounts& send, bool report_to_host,
-                  const MegaFront* front, hipStream_t stream)
+                  const MegaFront* front, const LayoutPayload* payload, bool* payload_launched, hipStream_t stream)
 {
     Workspace* w = as_workspace(ws);
     DPEP_REQUIRE(w != nullptr, "layout: not a live workspace");
@@ -807,6 +892,30 @@ int launch_layout(void* ws, const IdxT* idx, int num_tokens, int num_topk, int n
                                reinterpret_cast<unsigned long long*>(sync + kSyncTagged), blocks, blocks + w->exchange_extra_rows,
                                w->exchange_ticks, w->mailbox_device + kMailboxTimeout, w->layout_launches, f);
         };
+        // The payload rides along where the words have room for every route and the launch is not captured.
+        if (payload != nullptr && chunk <= 8 * kWave && num_local <= kRidingExperts && n_routes <= kSyncRowWords && !is_capturing(stream)) {
+            if constexpr (std::is_same_v<IdxT, int64_t>) {
+                const unsigned per = kThreads / payload->shape.threads, more = (payload->blocks + per - 1) / per;
+                auto ride = [&](auto kernel) {
+                    hipLaunchKernelGGL(kernel, dim3(blocks + 1 + more), dim3(kThreads), 0, stream, idx, n_routes, num_experts, expert_begin,
+                                       num_local, padded, chunk, num_chunks, counts, psum, offsets, num_rows, route_to_row, row_to_route,
+                                       idx_copy, send, mailbox, w->sequence, reinterpret_cast<unsigned long long*>(sync),
+                                       reinterpret_cast<unsigned long long*>(sync + kSyncTagged), blocks, blocks + w->exchange_extra_rows,
+                                       w->exchange_ticks, w->mailbox_device + kMailboxTimeout, w->layout_launches,
+                                       reinterpret_cast<unsigned long long*>(sync + kSyncTotal), reinterpret_cast<unsigned long long*>(sync + kSyncRows),
+                                       *payload);
+                };
+                auto ride_steps = [&](auto steps_constant) {
+                    constexpr int kSteps = decltype(steps_constant)::value;
+                    if (payload->row_major) payload->quantize ? ride(layout_payload_kernel<kSteps, true, true>) : ride(layout_payload_kernel<kSteps, false, true>);
+                    else payload->quantize ? ride(layout_payload_kernel<kSteps, true, false>) : ride(layout_payload_kernel<kSteps, false, false>);
+                };
+                if (chunk <= 4 * kWave) ride_steps(std::integral_constant<int, 4>{});
+                else ride_steps(std::integral_constant<int, 8>{});
+                *payload_launched = true;
+                return launch_status("layout_payload");
+            }
+        }
         auto launch_steps = [&](auto steps_constant) {
             constexpr int kSteps = decltype(steps_constant)::value;
             if (front != nullptr) launch(layout_fused_kernel<IdxT, true, kSteps>, front_blocks(*front, kFrontThreads), *front);
@@ -839,15 +948,15 @@ int layout_i32(void* ws, const int32_t* idx, int num_tokens, int num_topk, int n
 {
     DPEP_REQUIRE(num_local <= kMegaExperts, "layout: %d local experts, at most %d", num_local, kMegaExperts);
     return launch_layout<int32_t>(ws, idx, num_tokens, num_topk, num_experts, expert_begin, num_local, counts, psum,
-                                  offsets, route_to_row, row_to_route, num_rows, nullptr, SendCounts{}, /*report_to_host=*/false, &front, stream);
+                                  offsets, route_to_row, row_to_route, num_rows, nullptr, SendCounts{}, /*report_to_host=*/false, &front, nullptr, nullptr, stream);
 }
 
-// The layout of a fresh dispatch (dpep_dispatch_fresh).
-int layout_of_fresh(void* ws, const dpep_fresh_dispatch& c, hipStream_t stream)
+// The layout of a fresh dispatch (dpep_dispatch_fresh), and its payload, if it may ride along.
+int layout_of_fresh(void* ws, const dpep_fresh_dispatch& c, const LayoutPayload* payload, bool* payload_launched, hipStream_t stream)
 {
     return launch_layout<int64_t>(ws, c.topk_idx, c.num_tokens, c.num_topk, c.num_experts, c.expert_begin, c.num_local, c.counts,
                                   c.psum, c.offsets, c.route_to_row, c.row_to_route, c.num_rows, c.topk_idx_copy,
-                                  SendCounts{c.send_counts, c.expert_begin, c.num_experts}, c.report_to_host != 0, nullptr, stream);
+                                  SendCounts{c.send_counts, c.expert_begin, c.num_experts}, c.report_to_host != 0, nullptr, payload, payload_launched, stream);
 }
 
 }  // namespace dpep
@@ -904,7 +1013,7 @@ int dpep_layout(void* ws, const int64_t* topk_idx, int num_tokens, int num_topk,
 {
     return dpep::launch_layout<int64_t>(ws, topk_idx, num_tokens, num_topk, num_experts, expert_begin, num_local,
                                         counts, psum, offsets, route_to_row, row_to_route, num_rows, nullptr, dpep::SendCounts{},
-                                        /*report_to_host=*/true, nullptr, static_cast<hipStream_t>(stream));
+                                        /*report_to_host=*/true, nullptr, nullptr, nullptr, static_cast<hipStream_t>(stream));
 }
 
 int dpep_layout_static(const int64_t* topk_idx, int num_tokens, int num_topk, int num_experts, int expert_begin,

@@ -161,7 +161,7 @@ int dpep_layout_dispatch_small(void* ws, const int64_t* topk_idx, const void* x,
                                float* out_scales, float* out_weights, void* stream);
 
 /* One fresh dispatch as ElasticBuffer makes it (notify + dispatch, deep_ep/backends/mesh_clos/elastic.py:648-1008): the layout
- * and, queued behind it before the host knows R, the payload; for a small batch both in one launch (see above).  The
+ * and, queued behind it or in the same grid before the host knows R, the payload; for a small batch both in one launch (see above).  The
  * payload outputs hold capacity_rows rows, of which the first min(R, capacity_rows) are written: a caller that finds
  * R > capacity_rows allocates R rows and calls dpep_dispatch_copy / dpep_dispatch_quant_fp8 with the same maps.  One that does
  * so whenever DPEP_ROWS_KEPT says that the outputs are too small, or mostly unused, sets report_to_host to
