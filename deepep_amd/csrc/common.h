@@ -72,7 +72,7 @@ constexpr size_t kSyncTagged = 256;
 constexpr size_t kSyncTaggedWords = 4096 + DPEP_MAX_LOCAL_EXPERTS;  // (workgroups + 1) * experts never exceeds this
 constexpr size_t kSyncTotal = kSyncTagged + kSyncTaggedWords * 8;
 constexpr size_t kSyncRows = kSyncTotal + 256;
-constexpr int kSyncRowWords = 131072;
+constexpr int kSyncRowWords = 65536;
 constexpr size_t kSyncBytes = kSyncRows + static_cast<size_t>(kSyncRowWords) * 8;
 // The host mailbox (pinned memory, 32-bit words): word 0 = number of rows and word 1 = sequence number of the layout
 // that reported last (one 8-byte store); word kMailboxTimeout = launch number of a layout kernel whose wait for the

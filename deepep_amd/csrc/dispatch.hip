@@ -48,13 +48,51 @@ __global__ __launch_bounds__(kMaxThreads) void dispatch_copy_token_kernel(
     copy_token<kPolicy>(x, scales, weights, out, out_scales, out_weights, p, tokens, blockIdx.x, threadIdx.x, lds);
 }
 
+// ---- row-major: one workgroup per (output row, column part); for sparse receive shares -------------
+// Rows [0, rows): `rows` from the host, or, rows_on_device, the smaller of that bound and the count the layout left on the
+// device (a payload queued before the host knows R); all_or_none, the outputs' capacity: no rows at all unless DPEP_ROWS_KEPT
+// (0: the first rows in any case).  Such a launch has workgroups for about the expected number of rows;
+// they walk on by the grid's rows until the real count is reached, and the first row's route is asked for together with
+// the count (row_to_route has an entry for every row of the grid, so the load is in bounds whatever the count says).
+struct RowRange {
+    int rows;
+    const int* rows_on_device;
+    int all_or_none;
+    __device__ __forceinline__ int count() const
+    {
+        if (rows_on_device == nullptr) return rows;
+        const int all = *rows_on_device;
+        return all_or_none == 0 || DPEP_ROWS_KEPT(all, all_or_none) ? min(all, rows) : 0;
+    }
+};
+
 template <int kPolicy>
 __global__ __launch_bounds__(kMaxThreads) void dispatch_copy_row_kernel(
-    const u32x4* __restrict__ x, const float* __restrict__ scales, const float* __restrict__ weights, u32x4* __restrict__ out,
-    float* __restrict__ out_scales, float* __restrict__ out_weights, PayloadShape p, const int* __restrict__ row_to_route,
-    RowRange range)
+    const u32x4* __restrict__ x, const float* __restrict__ scales, const float* __restrict__ weights,
+    const int* __restrict__ row_to_route, RowRange range, int num_tokens, int num_topk, int vec_per_row, int vec_per_part,
+    int parts, int scale_cols, u32x4* __restrict__ out, float* __restrict__ out_scales, float* __restrict__ out_weights)
 {
-    copy_rows<kPolicy>(x, scales, weights, out, out_scales, out_weights, p, MappedRows<false>{row_to_route, range}, blockIdx.x, gridDim.x / p.parts, threadIdx.x);
+    const int part = blockIdx.x % parts, stride = gridDim.x / parts;
+    const int v_begin = part * vec_per_part;
+    const int v_end = min(v_begin + vec_per_part, vec_per_row);
+    int row = blockIdx.x / parts;
+    int next_route = row_to_route[row];
+    const int rows = range.count();
+    for (; row < rows; row += stride) {
+        // (clamped: a map left incomplete by a layout launch that reported a time-out must not become a wild address)
+        const int route = min(max(next_route, 0), num_tokens * num_topk - 1);
+        if (row + stride < rows) next_route = row_to_route[row + stride];
+        const int token = route / num_topk;
+        const u32x4* src = x + static_cast<size_t>(token) * vec_per_row;
+        u32x4* dst = out + static_cast<size_t>(row) * vec_per_row;
+        for (int v = v_begin + threadIdx.x; v < v_end; v += blockDim.x) store16_as<kPolicy>(dst + v, load16(src + v));
+        if (part == 0) {
+            if (scales != nullptr)
+                for (int c = threadIdx.x; c < scale_cols; c += blockDim.x)
+                    out_scales[static_cast<size_t>(row) * scale_cols + c] = scales[static_cast<size_t>(token) * scale_cols + c];
+            if (weights != nullptr && threadIdx.x == 0) out_weights[row] = weights[route];
+        }
+    }
 }
 
 template <int kPolicy>
@@ -67,13 +105,33 @@ __global__ __launch_bounds__(kMaxThreads) void dispatch_quant_token_kernel(
     quant_token<kPolicy>(x, weights, out, out_scales, out_weights, p, tokens, blockIdx.x, threadIdx.x, lds, part_scales);
 }
 
+// row-major: one workgroup per (output row, column part), rows as above; row_to_route == nullptr means identity
+// (row == token), which is the stand-alone quantiser.
 template <int kPolicy>
 __global__ __launch_bounds__(kMaxThreads) void dispatch_quant_row_kernel(
-    const u32x4* __restrict__ x, const float* __restrict__ weights, u32x4* __restrict__ out, float* __restrict__ out_scales,
-    float* __restrict__ out_weights, PayloadShape p, const int* __restrict__ row_to_route,
-    RowRange range)
+    const u32x4* __restrict__ x, const float* __restrict__ weights, const int* __restrict__ row_to_route, RowRange range,
+    int num_tokens, int num_topk, int units_per_row, int units_per_part, int parts, u32x4* __restrict__ out,
+    float* __restrict__ out_scales, float* __restrict__ out_weights)
 {
-    quant_rows<kPolicy>(x, weights, out, out_scales, out_weights, p, MappedRows<true>{row_to_route, range}, blockIdx.x, gridDim.x / p.parts, threadIdx.x);
+    const int part = blockIdx.x % parts, stride = gridDim.x / parts;
+    const int u_begin = part * units_per_part;
+    const int u_end = min(u_begin + units_per_part, units_per_row);
+    const int scale_cols = units_per_row / 8;
+    int row = blockIdx.x / parts;
+    int next_route = row_to_route != nullptr ? row_to_route[row] : row;
+    const int rows = range.count();
+    for (; row < rows; row += stride) {
+        const int route = row_to_route != nullptr ? min(max(next_route, 0), num_tokens * num_topk - 1) : row;
+        if (row_to_route != nullptr && row + stride < rows) next_route = row_to_route[row + stride];
+        const int token = row_to_route != nullptr ? route / num_topk : row;
+        const u32x4* src = x + static_cast<size_t>(token) * units_per_row * 2;
+        for (int u = u_begin + threadIdx.x; u < u_end; u += blockDim.x) {
+            const Quant16 q = quantize16(load16(src + 2 * u), load16(src + 2 * u + 1));
+            store16_as<kPolicy>(out + static_cast<size_t>(row) * units_per_row + u, q.codes);
+            if ((u & 7) == 0) out_scales[static_cast<size_t>(row) * scale_cols + (u >> 3)] = q.scale;
+        }
+        if (part == 0 && weights != nullptr && threadIdx.x == 0) out_weights[row] = weights[route];
+    }
 }
 
 // Stand-alone quantiser for rows whose width is not a multiple of 128: the last block of a row is short and is
@@ -309,15 +367,14 @@ __global__ __launch_bounds__(kMaxThreads) void layout_dispatch_small_kernel(
 }
 
 // Split a row of `units` work items over `parts` workgroups so that a launch of `rows` rows has
-// enough workgroups to fill 256 CUs; each part is a multiple of `granule` units.
+// enough workgroups (target_blocks) to fill 256 CUs; each part is a multiple of `granule` units.
 struct Split {
     int parts, per_part, threads;
 };
 
-Split choose_split(int rows, int units, int granule)
+Split choose_split(int rows, int units, int granule, int target_blocks = kTargetBlocks)
 {
     Split s;
-    const int target_blocks = kTargetBlocks;
     int parts = 1;
     while (rows * parts < target_blocks && units / (parts * 2) >= 64 && parts < 16) parts *= 2;
     int per_part = (units + parts - 1) / parts;
@@ -353,21 +410,37 @@ struct Payload {
     float* out_weights;
 };
 
+// The split of a payload launch over `lines` tokens or rows.  Parts end at multiples of 128 bytes.  Where the rows themselves do not,
+// every part boundary is two partial lines to HBM in each of a token's rows, and a token-major launch has parts only while it would
+// have fewer than 2048 workgroups (dispatch and combine, BF16: 6045 tokens x top-10 of 6064 columns 353 -> 335 us, 7421 x 7 of 2848 280 -> 264, 1874 x 7 of
+// 2400 38.7 -> 36.3; rows of whole lines are better off with the finer split: 4096 x 8 of 4096 106.7 against 108.6, of 7168 to FP8 136.9 against 138.1).
+Split payload_split(const Payload& p, bool token_major, int lines)
+{
+    const bool whole_lines = p.quantize || p.units % 8 == 0;
+    return choose_split(lines, p.units, whole_lines ? 8 : 1, token_major && !whole_lines ? 2048 : kTargetBlocks);
+}
+
 PayloadShape payload_shape(const Payload& p, const Split& sp)
 {
     return {p.num_tokens, p.num_topk, p.units, sp.per_part, sp.parts, sp.threads, p.scale_cols};
 }
 
-// token-major: the grid does not depend on R; rows at or beyond `capacity` are dropped; all_rows: all of them unless DPEP_ROWS_KEPT.
-int launch_token_major(const Payload& p, const int32_t* route_to_row, int capacity, const int32_t* all_rows, hipStream_t s)
+// token-major: the grid does not depend on R; rows at or beyond `capacity` are dropped; all_rows: all of them unless DPEP_ROWS_KEPT.  rows:
+// their number, about.
+int launch_token_major(const Payload& p, const int32_t* route_to_row, int capacity, const int32_t* all_rows, long long rows, hipStream_t s)
 {
-    const Split sp = choose_split(p.num_tokens, p.units, p.quantize ? 8 : 1);
+    const Split sp = payload_split(p, true, p.num_tokens);
     const dim3 grid(p.num_tokens * sp.parts), block(sp.threads);
+    // A launch that mostly writes is faster with sixteen waves to a CU than with as many as there is room for (fewer rows open at a time;
+    // 6045 tokens x top-10 of 6064 BF16 columns 335 -> 328 us, 6249 x 7 of 1552 145.7 -> 141.3; 1.25 rows per
+    // token 39.6 -> 47.3; to FP8, whose reads are half of its rows' bytes, 146.6 -> 150.7): the LDS that it asks for keeps others out.
+    const bool mostly_writes = !p.quantize && rows >= 5LL * p.num_tokens && rows * p.units * 16 >= (32LL << 20);
+    const unsigned room = mostly_writes ? 40960 / kMaxThreads * sp.threads : 0;
     const MappedTokens tokens = {route_to_row, capacity, all_rows};
     with_store_policy([&](auto policy) {
         constexpr int kPolicy = decltype(policy)::value;
         if (p.quantize) hipLaunchKernelGGL(dispatch_quant_token_kernel<kPolicy>, grid, block, 0, s, p.x, p.weights, p.out, p.out_scales, p.out_weights, payload_shape(p, sp), tokens);
-        else hipLaunchKernelGGL(dispatch_copy_token_kernel<kPolicy>, grid, block, 0, s, p.x, p.scales, p.weights, p.out, p.out_scales, p.out_weights,
+        else hipLaunchKernelGGL(dispatch_copy_token_kernel<kPolicy>, grid, block, room, s, p.x, p.scales, p.weights, p.out, p.out_scales, p.out_weights,
                                 payload_shape(p, sp), tokens);
     });
     return launch_status("dispatch_token");
@@ -376,14 +449,16 @@ int launch_token_major(const Payload& p, const int32_t* route_to_row, int capaci
 // row-major: workgroups for `grid_rows` rows (row_to_route has at least as many entries), which walk on to the range's end.
 int launch_row_major(const Payload& p, const int32_t* row_to_route, const RowRange& range, int grid_rows, hipStream_t s)
 {
-    const Split sp = choose_split(grid_rows, p.units, p.quantize ? 8 : 1);
+    const Split sp = payload_split(p, false, grid_rows);
     const dim3 grid(grid_rows * sp.parts), block(sp.threads);
     with_store_policy([&](auto policy) {
         constexpr int kPolicy = decltype(policy)::value;
-        if (p.quantize) hipLaunchKernelGGL(dispatch_quant_row_kernel<kPolicy>, grid, block, 0, s, p.x, p.weights, p.out, p.out_scales, p.out_weights, payload_shape(p, sp),
-                               row_to_route, range);
-        else hipLaunchKernelGGL(dispatch_copy_row_kernel<kPolicy>, grid, block, 0, s, p.x, p.scales, p.weights, p.out, p.out_scales, p.out_weights,
-                                payload_shape(p, sp), row_to_route, range);
+        if (p.quantize)
+            hipLaunchKernelGGL(dispatch_quant_row_kernel<kPolicy>, grid, block, 0, s, p.x, p.weights, row_to_route, range, p.num_tokens, p.num_topk,
+                               p.units, sp.per_part, sp.parts, p.out, p.out_scales, p.out_weights);
+        else
+            hipLaunchKernelGGL(dispatch_copy_row_kernel<kPolicy>, grid, block, 0, s, p.x, p.scales, p.weights, row_to_route, range, p.num_tokens,
+                               p.num_topk, p.units, sp.per_part, sp.parts, p.scale_cols, p.out, p.out_scales, p.out_weights);
     });
     return launch_status("dispatch_row");
 }
@@ -393,7 +468,7 @@ int launch_row_major(const Payload& p, const int32_t* row_to_route, const RowRan
 int launch_payload(const Payload& p, const int32_t* route_to_row, const int32_t* row_to_route, int num_rows, hipStream_t s)
 {
     if (num_rows < 0 || static_cast<long long>(num_rows) > static_cast<long long>(kRowMajorRatio) * p.num_tokens)
-        return launch_token_major(p, route_to_row, 0x7fffffff, nullptr, s);
+        return launch_token_major(p, route_to_row, 0x7fffffff, nullptr, num_rows < 0 ? 0 : num_rows, s);
     return launch_row_major(p, row_to_route, RowRange{num_rows, nullptr, 0}, num_rows, s);
 }
 
@@ -557,14 +632,17 @@ int dpep_dispatch_fresh(void* ws, const dpep_fresh_dispatch* call, void* stream)
         const bool may_ride = worth_it && c.capacity_rows > 0 && dpep_dispatch_store_policy(DPEP_STORE_QUERY) == DPEP_STORE_STREAMING;
         if (may_ride) {
             const int lines = token_major ? c.num_tokens : static_cast<int>(grid_rows);
-            const Split sp = choose_split(lines, units, c.quantize ? 8 : 1);
+            Split sp = payload_split(p, token_major, lines);
+            // (A workgroup of the layout's has 256 threads; parts that leave a third of them idle are too fine: 3596 tokens x top-5 of 4608
+            // columns to FP8, two parts of 144 units 56.8 us, one 54.3.)
+            if (token_major && kMaxThreads / sp.threads * sp.per_part < 176) sp = choose_split(lines, units, p.quantize || units % 8 == 0 ? 8 : 1, 2048);
             riding = {p.x, p.scales, p.weights, p.out, p.out_scales, p.out_weights, payload_shape(p, sp), c.quantize != 0, !token_major, static_cast<unsigned>(lines) * sp.parts, bound, c.capacity_rows,
                       all_or_none ? c.capacity_rows : 0};
         }
         bool launched = false;
         if (int rc = layout_of_fresh(ws, c, may_ride ? &riding : nullptr, &launched, s)) return rc;  // (checks the routing arguments)
         if (launched || c.capacity_rows == 0) return DPEP_OK;
-        if (token_major) return launch_token_major(p, c.route_to_row, c.capacity_rows, all_or_none ? c.num_rows : nullptr, s);
+        if (token_major) return launch_token_major(p, c.route_to_row, c.capacity_rows, all_or_none ? c.num_rows : nullptr, expected, s);
         return launch_row_major(p, c.row_to_route, RowRange{bound, c.num_rows, all_or_none ? c.capacity_rows : 0}, static_cast<int>(grid_rows), s);
     }
     return fresh_in_one_launch(w, c, s);
@@ -603,11 +681,11 @@ int dpep_cast_to_fp8(const void* x, int num_tokens, int hidden, void* out, float
         return launch_status("cast_to_fp8");
     }
     const Split sp = choose_split(num_tokens, units, 8);
-    const PayloadShape shape = {num_tokens, 1, units, sp.per_part, sp.parts, sp.threads, 0};
     auto launch = [&](auto policy) {
-        hipLaunchKernelGGL(dispatch_quant_row_kernel<decltype(policy)::value>, dim3(num_tokens * sp.parts), dim3(sp.threads), 0,
-                           static_cast<hipStream_t>(stream), static_cast<const u32x4*>(x), nullptr, static_cast<u32x4*>(out), out_scales, nullptr, shape,
-                           nullptr, RowRange{num_tokens, nullptr, 0});
+        hipLaunchKernelGGL(dispatch_quant_row_kernel<decltype(policy)::value>, dim3(num_tokens * sp.parts),
+                           dim3(sp.threads), 0, static_cast<hipStream_t>(stream), static_cast<const u32x4*>(x), nullptr,
+                           nullptr, RowRange{num_tokens, nullptr, 0}, num_tokens, 1, units, sp.per_part, sp.parts,
+                           static_cast<u32x4*>(out), out_scales, nullptr);
     };
     // (codes that the memory-side cache takes are written through, whatever the dispatch's policy: the quantiser's reader is next.
     // 10007 x 5120: quantise and dequantise 47.7 us instead of 53.2)

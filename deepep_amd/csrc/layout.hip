@@ -610,8 +610,9 @@ __global__ __launch_bounds__(kThreads) void layout_fused_kernel(
 // Bound by HBM once the words are there.  Dispatch and combine, launches back to back, one grid / two: 1000 tokens x top-6 of 5120 BF16 30.5 / 31.7 us,
 // 618 x 7 of 5824 28.8 / 32.7, 3407 x 6 of 1584 37.5 / 42.5, 4372 x 7 of 5840 169.5 / 177.2.  Up to kSingleRoutes routes the layout's
 // workgroup of its own is the better one (710 x 4 of 2672 20.1 / 18.7).
-constexpr int kRidingExperts = 256;
-template <int kSteps, bool kQuant, bool kRowMajor>
+// Chunks of at most four steps: with eight (32 768 routes over 256 experts, skewed popularity, 235 MB) one grid took 149.9 us, two 146.6.
+constexpr int kRidingExperts = 256, kRidingSteps = 4;
+template <bool kQuant, bool kRowMajor>
 __global__ __launch_bounds__(kThreads, 4) void layout_payload_kernel(
     const int64_t* __restrict__ idx, int n_routes, int num_experts, int expert_begin, int num_local, int padded_local,
     int chunk, int num_chunks, int* __restrict__ counts, int* __restrict__ psum, int* __restrict__ offsets,
@@ -632,7 +633,7 @@ __global__ __launch_bounds__(kThreads, 4) void layout_payload_kernel(
         __device__ Both() {}
     } lds;
     if (static_cast<int>(blockIdx.x) <= num_blocks) {
-        fused_layout<int64_t, false, kSteps, kRowMajor ? 2 : 1>(lds.layout, idx, n_routes, num_experts, expert_begin, num_local, padded_local, chunk, num_chunks, counts, psum, offsets, num_rows, route_to_row, row_to_route, idx_copy, send, mailbox, sequence, epoch, tagged, num_blocks, rows, limit_ticks, timeouts, launch_id, MegaFront{}, total_word, row_words);
+        fused_layout<int64_t, false, kRidingSteps, kRowMajor ? 2 : 1>(lds.layout, idx, n_routes, num_experts, expert_begin, num_local, padded_local, chunk, num_chunks, counts, psum, offsets, num_rows, route_to_row, row_to_route, idx_copy, send, mailbox, sequence, epoch, tagged, num_blocks, rows, limit_ticks, timeouts, launch_id, MegaFront{}, total_word, row_words);
         return;
     }
     // Payload workgroups of fewer threads share one of these: `per` of them, each of whole waves.
@@ -893,7 +894,7 @@ int launch_layout(void* ws, const IdxT* idx, int num_tokens, int num_topk, int n
                                w->exchange_ticks, w->mailbox_device + kMailboxTimeout, w->layout_launches, f);
         };
         // The payload rides along where the words have room for every route and the launch is not captured.
-        if (payload != nullptr && chunk <= 8 * kWave && num_local <= kRidingExperts && n_routes <= kSyncRowWords && !is_capturing(stream)) {
+        if (payload != nullptr && chunk <= kRidingSteps * kWave && num_local <= kRidingExperts && n_routes <= kSyncRowWords && !is_capturing(stream)) {
             if constexpr (std::is_same_v<IdxT, int64_t>) {
                 const unsigned per = kThreads / payload->shape.threads, more = (payload->blocks + per - 1) / per;
                 auto ride = [&](auto kernel) {
@@ -905,13 +906,8 @@ int launch_layout(void* ws, const IdxT* idx, int num_tokens, int num_topk, int n
                                        reinterpret_cast<unsigned long long*>(sync + kSyncTotal), reinterpret_cast<unsigned long long*>(sync + kSyncRows),
                                        *payload);
                 };
-                auto ride_steps = [&](auto steps_constant) {
-                    constexpr int kSteps = decltype(steps_constant)::value;
-                    if (payload->row_major) payload->quantize ? ride(layout_payload_kernel<kSteps, true, true>) : ride(layout_payload_kernel<kSteps, false, true>);
-                    else payload->quantize ? ride(layout_payload_kernel<kSteps, true, false>) : ride(layout_payload_kernel<kSteps, false, false>);
-                };
-                if (chunk <= 4 * kWave) ride_steps(std::integral_constant<int, 4>{});
-                else ride_steps(std::integral_constant<int, 8>{});
+                if (payload->row_major) payload->quantize ? ride(layout_payload_kernel<true, true>) : ride(layout_payload_kernel<false, true>);
+                else payload->quantize ? ride(layout_payload_kernel<true, false>) : ride(layout_payload_kernel<false, false>);
                 *payload_launched = true;
                 return launch_status("layout_payload");
             }

@@ -43,44 +43,6 @@ struct MappedTokens {
     }
 };
 
-// Row-major: rows [0, rows): `rows` from the host, or, rows_on_device, the smaller of that bound and the count the layout left on the
-// device (a payload queued before the host knows R); all_or_none, the outputs' capacity: no rows at all unless DPEP_ROWS_KEPT
-// (0: the first rows in any case).  Such a launch has workgroups for about the expected number of rows;
-// they walk on by the grid's rows until the real count is reached, and the first row's route is asked for together with
-// the count (row_to_route has an entry for every row of the grid, so the load is in bounds whatever the count says).
-// kIdentity: row_to_route may be nullptr, which means identity (row == token): the stand-alone quantiser.
-struct RowRange {
-    int rows;
-    const int* rows_on_device;
-    int all_or_none;
-    __device__ __forceinline__ int count() const
-    {
-        if (rows_on_device == nullptr) return rows;
-        const int all = *rows_on_device;
-        return all_or_none == 0 || DPEP_ROWS_KEPT(all, all_or_none) ? min(all, rows) : 0;
-    }
-};
-template <bool kIdentity>
-struct MappedRows {
-    const int* row_to_route;
-    RowRange range;
-    struct Walk {
-        const int* map;
-        int next, rows;
-        __device__ __forceinline__ bool has(int row) const { return row < rows; }
-        __device__ __forceinline__ int route(int row) const { return !kIdentity || map != nullptr ? next : row; }
-        __device__ __forceinline__ void ask(int row)
-        {
-            if ((!kIdentity || map != nullptr) && row < rows) next = map[row];
-        }
-    };
-    __device__ __forceinline__ Walk begin(int row) const
-    {
-        const int first = !kIdentity || row_to_route != nullptr ? row_to_route[row] : row;
-        return {row_to_route, first, range.count()};
-    }
-};
-
 // In the layout's own grid (layout.hip) a route's row, or a row's route, comes as a word that says itself which launch it belongs to:
 // the launch's number above, the value (-1: no row) below.  `total` gets R the same way.  A wait is bounded; one that runs out moves
 // nothing and leaves the launch's number in the host mailbox, as a layout's own wait does.
@@ -138,34 +100,24 @@ struct AwaitedTokens {
 struct AwaitedRows {
     AwaitedWords from;
     int rows;         // bound of R
-    int all_or_none;  // as in RowRange
-    struct Walk {
-        AwaitedWords from;
-        int rows, next;
-        __device__ __forceinline__ bool has(int row)
-        {
-            if (row >= rows) return false;
-            long long start = 0;
-            for (int spins = 0;; ++spins) {
-                const unsigned long long v = __hip_atomic_load(from.words + row, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                const unsigned long long total = __hip_atomic_load(from.total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                next = static_cast<int>(static_cast<uint32_t>(v));
-                if (static_cast<uint32_t>(v >> 32) == from.launch) return true;
-                if (static_cast<uint32_t>(total >> 32) == from.launch && row >= static_cast<int>(static_cast<uint32_t>(total))) return false;
-                if (!from.patient(spins, start)) return false;
-            }
-        }
-        __device__ __forceinline__ int route(int) const { return next; }
-        __device__ __forceinline__ void ask(int) {}
-    };
-    __device__ __forceinline__ Walk begin(int) const
+    int all_or_none;  // the outputs' capacity: no rows at all unless DPEP_ROWS_KEPT; 0: the first rows in any case
+    __device__ __forceinline__ int bound() const
     {
-        int bound = rows;
-        if (all_or_none != 0) {
-            const int all = from.await(from.total, 0);
-            bound = DPEP_ROWS_KEPT(all, all_or_none) ? min(all, rows) : 0;
+        if (all_or_none == 0) return rows;
+        const int all = from.await(from.total, 0);
+        return DPEP_ROWS_KEPT(all, all_or_none) ? min(all, rows) : 0;
+    }
+    // The route of row `row` below the bound; -1: there is no such row.
+    __device__ __forceinline__ int route_of(int row) const
+    {
+        long long start = 0;
+        for (int spins = 0;; ++spins) {
+            const unsigned long long v = __hip_atomic_load(from.words + row, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            const unsigned long long total = __hip_atomic_load(from.total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (static_cast<uint32_t>(v >> 32) == from.launch) return static_cast<int>(static_cast<uint32_t>(v));
+            if (static_cast<uint32_t>(total >> 32) == from.launch && row >= static_cast<int>(static_cast<uint32_t>(total))) return -1;
+            if (!from.patient(spins, start)) return -1;
         }
-        return {from, bound, 0};
     }
 };
 
@@ -199,13 +151,26 @@ __device__ __forceinline__ void copy_token(const u32x4* __restrict__ x, const fl
     const int all = tokens.begin();
     const int v_begin = part * p.per_part, v_end = min(v_begin + p.per_part, p.units);
     const u32x4* src = x + static_cast<size_t>(token) * p.units;
-    // The token's first values are asked for before its routes are known (see the quantising one below).
+    // The token's first values are asked for before its routes are known (see the quantising one below), and written row by row: 4 KB and
+    // more of one row at a time instead of 1 KB of every row in turn (6045 tokens x top-10 of 6064 BF16 columns, dispatch and
+    // combine 357 -> 353 us, 4372 x 7 of 5840 178 -> 173).
     const int v_first = v_begin + t;
-    u32x4 first = {0u, 0u, 0u, 0u};
-    if (v_first < v_end) first = load16(src + v_first);
+    constexpr int kEarly = 2;
+    u32x4 early[kEarly];
+#pragma unroll
+    for (int j = 0; j < kEarly; ++j)
+        if (v_first + j * p.threads < v_end) early[j] = load16(src + v_first + j * p.threads);
     if (!rows_of_token(p, tokens, all, token, t, lds)) return;
-    for (int v = v_first; v < v_end; v += p.threads) {
-        const u32x4 value = v == v_first ? first : load16(src + v);
+    for (int s = 0; s < p.num_topk; ++s) {
+        const int row = lds.rows[s];
+        if (row < 0) continue;
+        u32x4* dst = out + static_cast<size_t>(row) * p.units;
+#pragma unroll
+        for (int j = 0; j < kEarly; ++j)
+            if (v_first + j * p.threads < v_end) store16_as<kPolicy>(dst + v_first + j * p.threads, early[j]);
+    }
+    for (int v = v_first + kEarly * p.threads; v < v_end; v += p.threads) {  // rows wider than that
+        const u32x4 value = load16(src + v);
         for (int s = 0; s < p.num_topk; ++s) {
             const int row = lds.rows[s];
             if (row >= 0) store16_as<kPolicy>(out + static_cast<size_t>(row) * p.units + v, value);
@@ -226,21 +191,20 @@ __device__ __forceinline__ void copy_token(const u32x4* __restrict__ x, const fl
     }
 }
 
-// ---- row-major: one output row and column part to `p.threads` threads; for sparse receive shares -----------------------------
-// stride: rows between two of a workgroup.
-template <int kPolicy, typename Rows>
+// ---- row-major, in the layout's grid: one output row and column part to `p.threads` threads; for sparse receive shares --------
+// stride: rows between two of a workgroup.  (dispatch.hip has the same for maps that are there already: in one piece with this its prologue
+// grew by 0.1 us, a fortieth of what a few hundred rows take.)
+template <int kPolicy>
 __device__ __forceinline__ void copy_rows(const u32x4* __restrict__ x, const float* __restrict__ scales, const float* __restrict__ weights,
                                           u32x4* __restrict__ out, float* __restrict__ out_scales, float* __restrict__ out_weights,
-                                          const PayloadShape& p, const Rows& source, unsigned block, int stride, int t)
+                                          const PayloadShape& p, const AwaitedRows& source, unsigned block, int stride, int t)
 {
     const int part = block % static_cast<unsigned>(p.parts);
     const int v_begin = part * p.per_part, v_end = min(v_begin + p.per_part, p.units);
     int row = block / static_cast<unsigned>(p.parts);
-    auto walk = source.begin(row);
-    for (; walk.has(row); row += stride) {
-        // (clamped: a map left incomplete by a layout launch that reported a time-out must not become a wild address)
-        const int route = min(max(walk.route(row), 0), p.num_tokens * p.num_topk - 1);
-        walk.ask(row + stride);
+    for (const int bound = source.bound(); row < bound; row += stride) {
+        const int route = source.route_of(row);
+        if (route < 0) return;
         const int token = route / p.num_topk;
         const u32x4* src = x + static_cast<size_t>(token) * p.units;
         u32x4* dst = out + static_cast<size_t>(row) * p.units;
@@ -385,20 +349,19 @@ __device__ __forceinline__ void quant_token(const u32x4* __restrict__ x, const f
         out_weights[lds.rows[t]] = weights[static_cast<size_t>(token) * p.num_topk + t];
 }
 
-// row-major
-template <int kPolicy, typename Rows>
+// row-major, in the layout's grid
+template <int kPolicy>
 __device__ __forceinline__ void quant_rows(const u32x4* __restrict__ x, const float* __restrict__ weights, u32x4* __restrict__ out,
                                            float* __restrict__ out_scales, float* __restrict__ out_weights, const PayloadShape& p,
-                                           const Rows& source, unsigned block, int stride, int t)
+                                           const AwaitedRows& source, unsigned block, int stride, int t)
 {
     const int part = block % static_cast<unsigned>(p.parts);
     const int u_begin = part * p.per_part, u_end = min(u_begin + p.per_part, p.units);
     const int scale_cols = p.units / 8;
     int row = block / static_cast<unsigned>(p.parts);
-    auto walk = source.begin(row);
-    for (; walk.has(row); row += stride) {
-        const int route = min(max(walk.route(row), 0), p.num_tokens * p.num_topk - 1);
-        walk.ask(row + stride);
+    for (const int bound = source.bound(); row < bound; row += stride) {
+        const int route = source.route_of(row);
+        if (route < 0) return;
         const int token = route / p.num_topk;
         const u32x4* src = x + static_cast<size_t>(token) * p.units * 2;
         for (int u = u_begin + t; u < u_end; u += p.threads) {

@@ -64,7 +64,10 @@ class _Call:
     (8200, 2, 16, 0, 16, 2560, 0, False, 1, 0),       # 160 vectors: 192 threads, one to a workgroup
     (700, 32, 64, 0, 64, 1536, 0, False, 1, 100),     # top-32, more room than rows
     (260, 16, 64, 0, 64, 9216, 0, False, 1, -300),    # the last rows have no room
-    (3900, 8, 256, 0, 256, 1088, 0, False, 1, 0),     # eight steps to a chunk, as many experts as ride
+    (420, 10, 40, 0, 40, 12128, 0, False, 1, 0),      # 758 vectors, not whole lines: parts that are not either
+    (2100, 5, 24, 0, 24, 9232, 0, False, 1, 0),       # 577 in one part: two rounds from registers and one behind them
+    (2040, 8, 256, 0, 256, 2176, 0, False, 1, 0),     # as many experts and routes per wave as ride
+    (3900, 8, 256, 0, 256, 1088, 0, False, 1, 0),     # and more
     (1700, 12, 96, 48, 48, 4096, 5, False, 2, 0),     # half of the experts: all of the rows,
     (1700, 12, 96, 48, 48, 4096, 5, False, 2, -1),    # or none
     (10000, 3, 12, 0, 12, 2304, 0, True, 1, 0),       # quantised: 72 units, 128 threads
@@ -74,7 +77,7 @@ class _Call:
     (6000, 4, 256, 12, 4, 7168, 56, False, 0, 1000),  # row-major
     (6000, 4, 256, 12, 4, 7168, 0, False, 0, -100),
     (6000, 4, 256, 252, 4, 14336, 0, True, 0, 1000),
-    (8000, 4, 1024, 800, 200, 464, 0, False, 0, 0),   # eight steps
+    (4000, 4, 1024, 800, 200, 464, 0, False, 0, 0),
     (32768, 2, 256, 0, 1, 256, 0, True, 0, 0),        # one expert
 ])
 def test_riding_payload_equals_one_of_its_own_launch(tokens, topk, experts, begin, local, row_bytes, scale_cols, quantize, report, spare):
