@@ -5,6 +5,7 @@
 //
 // Observable contract: tests/elastic/test_dispatch.py:1391-1416 (payload, scales and weights arrive
 // bit-exactly in row order), tests/clos/common.py:276-279; quantiser deep_ep/utils/math.py:45-61.
+#include <algorithm>
 #include <type_traits>
 
 #include "common.h"
@@ -39,13 +40,14 @@ void with_store_policy(Launch&& launch)
     }
 }
 
-template <int kPolicy>
+template <int kPolicy, bool kStaged>
 __global__ __launch_bounds__(kMaxThreads) void dispatch_copy_token_kernel(
     const u32x4* __restrict__ x, const float* __restrict__ scales, const float* __restrict__ weights, u32x4* __restrict__ out,
     float* __restrict__ out_scales, float* __restrict__ out_weights, PayloadShape p, MappedTokens tokens)
 {
     __shared__ TokenLds lds;
-    copy_token<kPolicy>(x, scales, weights, out, out_scales, out_weights, p, tokens, blockIdx.x, threadIdx.x, lds);
+    __shared__ u32x4 stage[kStaged ? kStagedVec : 1];
+    copy_token<kPolicy, kStaged>(x, scales, weights, out, out_scales, out_weights, p, tokens, blockIdx.x, threadIdx.x, lds, stage);
 }
 
 // ---- row-major: one workgroup per (output row, column part); for sparse receive shares -------------
@@ -411,13 +413,21 @@ struct Payload {
 };
 
 // The split of a payload launch over `lines` tokens or rows.  Parts end at multiples of 128 bytes.  Where the rows themselves do not,
-// every part boundary is two partial lines to HBM in each of a token's rows, and a token-major launch has parts only while it would
-// have fewer than 2048 workgroups (dispatch and combine, BF16: 6045 tokens x top-10 of 6064 columns 353 -> 335 us, 7421 x 7 of 2848 280 -> 264, 1874 x 7 of
-// 2400 38.7 -> 36.3; rows of whole lines are better off with the finer split: 4096 x 8 of 4096 106.7 against 108.6, of 7168 to FP8 136.9 against 138.1).
-Split payload_split(const Payload& p, bool token_major, int lines)
+// every part boundary is two partial lines to HBM in each of a token's rows, and a token-major launch with four and more rows per token has
+// parts only while it would have fewer than 2048 workgroups (dispatch and combine, BF16: 6045 tokens x top-10 of 6064 columns 353 -> 335 us, 7421 x 7 of 2848 280 -> 264, 1874 x 7 of
+// 2400 38.7 -> 36.3; rows of whole lines are better off with the finer split: 4096 x 8 of 4096 106.7 against 108.6, of 7168 to FP8 136.9 against 138.1; two
+// rows per token are too few for it: 2264 of 4464 30.3 against 31.6).
+Split payload_split(const Payload& p, int lines, long long rows_to_write)
 {
     const bool whole_lines = p.quantize || p.units % 8 == 0;
-    return choose_split(lines, p.units, whole_lines ? 8 : 1, token_major && !whole_lines ? 2048 : kTargetBlocks);
+    return choose_split(lines, p.units, whole_lines ? 8 : 1, !whole_lines && rows_to_write >= 4LL * lines ? 2048 : kTargetBlocks);
+}
+
+// Whether a token-major copy goes through LDS (dispatch and combine, BF16: 6045 tokens x top-10 of 6064 columns 343.2 -> 321.6 us, 3054 x 9 of 3152 there
+// and back 174.5 -> 166.7, 6249 x 7 of 1552 71.3 -> 69.8; 7782 x 5 of 1232, 154 vectors, 45.5 against 48.3).
+bool payload_staged(const Payload& p, const Split& sp)
+{
+    return !p.quantize && p.units % 8 != 0 && sp.threads == kMaxThreads && sp.per_part <= kStagedVec;
 }
 
 PayloadShape payload_shape(const Payload& p, const Split& sp)
@@ -429,7 +439,7 @@ PayloadShape payload_shape(const Payload& p, const Split& sp)
 // their number, about.
 int launch_token_major(const Payload& p, const int32_t* route_to_row, int capacity, const int32_t* all_rows, long long rows, hipStream_t s)
 {
-    const Split sp = payload_split(p, true, p.num_tokens);
+    const Split sp = payload_split(p, p.num_tokens, rows);
     const dim3 grid(p.num_tokens * sp.parts), block(sp.threads);
     // A launch that mostly writes is faster with sixteen waves to a CU than with as many as there is room for (fewer rows open at a time;
     // 6045 tokens x top-10 of 6064 BF16 columns 335 -> 328 us, 6249 x 7 of 1552 145.7 -> 141.3; 1.25 rows per
@@ -440,8 +450,12 @@ int launch_token_major(const Payload& p, const int32_t* route_to_row, int capaci
     with_store_policy([&](auto policy) {
         constexpr int kPolicy = decltype(policy)::value;
         if (p.quantize) hipLaunchKernelGGL(dispatch_quant_token_kernel<kPolicy>, grid, block, 0, s, p.x, p.weights, p.out, p.out_scales, p.out_weights, payload_shape(p, sp), tokens);
-        else hipLaunchKernelGGL(dispatch_copy_token_kernel<kPolicy>, grid, block, room, s, p.x, p.scales, p.weights, p.out, p.out_scales, p.out_weights,
-                                payload_shape(p, sp), tokens);
+        else if (kPolicy == DPEP_STORE_STREAMING && payload_staged(p, sp))
+            hipLaunchKernelGGL((dispatch_copy_token_kernel<kPolicy, true>), grid, block, room - std::min(room, kStagedVec * 16u), s, p.x, p.scales, p.weights,
+                               p.out, p.out_scales, p.out_weights, payload_shape(p, sp), tokens);
+        else
+            hipLaunchKernelGGL((dispatch_copy_token_kernel<kPolicy, false>), grid, block, room, s, p.x, p.scales, p.weights, p.out, p.out_scales,
+                               p.out_weights, payload_shape(p, sp), tokens);
     });
     return launch_status("dispatch_token");
 }
@@ -449,7 +463,7 @@ int launch_token_major(const Payload& p, const int32_t* route_to_row, int capaci
 // row-major: workgroups for `grid_rows` rows (row_to_route has at least as many entries), which walk on to the range's end.
 int launch_row_major(const Payload& p, const int32_t* row_to_route, const RowRange& range, int grid_rows, hipStream_t s)
 {
-    const Split sp = payload_split(p, false, grid_rows);
+    const Split sp = payload_split(p, grid_rows, grid_rows);
     const dim3 grid(grid_rows * sp.parts), block(sp.threads);
     with_store_policy([&](auto policy) {
         constexpr int kPolicy = decltype(policy)::value;
@@ -632,11 +646,11 @@ int dpep_dispatch_fresh(void* ws, const dpep_fresh_dispatch* call, void* stream)
         const bool may_ride = worth_it && c.capacity_rows > 0 && dpep_dispatch_store_policy(DPEP_STORE_QUERY) == DPEP_STORE_STREAMING;
         if (may_ride) {
             const int lines = token_major ? c.num_tokens : static_cast<int>(grid_rows);
-            Split sp = payload_split(p, token_major, lines);
+            Split sp = payload_split(p, lines, token_major ? expected : lines);
             // (A workgroup of the layout's has 256 threads; parts that leave a third of them idle are too fine: 3596 tokens x top-5 of 4608
             // columns to FP8, two parts of 144 units 56.8 us, one 54.3.)
             if (token_major && kMaxThreads / sp.threads * sp.per_part < 176) sp = choose_split(lines, units, p.quantize || units % 8 == 0 ? 8 : 1, 2048);
-            riding = {p.x, p.scales, p.weights, p.out, p.out_scales, p.out_weights, payload_shape(p, sp), c.quantize != 0, !token_major, static_cast<unsigned>(lines) * sp.parts, bound, c.capacity_rows,
+            riding = {p.x, p.scales, p.weights, p.out, p.out_scales, p.out_weights, payload_shape(p, sp), c.quantize != 0, payload_staged(p, sp), !token_major, static_cast<unsigned>(lines) * sp.parts, bound, c.capacity_rows,
                       all_or_none ? c.capacity_rows : 0};
         }
         bool launched = false;

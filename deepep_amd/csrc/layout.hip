@@ -612,7 +612,7 @@ __global__ __launch_bounds__(kThreads) void layout_fused_kernel(
 // workgroup of its own is the better one (710 x 4 of 2672 20.1 / 18.7).
 // Chunks of at most four steps: with eight (32 768 routes over 256 experts, skewed popularity, 235 MB) one grid took 149.9 us, two 146.6.
 constexpr int kRidingExperts = 256, kRidingSteps = 4;
-template <bool kQuant, bool kRowMajor>
+template <bool kQuant, bool kRowMajor, bool kStaged>
 __global__ __launch_bounds__(kThreads, 4) void layout_payload_kernel(
     const int64_t* __restrict__ idx, int n_routes, int num_experts, int expert_begin, int num_local, int padded_local,
     int chunk, int num_chunks, int* __restrict__ counts, int* __restrict__ psum, int* __restrict__ offsets,
@@ -626,6 +626,7 @@ __global__ __launch_bounds__(kThreads, 4) void layout_payload_kernel(
     struct Riding {
         TokenLds tokens[kWaves];
         float scales[kQuant && !kRowMajor ? kMaxScaleCols : 1];
+        u32x4 stage[kStaged ? kStagedVec : 1];
     };
     __shared__ union Both {
         Lds layout;
@@ -649,7 +650,8 @@ __global__ __launch_bounds__(kThreads, 4) void layout_payload_kernel(
     } else {
         const AwaitedTokens tokens = {words, payload.capacity, payload.all_or_none};
         if (kQuant) quant_token<DPEP_STORE_STREAMING>(payload.x, payload.weights, payload.out, payload.out_scales, payload.out_weights, p, tokens, block, t, lds.riding.tokens[sub], lds.riding.scales + sub * (p.threads / 8));
-        else copy_token<DPEP_STORE_STREAMING>(payload.x, payload.scales, payload.weights, payload.out, payload.out_scales, payload.out_weights, p, tokens, block, t, lds.riding.tokens[sub]);
+        else copy_token<DPEP_STORE_STREAMING, kStaged>(payload.x, payload.scales, payload.weights, payload.out, payload.out_scales, payload.out_weights, p, tokens, block, t,
+                                                       lds.riding.tokens[sub], lds.riding.stage);
     }
 }
 
@@ -906,8 +908,9 @@ int launch_layout(void* ws, const IdxT* idx, int num_tokens, int num_topk, int n
                                        reinterpret_cast<unsigned long long*>(sync + kSyncTotal), reinterpret_cast<unsigned long long*>(sync + kSyncRows),
                                        *payload);
                 };
-                if (payload->row_major) payload->quantize ? ride(layout_payload_kernel<true, true>) : ride(layout_payload_kernel<false, true>);
-                else payload->quantize ? ride(layout_payload_kernel<true, false>) : ride(layout_payload_kernel<false, false>);
+                if (payload->row_major) payload->quantize ? ride(layout_payload_kernel<true, true, false>) : ride(layout_payload_kernel<false, true, false>);
+                else if (payload->quantize) ride(layout_payload_kernel<true, false, false>);
+                else payload->staged ? ride(layout_payload_kernel<false, false, true>) : ride(layout_payload_kernel<false, false, false>);
                 *payload_launched = true;
                 return launch_status("layout_payload");
             }

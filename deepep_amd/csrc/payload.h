@@ -142,10 +142,17 @@ __device__ __forceinline__ bool rows_of_token(const PayloadShape& p, const Token
     return lds.any_valid != 0;
 }
 
-template <int kPolicy, typename Tokens>
+// How far (in 16-byte vectors) an address lies behind the start of its cache line.
+__device__ __forceinline__ int behind_line(const void* p) { return static_cast<int>(reinterpret_cast<uintptr_t>(p) >> 4 & 7); }
+
+// kStaged: rows that are no whole lines.  A wave's 1 KB would begin and end inside a line of every such row, two partial writes to HBM each: the
+// piece goes through LDS (`stage`, kStagedVec vectors), and each row is written from the start of a line on.
+constexpr int kStagedVec = 4 * kMaxThreads;
+template <int kPolicy, bool kStaged, typename Tokens>
 __device__ __forceinline__ void copy_token(const u32x4* __restrict__ x, const float* __restrict__ scales, const float* __restrict__ weights,
                                            u32x4* __restrict__ out, float* __restrict__ out_scales, float* __restrict__ out_weights,
-                                           const PayloadShape& p, const Tokens& tokens, unsigned block, int t, TokenLds& lds)
+                                           const PayloadShape& p, const Tokens& tokens, unsigned block, int t, TokenLds& lds,
+                                           u32x4* stage = nullptr)
 {
     const int token = block / static_cast<unsigned>(p.parts), part = block % static_cast<unsigned>(p.parts);
     const int all = tokens.begin();
@@ -160,16 +167,27 @@ __device__ __forceinline__ void copy_token(const u32x4* __restrict__ x, const fl
 #pragma unroll
     for (int j = 0; j < kEarly; ++j)
         if (v_first + j * p.threads < v_end) early[j] = load16(src + v_first + j * p.threads);
-    if (!rows_of_token(p, tokens, all, token, t, lds)) return;
+    if constexpr (kStaged) {
+#pragma unroll
+        for (int j = 0; j < kEarly; ++j)
+            if (v_first + j * p.threads < v_end) stage[t + j * p.threads] = early[j];
+        for (int v = v_first + kEarly * p.threads; v < v_end; v += p.threads) stage[v - v_begin] = load16(src + v);
+    }
+    if (!rows_of_token(p, tokens, all, token, t, lds)) return;  // (with a barrier behind the staging)
     for (int s = 0; s < p.num_topk; ++s) {
         const int row = lds.rows[s];
         if (row < 0) continue;
         u32x4* dst = out + static_cast<size_t>(row) * p.units;
+        if constexpr (kStaged) {
+            for (int i = t - behind_line(dst + v_begin); i < v_end - v_begin; i += p.threads)
+                if (i >= 0) store16_as<kPolicy>(dst + v_begin + i, stage[i]);
+        } else {
 #pragma unroll
-        for (int j = 0; j < kEarly; ++j)
-            if (v_first + j * p.threads < v_end) store16_as<kPolicy>(dst + v_first + j * p.threads, early[j]);
+            for (int j = 0; j < kEarly; ++j)
+                if (v_first + j * p.threads < v_end) store16_as<kPolicy>(dst + v_first + j * p.threads, early[j]);
+        }
     }
-    for (int v = v_first + kEarly * p.threads; v < v_end; v += p.threads) {  // rows wider than that
+    for (int v = v_first + kEarly * p.threads; v < v_end && !kStaged; v += p.threads) {  // rows wider than that
         const u32x4 value = load16(src + v);
         for (int s = 0; s < p.num_topk; ++s) {
             const int row = lds.rows[s];
@@ -382,7 +400,7 @@ struct LayoutPayload {
     float* out_scales;
     float* out_weights;
     PayloadShape shape;
-    bool quantize, row_major;
+    bool quantize, staged, row_major;
     unsigned blocks;
     int rows, capacity, all_or_none;  // rows: row-major, the bound of R; capacity: token-major
 };

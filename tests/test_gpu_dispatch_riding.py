@@ -66,6 +66,8 @@ class _Call:
     (260, 16, 64, 0, 64, 9216, 0, False, 1, -300),    # the last rows have no room
     (420, 10, 40, 0, 40, 12128, 0, False, 1, 0),      # 758 vectors, not whole lines: parts that are not either
     (2100, 5, 24, 0, 24, 9232, 0, False, 1, 0),       # 577 in one part: two rounds from registers and one behind them
+    (2100, 5, 24, 0, 24, 16368, 0, False, 1, 0),      # 1023: all that LDS is lent, and (the next) one more than that
+    (2100, 5, 24, 0, 24, 16400, 0, False, 1, 0),
     (2040, 8, 256, 0, 256, 2176, 0, False, 1, 0),     # as many experts and routes per wave as ride
     (3900, 8, 256, 0, 256, 1088, 0, False, 1, 0),     # and more
     (1700, 12, 96, 48, 48, 4096, 5, False, 2, 0),     # half of the experts: all of the rows,
@@ -81,7 +83,7 @@ class _Call:
     (32768, 2, 256, 0, 1, 256, 0, True, 0, 0),        # one expert
 ])
 def test_riding_payload_equals_one_of_its_own_launch(tokens, topk, experts, begin, local, row_bytes, scale_cols, quantize, report, spare):
-    from deepep_amd import ops
+    from deepep_amd import _lib, ops
 
     rng = np.random.default_rng(tokens + topk)
     workspace = ops.Workspace(4 << 20)
@@ -105,6 +107,14 @@ def test_riding_payload_equals_one_of_its_own_launch(tokens, topk, experts, begi
                 ops.dispatch_store_policy(before)
             riding.same_as(plain, want["num_rows"])
             np.testing.assert_array_equal(riding.forward.cpu().numpy().reshape(tokens, topk), want["route_to_row"])
+            if not quantize and report == 1 and spare >= 0:  # (a launch of its own by the default policy, into rows that begin 16 bytes behind a line)
+                moved = torch.full((want["num_rows"] * row_bytes + 32,), 0x55, dtype=torch.uint8, device="cuda")
+                _lib.check(_lib.load().dpep_dispatch_copy(
+                    x.data_ptr(), None, None, riding.forward.data_ptr(), riding.back.data_ptr(), tokens, topk, want["num_rows"], row_bytes, 0,
+                    moved.data_ptr() + 16, None, None, torch.cuda.current_stream().cuda_stream), "dispatch_copy")
+                torch.cuda.synchronize()
+                assert torch.equal(moved[16:-16].view(-1, row_bytes), riding.out[: want["num_rows"]])
+                assert bool((moved[:16] == 0x55).all()) and bool((moved[-16:] == 0x55).all())
             if report == 2 and spare < 0:
                 assert bool((riding.out == 0x55).all())
     finally:
