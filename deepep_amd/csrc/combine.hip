@@ -17,10 +17,47 @@ namespace dpep {
 namespace {
 
 constexpr int kMaxThreads = 256;
-constexpr int kDenseTargetBlocks = 1000000;  // dense routing: always split the token rows
-constexpr int kDenseVec = 64;                // ... into parts of 64 16-byte vectors
 constexpr int kSparseTargetBlocks = 2048;    // sparse shares: a workgroup per token while that fills the chip
 constexpr int kBatch = 8;  // rows fetched per thread before the dependent adds start
+
+// One vector of a token: the sum over its slots (rows[s] < 0: none), kBatch rows in flight.  Slots ascending, separate fp32 multiply and
+// add, one rounding.
+template <int kWeights, bool kHalf>
+__device__ __forceinline__ u32x4 combined(const u32x4* __restrict__ y, const int* rows, const float* wts, int num_slots, int vec_per_row, int v)
+{
+    float acc[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) acc[i] = 0.0f;
+    for (int s0 = 0; s0 < num_slots; s0 += kBatch) {
+        u32x4 val[kBatch];
+#pragma unroll
+        for (int j = 0; j < kBatch; ++j) {
+            const int row = rows[s0 + j];
+            if (row >= 0) val[j] = load16_nt(y + static_cast<size_t>(row) * vec_per_row + v);
+        }
+#pragma unroll
+        for (int j = 0; j < kBatch; ++j) {
+            if (rows[s0 + j] < 0) continue;
+            const float w = kWeights != 0 ? wts[s0 + j] : 1.0f;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                float lo = kHalf ? f16_to_f32(val[j][i] & 0xffffu) : bf16_to_f32(val[j][i] & 0xffffu);
+                float hi = kHalf ? f16_to_f32(val[j][i] >> 16) : bf16_to_f32(val[j][i] >> 16);
+                if (kWeights != 0) {
+                    lo = __fmul_rn(lo, w);
+                    hi = __fmul_rn(hi, w);
+                }
+                acc[2 * i] = __fadd_rn(acc[2 * i], lo);
+                acc[2 * i + 1] = __fadd_rn(acc[2 * i + 1], hi);
+            }
+        }
+    }
+    u32x4 packed;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        packed[i] = kHalf ? pack_f16x2(acc[2 * i], acc[2 * i + 1]) : pack_bf16x2(acc[2 * i], acc[2 * i + 1]);
+    return packed;
+}
 
 // kWeights: 0 = plain sum, 1 = weight per expert row (w[row]), 2 = weight per route (w[t*K + s]).
 // kHalf: rows and output are IEEE half instead of BF16.
@@ -70,39 +107,57 @@ __global__ __launch_bounds__(kMaxThreads) void combine_kernel(
         return;
     }
     for (int v = v_begin + threadIdx.x; v < v_end; v += blockDim.x) {
-        float acc[8];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) acc[i] = 0.0f;
-        for (int s0 = 0; s0 < num_slots; s0 += kBatch) {
-            u32x4 val[kBatch];
-#pragma unroll
-            for (int j = 0; j < kBatch; ++j) {
-                const int row = rows[s0 + j];
-                if (row >= 0) val[j] = load16_nt(y + static_cast<size_t>(row) * vec_per_row + v);
-            }
-#pragma unroll
-            for (int j = 0; j < kBatch; ++j) {
-                if (rows[s0 + j] < 0) continue;
-                const float w = kWeights != 0 ? wts[s0 + j] : 1.0f;
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    float lo = kHalf ? f16_to_f32(val[j][i] & 0xffffu) : bf16_to_f32(val[j][i] & 0xffffu);
-                    float hi = kHalf ? f16_to_f32(val[j][i] >> 16) : bf16_to_f32(val[j][i] >> 16);
-                    if (kWeights != 0) {
-                        lo = __fmul_rn(lo, w);
-                        hi = __fmul_rn(hi, w);
-                    }
-                    acc[2 * i] = __fadd_rn(acc[2 * i], lo);
-                    acc[2 * i + 1] = __fadd_rn(acc[2 * i + 1], hi);
-                }
-            }
-        }
-        u32x4 packed;
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-            packed[i] = kHalf ? pack_f16x2(acc[2 * i], acc[2 * i + 1]) : pack_bf16x2(acc[2 * i], acc[2 * i + 1]);
-        store16_through(out + static_cast<size_t>(token) * vec_per_row + v, packed);
+        store16_through(out + static_cast<size_t>(token) * vec_per_row + v, combined<kWeights, kHalf>(y, rows, wts, num_slots, vec_per_row, v));
     }
+}
+
+// Dense routing, rows of more than 64 vectors that are no multiple of that: the output's vectors one after the other, 64 to a one-wave workgroup, which holds the slots
+// of the two tokens that it may touch.  No wave has lanes behind a row's end, and every store is whole lines.
+// Bound by HBM: rows read at 6 TB/s.  Against a workgroup for every started 64 vectors of a row (dispatch and combine, BF16): 6000 tokens x top-10 of 528
+// columns 43.5 -> 38.1 us, 6249 x 7 of 1552 69.1 -> 65.3, 5000 x 6 of 832 29.4 -> 27.6.
+template <int kWeights, bool kHalf = false>
+__global__ __launch_bounds__(64) void combine_dense_kernel(
+    const u32x4* __restrict__ y, const float* __restrict__ row_weights, const int* __restrict__ route_to_row,
+    int num_topk, int vec_per_row, u32x4* __restrict__ out,
+    const float* __restrict__ return_in, float* __restrict__ return_out, const int* __restrict__ shared_first_row,
+    int num_shared, int num_tokens, const int* __restrict__ fill_state, int num_rows, int leave_unserved)
+{
+    __shared__ int rows[2][DPEP_MAX_TOPK + kBatch];
+    __shared__ float wts[2][DPEP_MAX_TOPK + kBatch];
+    static_assert(DPEP_MAX_TOPK == 32, "a half wave looks up a token's slots");
+    const int lane = threadIdx.x, half = lane >> 5, slot = lane & 31;
+    const unsigned first = blockIdx.x * 64u, vec = vec_per_row;
+    const int token0 = static_cast<int>(first / vec), v0 = static_cast<int>(first - token0 * vec);
+    const int looked_up = token0 + half;
+    int row = -1;
+    if (looked_up < num_tokens && slot < num_topk && (half == 0 || v0 + 64 > vec_per_row)) {
+        const size_t route = static_cast<size_t>(looked_up) * num_topk + slot;
+        row = route_to_row[route];
+        if (row >= num_rows) row = -1;  // a row the caller's y does not hold (capacity layouts drop surplus rows)
+        if (kWeights == 1) wts[half][slot] = row >= 0 ? row_weights[row] : 0.0f;
+        if (kWeights == 2) wts[half][slot] = row >= 0 ? row_weights[route] : 0.0f;
+        if (return_out != nullptr && (half == 1 || v0 == 0)) return_out[route] = row >= 0 ? return_in[row] : 0.0f;  // (where the token begins)
+    }
+    // Shared experts (MegaMoE): slot K + j is row first + j * B + token with weight 1, summed after the routes.
+    if (kWeights == 2 && slot >= num_topk && slot < num_topk + num_shared) {
+        row = shared_first_row[0] + (slot - num_topk) * num_tokens + looked_up;
+        wts[half][slot] = 1.0f;
+    }
+    rows[half][slot] = row;
+    if (slot < kBatch) rows[half][DPEP_MAX_TOPK + slot] = -1;
+    const unsigned long long any = __ballot(row >= 0);
+    __syncthreads();
+    const int num_slots = num_topk + (kWeights == 2 ? num_shared : 0);
+    const int mine = v0 + lane >= vec_per_row ? 1 : 0, token = token0 + mine, v = v0 + lane - (mine != 0 ? vec_per_row : 0);
+    if (token >= num_tokens) return;
+    if (static_cast<uint32_t>(any >> (32 * mine)) == 0u) {  // no row: zeros, unless
+        if (leave_unserved) return;                          // the caller wants only the tokens that own a row written,
+        if (kWeights == 2 && fill_state != nullptr) {        // or idle workgroups of the first GEMM have written them (see above)
+            const int fillers = fill_state[0];
+            if (fillers > 0 && token / fillers < fill_state[1 + token % fillers]) return;
+        }
+    }
+    store16_through(out + first + lane, combined<kWeights, kHalf>(y, rows[mine], wts[mine], num_slots, vec_per_row, v));
 }
 
 // Sparse shares: most tokens own no row (one rank's part of an EP job).  A workgroup takes a few consecutive tokens, at most
@@ -246,39 +301,31 @@ void launch_combine_share(hipStream_t stream, const void* y, const float* weight
                        fill_state, static_cast<size_t>(num_tokens) * vec * 16 > kStreamBytes);
 }
 
-struct CombineGrid {
-    int parts, per_part, threads, blocks;
-};
-
-
-// Dense routing (at least one row per token on average): split every token row into 1-2 KiB parts.
-// Sparse receive shares (most tokens own no row and only get zero-filled): one workgroup per token
-// while that still fills the chip.
-CombineGrid combine_grid(int num_tokens, int num_rows, int vec)
-{
-    CombineGrid g;
-    const int target = num_rows >= num_tokens ? kDenseTargetBlocks : kSparseTargetBlocks;
-    int parts = 1;
-    while (num_tokens * parts < target && vec / (parts * 2) >= 64 && parts < 16) parts *= 2;
-    g.per_part = (vec + parts - 1) / parts;
-    // Dense routing: 1 KiB parts, one full wave each (at 4096 tokens x top-8 x 14 KiB rows 84 us, against 87 us for parts of
-    // 0.875 or 3.5 KiB, 90 us for 1.75 KiB on two waves and 125 us for 0.5 KiB).
-    if (num_rows >= num_tokens && vec >= kDenseVec) g.per_part = kDenseVec;
-    g.parts = (vec + g.per_part - 1) / g.per_part;
-    int threads = (g.per_part + 63) / 64 * 64;
-    g.threads = threads > kMaxThreads ? kMaxThreads : (threads < 64 ? 64 : threads);
-    g.blocks = num_tokens * g.parts;
-    return g;
-}
-
+// Dense routing (at least one row per token on average): a wave for every 64 vectors of the output, or of a token's row (at 4096 tokens x top-8 x 14 KiB rows parts of 1 KiB take
+// 84 us, of 0.875 or 3.5 KiB 87, of 1.75 KiB on two waves 90 and of 0.5 KiB 125).  Sparse receive shares (most tokens own no row and only get
+// zero-filled), and rows of less than 1 KiB: a workgroup per token while that still fills the chip.
 template <int kWeights, bool kHalf = false>
-void launch_combine(const CombineGrid& g, hipStream_t stream, const void* y, const float* weights, const int32_t* route_to_row,
-                    int num_topk, int vec, void* out, const float* return_in, float* return_out,
-                    int num_rows, const int32_t* shared_first_row = nullptr, int num_shared = 0, int num_tokens = 0,
-                    const int32_t* fill_state = nullptr, int leave_unserved = 0)
+void launch_combine(hipStream_t stream, const void* y, const float* weights, const int32_t* route_to_row, int num_tokens, int num_topk, int expected_rows,
+                    int vec, void* out, const float* return_in, float* return_out, int num_rows, const int32_t* shared_first_row = nullptr,
+                    int num_shared = 0, const int32_t* fill_state = nullptr, int leave_unserved = 0)
 {
-    hipLaunchKernelGGL((combine_kernel<kWeights, kHalf>), dim3(g.blocks), dim3(g.threads), 0, stream, static_cast<const u32x4*>(y),
-                       weights, route_to_row, num_topk, vec, g.per_part, g.parts, static_cast<u32x4*>(out), return_in,
+    const long long vectors = static_cast<long long>(num_tokens) * vec;
+    // (Rows of whole kilobytes gain nothing from it: 4096 tokens x top-8 of 4096 columns there and back 220.4 and 220.1 us, with the communication
+    // stream 256 against 252.)
+    if (expected_rows >= num_tokens && vec >= 64 && vec % 64 != 0 && vectors < (1LL << 31)) {
+        hipLaunchKernelGGL((combine_dense_kernel<kWeights, kHalf>), dim3(static_cast<unsigned>((vectors + 63) / 64)), dim3(64), 0, stream,
+                           static_cast<const u32x4*>(y), weights, route_to_row, num_topk, vec, static_cast<u32x4*>(out), return_in, return_out,
+                           shared_first_row, num_shared, num_tokens, fill_state, num_rows, leave_unserved);
+        return;
+    }
+    int parts = 1;
+    while (num_tokens * parts < kSparseTargetBlocks && vec / (parts * 2) >= 64 && parts < 16) parts *= 2;
+    int per_part = (vec + parts - 1) / parts;
+    if (expected_rows >= num_tokens && vec >= 64) per_part = 64;
+    parts = (vec + per_part - 1) / per_part;
+    const int threads = std::min(kMaxThreads, (per_part + 63) / 64 * 64);
+    hipLaunchKernelGGL((combine_kernel<kWeights, kHalf>), dim3(num_tokens * parts), dim3(threads), 0, stream, static_cast<const u32x4*>(y),
+                       weights, route_to_row, num_topk, vec, per_part, parts, static_cast<u32x4*>(out), return_in,
                        return_out, shared_first_row, num_shared, num_tokens, fill_state, num_rows, leave_unserved);
 }
 
@@ -295,9 +342,8 @@ int combine_routes(const void* y, const float* route_weights, const int32_t* rou
                                       0x7fffffff, leave_unserved, fill_state);
         return launch_status("combine_routes_share");
     }
-    const CombineGrid g = combine_grid(num_tokens, num_rows_hint, vec);
-    launch_combine<2>(g, stream, y, route_weights, route_to_row, num_topk, vec, out, nullptr, nullptr, 0x7fffffff,
-                      shared_first_row, num_shared, num_tokens, fill_state, leave_unserved);
+    launch_combine<2>(stream, y, route_weights, route_to_row, num_tokens, num_topk, num_rows_hint, vec, out, nullptr, nullptr, 0x7fffffff,
+                      shared_first_row, num_shared, fill_state, leave_unserved);
     return launch_status("combine_routes");
 }
 
@@ -338,12 +384,11 @@ int combine_entry(const char* what, const void* y, const float* row_weights, con
                                                   num_rows, leave_unserved);
         return launch_status(what);
     }
-    const CombineGrid g = combine_grid(num_tokens, hint, vec);
     if (row_weights != nullptr)
-        launch_combine<1, kHalf>(g, s, y, row_weights, route_to_row, num_topk, vec, out, return_in, return_out, num_rows, nullptr, 0,
-                                 0, nullptr, leave_unserved);
+        launch_combine<1, kHalf>(s, y, row_weights, route_to_row, num_tokens, num_topk, hint, vec, out, return_in, return_out, num_rows, nullptr, 0,
+                                 nullptr, leave_unserved);
     else
-        launch_combine<0, kHalf>(g, s, y, nullptr, route_to_row, num_topk, vec, out, return_in, return_out, num_rows, nullptr, 0, 0,
+        launch_combine<0, kHalf>(s, y, nullptr, route_to_row, num_tokens, num_topk, hint, vec, out, return_in, return_out, num_rows, nullptr, 0,
                                  nullptr, leave_unserved);
     return launch_status(what);
 }

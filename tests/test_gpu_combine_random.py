@@ -68,3 +68,33 @@ def test_combine_forms_at_random_shapes(seed):
         assert not got_bits[~served].any(), case
     if returned:
         np.testing.assert_array_equal(f32_bits(got_values), ocombine.return_weights(values, held).view(np.uint32), err_msg=str(case))
+
+
+@pytest.mark.parametrize("tokens,topk,hidden,density", [
+    (1, 3, 520, 1.0),      # one token: the last wave has one vector
+    (7, 32, 776, 0.3),     # 97 vectors: waves with a token's end and the next one's beginning at every lane
+    (64, 2, 1016, 0.7),    # 127; tokens without a row next to served ones
+    (333, 8, 1552, 0.9),
+    (130, 4, 512, 0.6),    # whole waves
+])
+def test_dense_rows_whose_waves_hold_two_tokens(tokens, topk, hidden, density):
+    from deepep_amd import ops
+
+    rng = np.random.default_rng(hidden)
+    valid = rng.random((tokens, topk)) < density
+    rows = int(valid.sum())
+    assert rows >= tokens
+    route_to_row = np.full((tokens, topk), -1, dtype=np.int32)
+    route_to_row[valid] = rng.permutation(rows).astype(np.int32)
+    y = torch.from_numpy(rng.normal(size=(rows, hidden)).astype(np.float32)).bfloat16()
+    weights, values = rng.random(rows).astype(np.float32), rng.random(rows).astype(np.float32)
+    served = torch.from_numpy((route_to_row >= 0).any(axis=1))
+    for served_only in (False, True):
+        out = torch.full((tokens + 1, hidden), 5.0, dtype=torch.bfloat16, device="cuda")  # (a row more than is written)
+        _, got_values = ops.combine(y.cuda(), torch.from_numpy(route_to_row).cuda(), torch.from_numpy(weights).cuda(),
+                                    torch.from_numpy(values).cuda(), out=out[:tokens], served_only=served_only)
+        want = ocombine.combine(bf16_bits(y), route_to_row, weights)
+        np.testing.assert_array_equal(bf16_bits(out[:tokens])[served.numpy()], want[served.numpy()])
+        others = out[:tokens][~served.cuda()]
+        assert bool((others == (5.0 if served_only else 0.0)).all()) and bool((out[tokens] == 5.0).all())
+        np.testing.assert_array_equal(f32_bits(got_values), ocombine.return_weights(values, route_to_row).view(np.uint32))
