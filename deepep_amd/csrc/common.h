@@ -69,7 +69,7 @@ struct Workspace {
 constexpr size_t kSyncFillStop = 64;
 constexpr size_t kSyncReporterTag = 128;
 constexpr size_t kSyncTagged = 256;
-constexpr size_t kSyncTaggedWords = 4096 + DPEP_MAX_LOCAL_EXPERTS;  // (workgroups + 1) * experts never exceeds this
+constexpr size_t kSyncTaggedWords = 8192 + DPEP_MAX_LOCAL_EXPERTS;  // (workgroups + 1) * experts never exceeds this
 constexpr size_t kSyncTotal = kSyncTagged + kSyncTaggedWords * 8;
 constexpr size_t kSyncRows = kSyncTotal + 256;
 constexpr int kSyncRowWords = 65536;

@@ -16,12 +16,13 @@
 //            lives in LDS.  There is no separate scan launch.
 // The smallest inputs take one workgroup, which holds everything (see "one workgroup" below).
 // Inputs whose chunks fit a wave's registers (at most kKeep steps of 64 routes) take ONE launch: the workgroups
-// (at most 65, far fewer than there are CUs, so all are resident together) count, publish their histograms as
+// (at most 129, far fewer than there are CUs, so all are resident together) count, publish their histograms as
 // self-validating words (count + the launch's tag in one 64-bit store), read each other's as soon as they appear, and
 // assign from the ids they still hold: no barrier, no counter that anybody has to reset.  The wait for the others'
 // words is bounded; a launch whose wait runs out assigns nothing (a histogram is missing): it reports no rows, marks
 // every route as having none, and leaves its number in the workspace's mailbox, where the host finds it; later layouts
 // on that workspace take two launches.  Larger inputs take two launches anyway.
+#include <algorithm>
 #include <mutex>
 #include <type_traits>
 
@@ -43,7 +44,8 @@ constexpr int kPrefetch = 8;          // 64-route steps whose ids are fetched at
 constexpr int kKeep = 16;             // 64-route steps of a chunk that the one-launch kernel holds in registers
 constexpr int kMegaExperts = 128;     // local experts of a MegaMoE forward, at most
 constexpr int kColumnBatch = 16;      // histogram loads in flight per thread
-static_assert(kSyncTaggedWords >= static_cast<size_t>(kBlockHistInts), "the tagged histograms need a word per (workgroup, expert)");
+constexpr int kTaggedInts = 32768;    // chunks * padded experts of the one-launch form
+static_assert(kSyncTaggedWords >= static_cast<size_t>(kTaggedInts / kWaves + DPEP_MAX_LOCAL_EXPERTS), "the tagged histograms need a word per (workgroup, expert)");
 
 __device__ __forceinline__ uint64_t lanes_below()
 {
@@ -477,7 +479,7 @@ __global__ __launch_bounds__(kThreads) void layout_assign_kernel(
 // out of time may use two tags, and the atomic max still leaves the epoch above both.  Replays of a captured launch
 // therefore get fresh tags without any host involvement.  40 tag bits last 10^12 launches.
 // Count, exchange, assign in one launch; every wave keeps the ids of its chunk (at most kSteps steps) in registers, and ranks
-// them within (wave, expert) while the words travel.  kSteps is the smallest of 4, 8 and kKeep that holds the chunk: the code is
+// them within (wave, expert) while the words travel.  kSteps is the smallest of 2, 4, 8 and kKeep that holds the chunk: the code is
 // straight-line, every launch finds the instruction caches cold, and steps that do nothing still had to be fetched (65 536
 // routes, 256 per wave, launches back to back: 6.8 us with sixteen steps that assigned behind the exchange, 6.3 with four
 // ranked ahead of it; with sixteen ranked ahead of it 7.7).
@@ -786,6 +788,17 @@ int chunk_routes(int n_routes, int padded_local, int hist_ints = kHistInts)
     return chunk < kMinChunk ? kMinChunk : chunk;
 }
 
+// The one-launch form's: 128 to 256 routes a wave, so that 128 waves share what there is; then 256, as long as that is at most 512 waves and the
+// histograms have room; then longer ones.  Shorter chunks than two-launch ones, because a wave's steps are a serial chain and the exchange costs
+// the same for 16 and for 128 workgroups (whole passes: 98 304 routes over 6 experts 144.5 -> 143.0 us, 32 768 over 256 147.9 -> 146.2, 36 864 over 6
+// 28.4 -> 28.2, 6000 over 160 30.8 -> 30.2; with 128 everywhere 32 768 over 128 experts 255.3 against 253.2).
+int one_launch_chunk(int n_routes, int padded_local)
+{
+    const int max_chunks = std::clamp(kTaggedInts / padded_local, 16, 512);
+    const int even = std::clamp((n_routes + 127) / 128, kMinChunk / 2, kMinChunk);
+    return (std::max(even, (n_routes + max_chunks - 1) / max_chunks) + kWave - 1) / kWave * kWave;
+}
+
 int check_layout_arguments(const void* idx, int num_tokens, int num_topk, int num_experts, int expert_begin, int num_local,
                            const int32_t* counts, const int32_t* psum, const int32_t* offsets, const int32_t* route_to_row,
                            const int32_t* row_to_route, const int32_t* num_rows)
@@ -856,8 +869,8 @@ int launch_layout(void* ws, const IdxT* idx, int num_tokens, int num_topk, int n
     }
     w->layout_launches = w->layout_launches == 0xffffffffu ? 1u : w->layout_launches + 1u;  // never 0
     const int padded = padded_experts(num_local);
-    int chunk = chunk_routes(n_routes, padded);
-    const bool one_launch = n_routes > 0 && chunk <= kKeep * kWave && w->layout_one_launch;
+    int chunk = one_launch_chunk(n_routes, padded);
+    const bool one_launch = n_routes > 0 && chunk_routes(n_routes, padded) <= kKeep * kWave && w->layout_one_launch;
     // Inputs that take two launches anyway get shorter chunks (more waves at work), with the larger histograms the
     // workspace has room for: 131 072 routes over 256 local experts 16 -> 64 workgroups.
     int hist_ints = kHistInts;
@@ -920,7 +933,8 @@ int launch_layout(void* ws, const IdxT* idx, int num_tokens, int num_topk, int n
             if (front != nullptr) launch(layout_fused_kernel<IdxT, true, kSteps>, front_blocks(*front, kFrontThreads), *front);
             else launch(layout_fused_kernel<IdxT, false, kSteps>, 0u, MegaFront{});
         };
-        if (chunk <= 4 * kWave) launch_steps(std::integral_constant<int, 4>{});
+        if (chunk <= 2 * kWave) launch_steps(std::integral_constant<int, 2>{});
+        else if (chunk <= 4 * kWave) launch_steps(std::integral_constant<int, 4>{});
         else if (chunk <= 8 * kWave) launch_steps(std::integral_constant<int, 8>{});
         else launch_steps(std::integral_constant<int, kKeep>{});
         return launch_status("layout_fused");
