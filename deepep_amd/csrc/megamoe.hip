@@ -2424,7 +2424,11 @@ GemmChoice choose_gemm(const GemmParams& p, const ExpectedRows& expected, int cu
             unfilled = std::min(zeros, (cus - tiles_of[best]) * 30e3 * best_cost) / 11e6;
         }
         const double few = std::min(one, four);
-        if (paired + unfilled < std::min(few, best_cost)) return pair_choice;
+        // (Against 64-row tiles, whose model is the worst of these where an expert has one of them, the paired kernel has to be a tenth ahead, but for
+        // the shortest k: whole forwards 336 tokens x top-1 of 8000 x 2688 over 14 experts and a shared one 159.3 -> 147.0 us, 888 x 4 of 5312 x 512 over 40
+        // 77.8 -> 67.7, 1000 x 2 of 7168 x 1024 over 48 146.2 -> 135.3; with k of 256, 1424 x 6 of 4224 x 256 over 26 46.9 and 56.5.)
+        const double margin = best == 1 && p.k_real > 384 ? 1.1 : 1.0;
+        if (paired + unfilled < few && (paired + unfilled) * margin < best_cost) return pair_choice;
         if (few < best_cost) return {32, one < four ? 1 : kGemmWaves, tiles, false, false, one < four && direct, row_tiles_per_expert};
     }
     if ((p.forced & 0xff) == 32) return {32, p.forced >> 8, tiles, false, false, (p.forced >> 8) == 1 && direct, row_tiles_per_expert};
