@@ -2408,7 +2408,9 @@ GemmChoice choose_gemm(const GemmParams& p, const ExpectedRows& expected, int cu
     // One-wave workgroups without LDS while there is at most one to a CU (16 % faster than with it over 167 launches, a tenth where tiles are
     // full), or two with about half a dozen rows per tile (4 % over 67); with more of either they are 1 to 20 % slower.
     const double waves = kGemmWaves * tiles, rows_per_tile = (p.num_routed * mean + static_cast<double>(num_shared) * expected.shared) * p.live_n_tiles / std::max(tiles, 1e-3);
-    const bool direct = waves <= cus || (waves <= 2.0 * cus && rows_per_tile <= 6.0);
+    // And while k is long enough for its requests to run ahead: up to four k tiles (one span) it is no faster, up to eight 6 % slower with more waves
+    // than CUs (42 launches with more than eight there: 9 % faster; 9 tokens over 38 experts of 1216 x 512, second GEMM 4.4 us with LDS, 5.6).
+    const bool direct = (waves <= cus && p.k_real > 4 * kBK) || (waves <= 2.0 * cus && rows_per_tile <= 6.0 && p.k_real > 8 * kBK);
     if (p.column_waves && p.forced == 0) {
         // (by the padded sizes, as fitted: by the real ones these kernels look too good where little of a tile is real)
         const double all_tiles = live_row_tiles * n_tiles;
