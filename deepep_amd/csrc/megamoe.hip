@@ -2320,7 +2320,7 @@ struct ExpectedRows {
 // rounds on 256 CUs, 192-row tiles need 2 = one round; measured 94 vs 67 us.)
 // Times are in microseconds, fitted to kernel traces of both GEMMs on an MI355X at 263 shapes (2 to 100 experts, k from 512 to
 // 8192): once per launch; per round of one tile per CU its epilogue and switch, and per k tile the main loop and the weights'
-// way from memory, which the row tiles of an expert share; nothing below the time to read the weights once.  What it picks is 1.1 %
+// way from memory, which the row tiles of an expert share; nothing below the time to read the weights once.  What it picks is 1.3 %
 // slower than the best on average.  How to refit: force each height with the workspace setting "gemm_tile_rows" and
 // take a kernel trace.
 // The few-rows kernel is the better one for small launches whatever the rows: a CU draws no more than about 50 GB/s from
