@@ -50,6 +50,7 @@ struct Workspace {
     long long exchange_ticks;
     int exchange_extra_rows;
     int layout_one_launch;
+    int payload_looks;         // of a payload in the layout's grid for a word of the layout's, before it works its rows out itself
     uint32_t layout_launches;  // number of the most recent layout launch (never 0)
     uint32_t timeout_seen;     // number of the last timed-out launch the host has been told about
     int gemm_zero_fill;        // 1 (default): idle workgroups of the first GEMM zero rows of unserved tokens; 0: the reduce does
@@ -89,6 +90,7 @@ constexpr int kMailboxBlock = DPEP_MAX_LOCAL_EXPERTS;  // words of one block of 
 constexpr int kMailboxWords = kMailboxCounts + 2 * kMailboxBlock;
 inline __host__ __device__ bool mailbox_narrow(int n_routes) { return n_routes < 65536; }
 constexpr long long kLayoutExchangeTicks = 200000000;  // 2 s
+constexpr int kPayloadLooks = 64;  // one or two microseconds apart; the words are there after about six
 constexpr uint32_t kWorkspaceMagic = 0x44504550u;  // "DPEP"
 Workspace* as_workspace(void* ws);
 

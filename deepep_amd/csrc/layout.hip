@@ -603,10 +603,12 @@ __global__ __launch_bounds__(kThreads) void layout_fused_kernel(
 }
 
 // ---- layout and payload in one grid ------------------------------------------------------------------------------------
-// The payload's workgroups, behind the layout's in the same grid, ask for their tokens at once and wait for the words that say where
+// The payload's workgroups, behind the layout's in the same grid, ask for their tokens at once and look for the words that say where
 // these go: between the routes' ids and the first payload store there is no second launch, whose ramp and first loads would follow
-// the layout's last store.  A wait is short of a deadlock whatever else runs: the layout's workgroups come first in
-// the grid and wait for no payload, and every wait is bounded.  The words carry the number of the launch, which comes from the host, so a
+// the layout's last store.  A payload workgroup looks for a while only (kPayloadLooks); where the words do not come it works its rows out
+// from the ids itself and waits for nobody.  It must not wait without such a bound: a grid is dealt over eight XCDs, each of which starts
+// its share by itself, the layout's workgroups need each other across them, and two such grids at once could each hold an
+// XCD that the other's layout has yet to enter.  The words carry the number of the launch, which comes from the host, so a
 // captured launch (whose replays would repeat it) takes two.  128 registers, as the layout wants: four workgroups to a CU carry the payload
 // as fast as eight (with 64 the layout spills, and the kernel takes 7 us longer).
 // Bound by HBM once the words are there.  Dispatch and combine, launches back to back, one grid / two: 1000 tokens x top-6 of 5120 BF16 30.5 / 31.7 us,
@@ -614,6 +616,150 @@ __global__ __launch_bounds__(kThreads) void layout_fused_kernel(
 // workgroup of its own is the better one (710 x 4 of 2672 20.1 / 18.7).
 // Chunks of at most four steps: with eight (32 768 routes over 256 experts, skewed popularity, 235 MB) one grid took 149.9 us, two 146.6.
 constexpr int kRidingExperts = 256, kRidingSteps = 4;
+
+// What the rows follow from.
+struct Routing {
+    const int64_t* idx;
+    int n_routes, num_experts, expert_begin, num_local;
+    // Calls visit(local expert or -1, route) for the routes that this one of `waves` waves goes through, in order.
+    template <typename Visit>
+    __device__ __forceinline__ void scan(int wave, int waves, Visit&& visit) const
+    {
+        for (int base = wave * kPrefetch * kWave; base < n_routes; base += waves * kPrefetch * kWave) {
+            int experts[kPrefetch];
+            fetch_experts(experts, idx, base, n_routes, n_routes, num_experts, expert_begin, num_local);
+#pragma unroll
+            for (int i = 0; i < kPrefetch; ++i) visit(experts[i], base + i * kWave + (static_cast<int>(threadIdx.x) & 63));
+        }
+    }
+};
+
+// One look: whether the word is this launch's, and its value.
+__device__ __forceinline__ bool look(const unsigned long long* word, uint32_t launch, int& value)
+{
+    const unsigned long long v = load_word(word);
+    value = static_cast<int>(static_cast<uint32_t>(v));
+    return static_cast<uint32_t>(v >> 32) == launch;
+}
+
+// Looks past the caches, by a thousand workgroups, delay the layout that they wait for: kNaps of 256 cycles lie between two (1000 tokens x top-6
+// 31.0 us with one look per microsecond, 32.3 with one per two; a few hundred rows of 6144 tokens 28.6 with one per two, 28.8 with
+// one, 29.7 with three).
+template <int kNaps>
+__device__ __forceinline__ void nap()
+{
+    for (int i = 0; i < kNaps; ++i) __builtin_amdgcn_s_sleep(4);
+}
+
+// Where a token's rows come from: row_of(), by one thread for each route, between two barriers of the workgroup; where any of its threads gave
+// up, all of them go through work_out().
+struct AwaitedTokens {
+    static constexpr bool kAwaits = true;
+    Routing routing;
+    const unsigned long long* words;
+    const unsigned long long* total;
+    uint32_t launch;
+    int looks;
+    int capacity, all_or_none;
+    int* late;                       // LDS of the workgroup
+    int (*rows_of)[kRidingExperts];  // LDS of this token's threads: rows of every expert, and those of them from tokens before
+    __device__ __forceinline__ int begin() const { return 0; }
+    __device__ __forceinline__ void before_the_wait() const
+    {
+        if (threadIdx.x == 0) *late = 0;
+    }
+    __device__ __forceinline__ bool gave_up() const { return *late != 0; }
+    __device__ __forceinline__ bool await(const unsigned long long* word, int& value) const
+    {
+        for (int i = 0; i < looks; ++i, nap<8>())
+            if (look(word, launch, value)) return true;
+        *late = 1;
+        return false;
+    }
+    __device__ __forceinline__ int kept(int row, int all) const
+    {
+        return row < capacity && (all_or_none == 0 || DPEP_ROWS_KEPT(all, capacity)) ? row : -1;
+    }
+    __device__ __forceinline__ int row_of(size_t route, int) const
+    {
+        int row, all = 0;
+        if (!await(words + route, row) || row < 0 || row >= capacity) return -1;
+        if (all_or_none != 0 && !await(total, all)) return -1;
+        return kept(row, all);
+    }
+    // The same rows without the words: row = rows of the experts before + earlier routes to the same expert.
+    __device__ __forceinline__ void work_out(const PayloadShape& p, int token, int t, TokenLds& lds) const
+    {
+        const int first = token * p.num_topk;
+        if (t == 0) lds.any_valid = 0;
+        for (int e = t; e < routing.num_local; e += p.threads) rows_of[0][e] = rows_of[1][e] = 0;
+        __syncthreads();
+        routing.scan(t >> 6, p.threads >> 6, [&](int e, int route) {
+            if (e < 0) return;
+            atomicAdd(&rows_of[0][e], 1);
+            if (route < first) atomicAdd(&rows_of[1][e], 1);
+        });
+        __syncthreads();
+        if (t < p.num_topk) {
+            auto expert_of = [&](int s) {
+                return local_expert(routing.idx[first + s], first + s, routing.n_routes, routing.num_experts, routing.expert_begin, routing.num_local);
+            };
+            const int mine = expert_of(t);
+            int all = 0, row = mine < 0 ? -1 : rows_of[1][mine];
+            for (int e = 0; e < routing.num_local; ++e) {
+                if (e < mine) row += rows_of[0][e];
+                all += rows_of[0][e];
+            }
+            for (int s = 0; s < t && mine >= 0; ++s) row += expert_of(s) == mine ? 1 : 0;
+            row = row < 0 ? -1 : kept(row, all);
+            lds.rows[t] = row;
+            if (row >= 0) lds.any_valid = 1;
+        }
+        __syncthreads();
+    }
+};
+
+// Where a row's route comes from; every wave looks by itself.
+struct AwaitedRows {
+    Routing routing;
+    const unsigned long long* words;
+    const unsigned long long* total;
+    uint32_t launch;
+    int looks;
+    int rows;      // bound of R
+    int* rows_of;  // LDS of this wave: rows of every expert
+    // The route of row `row` below the bound; -1: there is no such row.  Called by whole waves.
+    __device__ __forceinline__ int route_of(int row) const
+    {
+        for (int i = 0; i < looks; ++i, nap<16>()) {
+            int route, all;
+            const bool has_route = look(words + row, launch, route), has_total = look(total, launch, all);
+            if (__builtin_amdgcn_readfirstlane(has_route ? 1 : 0)) return __builtin_amdgcn_readfirstlane(route);
+            if (__builtin_amdgcn_readfirstlane(has_total && row >= all ? 1 : 0)) return -1;
+        }
+        return work_out(row);
+    }
+    // The same without the words: the expert whose rows hold `row`, then that expert's route by its rank.
+    __device__ __forceinline__ int work_out(int row) const
+    {
+        for (int e = threadIdx.x & 63; e < routing.num_local; e += kWave) rows_of[e] = 0;
+        wave_sync();
+        routing.scan(0, 1, [&](int e, int) { count_step(e, rows_of); });
+        wave_sync();
+        int expert = 0, rank = row, route = -1;
+        while (expert < routing.num_local && rank >= rows_of[expert]) rank -= rows_of[expert++];
+        wave_sync();  // (the next row's counts go to the same place)
+        if (expert == routing.num_local) return -1;
+        routing.scan(0, 1, [&](int e, int at) {
+            const unsigned long long same = __ballot(e == expert);
+            const unsigned long long it = __ballot(e == expert && __popcll(same & lanes_below()) == rank);
+            if (it != 0) route = at - (static_cast<int>(threadIdx.x) & 63) + __ffsll(it) - 1;  // (once: the rank falls below zero)
+            rank -= __popcll(same);
+        });
+        return __builtin_amdgcn_readfirstlane(route);
+    }
+};
+
 template <bool kQuant, bool kRowMajor, bool kStaged>
 __global__ __launch_bounds__(kThreads, 4) void layout_payload_kernel(
     const int64_t* __restrict__ idx, int n_routes, int num_experts, int expert_begin, int num_local, int padded_local,
@@ -622,13 +768,15 @@ __global__ __launch_bounds__(kThreads, 4) void layout_payload_kernel(
     SendCounts send, uint32_t* __restrict__ mailbox, uint32_t sequence, unsigned long long* __restrict__ epoch,
     unsigned long long* __restrict__ tagged, int num_blocks, int rows, long long limit_ticks, uint32_t* __restrict__ timeouts,
     uint32_t launch_id,
-    unsigned long long* __restrict__ total_word, unsigned long long* __restrict__ row_words, LayoutPayload payload)
+    unsigned long long* __restrict__ total_word, unsigned long long* __restrict__ row_words, int looks, LayoutPayload payload)
 {
     using Lds = LayoutLds<kRidingExperts, true>;
     struct Riding {
         TokenLds tokens[kWaves];
         float scales[kQuant && !kRowMajor ? kMaxScaleCols : 1];
         u32x4 stage[kStaged ? kStagedVec : 1];
+        int late;
+        int rows_of[kStaged ? 1 : kWaves][2][kRidingExperts];
     };
     __shared__ union Both {
         Lds layout;
@@ -644,13 +792,13 @@ __global__ __launch_bounds__(kThreads, 4) void layout_payload_kernel(
     const int per = kThreads / p.threads, sub = threadIdx.x / p.threads, t = threadIdx.x - sub * p.threads;
     const unsigned block = (blockIdx.x - num_blocks - 1) * per + sub;
     if (sub >= per || block >= payload.blocks) return;  // (whole waves)
-    const AwaitedWords words = {row_words, total_word, launch_id, 4 * limit_ticks, timeouts, kRowMajor ? 16 : 8};
+    const Routing routing = {idx, n_routes, num_experts, expert_begin, num_local};
     if (kRowMajor) {
-        const AwaitedRows rows = {words, payload.rows, payload.all_or_none};
+        const AwaitedRows rows = {routing, row_words, total_word, launch_id, looks, payload.rows, lds.riding.rows_of[threadIdx.x >> 6][0]};
         if (kQuant) quant_rows<DPEP_STORE_STREAMING>(payload.x, payload.weights, payload.out, payload.out_scales, payload.out_weights, p, rows, block, payload.blocks / p.parts, t);
         else copy_rows<DPEP_STORE_STREAMING>(payload.x, payload.scales, payload.weights, payload.out, payload.out_scales, payload.out_weights, p, rows, block, payload.blocks / p.parts, t);
     } else {
-        const AwaitedTokens tokens = {words, payload.capacity, payload.all_or_none};
+        const AwaitedTokens tokens = {routing, row_words, total_word, launch_id, looks, payload.capacity, payload.all_or_none, &lds.riding.late, lds.riding.rows_of[sub]};
         if (kQuant) quant_token<DPEP_STORE_STREAMING>(payload.x, payload.weights, payload.out, payload.out_scales, payload.out_weights, p, tokens, block, t, lds.riding.tokens[sub], lds.riding.scales + sub * (p.threads / 8));
         else copy_token<DPEP_STORE_STREAMING, kStaged>(payload.x, payload.scales, payload.weights, payload.out, payload.out_scales, payload.out_weights, p, tokens, block, t,
                                                        lds.riding.tokens[sub], lds.riding.stage);
@@ -919,7 +1067,7 @@ int launch_layout(void* ws, const IdxT* idx, int num_tokens, int num_topk, int n
                                        reinterpret_cast<unsigned long long*>(sync + kSyncTagged), blocks, blocks + w->exchange_extra_rows,
                                        w->exchange_ticks, w->mailbox_device + kMailboxTimeout, w->layout_launches,
                                        reinterpret_cast<unsigned long long*>(sync + kSyncTotal), reinterpret_cast<unsigned long long*>(sync + kSyncRows),
-                                       *payload);
+                                       w->payload_looks, *payload);
                 };
                 if (payload->row_major) payload->quantize ? ride(layout_payload_kernel<true, true, false>) : ride(layout_payload_kernel<false, true, false>);
                 else if (payload->quantize) ride(layout_payload_kernel<true, false, false>);

@@ -1,5 +1,5 @@
 // The payload of a dispatch, out[row(t,s)] = x[t], as device functions: token-major or row-major, copied or quantised to FP8.  They run as
-// kernels of their own behind a layout that has ended (Mapped..., dispatch.hip), or in the layout's own grid, where they wait for the
+// kernels of their own behind a layout that has ended (Mapped..., dispatch.hip), or in the layout's own grid, where they look for the
 // places of their rows (Awaited..., layout.hip).
 //
 // Observable contract: as dispatch.hip.
@@ -32,6 +32,7 @@ struct PayloadShape {
 // Token-major, in the map that an earlier launch has left.  Rows at or beyond `capacity` are dropped; with all_rows (the layout's
 // count) nothing is moved unless DPEP_ROWS_KEPT.
 struct MappedTokens {
+    static constexpr bool kAwaits = false;
     const int* route_to_row;
     int capacity;
     const int* all_rows;
@@ -44,82 +45,11 @@ struct MappedTokens {
 };
 
 // In the layout's own grid (layout.hip) a route's row, or a row's route, comes as a word that says itself which launch it belongs to:
-// the launch's number above, the value (-1: no row) below.  `total` gets R the same way.  A wait is bounded; one that runs out moves
-// nothing and leaves the launch's number in the host mailbox, as a layout's own wait does.
+// the launch's number above, the value (-1: no row) below.  The number of rows comes the same way.
 __device__ __forceinline__ unsigned long long row_word(uint32_t launch, int value)
 {
     return static_cast<unsigned long long>(launch) << 32 | static_cast<uint32_t>(value);
 }
-struct AwaitedWords {
-    const unsigned long long* words;
-    const unsigned long long* total;
-    uint32_t launch;
-    long long limit_ticks;
-    uint32_t* timeouts;
-    int naps;  // of 256 cycles each, between two looks
-    // Called again and again with the number of the attempt: false when the time is up.
-    __device__ __forceinline__ bool patient(int spins, long long& start) const
-    {
-        if ((spins & 15) == 15) {
-            const long long now = wall_clock64();
-            if (start == 0) start = now;
-            if (now - start > limit_ticks) {
-                __hip_atomic_store(timeouts, launch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-                return false;
-            }
-        }
-        // (Looks past the caches, by a thousand workgroups, delay the layout that they wait for: 1000 tokens x top-6 31.0 us with one look per
-        // microsecond, 32.3 with one per two; a few hundred rows of 6144 tokens 28.6 with one per two, 28.8 with one, 29.7 with three.)
-        for (int i = 0; i < naps; ++i) __builtin_amdgcn_s_sleep(4);
-        return true;
-    }
-    __device__ __forceinline__ int await(const unsigned long long* word, int otherwise) const
-    {
-        long long start = 0;
-        for (int spins = 0;; ++spins) {
-            const unsigned long long v = __hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if (static_cast<uint32_t>(v >> 32) == launch) return static_cast<int>(static_cast<uint32_t>(v));
-            if (!patient(spins, start)) return otherwise;
-        }
-    }
-};
-struct AwaitedTokens {
-    AwaitedWords from;
-    int capacity;
-    int all_or_none;
-    __device__ __forceinline__ int begin() const { return 0; }
-    __device__ __forceinline__ int row_of(size_t route, int) const
-    {
-        const int row = from.await(from.words + route, -1);
-        if (row < 0 || row >= capacity) return -1;
-        if (all_or_none == 0) return row;
-        const int all = from.await(from.total, 0);
-        return DPEP_ROWS_KEPT(all, capacity) ? row : -1;
-    }
-};
-struct AwaitedRows {
-    AwaitedWords from;
-    int rows;         // bound of R
-    int all_or_none;  // the outputs' capacity: no rows at all unless DPEP_ROWS_KEPT; 0: the first rows in any case
-    __device__ __forceinline__ int bound() const
-    {
-        if (all_or_none == 0) return rows;
-        const int all = from.await(from.total, 0);
-        return DPEP_ROWS_KEPT(all, all_or_none) ? min(all, rows) : 0;
-    }
-    // The route of row `row` below the bound; -1: there is no such row.
-    __device__ __forceinline__ int route_of(int row) const
-    {
-        long long start = 0;
-        for (int spins = 0;; ++spins) {
-            const unsigned long long v = __hip_atomic_load(from.words + row, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            const unsigned long long total = __hip_atomic_load(from.total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if (static_cast<uint32_t>(v >> 32) == from.launch) return static_cast<int>(static_cast<uint32_t>(v));
-            if (static_cast<uint32_t>(total >> 32) == from.launch && row >= static_cast<int>(static_cast<uint32_t>(total))) return -1;
-            if (!from.patient(spins, start)) return -1;
-        }
-    }
-};
 
 // ---- token-major: one token and column part to `p.threads` threads; read once, write K times ----------------------------------
 // t: the thread's number among them.  Called by all threads of a workgroup whose `block` is in range.
@@ -132,6 +62,7 @@ template <typename Tokens>
 __device__ __forceinline__ bool rows_of_token(const PayloadShape& p, const Tokens& tokens, int all, int token, int t, TokenLds& lds)
 {
     if (t == 0) lds.any_valid = 0;
+    if constexpr (Tokens::kAwaits) tokens.before_the_wait();
     __syncthreads();
     if (t < p.num_topk) {
         const int row = tokens.row_of(static_cast<size_t>(token) * p.num_topk + t, all);
@@ -139,6 +70,8 @@ __device__ __forceinline__ bool rows_of_token(const PayloadShape& p, const Token
         if (row >= 0) lds.any_valid = 1;
     }
     __syncthreads();
+    if constexpr (Tokens::kAwaits)
+        if (tokens.gave_up()) tokens.work_out(p, token, t, lds);
     return lds.any_valid != 0;
 }
 
@@ -212,15 +145,15 @@ __device__ __forceinline__ void copy_token(const u32x4* __restrict__ x, const fl
 // ---- row-major, in the layout's grid: one output row and column part to `p.threads` threads; for sparse receive shares --------
 // stride: rows between two of a workgroup.  (dispatch.hip has the same for maps that are there already: in one piece with this its prologue
 // grew by 0.1 us, a fortieth of what a few hundred rows take.)
-template <int kPolicy>
+template <int kPolicy, typename Rows>
 __device__ __forceinline__ void copy_rows(const u32x4* __restrict__ x, const float* __restrict__ scales, const float* __restrict__ weights,
                                           u32x4* __restrict__ out, float* __restrict__ out_scales, float* __restrict__ out_weights,
-                                          const PayloadShape& p, const AwaitedRows& source, unsigned block, int stride, int t)
+                                          const PayloadShape& p, const Rows& source, unsigned block, int stride, int t)
 {
     const int part = block % static_cast<unsigned>(p.parts);
     const int v_begin = part * p.per_part, v_end = min(v_begin + p.per_part, p.units);
     int row = block / static_cast<unsigned>(p.parts);
-    for (const int bound = source.bound(); row < bound; row += stride) {
+    for (; row < source.rows; row += stride) {
         const int route = source.route_of(row);
         if (route < 0) return;
         const int token = route / p.num_topk;
@@ -368,16 +301,16 @@ __device__ __forceinline__ void quant_token(const u32x4* __restrict__ x, const f
 }
 
 // row-major, in the layout's grid
-template <int kPolicy>
+template <int kPolicy, typename Rows>
 __device__ __forceinline__ void quant_rows(const u32x4* __restrict__ x, const float* __restrict__ weights, u32x4* __restrict__ out,
                                            float* __restrict__ out_scales, float* __restrict__ out_weights, const PayloadShape& p,
-                                           const AwaitedRows& source, unsigned block, int stride, int t)
+                                           const Rows& source, unsigned block, int stride, int t)
 {
     const int part = block % static_cast<unsigned>(p.parts);
     const int u_begin = part * p.per_part, u_end = min(u_begin + p.per_part, p.units);
     const int scale_cols = p.units / 8;
     int row = block / static_cast<unsigned>(p.parts);
-    for (const int bound = source.bound(); row < bound; row += stride) {
+    for (; row < source.rows; row += stride) {
         const int route = source.route_of(row);
         if (route < 0) return;
         const int token = route / p.num_topk;
@@ -402,7 +335,7 @@ struct LayoutPayload {
     PayloadShape shape;
     bool quantize, staged, row_major;
     unsigned blocks;
-    int rows, capacity, all_or_none;  // rows: row-major, the bound of R; capacity: token-major
+    int rows, capacity, all_or_none;  // rows: row-major, the bound of R; the others: token-major
 };
 
 }  // namespace dpep

@@ -88,6 +88,7 @@ int dpep_workspace_create(size_t bytes, void** ws)
     w->exchange_ticks = dpep::kLayoutExchangeTicks;
     w->exchange_extra_rows = 0;
     w->layout_one_launch = 1;
+    w->payload_looks = dpep::kPayloadLooks;
     w->gemm_tile_rows = 0;
     w->gemm_few_rows_waves = 4;
     w->gemm_column_waves = 1;
@@ -185,6 +186,9 @@ int dpep_workspace_tune(void* ws, const char* key, long long value)
     } else if (strcmp(key, "layout_exchange_extra_rows") == 0) {
         DPEP_REQUIRE(value >= 0 && value <= 1, "workspace_tune: layout_exchange_extra_rows is 0 or 1");
         w->exchange_extra_rows = static_cast<int>(value);
+    } else if (strcmp(key, "layout_payload_looks") == 0) {
+        DPEP_REQUIRE(value >= 0 && value <= dpep::kPayloadLooks, "workspace_tune: layout_payload_looks is 0 to %d", dpep::kPayloadLooks);
+        w->payload_looks = static_cast<int>(value);
     } else if (strcmp(key, "gemm_zero_fill") == 0) {
         w->gemm_zero_fill = value != 0;
     } else if (strcmp(key, "megamoe_served_only") == 0) {

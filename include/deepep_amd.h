@@ -45,6 +45,8 @@ int dpep_workspace_capacity(void* ws, size_t* bytes);
  *   "layout_exchange_ticks"         bound of a workgroup's wait for the others' histograms in 10 ns ticks (default 2 s)
  *   "layout_exchange_extra_rows"    1: the workgroups wait for one histogram more than there are workgroups, so that
  *                                   the wait runs out (exercises the error path)
+ *   "layout_payload_looks"          how often a payload in the layout's grid looks for a word of the layout's, one or two
+ *                                   microseconds apart, before it works its rows out from the ids itself (0 to 64, the default)
  *   "gemm_zero_fill"                1 (default): workgroups of dpep_megamoe_forward's first GEMM that get no tile zero
  *                                   the output rows of tokens no local expert serves; 0: the weighted reduce writes them
  *   "megamoe_served_only"           1: dpep_megamoe_forward leaves the rows of y whose token no local expert serves

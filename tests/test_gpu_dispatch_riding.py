@@ -122,6 +122,94 @@ def test_riding_payload_equals_one_of_its_own_launch(tokens, topk, experts, begi
         workspace.destroy()
 
 
+# The payload may look for the layout's words `looks` times; with none it never sees one, as where the layout cannot start for whatever else
+# runs, and everything that it moves follows from the ids alone.  (Ids drawn with repetition: a route's row counts the token's own earlier ones.)
+@pytest.mark.parametrize("looks", [0, 1])
+@pytest.mark.parametrize("tokens,topk,experts,begin,local,row_bytes,scale_cols,quantize,report,spare", [
+    (1100, 8, 32, 0, 32, 4096, 0, False, 1, 0),       # four tokens' threads to a workgroup, the last workgroup not full
+    (1101, 8, 32, 0, 32, 4096, 3, False, 1, -300),
+    (420, 10, 40, 0, 40, 12128, 0, False, 1, 0),      # through LDS
+    (2040, 8, 256, 0, 256, 2176, 0, False, 1, 0),     # as many experts as ride
+    (700, 32, 64, 0, 64, 1536, 0, False, 1, 100),
+    (1700, 12, 96, 48, 48, 4096, 5, False, 2, 0),     # all of the rows, or none
+    (1700, 12, 96, 48, 48, 4096, 5, False, 2, -1),
+    (640, 8, 128, 0, 128, 14336, 0, True, 1, 0),
+    (3000, 20, 40, 0, 20, 2560, 0, True, 2, 0),
+    (6000, 4, 256, 12, 4, 7168, 56, False, 0, 1000),  # row-major: fewer rows than the grid has
+    (6000, 4, 256, 12, 4, 7168, 0, False, 0, -100),
+    (6000, 4, 256, 252, 4, 14336, 0, True, 0, 1000),
+    (1029, 4, 1024, 800, 200, 464, 0, False, 0, 0),   # a last step of 20 routes
+    (32768, 2, 256, 0, 1, 256, 0, True, 0, 0),
+])
+def test_payload_that_gives_up_its_wait_works_its_rows_out(tokens, topk, experts, begin, local, row_bytes, scale_cols, quantize, report, spare, looks):
+    from deepep_amd import ops
+
+    rng = np.random.default_rng(tokens + topk + looks)
+    workspace = ops.Workspace(4 << 20)
+    try:
+        workspace.tune("layout_payload_looks", looks)
+        ids, x, scales, weights = _inputs(rng, tokens, topk, experts, row_bytes, scale_cols, quantize, 0.0)
+        ids = np.where(rng.random(ids.shape) < 0.1, -1, rng.integers(0, experts, ids.shape))
+        want = olayout.layout(ids, experts, begin, local)
+        capacity = want["num_rows"] + (want["num_rows"] // 8 + 256 if report == 2 and spare == 0 else spare)
+        idx = torch.from_numpy(ids).cuda()
+        args = (idx, x, scales, weights, experts, begin, local, quantize, capacity, report)
+        riding, plain = _Call(*args), _Call(*args)
+        riding.launch(workspace)
+        torch.cuda.synchronize()
+        before = ops.dispatch_store_policy("through")
+        try:
+            plain.launch(workspace)
+            torch.cuda.synchronize()
+        finally:
+            ops.dispatch_store_policy(before)
+        riding.same_as(plain, want["num_rows"])
+        np.testing.assert_array_equal(riding.forward.cpu().numpy().reshape(tokens, topk), want["route_to_row"])
+    finally:
+        torch.cuda.synchronize()
+        workspace.destroy()
+
+
+@pytest.mark.parametrize("looks", [64, 1])
+def test_two_riding_grids_at_once(looks):
+    """Two workspaces on two streams, each grid with several times the workgroups that the GPU holds, queued with nothing between them."""
+    from deepep_amd import ops
+
+    rng = np.random.default_rng(9)
+    tokens, topk, experts = 4096, 8, 64
+    workspaces = [ops.Workspace(4 << 20) for _ in range(2)]
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    try:
+        for workspace in workspaces:
+            workspace.tune("layout_payload_looks", looks)
+        batches = []
+        for _ in range(2):
+            ids, x, _, weights = _inputs(rng, tokens, topk, experts, 2048, 0, False, 0.1)
+            want = olayout.layout(ids, experts, 0, experts)
+            args = (torch.from_numpy(ids).cuda(), x, None, weights, experts, 0, experts, False, want["num_rows"], 0)
+            batches.append((want["num_rows"], [_Call(*args) for _ in range(4)], _Call(*args)))
+        torch.cuda.synchronize()
+        for turn in range(4):
+            for workspace, stream, (_, calls, _) in zip(workspaces, streams, batches):
+                with torch.cuda.stream(stream):
+                    calls[turn].launch(workspace)
+        torch.cuda.synchronize()
+        before = ops.dispatch_store_policy("through")
+        try:
+            for workspace, (_, _, plain) in zip(workspaces, batches):
+                plain.launch(workspace)
+            torch.cuda.synchronize()
+        finally:
+            ops.dispatch_store_policy(before)
+        for rows, calls, plain in batches:
+            for call in calls:
+                call.same_as(plain, rows)
+    finally:
+        torch.cuda.synchronize()
+        for workspace in workspaces:
+            workspace.destroy()
+
+
 def test_captured_dispatch_takes_two_launches():
     """Replays with new ids, ordinary calls between them: a payload that waited for words would find those of the replay before."""
     from deepep_amd import ops
