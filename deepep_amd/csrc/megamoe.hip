@@ -245,8 +245,8 @@ struct GemmParams {
     int fill_tokens, fill_vec, fill_topk;
     int* fill_state;
     int* fill_stop;
-    int forced;                     // 64 / 128 / 192: that tile height whatever the cost model says (tests); 32: the few-rows kernel
-                                    //   with (1, 4) << 8 waves per workgroup; 0: the model decides
+    int forced;                     // 64 / 128 / 192: that tile height whatever the cost model says (tests), 128 | 1 << 8: the paired kernel; 32: the
+                                    //   few-rows kernel with (1, 4) << 8 waves per workgroup; 0: the model decides
     int column_waves;               // 1: the kernel whose waves split the tile's columns and load their weights straight into registers
     int n_real, k_real;             // what is not padding of n and k (first GEMM: n counts gate and up)
     int live_n_tiles;               // column tiles that the kernels that skip padding work on (first GEMM: all, unless the second reads none of it)
@@ -2285,11 +2285,13 @@ int launch_paired(const GemmParams& p, hipStream_t stream, const char* what)
     return launch_status(what);
 }
 
+bool column_waves(const GemmParams& p) { return p.column_waves && p.k % 512 == 0; }
+
 template <int RT, bool kGateUp>
 int launch_gemm_rt(const GemmParams& p, double expected_tiles, hipStream_t stream, const char* what)
 {
     constexpr int kMaxDevices = 64;
-    if (p.column_waves && p.k % 512 == 0) {
+    if (column_waves(p)) {
         constexpr int kLds = ColCfg<RT>::kLdsBytes;
         static std::atomic<bool> configured[kMaxDevices];
         if (int rc = allow_lds(&grouped_gemm_colwave_kernel<RT, kGateUp>, kLds, configured, kMaxDevices)) return rc;
@@ -2356,7 +2358,7 @@ GemmChoice choose_gemm(const GemmParams& p, const ExpectedRows& expected, int cu
     const double weight_bytes = (p.num_routed * routed_with_rows + num_shared) * n_tiles * ktiles * 16896.0;
     // Nothing ends before the weights are read; where that decides, the one that would be done first otherwise is still better.
     auto bounded = [&](double t) { return std::max(2.0 + weight_bytes / 6.3e6, t) + 0.05 * t; };
-    const int kind = p.column_waves && p.k % 512 == 0 ? 0 : 1;  // the kernel that launch_gemm_rt takes: column waves, 2 x 2
+    const int kind = column_waves(p) ? 0 : 1;  // the kernel that launch_gemm_rt takes: column waves, 2 x 2
     double paired_row_tiles = 0.0;
     int best = 2;
     double best_cost = 1e30, tiles_of[4] = {0.0, 0.0, 0.0, 0.0};
@@ -2434,7 +2436,7 @@ GemmChoice choose_gemm(const GemmParams& p, const ExpectedRows& expected, int cu
         if (few < best_cost) return {32, one < four ? 1 : kGemmWaves, tiles, false, false, one < four && direct, row_tiles_per_expert};
     }
     if ((p.forced & 0xff) == 32) return {32, p.forced >> 8, tiles, false, false, (p.forced >> 8) == 1 && direct, row_tiles_per_expert};
-    if (p.forced == 128 && p.column_waves && (p.fill_tokens == 0 || tiles_of[2] >= cus)) return pair_choice;
+    if (p.forced == (128 | 1 << 8)) return {128, kGemmWaves, paired_row_tiles * p.live_n_tiles, true, false, false, 0.0};
     if (p.forced != 0) best = p.forced / 64;
     return {64 * best, kGemmWaves, tiles_of[best], false, false, false, 0.0};
 }
@@ -2493,7 +2495,8 @@ GemmParams gemm_of(const MegaSizes& m, const Workspace* w, bool second)
     p.n_real = second ? m.hidden : 2 * m.intermediate;
     p.k_real = second ? m.intermediate : m.hidden;
     p.live_n_tiles = second ? (m.hidden + kBN - 1) / kBN : p.n / kBN;
-    p.forced = w == nullptr ? 0 : w->gemm_tile_rows == 32 ? 32 | w->gemm_few_rows_waves << 8 : w->gemm_tile_rows;
+    const int forced = w == nullptr ? 0 : w->gemm_tile_rows;
+    p.forced = forced == 32 ? 32 | w->gemm_few_rows_waves << 8 : forced == 128 ? 128 | w->gemm_paired << 8 : forced;
     p.column_waves = w != nullptr ? w->gemm_column_waves : 1;
     // Without shared experts most tokens of a share have no row: workgroups of the first GEMM that get no tile
     // zero those rows of y meanwhile, and the weighted reduce skips what they got through.  (Served-only: rows of y whose
@@ -2863,21 +2866,45 @@ size_t dpep_megamoe_workspace_bytes(int num_tokens, int num_topk, int hidden, in
     return mega_layout(num_tokens, num_topk, hidden, intermediate, num_local, num_shared).total;
 }
 
-int dpep_megamoe_gemm_choice(void* ws, int num_tokens, int hidden, int intermediate, int num_topk, int num_experts, int num_local,
-                             int num_shared, int second, int32_t* tile_rows, int32_t* waves)
+// What a forward of these sizes takes for its first or second GEMM: the choice, and whether the kernels of every height split the columns.
+static int choice_of(const char* what, void* ws, const dpep::MegaSizes& m, bool second, dpep::GemmChoice* choice, bool* by_columns)
 {
     using namespace dpep;
     const Workspace* w = as_workspace(ws);
-    DPEP_REQUIRE(ws == nullptr || w != nullptr, "megamoe_gemm_choice: not a live workspace");
+    DPEP_REQUIRE(ws == nullptr || w != nullptr, "%s: not a live workspace", what);
+    DPEP_REQUIRE(m.num_tokens >= 1 && m.hidden >= 1 && m.intermediate >= 1 && m.num_topk >= 1 && m.num_experts >= m.num_local && m.num_local >= 1 && m.num_shared >= 0,
+                 "%s: bad sizes", what);
+    GemmParams g1 = gemm_of(m, w, false), g2 = gemm_of(m, w, true);
+    const GemmChoices choices = choose_gemms(m, g1, g2);
+    *choice = second ? choices.second : choices.first;
+    *by_columns = column_waves(second ? g2 : g1);
+    return DPEP_OK;
+}
+
+int dpep_megamoe_gemm_choice(void* ws, int num_tokens, int hidden, int intermediate, int num_topk, int num_experts, int num_local,
+                             int num_shared, int second, int32_t* tile_rows, int32_t* waves)
+{
     DPEP_REQUIRE(tile_rows != nullptr && waves != nullptr, "megamoe_gemm_choice: NULL output");
-    DPEP_REQUIRE(num_tokens >= 1 && hidden >= 1 && intermediate >= 1 && num_topk >= 1 && num_experts >= num_local && num_local >= 1 && num_shared >= 0,
-                 "megamoe_gemm_choice: bad sizes");
-    const MegaSizes sizes = {num_tokens, hidden, intermediate, num_topk, num_experts, num_local, num_shared};
-    GemmParams g1 = gemm_of(sizes, w, false);
-    const GemmChoices choices = choose_gemms(sizes, g1, gemm_of(sizes, w, true));
-    const GemmChoice& choice = second != 0 ? choices.second : choices.first;
+    dpep::GemmChoice choice;
+    bool by_columns;
+    if (int rc = choice_of("megamoe_gemm_choice", ws, {num_tokens, hidden, intermediate, num_topk, num_experts, num_local, num_shared}, second != 0, &choice, &by_columns))
+        return rc;
     *tile_rows = choice.rows;
     *waves = choice.waves;
+    return DPEP_OK;
+}
+
+int dpep_megamoe_gemm_kernel(void* ws, int num_tokens, int hidden, int intermediate, int num_topk, int num_experts, int num_local,
+                             int num_shared, int second, int32_t* kernel)
+{
+    DPEP_REQUIRE(kernel != nullptr, "megamoe_gemm_kernel: NULL output");
+    dpep::GemmChoice choice;
+    bool by_columns;
+    if (int rc = choice_of("megamoe_gemm_kernel", ws, {num_tokens, hidden, intermediate, num_topk, num_experts, num_local, num_shared}, second != 0, &choice, &by_columns))
+        return rc;
+    if (choice.rows == 32) *kernel = choice.direct ? DPEP_GEMM_ONE_WAVE : DPEP_GEMM_FEW_ROWS;
+    else if (choice.paired) *kernel = choice.streamed ? DPEP_GEMM_PAIRED_STREAMED : DPEP_GEMM_PAIRED;
+    else *kernel = by_columns ? DPEP_GEMM_COLUMN_WAVES : DPEP_GEMM_TWO_BY_TWO;
     return DPEP_OK;
 }
 

@@ -91,6 +91,7 @@ int dpep_workspace_create(size_t bytes, void** ws)
     w->payload_looks = dpep::kPayloadLooks;
     w->gemm_tile_rows = 0;
     w->gemm_few_rows_waves = 4;
+    w->gemm_paired = 0;
     w->gemm_column_waves = 1;
     w->gemm_zero_fill = 1;
     w->megamoe_served_only = 0;
@@ -202,6 +203,9 @@ int dpep_workspace_tune(void* ws, const char* key, long long value)
     } else if (strcmp(key, "gemm_few_rows_waves") == 0) {
         DPEP_REQUIRE(value == 1 || value == 4, "workspace_tune: gemm_few_rows_waves is 1 or 4");
         w->gemm_few_rows_waves = static_cast<int>(value);
+    } else if (strcmp(key, "gemm_paired") == 0) {
+        DPEP_REQUIRE(value == 0 || value == 1, "workspace_tune: gemm_paired is 0 or 1");
+        w->gemm_paired = static_cast<int>(value);
     } else {
         return dpep::fail(DPEP_EINVAL, "workspace_tune: unknown key '%s'", key);
     }

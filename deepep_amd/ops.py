@@ -467,6 +467,22 @@ def megamoe_gemm_choice(num_tokens: int, hidden: int, intermediate: int, num_top
     return tuple(chosen)
 
 
+GEMM_KERNELS = ("two_by_two", "column_waves", "paired", "paired_streamed", "few_rows", "one_wave")
+
+
+def megamoe_gemm_kernels(num_tokens: int, hidden: int, intermediate: int, num_topk: int, num_experts: int, num_local: int,
+                         num_shared: int = 0, ws: Optional[Workspace] = None):
+    """The kernels (names of ``GEMM_KERNELS``) that a forward of these sizes takes for its first and its second GEMM.  Host arithmetic only."""
+    kernels = []
+    for second in (0, 1):
+        kernel = ctypes.c_int32()
+        status = _lib.load().dpep_megamoe_gemm_kernel(None if ws is None else ws.handle, num_tokens, hidden, intermediate, num_topk, num_experts,
+                                                      num_local, num_shared, second, ctypes.byref(kernel))
+        _lib.check(status, "megamoe_gemm_kernel")
+        kernels.append(GEMM_KERNELS[kernel.value])
+    return tuple(kernels)
+
+
 def megamoe_fill_report(ws, num_tokens, num_topk, hidden, intermediate, num_local, num_shared: int = 0):
     """(filler waves, tokens they looked at) of the most recent forward on ``ws``; waits for the current stream."""
     fillers, filled = ctypes.c_int32(0), ctypes.c_int64(0)

@@ -56,6 +56,8 @@ int dpep_workspace_capacity(void* ws, size_t* bytes);
  *                                   from the expected rows per expert; 64, 128 or 192: that height for both, 32: the
  *                                   kernel for few rows per expert for both
  *   "gemm_few_rows_waves"           its waves per workgroup when forced: 4 (default) or 1
+ *   "gemm_paired"                   with 128 forced: 0 (default) the kernel that the other heights take too, 1 the one with
+ *                                   two workgroups to a CU
  *   "gemm_column_waves"             1 (default): the GEMM whose waves split a tile's columns, where it takes the sizes;
  *                                   0: always the 2 x 2 form */
 int dpep_workspace_tune(void* ws, const char* key, long long value);
@@ -269,6 +271,15 @@ int dpep_megamoe_schedule_check_column_waves(int tile_rows, int tiles_per_workgr
  * and its waves per workgroup.  Host arithmetic only; no counterpart in the reference. */
 int dpep_megamoe_gemm_choice(void* ws, int num_tokens, int hidden, int intermediate, int num_topk, int num_experts, int num_local,
                              int num_shared, int second, int32_t* tile_rows, int32_t* waves);
+#define DPEP_GEMM_TWO_BY_TWO 0       /* 64, 128 or 192 rows: 2 x 2 waves, weights through LDS */
+#define DPEP_GEMM_COLUMN_WAVES 1     /* the same heights: the waves split the columns, weights straight to registers */
+#define DPEP_GEMM_PAIRED 2           /* 128 rows, two workgroups to a CU */
+#define DPEP_GEMM_PAIRED_STREAMED 3  /* the same, weights past the caches */
+#define DPEP_GEMM_FEW_ROWS 4         /* 32 rows, activations through LDS; four waves to a workgroup, or one */
+#define DPEP_GEMM_ONE_WAVE 5         /* 32 rows, one wave to a workgroup, no LDS */
+/* The same question, answered with the kernel's name. */
+int dpep_megamoe_gemm_kernel(void* ws, int num_tokens, int hidden, int intermediate, int num_topk, int num_experts, int num_local,
+                             int num_shared, int second, int32_t* kernel);
 
 /* Bytes of workspace dpep_megamoe_forward needs (buffer_size(), experiments/megamoe/csrc/forward.cpp:480).
  * num_shared = number of shared experts (0..8) whose rows (every token, each) are held next to the routed ones. */

@@ -21,7 +21,23 @@ def test_kernels_of_known_sizes(sizes, first, second):
     assert ops.megamoe_gemm_choice(*sizes) == (first, second)
 
 
-def test_choice_refuses_bad_sizes():
+@pytest.mark.parametrize("sizes,first,second", [
+    ((512, 7168, 2048, 8, 256, 32, 0), "few_rows", "few_rows"),
+    ((16384, 7168, 2048, 8, 384, 6, 0), "column_waves", "paired"),
+    ((777, 2880, 1408, 4, 32, 32, 1), "paired", "paired"),
+    ((8192, 7168, 2048, 8, 32, 32, 0), "column_waves", "column_waves"),
+    ((24, 7168, 2048, 2, 2, 2, 0), "one_wave", "one_wave"),
+    ((24, 1024, 512, 16, 16, 16, 0), "one_wave", "few_rows"),    # k = 512 is short for the one without LDS
+    ((5000, 7168, 2048, 1, 55, 55, 0), "paired_streamed", "paired_streamed"),  # 91 rows for each of 55, 850 and 425 MB of weights
+    ((5000, 7168, 2048, 1, 16, 16, 0), "paired", "paired"),
+    ((4096, 1280, 1280, 2, 4, 4, 0), "paired", "two_by_two"),
+])
+def test_kernels_by_name(sizes, first, second):
+    assert ops.megamoe_gemm_kernels(*sizes) == (first, second)
+
+
+@pytest.mark.parametrize("choice", [ops.megamoe_gemm_choice, ops.megamoe_gemm_kernels])
+def test_choice_refuses_bad_sizes(choice):
     for bad in ((0, 1024, 512, 2, 8, 8), (8, 1024, 512, 2, 4, 8), (8, 1024, 512, 0, 8, 8), (8, 1024, 512, 2, 8, 8, -1)):
         with pytest.raises(ValueError, match="bad sizes"):
-            ops.megamoe_gemm_choice(*bad)
+            choice(*bad)

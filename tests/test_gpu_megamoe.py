@@ -102,6 +102,11 @@ def _run(ops, x_codes, x_scales, l1, l2, idx, weights, experts, begin, local, ti
         sizes = (tokens, hidden, inter, idx.shape[1], experts, local)
         taken = (tile_rows, few_rows_waves if tile_rows == 32 else 4)
         assert ops.megamoe_gemm_choice(*sizes, ws=ws) == (taken, taken)
+        for kernel, size in zip(ops.megamoe_gemm_kernels(*sizes, ws=ws), (hidden, inter)):
+            if tile_rows == 32:
+                assert kernel == "few_rows" or (kernel == "one_wave" and few_rows_waves == 1)
+            else:
+                assert kernel == ("column_waves" if column_waves and ops.megamoe_padded_dim(size) % 512 == 0 else "two_by_two")
     y = torch.full((tokens, hidden), float("nan"), dtype=torch.bfloat16, device=dev)
     counts = torch.empty((local,), dtype=torch.int32, device=dev)
     ops.megamoe_forward(

@@ -14,7 +14,7 @@ pytestmark = pytest.mark.gpu
 EDGES = (1, 31, 32, 33, 0, 64, 65, 96, 97, 127, 128, 129, 160, 256, 257)
 
 
-def _forward(ops, x, l1, l2, shared, idx, weights, hidden, inter, local, tile_rows, few_rows_waves=4, experts=None, fill=0):
+def _forward(ops, x, l1, l2, shared, idx, weights, hidden, inter, local, tile_rows, few_rows_waves=4, experts=None, fill=0, paired=0):
     dev = "cuda"
     num_shared = 0 if shared is None else shared[0][0].shape[0]
 
@@ -27,7 +27,10 @@ def _forward(ops, x, l1, l2, shared, idx, weights, hidden, inter, local, tile_ro
     ws = ops.Workspace(ops.megamoe_workspace_bytes(len(idx), idx.shape[1], hidden, inter, local, num_shared))
     ws.tune("gemm_tile_rows", tile_rows)
     ws.tune("gemm_few_rows_waves", few_rows_waves)
-    ws.tune("gemm_zero_fill", fill)  # (a launch whose idle workgroups zero rows keeps the column-wave kernel)
+    ws.tune("gemm_paired", paired)
+    ws.tune("gemm_zero_fill", fill)
+    if paired:
+        assert ops.megamoe_gemm_kernels(len(idx), hidden, inter, idx.shape[1], experts or local, local, num_shared, ws=ws) == ("paired",) * 2
     y = torch.full((len(idx), hidden), float("nan"), dtype=torch.bfloat16, device=dev)
     counts = torch.empty((local,), dtype=torch.int32, device=dev)
     ops.megamoe_forward(ws, torch.from_numpy(x[0]).to(dev).view(torch.float8_e4m3fn), torch.from_numpy(x[1]).to(dev), torch.from_numpy(idx).to(dev),
@@ -60,7 +63,7 @@ def test_paired_kernel_at_its_edges(hidden, inter, rows, num_shared):
 
     l1, l2 = quantised(local, 2 * inter, hidden), quantised(local, hidden, inter)
     shared = (quantised(num_shared, 2 * inter, hidden), quantised(num_shared, hidden, inter)) if num_shared else None
-    got, counts = _forward(ops, x, l1, l2, shared, idx, weights, hidden, inter, local, 128)
+    got, counts = _forward(ops, x, l1, l2, shared, idx, weights, hidden, inter, local, 128, paired=1)
     want, _ = _forward(ops, x, l1, l2, shared, idx, weights, hidden, inter, local, 32)
     np.testing.assert_array_equal(counts, np.bincount(idx.ravel(), minlength=local))
     assert torch.equal(got.view(torch.int16), want.view(torch.int16))

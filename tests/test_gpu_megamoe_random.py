@@ -254,8 +254,8 @@ def _agreement_case(ops, seed, tokens, hidden, inter, experts, begin, local, top
     route_weights = torch.rand((tokens, topk), device=dev, generator=g, dtype=torch.float32)
     sentinel = 3.0
     first = None
-    for column_waves, tile_rows, few_rows_waves in [(1, 0, 4), (1, 64, 4), (1, 128, 4), (1, 192, 4), (0, 64, 4), (0, 128, 4), (0, 192, 4),
-                                                    (1, 32, 1), (1, 32, 4), (1, 0, 4)]:
+    for column_waves, tile_rows, few_rows_waves, paired in [(1, 0, 4, 0), (1, 64, 4, 0), (1, 128, 4, 0), (1, 128, 4, 1), (1, 192, 4, 0), (0, 64, 4, 0),
+                                                            (0, 128, 4, 0), (0, 192, 4, 0), (1, 32, 1, 0), (1, 32, 4, 0), (1, 0, 4, 0)]:
         ws = ops.Workspace(ops.megamoe_workspace_bytes(tokens, topk, hidden, inter, local, shared))
         y = torch.full((tokens, hidden), sentinel, dtype=torch.bfloat16, device=dev)
         counts = torch.empty((local,), dtype=torch.int32, device=dev)
@@ -263,6 +263,7 @@ def _agreement_case(ops, seed, tokens, hidden, inter, experts, begin, local, top
             ws.tune("gemm_tile_rows", tile_rows)
             ws.tune("gemm_column_waves", column_waves)
             ws.tune("gemm_few_rows_waves", few_rows_waves)
+            ws.tune("gemm_paired", paired)
             ws.tune("gemm_zero_fill", zero_fill)
             ws.tune("megamoe_served_only", served_only)
             ops.megamoe_forward(ws, x.view(torch.float8_e4m3fn), x_scales, idx, route_weights, w1, s1, w2, s2, experts, begin, local, y,
@@ -283,7 +284,7 @@ def _agreement_case(ops, seed, tokens, hidden, inter, experts, begin, local, top
                 assert bool((~written | served).all()), case
         else:
             differing = (bits != first[0]).any(dim=1).nonzero().flatten()
-            assert differing.numel() == 0, (column_waves, tile_rows, int(differing.numel()), differing[:8].tolist(), case)
+            assert differing.numel() == 0, (column_waves, tile_rows, paired, int(differing.numel()), differing[:8].tolist(), case)
             assert torch.equal(counts, first[1]), (column_waves, tile_rows, case)
 
 
