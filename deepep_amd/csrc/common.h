@@ -57,7 +57,7 @@ struct Workspace {
     int megamoe_served_only;   // 1: rows of y whose token no local expert serves are left untouched; 0 (default): zeroed
     int gemm_tile_rows;  // 0: the grouped GEMM chooses its tile height; 64 / 128 / 192, or 32 (the few-rows kernel): forced (tests)
     int gemm_few_rows_waves;  // waves per workgroup of a forced few-rows kernel: 4 (default) or 1
-    int gemm_paired;          // forced 128 rows: 0 (default) one of the kernels of every height, 1 the paired kernel
+    int gemm_paired;          // forced 128 rows: 0 (default) one of the kernels of every height, 1 the paired kernel, 2 that with streamed weights
     int gemm_column_waves;  // which grouped GEMM kernel runs: 1 = waves split the columns, weights straight to registers; 0 = 2 x 2 waves, weights through LDS
 };
 // Device memory the kernels synchronise through, behind the caller's bytes, zero when the workspace is created:

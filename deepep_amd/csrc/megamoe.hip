@@ -245,7 +245,7 @@ struct GemmParams {
     int fill_tokens, fill_vec, fill_topk;
     int* fill_state;
     int* fill_stop;
-    int forced;                     // 64 / 128 / 192: that tile height whatever the cost model says (tests), 128 | 1 << 8: the paired kernel; 32: the
+    int forced;                     // 64 / 128 / 192: that tile height whatever the cost model says (tests), 128 | (1, 2) << 8: the paired kernel, its weights cached or streamed; 32: the
                                     //   few-rows kernel with (1, 4) << 8 waves per workgroup; 0: the model decides
     int column_waves;               // 1: the kernel whose waves split the tile's columns and load their weights straight into registers
     int n_real, k_real;             // what is not padding of n and k (first GEMM: n counts gate and up)
@@ -2436,7 +2436,7 @@ GemmChoice choose_gemm(const GemmParams& p, const ExpectedRows& expected, int cu
         if (few < best_cost) return {32, one < four ? 1 : kGemmWaves, tiles, false, false, one < four && direct, row_tiles_per_expert};
     }
     if ((p.forced & 0xff) == 32) return {32, p.forced >> 8, tiles, false, false, (p.forced >> 8) == 1 && direct, row_tiles_per_expert};
-    if (p.forced == (128 | 1 << 8)) return {128, kGemmWaves, paired_row_tiles * p.live_n_tiles, true, false, false, 0.0};
+    if ((p.forced & 0xff) == 128 && p.forced >> 8 != 0) return {128, kGemmWaves, paired_row_tiles * p.live_n_tiles, true, p.forced >> 8 == 2, false, 0.0};
     if (p.forced != 0) best = p.forced / 64;
     return {64 * best, kGemmWaves, tiles_of[best], false, false, false, 0.0};
 }

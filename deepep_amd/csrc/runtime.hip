@@ -204,7 +204,7 @@ int dpep_workspace_tune(void* ws, const char* key, long long value)
         DPEP_REQUIRE(value == 1 || value == 4, "workspace_tune: gemm_few_rows_waves is 1 or 4");
         w->gemm_few_rows_waves = static_cast<int>(value);
     } else if (strcmp(key, "gemm_paired") == 0) {
-        DPEP_REQUIRE(value == 0 || value == 1, "workspace_tune: gemm_paired is 0 or 1");
+        DPEP_REQUIRE(value >= 0 && value <= 2, "workspace_tune: gemm_paired is 0, 1 or 2");
         w->gemm_paired = static_cast<int>(value);
     } else {
         return dpep::fail(DPEP_EINVAL, "workspace_tune: unknown key '%s'", key);

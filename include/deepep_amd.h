@@ -57,7 +57,7 @@ int dpep_workspace_capacity(void* ws, size_t* bytes);
  *                                   kernel for few rows per expert for both
  *   "gemm_few_rows_waves"           its waves per workgroup when forced: 4 (default) or 1
  *   "gemm_paired"                   with 128 forced: 0 (default) the kernel that the other heights take too, 1 the one with
- *                                   two workgroups to a CU
+ *                                   two workgroups to a CU, 2 that one with its weights past the caches
  *   "gemm_column_waves"             1 (default): the GEMM whose waves split a tile's columns, where it takes the sizes;
  *                                   0: always the 2 x 2 form */
 int dpep_workspace_tune(void* ws, const char* key, long long value);

@@ -14,7 +14,7 @@ pytestmark = pytest.mark.gpu
 EDGES = (1, 31, 32, 33, 0, 64, 65, 96, 97, 127, 128, 129, 160, 256, 257)
 
 
-def _forward(ops, x, l1, l2, shared, idx, weights, hidden, inter, local, tile_rows, few_rows_waves=4, experts=None, fill=0, paired=0):
+def _forward(ops, x, l1, l2, shared, idx, weights, hidden, inter, local, tile_rows, few_rows_waves=4, experts=None, fill=0, paired=0, kernels=None):
     dev = "cuda"
     num_shared = 0 if shared is None else shared[0][0].shape[0]
 
@@ -30,7 +30,9 @@ def _forward(ops, x, l1, l2, shared, idx, weights, hidden, inter, local, tile_ro
     ws.tune("gemm_paired", paired)
     ws.tune("gemm_zero_fill", fill)
     if paired:
-        assert ops.megamoe_gemm_kernels(len(idx), hidden, inter, idx.shape[1], experts or local, local, num_shared, ws=ws) == ("paired",) * 2
+        kernels = (("paired", "paired_streamed")[paired - 1],) * 2
+    if kernels:
+        assert ops.megamoe_gemm_kernels(len(idx), hidden, inter, idx.shape[1], experts or local, local, num_shared, ws=ws) == kernels
     y = torch.full((len(idx), hidden), float("nan"), dtype=torch.bfloat16, device=dev)
     counts = torch.empty((local,), dtype=torch.int32, device=dev)
     ops.megamoe_forward(ws, torch.from_numpy(x[0]).to(dev).view(torch.float8_e4m3fn), torch.from_numpy(x[1]).to(dev), torch.from_numpy(idx).to(dev),
@@ -63,23 +65,24 @@ def test_paired_kernel_at_its_edges(hidden, inter, rows, num_shared):
 
     l1, l2 = quantised(local, 2 * inter, hidden), quantised(local, hidden, inter)
     shared = (quantised(num_shared, 2 * inter, hidden), quantised(num_shared, hidden, inter)) if num_shared else None
-    got, counts = _forward(ops, x, l1, l2, shared, idx, weights, hidden, inter, local, 128, paired=1)
     want, _ = _forward(ops, x, l1, l2, shared, idx, weights, hidden, inter, local, 32)
-    np.testing.assert_array_equal(counts, np.bincount(idx.ravel(), minlength=local))
-    assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+    for paired in (1, 2):  # weights cached, and past the caches
+        got, counts = _forward(ops, x, l1, l2, shared, idx, weights, hidden, inter, local, 128, paired=paired)
+        np.testing.assert_array_equal(counts, np.bincount(idx.ravel(), minlength=local))
+        assert torch.equal(got.view(torch.int16), want.view(torch.int16)), paired
     if len(idx) * hidden * inter < 2e9 and not num_shared:
         oracle = mm.round_bf16(mm.local_reference(mm.mx_dequantize(*x), idx, weights, mm.unpack_weight(*l1), mm.unpack_weight(*l2), 0))
         assert mm.relative_frobenius(got.float().cpu().numpy(), oracle) <= 2e-2
 
 
-@pytest.mark.parametrize("hidden,inter,rows", [
-    (64, 128, (3, 1)),           # one k tile in both GEMMs
-    (960, 640, (5, 0, 2)),       # eight k tiles, the last half padding; five
-    (1664, 1152, (33, 1, 32)),   # 13 and nine: four and three spans of four
-    (2368, 3200, (5, 0, 33)),    # 19 and 25: five and seven spans
-    (2624, 2176, (1,) * 66),     # more experts than a wave has lanes
+@pytest.mark.parametrize("hidden,inter,rows,one_wave", [  # one_wave: the kernels that one-wave workgroups run
+    (64, 128, (3, 1), ("few_rows", "few_rows")),           # one k tile in both GEMMs
+    (960, 640, (5, 0, 2), ("one_wave", "one_wave")),       # eight k tiles, the last half padding; five
+    (1664, 1152, (33, 1, 32), ("one_wave", "one_wave")),   # 13 and nine: four and three spans of four
+    (2368, 3200, (5, 0, 33), ("few_rows", "one_wave")),    # 19 and 25: five and seven spans
+    (2624, 2176, (1,) * 66, ("few_rows", "few_rows")),     # more experts than a wave has lanes
 ])
-def test_few_rows_kernels_at_their_edges(hidden, inter, rows):
+def test_few_rows_kernels_at_their_edges(hidden, inter, rows, one_wave):
     """k tiles of every number behind the last whole span, and a span loop of none, one and several rounds: one-wave workgroups (without
     LDS where the launch is small) and four-wave ones against the 64-row kernel, bit for bit."""
     from deepep_amd import ops
@@ -96,7 +99,8 @@ def test_few_rows_kernels_at_their_edges(hidden, inter, rows):
     l1, l2 = random_weights(2 * inter, hidden), random_weights(hidden, inter)
     want, _ = _forward(ops, x, l1, l2, None, idx, weights, hidden, inter, local, 64)
     for waves in (1, 4):
-        got, counts = _forward(ops, x, l1, l2, None, idx, weights, hidden, inter, local, 32, waves)
+        got, counts = _forward(ops, x, l1, l2, None, idx, weights, hidden, inter, local, 32, waves,
+                               kernels=one_wave if waves == 1 else ("few_rows",) * 2)
         np.testing.assert_array_equal(counts, rows)
         assert torch.equal(got.view(torch.int16), want.view(torch.int16)), waves
 

@@ -254,7 +254,7 @@ def _agreement_case(ops, seed, tokens, hidden, inter, experts, begin, local, top
     route_weights = torch.rand((tokens, topk), device=dev, generator=g, dtype=torch.float32)
     sentinel = 3.0
     first = None
-    for column_waves, tile_rows, few_rows_waves, paired in [(1, 0, 4, 0), (1, 64, 4, 0), (1, 128, 4, 0), (1, 128, 4, 1), (1, 192, 4, 0), (0, 64, 4, 0),
+    for column_waves, tile_rows, few_rows_waves, paired in [(1, 0, 4, 0), (1, 64, 4, 0), (1, 128, 4, 0), (1, 128, 4, 1), (1, 128, 4, 2), (1, 192, 4, 0), (0, 64, 4, 0),
                                                             (0, 128, 4, 0), (0, 192, 4, 0), (1, 32, 1, 0), (1, 32, 4, 0), (1, 0, 4, 0)]:
         ws = ops.Workspace(ops.megamoe_workspace_bytes(tokens, topk, hidden, inter, local, shared))
         y = torch.full((tokens, hidden), sentinel, dtype=torch.bfloat16, device=dev)
