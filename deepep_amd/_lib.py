@@ -45,6 +45,7 @@ SIGNATURES = {
     "dpep_mx_quant": (_I, (_P, _I, _I, _P, _P, _P)),
     "dpep_megamoe_schedule_check": (_I, (_I, _I, _I, _I, _I)),
     "dpep_megamoe_schedule_check_column_waves": (_I, (_I, _I, _I, _I, _I)),
+    "dpep_megamoe_schedule_check_paired": (_I, (_I, _I, _I, _I, _I)),
     "dpep_megamoe_gemm_choice": (_I, (_P, _I, _I, _I, _I, _I, _I, _I, _I, ctypes.POINTER(ctypes.c_int32), ctypes.POINTER(ctypes.c_int32))),
     "dpep_megamoe_gemm_kernel": (_I, (_P, _I, _I, _I, _I, _I, _I, _I, _I, ctypes.POINTER(ctypes.c_int32))),
     "dpep_megamoe_workspace_bytes": (_Z, (_I, _I, _I, _I, _I, _I)),

@@ -36,6 +36,20 @@ struct ColumnRing {
     static constexpr int kPrologueWait = (kStages - 1) * kRequests;  // behind the prologue's four items: item 0 has arrived
 };
 
+// The paired kernel (two workgroups to a CU): activations, a span's scales and a tile's gather indices are asked for four items ahead, weights two.
+// Every item asks, in this order, for the first k step's weights of the item two ahead (behind its own first step), its LDS stage's next
+// activations (a span's first item for the next span's scales in front of them, a tile's first also for the indices of the tile after that), and
+// the second k step's weights.  An item's first weights have arrived when at most kWaitFirst later requests are in flight, its second ones
+// (and with them everything asked for by the items before the one two back) when at most kWaitSecond are.
+struct PairedRing {
+    static constexpr int kStages = 4;                   // LDS stages = items the activation copies run ahead = unroll of the item loop
+    static constexpr int kRing = 2;                     // items the weights run ahead
+    static constexpr int kActivations = 4, kWeights = 2;  // requests per thread and item; per thread, item and k step
+    static constexpr int kRequests = kActivations + 2 * kWeights;
+    static constexpr int kWaitFirst = (kRing - 1) * kRequests + kActivations + kWeights;
+    static constexpr int kWaitSecond = (kRing - 1) * kRequests + kWeights;
+};
+
 // When the copy cursor may trust the next tile's gather indices.  They are fetched (asynchronously, into LDS)
 // together with the first item of the current tile, and read when the cursor moves on to that next tile, right after
 // it has issued the current tile's last item.  Waits only happen in the main loop, one per consumed item, and the

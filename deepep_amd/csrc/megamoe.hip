@@ -1840,9 +1840,7 @@ __global__ __launch_bounds__(kGemmThreads, ColCfg<RT>::kWorkgroupsPerCu) void gr
 // for an item's second weights also covers everything that the items before the one two back asked for, which includes
 // the next item's activations and scales, and, at a tile's last item, the gather indices asked for at its first; the barrier
 // behind it makes them everybody's.  Requests of skipped work are issued all the same (for the last real k tile again), so the counts hold.
-struct PairCfg {
-    static constexpr int kStages = 4;                  // LDS stages = items the activation copies run ahead = unroll of the item loop
-    static constexpr int kRing = 2;                    // items the weights run ahead
+struct PairCfg : PairedRing {
     static constexpr int kBM = 128;
     static constexpr int kRowTiles = 4, kColTiles = 2;  // 32 x 32 MFMA tiles per wave
     static constexpr int kStageBytes = kBM * kBK;
@@ -1852,9 +1850,7 @@ struct PairCfg {
     static constexpr int kOffColScales = kOffRowScales + 2 * kRowScaleSlot;
     static constexpr int kLdsBytes = kOffColScales + 2 * kColScaleSlot;
     static constexpr int kWeightRegs = 96;  // first of the ordinary registers that hold weight fragments (v96..v127)
-    static constexpr int kRequests = kRowTiles + 2 * kColTiles;  // per thread and item
-    static constexpr int kWaitFirst = (kRing - 1) * kRequests + kRowTiles + kColTiles;
-    static constexpr int kWaitSecond = (kRing - 1) * kRequests + kColTiles;
+    static_assert(kActivations == kRowTiles && kWeights == kColTiles, "the waits count what the kernel asks for");
 };
 #define DPEP_PAIR_ACC_REGS \
     "a0", "a1", "a2", "a3", "a4", "a5", "a6", "a7", "a8", "a9", "a10", "a11", "a12", "a13", "a14", "a15", \
@@ -2540,7 +2536,7 @@ GemmChoices choose_gemms(const MegaSizes& m, GemmParams& g1, const GemmParams& g
 // forced, and checks that every item's copies have completed when its fragments are read and that the gather
 // indices of a tile have when the cursor reads them.
 struct ScheduleFault {
-    int item, what;  // what: 1 = an item's copies, 2 = gather indices
+    int item, what;  // what: 1 = an item's operands, 2 = gather indices, 3 = scale slots, 4 = weights of another item
 };
 
 // The rings of scale slots: a span's scales (the scales of item x are read during the body of item x - 1) must all have
@@ -2719,6 +2715,102 @@ bool replay_column_waves(int my_tiles, int ktiles, int epilogue_stores, int slac
     return ok;
 }
 
+// The same for the paired kernel, whose weights have a cursor of their own: the prologue asks for items 0..3 (weights: 0 and 1) and waits for all of it;
+// an item's body waits for its first weights, asks for the first weights of the item two ahead, waits for its second weights and
+// the next item's activations and scales, and asks for the activations of the item four ahead (their span's scales in front) and the rest
+// of the weights.  `first_slack`, `second_slack`: a kernel whose waits are laxer by that much.
+bool replay_paired(int my_tiles, int ktiles, int epilogue_stores, int first_slack, int second_slack, ScheduleFault* fault)
+{
+    using Ring = PairedRing;
+    const long long n_items = static_cast<long long>(my_tiles) * ktiles;
+    constexpr int kMost = 1 << 16;
+    if (n_items == 0) return true;
+    static thread_local long long activations_op[kMost], scales_op[kMost], weights_op[2][kMost];
+    if (n_items >= kMost) return true;  // not replayed (far beyond any real workgroup's share)
+    long long issued = 0, done = 0, body = -1;
+    bool ok = true;
+    auto broken = [&](long long item, int what) {
+        if (ok) *fault = {static_cast<int>(item), what};
+        ok = false;
+    };
+    auto wait = [&](long long in_flight) { done = issued - in_flight > done ? issued - in_flight : done; };
+    int copy_kt = 0, copy_tile = 0, weight_kt = 0, weight_tile = 0;  // k tile and tile under the two cursors
+    long long copy_item = 0, weight_item = 0, index_op = -1;
+    bool past_end = false;
+    ScaleSlots scales(2);
+    auto request_activations = [&](int pos) {
+        if (pos == 0) {
+            issued += 2;
+            if (!scales.take(past_end ? -1 : copy_item + 3, body)) broken(body, 3);
+            for (int i = 0; i < 4 && !past_end; ++i) scales_op[copy_item + i] = issued - 1;
+            if (copy_kt == 0) index_op = issued++;
+        }
+        issued += Ring::kActivations;
+        if (!past_end) activations_op[copy_item] = issued - 1;
+    };
+    auto request_weights = [&](int step) {
+        issued += Ring::kWeights;
+        if (weight_item < n_items) {
+            weights_op[step][weight_item] = issued - 1;
+            if (weight_item != static_cast<long long>(weight_tile) * ktiles + weight_kt) broken(weight_item, 4);
+        }
+    };
+    auto advance_activations = [&](bool in_prologue, bool last_of_four) {
+        ++copy_kt;
+        ++copy_item;
+        if (!last_of_four || copy_kt != ktiles) return;
+        if (copy_tile + 1 < my_tiles) {
+            if (switch_needs_drain(in_prologue, ktiles, Ring::kStages)) wait(0);
+            if (index_op >= done) broken(body, 2);
+            copy_kt = 0;
+            ++copy_tile;
+        } else {
+            copy_kt = ktiles - 4;
+            past_end = true;
+        }
+    };
+    auto advance_weights = [&](bool last_of_four) {
+        ++weight_kt;
+        ++weight_item;
+        if (last_of_four && weight_kt == ktiles) {
+            weight_kt = 0;
+            weight_tile = copy_tile;
+        }
+    };
+    ++issued;  // the first tile's own indices
+    wait(0);
+    for (int pos = 0; pos < Ring::kStages; ++pos) {
+        request_activations(pos);
+        advance_activations(true, pos == 3);
+    }
+    for (int item = 0; item < Ring::kRing; ++item) {
+        request_weights(0);
+        request_weights(1);
+        advance_weights(false);
+    }
+    wait(0);
+    int kt = 0;
+    for (long long item = 0; item < n_items; ++item) {
+        const int pos = static_cast<int>(item & 3);
+        body = item;
+        wait(Ring::kWaitFirst + first_slack);
+        if (weights_op[0][item] >= done || activations_op[item] >= done) broken(item, 1);
+        request_weights(0);
+        wait(Ring::kWaitSecond + second_slack);
+        if (weights_op[1][item] >= done) broken(item, 1);
+        if (item + 1 < n_items && (activations_op[item + 1] >= done || scales_op[item + 1] >= done)) broken(item + 1, 1);
+        request_activations(pos);
+        request_weights(1);
+        advance_activations(false, pos == 3);
+        advance_weights(((pos + Ring::kRing) & 3) == 3);
+        if (++kt == ktiles) {
+            issued += epilogue_stores;
+            kt = 0;
+        }
+    }
+    return ok;
+}
+
 int launch_gemm1(const GemmParams& p, const GemmChoice& choice, const ExpectedRows& expected, hipStream_t stream)
 {
     if (int rc = check_gemm("gemm1", p.n, p.k, p.num_local)) return rc;
@@ -2794,6 +2886,19 @@ int dpep_megamoe_schedule_check_column_waves(int tile_rows, int tiles_per_workgr
         return fail(DPEP_EINVAL, "schedule_check: %s read before any wait covers them (item %d)",
                     fault.what == 1 ? "an item's operands are" : "the next tile's gather indices are", fault.item);
     return DPEP_OK;
+}
+
+int dpep_megamoe_schedule_check_paired(int tiles_per_workgroup, int ktiles, int epilogue_stores, int first_slack, int second_slack)
+{
+    using namespace dpep;
+    DPEP_REQUIRE(tiles_per_workgroup >= 0 && ktiles >= 4 && ktiles % 4 == 0 && epilogue_stores >= 0 && first_slack >= 0 && second_slack >= 0,
+                 "schedule_check: bad arguments (the paired kernel takes k tiles in fours)");
+    ScheduleFault fault = {0, 0};
+    if (replay_paired(tiles_per_workgroup, ktiles, epilogue_stores, first_slack, second_slack, &fault)) return DPEP_OK;
+    if (fault.what == 3)
+        return fail(DPEP_EINVAL, "schedule_check: a span's scales are overwritten while they are still being read (behind item %d)", fault.item);
+    if (fault.what == 4) return fail(DPEP_EINVAL, "schedule_check: the weights asked for item %d are another item's", fault.item);
+    return fail(DPEP_EINVAL, "schedule_check: %s read before any wait covers them (item %d)", fault.what == 1 ? "operands" : "gather indices", fault.item);
 }
 
 int dpep_megamoe_padded_dim(int dim) { return dim < 1 ? 0 : dpep::padded_dim(dim); }

@@ -265,6 +265,10 @@ int dpep_megamoe_schedule_check(int tile_rows, int tiles_per_workgroup, int ktil
  * weights straight into registers; k tiles come in fours).  slack = operations the replayed wait allows in flight beyond
  * the kernel's own count: with slack > 0 the check has to fail, which is how the tests know that it can. */
 int dpep_megamoe_schedule_check_column_waves(int tile_rows, int tiles_per_workgroup, int ktiles, int epilogue_stores, int slack);
+/* The same check for the kernel with two workgroups to a CU (128 rows; k tiles in fours, those of padding included), whose
+ * weights have a cursor of their own: also that it asks for the right item's.  first_slack, second_slack: as slack, for the
+ * waits in front of an item's first and second k step. */
+int dpep_megamoe_schedule_check_paired(int tiles_per_workgroup, int ktiles, int epilogue_stores, int first_slack, int second_slack);
 
 /* Which grouped GEMM kernel a forward of these sizes takes on this workspace (NULL: one with default settings), for the
  * first or (second != 0) the second GEMM: its row-tile height (64, 128, 192, or 32 for the kernel for few rows per expert)

@@ -82,3 +82,22 @@ def test_replay_catches_scale_slots_reused_too_early(tile_rows, ahead):
         assert (status != 0) == must_fail, (tile_rows, ktiles, tiles, lib.dpep_last_error().decode())
         if must_fail:
             assert b"overwritten" in lib.dpep_last_error()
+
+
+def test_paired_schedule_holds_everywhere():
+    """The kernel with two workgroups to a CU: an item's weights before each of its k steps, the next item's activations and scales, a
+    tile's gather indices, and the weight cursor two items behind the activation cursor, at every k length (in fours) and number of tiles."""
+    lib = _lib.load()
+    for ktiles, tiles, epilogue in itertools.product((4, 8, 12, 16, 56, 64), (0, 1, 2, 3, 5, 24, 100), (0, 8, 96)):
+        status = lib.dpep_megamoe_schedule_check_paired(tiles, ktiles, epilogue, 0, 0)
+        assert status == 0, (ktiles, tiles, epilogue, lib.dpep_last_error().decode())
+    assert lib.dpep_megamoe_schedule_check_paired(3, 6, 0, 0, 0) == -1
+
+
+@pytest.mark.parametrize("first,second", [(1, 0), (0, 1), (2, 0), (0, 2), (8, 8)])
+def test_paired_replay_catches_a_wait_that_is_too_lax(first, second):
+    """One request more in flight than the kernel allows, in front of either k step, and operands are read that no wait covers."""
+    lib = _lib.load()
+    for ktiles, tiles in itertools.product((4, 8, 16, 56), (1, 2, 24)):
+        assert lib.dpep_megamoe_schedule_check_paired(tiles, ktiles, 12, first, second) == -1, (ktiles, tiles)
+        assert b"operands" in lib.dpep_last_error()
