@@ -651,7 +651,7 @@ int dpep_dispatch_fresh(void* ws, const dpep_fresh_dispatch* call, void* stream)
             // columns to FP8, two parts of 144 units 56.8 us, one 54.3.)
             if (token_major && kMaxThreads / sp.threads * sp.per_part < 176) sp = choose_split(lines, units, p.quantize || units % 8 == 0 ? 8 : 1, 2048);
             riding = {p.x, p.scales, p.weights, p.out, p.out_scales, p.out_weights, payload_shape(p, sp), c.quantize != 0, payload_staged(p, sp), !token_major, static_cast<unsigned>(lines) * sp.parts, bound, c.capacity_rows,
-                      all_or_none ? c.capacity_rows : 0};
+                      all_or_none ? c.capacity_rows : 0, w->payload_looks};
         }
         bool launched = false;
         if (int rc = layout_of_fresh(ws, c, may_ride ? &riding : nullptr, &launched, s)) return rc;  // (checks the routing arguments)

@@ -621,11 +621,11 @@ constexpr int kRidingExperts = 256, kRidingSteps = 4;
 struct Routing {
     const int64_t* idx;
     int n_routes, num_experts, expert_begin, num_local;
-    // Calls visit(local expert or -1, route) for the routes that this one of `waves` waves goes through, in order.
+    // Calls visit(local expert or -1, route) for all routes in order, 64 at a time.  Called by whole waves.
     template <typename Visit>
-    __device__ __forceinline__ void scan(int wave, int waves, Visit&& visit) const
+    __device__ __forceinline__ void scan(Visit&& visit) const
     {
-        for (int base = wave * kPrefetch * kWave; base < n_routes; base += waves * kPrefetch * kWave) {
+        for (int base = 0; base < n_routes; base += kPrefetch * kWave) {
             int experts[kPrefetch];
             fetch_experts(experts, idx, base, n_routes, n_routes, num_experts, expert_begin, num_local);
 #pragma unroll
@@ -651,71 +651,76 @@ __device__ __forceinline__ void nap()
     for (int i = 0; i < kNaps; ++i) __builtin_amdgcn_s_sleep(4);
 }
 
-// Where a token's rows come from: row_of(), by one thread for each route, between two barriers of the workgroup; where any of its threads gave
-// up, all of them go through work_out().
+// Where a token's rows come from.
 struct AwaitedTokens {
-    static constexpr bool kAwaits = true;
+    static constexpr int kGaveUp = -2;
     Routing routing;
     const unsigned long long* words;
     const unsigned long long* total;
     uint32_t launch;
     int looks;
     int capacity, all_or_none;
-    int* late;                       // LDS of the workgroup
-    int (*rows_of)[kRidingExperts];  // LDS of this token's threads: rows of every expert, and those of them from tokens before
+    int (*rows_of)[kRidingExperts];  // LDS of this wave: rows of every expert, and those of them from tokens before
     __device__ __forceinline__ int begin() const { return 0; }
-    __device__ __forceinline__ void before_the_wait() const
+    __device__ __forceinline__ int await(const unsigned long long* word) const
     {
-        if (threadIdx.x == 0) *late = 0;
-    }
-    __device__ __forceinline__ bool gave_up() const { return *late != 0; }
-    __device__ __forceinline__ bool await(const unsigned long long* word, int& value) const
-    {
-        for (int i = 0; i < looks; ++i, nap<8>())
-            if (look(word, launch, value)) return true;
-        *late = 1;
-        return false;
+        for (int i = 0; i < looks; ++i, nap<8>()) {
+            int value;
+            if (look(word, launch, value)) return value;
+        }
+        return kGaveUp;
     }
     __device__ __forceinline__ int kept(int row, int all) const
     {
         return row < capacity && (all_or_none == 0 || DPEP_ROWS_KEPT(all, capacity)) ? row : -1;
     }
-    __device__ __forceinline__ int row_of(size_t route, int) const
+    // The token's rows into lds.rows; whether there is any.  Called by all threads of the workgroup.
+    __device__ __forceinline__ bool find_rows(const PayloadShape& p, int, int token, int t, TokenLds& lds) const
     {
-        int row, all = 0;
-        if (!await(words + route, row) || row < 0 || row >= capacity) return -1;
-        if (all_or_none != 0 && !await(total, all)) return -1;
-        return kept(row, all);
-    }
-    // The same rows without the words: row = rows of the experts before + earlier routes to the same expert.
-    __device__ __forceinline__ void work_out(const PayloadShape& p, int token, int t, TokenLds& lds) const
-    {
-        const int first = token * p.num_topk;
-        if (t == 0) lds.any_valid = 0;
-        for (int e = t; e < routing.num_local; e += p.threads) rows_of[0][e] = rows_of[1][e] = 0;
-        __syncthreads();
-        routing.scan(t >> 6, p.threads >> 6, [&](int e, int route) {
-            if (e < 0) return;
-            atomicAdd(&rows_of[0][e], 1);
-            if (route < first) atomicAdd(&rows_of[1][e], 1);
-        });
-        __syncthreads();
         if (t < p.num_topk) {
+            int row = await(words + static_cast<size_t>(token) * p.num_topk + t);
+            if (row >= 0 && all_or_none != 0) {
+                const int all = await(total);
+                row = all == kGaveUp ? kGaveUp : kept(row, all);
+            }
+            lds.rows[t] = row < capacity ? row : -1;
+        }
+        __syncthreads();
+        const int lane = threadIdx.x & 63;
+        int row = lane < p.num_topk ? lds.rows[lane] : -1;
+        if (__ballot(row == kGaveUp) != 0) row = work_out(p, token, lds.rows);
+        return __ballot(row >= 0) != 0;
+    }
+    // The same rows without the words: row = rows of the experts before + earlier routes to the same expert.  Each of the token's waves works
+    // all of them out for itself (they write the same values, and one that finds nothing missing any more finds these).
+    __device__ __forceinline__ int work_out(const PayloadShape& p, int token, int* rows) const
+    {
+        const int lane = threadIdx.x & 63, first = token * p.num_topk;
+        for (int e = lane; e < routing.num_local; e += kWave) rows_of[0][e] = rows_of[1][e] = 0;
+        wave_sync();
+        routing.scan([&](int e, int route) {
+            count_step(e, rows_of[0]);
+            count_step(route < first ? e : -1, rows_of[1]);
+        });
+        wave_sync();
+        int row = -1;
+        if (lane < p.num_topk) {
             auto expert_of = [&](int s) {
                 return local_expert(routing.idx[first + s], first + s, routing.n_routes, routing.num_experts, routing.expert_begin, routing.num_local);
             };
-            const int mine = expert_of(t);
-            int all = 0, row = mine < 0 ? -1 : rows_of[1][mine];
+            const int mine = expert_of(lane);
+            int all = 0;
+            row = mine < 0 ? -1 : rows_of[1][mine];
             for (int e = 0; e < routing.num_local; ++e) {
                 if (e < mine) row += rows_of[0][e];
                 all += rows_of[0][e];
             }
-            for (int s = 0; s < t && mine >= 0; ++s) row += expert_of(s) == mine ? 1 : 0;
+            for (int s = 0; s < lane && mine >= 0; ++s) row += expert_of(s) == mine ? 1 : 0;
             row = row < 0 ? -1 : kept(row, all);
-            lds.rows[t] = row;
-            if (row >= 0) lds.any_valid = 1;
+            rows[lane] = row;
         }
-        __syncthreads();
+        wave_sync();
+        return row;
     }
 };
 
@@ -744,13 +749,13 @@ struct AwaitedRows {
     {
         for (int e = threadIdx.x & 63; e < routing.num_local; e += kWave) rows_of[e] = 0;
         wave_sync();
-        routing.scan(0, 1, [&](int e, int) { count_step(e, rows_of); });
+        routing.scan([&](int e, int) { count_step(e, rows_of); });
         wave_sync();
         int expert = 0, rank = row, route = -1;
         while (expert < routing.num_local && rank >= rows_of[expert]) rank -= rows_of[expert++];
         wave_sync();  // (the next row's counts go to the same place)
         if (expert == routing.num_local) return -1;
-        routing.scan(0, 1, [&](int e, int at) {
+        routing.scan([&](int e, int at) {
             const unsigned long long same = __ballot(e == expert);
             const unsigned long long it = __ballot(e == expert && __popcll(same & lanes_below()) == rank);
             if (it != 0) route = at - (static_cast<int>(threadIdx.x) & 63) + __ffsll(it) - 1;  // (once: the rank falls below zero)
@@ -768,15 +773,14 @@ __global__ __launch_bounds__(kThreads, 4) void layout_payload_kernel(
     SendCounts send, uint32_t* __restrict__ mailbox, uint32_t sequence, unsigned long long* __restrict__ epoch,
     unsigned long long* __restrict__ tagged, int num_blocks, int rows, long long limit_ticks, uint32_t* __restrict__ timeouts,
     uint32_t launch_id,
-    unsigned long long* __restrict__ total_word, unsigned long long* __restrict__ row_words, int looks, LayoutPayload payload)
+    unsigned long long* __restrict__ total_word, unsigned long long* __restrict__ row_words, LayoutPayload payload)
 {
     using Lds = LayoutLds<kRidingExperts, true>;
     struct Riding {
         TokenLds tokens[kWaves];
         float scales[kQuant && !kRowMajor ? kMaxScaleCols : 1];
         u32x4 stage[kStaged ? kStagedVec : 1];
-        int late;
-        int rows_of[kStaged ? 1 : kWaves][2][kRidingExperts];
+        int rows_of[kWaves][2][kRidingExperts];
     };
     __shared__ union Both {
         Lds layout;
@@ -794,11 +798,11 @@ __global__ __launch_bounds__(kThreads, 4) void layout_payload_kernel(
     if (sub >= per || block >= payload.blocks) return;  // (whole waves)
     const Routing routing = {idx, n_routes, num_experts, expert_begin, num_local};
     if (kRowMajor) {
-        const AwaitedRows rows = {routing, row_words, total_word, launch_id, looks, payload.rows, lds.riding.rows_of[threadIdx.x >> 6][0]};
+        const AwaitedRows rows = {routing, row_words, total_word, launch_id, payload.looks, payload.rows, lds.riding.rows_of[threadIdx.x >> 6][0]};
         if (kQuant) quant_rows<DPEP_STORE_STREAMING>(payload.x, payload.weights, payload.out, payload.out_scales, payload.out_weights, p, rows, block, payload.blocks / p.parts, t);
         else copy_rows<DPEP_STORE_STREAMING>(payload.x, payload.scales, payload.weights, payload.out, payload.out_scales, payload.out_weights, p, rows, block, payload.blocks / p.parts, t);
     } else {
-        const AwaitedTokens tokens = {routing, row_words, total_word, launch_id, looks, payload.capacity, payload.all_or_none, &lds.riding.late, lds.riding.rows_of[sub]};
+        const AwaitedTokens tokens = {routing, row_words, total_word, launch_id, payload.looks, payload.capacity, payload.all_or_none, lds.riding.rows_of[threadIdx.x >> 6]};
         if (kQuant) quant_token<DPEP_STORE_STREAMING>(payload.x, payload.weights, payload.out, payload.out_scales, payload.out_weights, p, tokens, block, t, lds.riding.tokens[sub], lds.riding.scales + sub * (p.threads / 8));
         else copy_token<DPEP_STORE_STREAMING, kStaged>(payload.x, payload.scales, payload.weights, payload.out, payload.out_scales, payload.out_weights, p, tokens, block, t,
                                                        lds.riding.tokens[sub], lds.riding.stage);
@@ -1067,7 +1071,7 @@ int launch_layout(void* ws, const IdxT* idx, int num_tokens, int num_topk, int n
                                        reinterpret_cast<unsigned long long*>(sync + kSyncTagged), blocks, blocks + w->exchange_extra_rows,
                                        w->exchange_ticks, w->mailbox_device + kMailboxTimeout, w->layout_launches,
                                        reinterpret_cast<unsigned long long*>(sync + kSyncTotal), reinterpret_cast<unsigned long long*>(sync + kSyncRows),
-                                       w->payload_looks, *payload);
+                                       *payload);
                 };
                 if (payload->row_major) payload->quantize ? ride(layout_payload_kernel<true, true, false>) : ride(layout_payload_kernel<false, true, false>);
                 else if (payload->quantize) ride(layout_payload_kernel<true, false, false>);

@@ -29,18 +29,32 @@ struct PayloadShape {
 };
 
 // ---- where a payload's workgroups find its rows -------------------------------------------------------------------------
+// LDS of a token's threads: its rows (-1: none), and whether there is any.
+struct TokenLds {
+    int rows[DPEP_MAX_TOPK];
+    int any_valid;
+};
+
 // Token-major, in the map that an earlier launch has left.  Rows at or beyond `capacity` are dropped; with all_rows (the layout's
 // count) nothing is moved unless DPEP_ROWS_KEPT.
 struct MappedTokens {
-    static constexpr bool kAwaits = false;
     const int* route_to_row;
     int capacity;
     const int* all_rows;
     __device__ __forceinline__ int begin() const { return all_rows != nullptr ? *all_rows : capacity; }  // (travels with the values and the routes)
-    __device__ __forceinline__ int row_of(size_t route, int all) const
+    // The token's rows into lds.rows; whether there is any.  Called by all threads of the workgroup.
+    __device__ __forceinline__ bool find_rows(const PayloadShape& p, int all, int token, int t, TokenLds& lds) const
     {
-        const int row = route_to_row[route];
-        return row >= capacity || !DPEP_ROWS_KEPT(all, capacity) ? -1 : row;  // outputs allocated before R was known
+        if (t == 0) lds.any_valid = 0;
+        __syncthreads();
+        if (t < p.num_topk) {
+            int row = route_to_row[static_cast<size_t>(token) * p.num_topk + t];
+            if (row >= capacity || !DPEP_ROWS_KEPT(all, capacity)) row = -1;  // outputs allocated before R was known
+            lds.rows[t] = row;
+            if (row >= 0) lds.any_valid = 1;
+        }
+        __syncthreads();
+        return lds.any_valid != 0;
     }
 };
 
@@ -53,27 +67,6 @@ __device__ __forceinline__ unsigned long long row_word(uint32_t launch, int valu
 
 // ---- token-major: one token and column part to `p.threads` threads; read once, write K times ----------------------------------
 // t: the thread's number among them.  Called by all threads of a workgroup whose `block` is in range.
-struct TokenLds {
-    int rows[DPEP_MAX_TOPK];
-    int any_valid;
-};
-
-template <typename Tokens>
-__device__ __forceinline__ bool rows_of_token(const PayloadShape& p, const Tokens& tokens, int all, int token, int t, TokenLds& lds)
-{
-    if (t == 0) lds.any_valid = 0;
-    if constexpr (Tokens::kAwaits) tokens.before_the_wait();
-    __syncthreads();
-    if (t < p.num_topk) {
-        const int row = tokens.row_of(static_cast<size_t>(token) * p.num_topk + t, all);
-        lds.rows[t] = row;
-        if (row >= 0) lds.any_valid = 1;
-    }
-    __syncthreads();
-    if constexpr (Tokens::kAwaits)
-        if (tokens.gave_up()) tokens.work_out(p, token, t, lds);
-    return lds.any_valid != 0;
-}
 
 // How far (in 16-byte vectors) an address lies behind the start of its cache line.
 __device__ __forceinline__ int behind_line(const void* p) { return static_cast<int>(reinterpret_cast<uintptr_t>(p) >> 4 & 7); }
@@ -106,7 +99,7 @@ __device__ __forceinline__ void copy_token(const u32x4* __restrict__ x, const fl
             if (v_first + j * p.threads < v_end) stage[t + j * p.threads] = early[j];
         for (int v = v_first + kEarly * p.threads; v < v_end; v += p.threads) stage[v - v_begin] = load16(src + v);
     }
-    if (!rows_of_token(p, tokens, all, token, t, lds)) return;  // (with a barrier behind the staging)
+    if (!tokens.find_rows(p, all, token, t, lds)) return;  // (with a barrier behind the staging)
     for (int s = 0; s < p.num_topk; ++s) {
         const int row = lds.rows[s];
         if (row < 0) continue;
@@ -256,7 +249,7 @@ __device__ __forceinline__ void quant_token(const u32x4* __restrict__ x, const f
             hi[j] = load16(src + 2 * u + 1);
         }
     }
-    if (!rows_of_token(p, tokens, all, token, t, lds)) return;
+    if (!tokens.find_rows(p, all, token, t, lds)) return;
     const int scale_cols = p.units / 8;
     // per_part is a multiple of 8 and the threads of 64, so the 8 lanes of a block stay together.
     // Quantise first, then write row by row: at any moment the workgroup's stores run along ONE output row.
@@ -336,6 +329,7 @@ struct LayoutPayload {
     bool quantize, staged, row_major;
     unsigned blocks;
     int rows, capacity, all_or_none;  // rows: row-major, the bound of R; the others: token-major
+    int looks;                        // of a workgroup for a word of the layout's
 };
 
 }  // namespace dpep
