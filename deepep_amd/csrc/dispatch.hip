@@ -415,8 +415,10 @@ struct Payload {
 // The split of a payload launch over `lines` tokens or rows.  Parts end at multiples of 128 bytes.  Where the rows themselves do not,
 // every part boundary is two partial lines to HBM in each of a token's rows, and a token-major launch with four and more rows per token has
 // parts only while it would have fewer than 2048 workgroups (dispatch and combine, BF16: 6045 tokens x top-10 of 6064 columns 353 -> 335 us, 7421 x 7 of 2848 280 -> 264, 1874 x 7 of
-// 2400 38.7 -> 36.3; rows of whole lines are better off with the finer split: 4096 x 8 of 4096 106.7 against 108.6, of 7168 to FP8 136.9 against 138.1; two
-// rows per token are too few for it: 2264 of 4464 30.3 against 31.6).
+// 2400 38.7 -> 36.3; rows of whole lines are better off with the finer split: 4096 x 8 of 4096 106.7 against 108.6, of 7168 to FP8 136.9 against 138.1).
+// On both sides of the four rows, 2048 / 8192 workgroups: 3000 tokens of 5840 columns x top-2 43.0 / 42.3 us, 3 56.2 / 58.4, 4 68.1 / 71.9, 5 79.5 /
+// 85.9; 4096 of 2832 32.7 / 32.1, 40.4 / 40.4, 50.4 / 52.9, 56.5 / 60.2; 6000 of 1552 28.5 / 28.3, 35.6 / 37.5, 42.5 / 45.9, 49.5 / 49.3.  Two rows per token
+// are too few for it (2264 of 4464 too: 31.6 against 30.3), three are as good or better in these, four and more nearly always.
 Split payload_split(const Payload& p, int lines, long long rows_to_write)
 {
     const bool whole_lines = p.quantize || p.units % 8 == 0;
@@ -441,9 +443,13 @@ int launch_token_major(const Payload& p, const int32_t* route_to_row, int capaci
 {
     const Split sp = payload_split(p, p.num_tokens, rows);
     const dim3 grid(p.num_tokens * sp.parts), block(sp.threads);
-    // A launch that mostly writes is faster with sixteen waves to a CU than with as many as there is room for (fewer rows open at a time;
+    // A launch that mostly writes is faster with twelve waves to a CU than with as many as there is room for (fewer rows open at a time;
     // 6045 tokens x top-10 of 6064 BF16 columns 335 -> 328 us, 6249 x 7 of 1552 145.7 -> 141.3; 1.25 rows per
-    // token 39.6 -> 47.3; to FP8, whose reads are half of its rows' bytes, 146.6 -> 150.7): the LDS that it asks for keeps others out.
+    // token 39.6 -> 47.3; to FP8, whose reads are half of its rows' bytes, 146.6 -> 150.7): the LDS that it asks for keeps others out.  A quarter of
+    // the CU's 160 KiB for 256 threads, beside the kernel's own 132 bytes: three workgroups fit (of 192 threads five, of 128 seven, of 64 fifteen).
+    // On both sides of the five rows, so / without it, BF16, a cached dispatch and its combine: 4096 tokens of 4096 columns x top-2 34.9 / 33.2 us, 3
+    // 43.4 / 43.5, 4 57.8 / 58.3, 5 62.8 / 64.0; 2000 of 5120 24.5 / 22.0, 29.7 / 28.1, 34.3 / 34.6, 40.1 / 41.1; 3000 of 5840 36.3 / 36.6, 51.4 / 52.8,
+    // 59.9 / 62.1, 74.9 / 77.3.  Behind a layout four rows are too few: 65.8 / 64.6 and 42.4 / 40.2 for the first two, 66.4 / 68.1 for the third.
     const bool mostly_writes = !p.quantize && rows >= 5LL * p.num_tokens && rows * p.units * 16 >= (32LL << 20);
     const unsigned room = mostly_writes ? 40960 / kMaxThreads * sp.threads : 0;
     const MappedTokens tokens = {route_to_row, capacity, all_rows};
@@ -636,7 +642,11 @@ int dpep_dispatch_fresh(void* ws, const dpep_fresh_dispatch* call, void* stream)
         // In the layout's grid (launch_layout), where that is the better place.  A large token-major payload with several rows to a token ends
         // 1 to 15 us sooner there; beside a small one the GPU waits for the host, and the layout reports to it 0.5 to 3 us later with a
         // payload in its grid (dispatch and combine: 39 MB 33.0 -> 31.9 us, 43 MB 39.0 -> 34.6, 152 MB 91.8 -> 87.8, 18 MB 22.7 -> 23.5, 13 MB
-        // 25.2 -> 28.1; 1.25 rows per token, 41 MB 39.8 -> 46.8, 142 MB 197.5 and 196.7).  Row-major workgroups wait for their row before they
+        // 25.2 -> 28.1; 1.25 rows per token, 41 MB 39.8 -> 46.8, 142 MB 197.5 and 196.7.  On both sides of the five rows per token, one grid / two: BF16, 4096
+        // tokens of 4096 columns x top-2 39.9 / 38.7, 3 48.2 / 49.8, 4 62.2 / 64.8, 5 68.4 / 70.8; 1500 of 7168 27.4 / 27.4, 34.8 / 35.0, 40.2 / 42.0, 47.4 /
+        // 48.8; 6000 of 1552 29.6 / 28.4, 35.5 / 37.7, 42.0 / 42.6, 48.7 / 53.3; to FP8, 2500 of 5120 31.4 / 31.3, 35.9 / 37.1, 41.2 / 42.4, 47.0 / 48.3, 4096 of
+        // 7168 62.6 / 57.8, 74.4 / 71.1, 89.6 / 88.7, 102.1 / 100.5 and, 6, 116.5 / 116.7.  The line lies where the largest quantised payloads stop losing;
+        // 18 others of five to ten rows gain 1 to 4 %, 10 that are FP8 already 3 to 9 %.  BF16 gains 1 to 6 % with three and four rows too.)  Row-major workgroups wait for their row before they
         // can ask for its values, so it is only the launch that is saved, which counts where nothing is reported and the host is
         // the one to wait for: 0.4 to 2 MB 17 -> 14 us, 4 MB 28.3 and 28.4, 10 MB 60.5 -> 63.1, 117 MB 124 -> 156.
         LayoutPayload riding = {};

@@ -1824,7 +1824,7 @@ __global__ __launch_bounds__(kGemmThreads, ColCfg<RT>::kWorkgroupsPerCu) void gr
 // workgroup), by streaming the weights where an expert has about one row tile, and by a tile's start and end where a launch is
 // a single round.  Measured on an MI355X against the best of the other heights, whole forwards, us: 4584 tokens over 29 + 2 experts of
 // 1600 x 2944 243 -> 198, 8512 over 3 + 2 of 3264 x 3840 672 -> 565, 4560 x top-8 over 59 + 2 of 1088 x 384 77 -> 63, 777 x top-4 over
-// 32 + 1 of 2880 x 1408 97 -> 91; 8192 x top-8 over 32 of 7168 x 2048: 2336 with 192 rows, 2408 with this.
+// 32 + 1 of 2880 x 1408 101 -> 94; 8192 x top-8 over 32 of 7168 x 2048: 2336 with 192 rows, 2408 with this.
 //
 // Accumulators and weight fragments live in registers that only the assembly statements name (a0..a127, v96..v127): with two
 // workgroups to a CU the accumulators are all the accumulation registers there are, and the register allocator, which may not
@@ -2390,7 +2390,7 @@ GemmChoice choose_gemm(const GemmParams& p, const ExpectedRows& expected, int cu
         const double pair = 5.0 + items * (0.652 + 0.147 * live + 0.269 * share), single = 3.37 + items * (0.236 + 0.112 * live + 0.135 * share);
         const double t = 2.94 + full * pair + (rest > 1.01 ? pair : rest > 0.0 ? single : 0.0);
         const double live_bytes = experts_with_rows * p.live_n_tiles * ((steps + 1) / 2) * 16896.0;
-        // A long launch runs at the power limit, and where it has nothing to jump over, 192-row tiles win by moving a third fewer
+        // A long launch pulls its own clock down (1.8 to 1.9 GHz where a reduce has 2.3), and where it has nothing to jump over, 192-row tiles win by moving a third fewer
         // weights: of nine launches of 8 and more rounds with less than 6 % of padding in those tiles they were 1.6 % faster on average
         // (8192 x top-8 over 32 experts of 7168 x 2048: first GEMM 1343 us against 1375, second 803 against 840).
         const double tall_work = tiles_of[3] * 6.0 * ktiles * 2.0, live_work = live_row_tiles * p.live_n_tiles * steps;
