@@ -16,7 +16,8 @@
 //            lives in LDS.  There is no separate scan launch.
 // The smallest inputs take one workgroup, which holds everything (see "one workgroup" below).
 // Inputs whose chunks fit a wave's registers (at most kKeep steps of 64 routes) take ONE launch: the workgroups
-// (at most 129, far fewer than there are CUs, so all are resident together) count, publish their histograms as
+// (at most 129, 17 to an XCD with room for 64 of the largest; whatever else runs ends by itself, so all become resident together unless four
+// such launches are at work at once, and then the wait has its bound) count, publish their histograms as
 // self-validating words (count + the launch's tag in one 64-bit store), read each other's as soon as they appear, and
 // assign from the ids they still hold: no barrier, no counter that anybody has to reset.  The wait for the others'
 // words is bounded; a launch whose wait runs out assigns nothing (a histogram is missing): it reports no rows, marks
